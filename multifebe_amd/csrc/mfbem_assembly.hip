@@ -100,7 +100,13 @@ struct DevMesh {
   const int* cel;               // (ncp) element holding an MCA point, -1 for a nodal point
   const double* cxi;            // (ncp, 2) local coordinates of an MCA point in cel
   const unsigned char* nmca;    // (nn) 1 for a node collocated by MCA points
+  const unsigned char* ekind;   // (ne) kNeedH | kNeedG: kernels that element's conditions need
 };
+
+// What an element contributes: with h (t*) to columns of unknown u and, where u is prescribed and not
+// zero, to b; with g (u*) to columns of unknown t and, where t is prescribed and not zero, to b.  A
+// traction-free element needs h alone, one held at zero g alone.
+constexpr int kNeedH = 1, kNeedG = 2;
 
 // ------------------------------------------------------------------------------------------------
 // small helpers
@@ -160,11 +166,12 @@ __device__ inline void ext_kernel_row(const KernelParams& k, const double* x, co
 __device__ inline void ext_kernel_row(const KernelParams& k, const double* x, const double* n,
                                       const double* x_i, zd* row, int stride = 1) {
   double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
-  double r = sqrt(dot3(rv, rv)), d1r = 1.0 / r;
+  double r, d1r;
+  dist_and_inverse(dot3(rv, rv), r, d1r);
   double dr[3] = {rv[0] * d1r, rv[1] * d1r, rv[2] * d1r};
   double drdn = dot3(dr, n);
   zd psi, chi, TT1, TT2, TT3;
-  har_factors(k.h, r, true, psi, chi, TT1, TT2, TT3);
+  har_factors<true, true>(&k.h, r, d1r, true, psi, chi, TT1, TT2, TT3);
   for (int il = 0; il < 3; il++)
     for (int ik = 0; ik < 3; ik++) {
       double dk = il == ik ? 1.0 : 0.0;
@@ -192,12 +199,14 @@ __device__ inline void sing_kernel_row(const KernelParams& k, const double* x, c
 __device__ inline void sing_kernel_row(const KernelParams& k, const double* x, const double* n,
                                        const double* x_i, zd* row) {
   double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
-  double r = sqrt(dot3(rv, rv)), d1r = 1.0 / r, d1r2 = d1r * d1r;
+  double r, d1r;
+  dist_and_inverse(dot3(rv, rv), r, d1r);
+  const double d1r2 = d1r * d1r;
   double dr[3] = {rv[0] * d1r, rv[1] * d1r, rv[2] * d1r};
   double drdn = dot3(dr, n);
   zd psi, chi, TT1, TT2, TT3;
-  har_factors(k.h, r, false, psi, chi, TT1, TT2, TT3);
-  zd t1s = mkz(k.h.T1[0][0], k.h.T1[0][1]) * d1r2, t2s = mkz(k.h.T2[0][0], k.h.T2[0][1]) * d1r2;
+  har_factors<true, true>(&k.h, r, d1r, false, psi, chi, TT1, TT2, TT3);
+  zd t1s = mkz(k.h.lead[2][0], k.h.lead[2][1]) * d1r2, t2s = mkz(k.h.lead[3][0], k.h.lead[3][1]) * d1r2;
   for (int il = 0; il < 3; il++)
     for (int ik = 0; ik < 3; ik++) {
       double dk = il == ik ? 1.0 : 0.0;
@@ -563,7 +572,7 @@ __global__ void __launch_bounds__(256) k_fill_lists(DevMesh m, const unsigned ch
 // Tiles of the scatter kernel (k_regular_tile): element e's run of precalculated rule c is cut
 // into tiles of at most kTileP consecutive list entries; toff[e*(kMaxPrecalsets+2)+c] is the
 // run's first tile.  A tile is (first list entry, count | rule << 8).
-constexpr int kTileP = 14;
+constexpr int kTileP = 16;
 __global__ void k_fill_tiles(DevMesh m, const int* counts, const long long* offsets,
                              const long long* toff, int2* tiles) {
   constexpr int S = kMaxPrecalsets + 2;
@@ -708,106 +717,232 @@ __global__ void __launch_bounds__(kWave) k_regular(DevMesh m, const KernelParams
   }
 }
 
+// kernel constants through the constant address space (scalar loads)
+typedef const __attribute__((address_space(4))) KernelParams* ConstKP;
+
+// Exterior kernel values at one point, handed to f(l, k, ft) for the nine components of t* and to
+// g(c, fu), c = 0..5 for (0,0) (0,1) (0,2) (1,1) (1,2) (2,2), of the symmetric u* (before the
+// constants; the values of ext_kernel_row).
+template <bool F, bool G, class EmitF, class EmitG>
+__device__ inline void ext_point(ConstKP k, const double* x, const double* n,
+                                 const double* x_i, double, EmitF&& f, EmitG&& g) {
+  const double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
+  const double s = rsqrt(dot3(rv, rv));
+  const double dr[3] = {rv[0] * s, rv[1] * s, rv[2] * s};
+  if (F) {
+    const double s2 = s * s, a = 3.0 * s2 * dot3(dr, n), c = s2 * k->ctet2;
+    const double d = c * dot3(dr, n);
+    const double cn[3] = {c * n[0], c * n[1], c * n[2]}, ad[3] = {a * dr[0], a * dr[1], a * dr[2]};
+#pragma unroll
+    for (int l = 0; l < 3; l++)
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        double v = ad[l] * dr[q];
+        if (l == q) v += d;
+        else v += cn[l] * dr[q] - cn[q] * dr[l];
+        f(3 * l + q, v);
+      }
+  }
+  if (G) {
+    const double a = s * k->cteu2, sd[3] = {s * dr[0], s * dr[1], s * dr[2]};
+    int c = 0;
+#pragma unroll
+    for (int l = 0; l < 3; l++)
+#pragma unroll
+      for (int q = l; q < 3; q++) g(c++, l == q ? a + sd[l] * dr[q] : sd[l] * dr[q]);
+  }
+}
+
+template <bool F, bool G, class EmitF, class EmitG>
+__device__ inline void ext_point(ConstKP k, const double* x, const double* n,
+                                 const double* x_i, zd, EmitF&& f, EmitG&& g) {
+  const double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
+  double r, s;
+  dist_and_inverse(dot3(rv, rv), r, s);
+  const double dr[3] = {rv[0] * s, rv[1] * s, rv[2] * s};
+  zd psi, chi, TT1, TT2, TT3;
+  har_factors<F, G>(&k->h, r, s, true, psi, chi, TT1, TT2, TT3);
+  if (F) {
+    const double drdn = dot3(dr, n);
+    const zd a = TT1 * drdn, d = TT2 * drdn;
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+      // row l: dr_k (a dr_l + TT2 n_l) + n_k (TT3 dr_l) + d delta
+      const zd u = a * dr[l] + TT2 * n[l], w = TT3 * dr[l];
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        zd v = u * dr[q] + w * n[q];
+        if (l == q) v += d;
+        f(3 * l + q, v);
+      }
+    }
+  }
+  if (G) {
+    int c = 0;
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+      const zd u = -(chi * dr[l]);
+#pragma unroll
+      for (int q = l; q < 3; q++) g(c++, l == q ? psi + u * dr[q] : u * dr[q]);
+    }
+  }
+}
+
+__device__ constexpr int kSym[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};
+
+// Sums over the points of one rule of one element for 16 collocation points, one wave, on the FP64
+// matrix cores (v_mfma_f64_4x4x4_4b).  A lane evaluates the kernel of pair lane % 16 at point
+// p0 + lane / 16: its values are, as they stand, the 16 x 4 left operand, and the weights
+// phi_n J w of the four points the 4 x 4 right operands (nodes 0..3, 4..7, 8), so no value goes
+// through LDS and no barrier is met.  Per value three of them (48 cycles of the FP64 pipe per SIMD,
+// which vector FP64 shares) stand for nine FMAs (36) and the LDS store and loads that those need.
+// Result layout: lane holds pair 4 ((lane / 4) % 4) + lane / 16, node 4 m + lane % 4.
+// pe: the rule's first point record of the element.
+template <bool H, int KIND>
+struct TileAcc {
+  static constexpr int RC = H ? 2 : 1;
+  static constexpr int NF = KIND & kNeedH ? 9 * RC : 1, NG = KIND & kNeedG ? 6 * RC : 1;
+  double f[NF][3], g[NG][3];
+  __device__ inline void clear() {
+#pragma unroll
+    for (int c = 0; c < NF; c++) f[c][0] = f[c][1] = f[c][2] = 0.0;
+#pragma unroll
+    for (int c = 0; c < NG; c++) g[c][0] = g[c][1] = g[c][2] = 0.0;
+  }
+};
+__device__ inline double mfma4(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+__device__ inline void mfma_row(double v, const double* w, double (*acc)[3], int c) {
+#pragma unroll
+  for (int m = 0; m < 3; m++) acc[c][m] = mfma4(v, w[m], acc[c][m]);
+}
+__device__ inline void mfma_row(zd v, const double* w, double (*acc)[3], int c) {
+#pragma unroll
+  for (int m = 0; m < 3; m++) {
+    acc[2 * c][m] = mfma4(v.re, w[m], acc[2 * c][m]);
+    acc[2 * c + 1][m] = mfma4(v.im, w[m], acc[2 * c + 1][m]);
+  }
+}
+
+template <bool H, int KIND>
+__device__ inline void tile_points(ConstKP kp, const double* __restrict__ pe, int P,
+                                   const double* xi, int lane, TileAcc<H, KIND>& acc) {
+  typedef typename Val<H>::T T;
+  const int k = lane >> 4, j = lane & 3;
+  for (int p0 = 0; p0 < P; p0 += 4) {
+    // past the last point: the first point's values with zero weights
+    const bool in = p0 + k < P;
+    const double* q = pe + (in ? p0 + k : 0) * kPsStride;
+    const double x[3] = {q[0], q[1], q[2]}, nv[3] = {q[3], q[4], q[5]};
+    const double w[3] = {in ? q[6 + j] : 0.0, in ? q[10 + j] : 0.0, in && j == 0 ? q[14] : 0.0};
+    ext_point<(KIND & kNeedH) != 0, (KIND & kNeedG) != 0>(
+        kp, x, nv, xi, T(), [&](int c, T v) { mfma_row(v, w, acc.f, c); },
+        [&](int c, T v) { mfma_row(v, w, acc.g, c); });
+  }
+}
+
+__device__ inline double tile_value(const double (*a)[3], int c, int m, double) { return a[c][m]; }
+__device__ inline zd tile_value(const double (*a)[3], int c, int m, zd) {
+  return mkz(a[2 * c][m], a[2 * c + 1][m]);
+}
+
+template <typename T>
+__device__ inline T lane_xor_add(T v, int mask);
+template <>
+__device__ inline double lane_xor_add(double v, int mask) { return v + __shfl_xor(v, mask); }
+template <>
+__device__ inline zd lane_xor_add(zd v, int mask) {
+  return mkz(v.re + __shfl_xor(v.re, mask), v.im + __shfl_xor(v.im, mask));
+}
+
+template <bool H, int KIND>
+__device__ inline void tile_body(const DevMesh& m, const KernelParams& kp,
+                                 const int* __restrict__ list, int2 tile, int e,
+                                 typename Val<H>::T* A, long long lda, typename Val<H>::T* b) {
+  typedef typename Val<H>::T T;
+  const int cnt = tile.y & 0xff, rule = tile.y >> 8, lane = threadIdx.x;
+  const int P = m.ps_gln[rule] * m.ps_gln[rule], first = e * m.ncp;
+  const double* pe = m.ps + ((long long)e * m.npts + m.ps_off[rule]) * kPsStride;
+  // a slot past the tile's pairs repeats the first one; its rows of the result are not stored
+  const int slot = lane & 15, cpi = list[tile.x + (slot < cnt ? slot : 0)] - first;
+  const double xi[3] = {m.xc[3 * cpi], m.xc[3 * cpi + 1], m.xc[3 * cpi + 2]};
+  TileAcc<H, KIND> acc;
+  acc.clear();
+  tile_points<H, KIND>((ConstKP)&kp, pe, P, xi, lane, acc);
+  const int po = 4 * ((lane >> 2) & 3) + (lane >> 4), j = lane & 3;
+  const bool live = po < cnt;
+  const int cp = list[tile.x + (live ? po : 0)] - first;
+  const long long row = 3LL * m.crow[cp];
+  const bool shared = m.cshared[cp] != 0;
+  T bs[3] = {zero_of(T()), zero_of(T()), zero_of(T())};
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    const int n = 4 * q + j;
+    if (!live || n >= 9) continue;
+    const int sn = m.conn[9 * e + n];
+#pragma unroll
+    for (int ik = 0; ik < 3; ik++) {
+      const long long col = 3LL * sn + ik;
+      T v[3];
+      if (KIND == kNeedH) {
+#pragma unroll
+        for (int il = 0; il < 3; il++)
+          v[il] = scale_h(kp, tile_value(acc.f, 3 * il + ik, q, T()));
+      } else if (KIND == kNeedG) {
+#pragma unroll
+        for (int il = 0; il < 3; il++)
+          v[il] = -scale_g(kp, tile_value(acc.g, kSym[3 * il + ik], q, T()));
+      } else {
+        const int ct = m.ctype[col];
+        const double cv = m.cval[col];
+        const double cb = ct == 0 ? -cv : ct == 1 ? cv : cv == 0.0 ? 0.0 : cv * m.nfn[col];
+#pragma unroll
+        for (int il = 0; il < 3; il++) {
+          const T h = scale_h(kp, tile_value(acc.f, 3 * il + ik, q, T()));
+          const T g = scale_g(kp, tile_value(acc.g, kSym[3 * il + ik], q, T()));
+          v[il] = ct == 0 ? -g : h;
+          if (cv != 0.0) bs[il] = bs[il] + (ct == 0 ? h : g) * cb;
+        }
+      }
+      T* a = A + row + lda * col;
+      if (shared) {
+        for (int il = 0; il < 3; il++) atomic_add(a + il, v[il]);
+      } else {
+        const T a0 = a[0], a1 = a[1], a2 = a[2];
+        a[0] = a0 + v[0];
+        a[1] = a1 + v[1];
+        a[2] = a2 + v[2];
+      }
+    }
+  }
+  if (KIND == (kNeedH | kNeedG)) {
+#pragma unroll
+    for (int il = 0; il < 3; il++) {
+      bs[il] = lane_xor_add(lane_xor_add(bs[il], 1), 2);
+      if (live && j == 0) atomic_add(&b[row + il], bs[il]);
+    }
+  }
+}
+
 // Precalculated-rule pairs scattered into A and b (ext_pre: bem_staela3d.f90:592-650,
 // bem_harela3d.f90:628-700; scatter: src/assemble_bem_staela_equation.f90,
-// src/assemble_bem_harela_equation.f90), one tile per workgroup: up to kTileP pairs of one element
-// and one rule, consecutive entries of the class list (ascending collocation points, so mostly
-// consecutive matrix rows).  The rule's P points run in chunks of PC <= kTileG points
-// (ceil(P / kTileG) chunks of near-equal size):
-//   kernel:   thread (slot, g) evaluates the 18 kernel values of pair `slot` at point p0 + g into
-//             LDS, F[value][g][slot];
-//   contract: thread (kind, ik, slot, il) -- one matrix row 3 crow + il of its pair, kind 0 t* -> h,
-//             1 u* -> g, direction ik -- sums its kernel value times the weights phi_n J w of the
-//             9 element nodes over the points, in rule order (weights: uniform loads).
-// Each thread then adds its 9 entries to A (or b).  Consecutive threads hold consecutive rows of
-// one column.  The tiles of one launch belong to elements of one colour (no shared node): two of
+// src/assemble_bem_harela_equation.f90), one tile per wave: up to 16 pairs of one element and one
+// rule, consecutive entries of the class list (ascending collocation points, so mostly consecutive
+// matrix rows).  The tiles of one launch belong to elements of one colour (no shared node): two of
 // them touch the same entry only if their points share rows (MCA points of one node), which add
-// atomically.  Chunks of at most 13 points keep F within 53 KB (harmonic), so three workgroups
-// share a CU's LDS; registers are held to 168 per thread to match (three waves per SIMD: ~11 %
-// faster than two with 18-point chunks; a 25-point rule still runs in two chunks).
-constexpr int kTileG = 13, kTileThreads = 256, kTileRows = 18 * kTileP;
-static_assert(kTileRows <= kTileThreads && kTileP * kTileG <= kTileThreads, "tile shape");
+// atomically.
 template <bool H>
-__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
     k_regular_tile(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
                    const int2* __restrict__ tiles, typename Val<H>::T* A, long long lda,
                    typename Val<H>::T* b) {
-  typedef typename Val<H>::T T;
-  constexpr int kStride = kTileG * kTileP + 1;  // values of one kind/component (padded)
-  __shared__ T F[18 * kStride];
-  const KernelParams& kp = *kpp;
   const int2 tile = tiles[blockIdx.x];
-  const int cnt = tile.y & 0xff, rule = tile.y >> 8;
-  const int t = threadIdx.x;
-  const int e = list[tile.x] / m.ncp;
-  const int P = m.ps_gln[rule] * m.ps_gln[rule];
-  const int nch = (P + kTileG - 1) / kTileG, PC = (P + nch - 1) / nch;
-  const double* pe = m.ps + ((long long)e * m.npts + m.ps_off[rule]) * kPsStride;
-  // kernel evaluation item of this thread
-  const int aslot = t % kTileP, ag = t / kTileP;
-  const bool aact = aslot < cnt && ag < PC;
-  double xi[3] = {0.0, 0.0, 0.0};
-  if (aact) {
-    const int cp = list[tile.x + aslot] % m.ncp;
-    xi[0] = m.xc[3 * cp];
-    xi[1] = m.xc[3 * cp + 1];
-    xi[2] = m.xc[3 * cp + 2];
-  }
-  // contraction row of this thread: t = ((kind * 3 + ik) * kTileP + slot) * 3 + il
-  const int il = t % 3, slot = (t / 3) % kTileP, kk = min(t / (3 * kTileP), 5);
-  const int kind = kk / 3, ik = kk % 3;
-  const bool live = t < kTileRows && slot < cnt;  // threads past kTileRows contract row 5 idly
-  const T* fr = &F[(kind * 9 + 3 * il + ik) * kStride + slot];
-  T acc[9];
-#pragma unroll
-  for (int n = 0; n < 9; n++) acc[n] = zero_of(T());
-  for (int p0 = 0; p0 < P; p0 += PC) {
-    const int np = min(PC, P - p0);
-    __syncthreads();  // the previous chunk is consumed
-    if (aact && ag < np) {
-      const double* q = pe + (long long)(p0 + ag) * kPsStride;
-      const double x[3] = {q[0], q[1], q[2]}, nv[3] = {q[3], q[4], q[5]};
-      ext_kernel_row(kp, x, nv, xi, &F[ag * kTileP + aslot], kStride);
-    }
-    __syncthreads();
-    for (int g = 0; g < np; g++) {
-      const double* w = pe + (long long)(p0 + g) * kPsStride + 6;
-      const T f = fr[g * kTileP];
-#pragma unroll
-      for (int n = 0; n < 9; n++) acc[n] += f * w[n];
-    }
-  }
-  if (!live) return;
-  const int cp = list[tile.x + slot] % m.ncp;
-  const long long row = 3LL * m.crow[cp] + il;
-  const bool shared = m.cshared[cp] != 0;
-  T bs = zero_of(T());
-  bool has_b = false;
-#pragma unroll
-  for (int n = 0; n < 9; n++) {
-    const T v = kind ? scale_g(kp, acc[n]) : scale_h(kp, acc[n]);
-    const long long col = 3LL * m.conn[9 * e + n] + ik;
-    const int ct = m.ctype[col];
-    const double cv = m.cval[col];
-    if (kind == 0) {
-      if (ct != 0) {
-        if (shared) atomic_add(&A[row + lda * col], v);
-        else A[row + lda * col] += v;
-      } else if (cv != 0.0) {
-        bs = bs - v * cv;
-        has_b = true;
-      }
-    } else {
-      if (ct == 0) {
-        if (shared) atomic_add(&A[row + lda * col], -v);
-        else A[row + lda * col] += -v;
-      } else if (cv != 0.0) {
-        bs = bs + (ct == 1 ? v * cv : v * (cv * m.nfn[col]));
-        has_b = true;
-      }
-    }
-  }
-  if (has_b) atomic_add(&b[row], bs);
+  const int e = __builtin_amdgcn_readfirstlane(list[tile.x] / m.ncp);
+  const int kind = __builtin_amdgcn_readfirstlane(m.ekind[e]);
+  if (kind == kNeedH) tile_body<H, kNeedH>(m, *kpp, list, tile, e, A, lda, b);
+  else if (kind == kNeedG) tile_body<H, kNeedG>(m, *kpp, list, tile, e, A, lda, b);
+  else tile_body<H, kNeedH | kNeedG>(m, *kpp, list, tile, e, A, lda, b);
 }
 
 // Interior-displacement contribution of one pair held as the per-lane outputs o = lane + 64 t
@@ -1236,7 +1371,7 @@ __global__ void __launch_bounds__(kWave) k_singular(DevMesh m, const QsiParams* 
       if (o < 81) {
         const int c = o / 9, n = o % 9;
         const double f = pf_i[n] * hli[c / 3][c % 3];
-        if constexpr (H) fin[t] += mkz(kp.h.T2[0][0], kp.h.T2[0][1]) * f;
+        if constexpr (H) fin[t] += mkz(kp.h.lead[3][0], kp.h.lead[3][1]) * f;
         else fin[t] += kp.ctet2 * f;
       }
     }
@@ -1252,7 +1387,7 @@ __global__ void __launch_bounds__(kWave) k_singular(DevMesh m, const QsiParams* 
       T v = acc[t];
       if (kind == 0) {
         double f = pf_i[n] * hli[il][ik];
-        if constexpr (H) v += mkz(kp.h.T2[0][0], kp.h.T2[0][1]) * f;
+        if constexpr (H) v += mkz(kp.h.lead[3][0], kp.h.lead[3][1]) * f;
         else v += kp.ctet2 * f;
       }
       v = kind ? scale_g(kp, v) : scale_h(kp, v);
@@ -1575,7 +1710,7 @@ struct mfb_mesh_s {
   // collocation points (device) and host copies of their rows / elements / coordinates
   double *xc = nullptr, *cxi = nullptr;
   int *crow = nullptr, *cel = nullptr;
-  unsigned char *cshared = nullptr, *nmca = nullptr;
+  unsigned char *cshared = nullptr, *nmca = nullptr, *ekind = nullptr;
   std::vector<int> h_crow, h_cel;
   std::vector<double> h_xc;
   int n_mca = 0;
@@ -1615,7 +1750,7 @@ static void mesh_release(mfb_mesh_s* m) {
                 m->qcls, m->lcls, m->llists, m->judge_counters, m->judge_err,
                 m->xc, m->cxi, m->crow, m->cel, m->cshared, m->nmca,
                 m->ws[0], m->ws[1], m->ws[2], m->ws[3], m->ws[4], m->ws[5], m->ws[6], m->ws[7],
-                m->tiles.d, m->ltiles.d, m->d_promo};
+                m->tiles.d, m->ltiles.d, m->d_promo, m->ekind};
   for (void* p : ps)
     if (p) (void)hipFree(p);
 }
@@ -1913,6 +2048,7 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
   TRY(dalloc(&m->cel, ncp));
   TRY(dalloc(&m->cshared, ncp));
   TRY(dalloc(&m->nmca, nn));
+  TRY(dalloc(&m->ekind, ne));
   TRY(dalloc(&m->err, 1));
   TRY(dalloc(&m->counters, 2));
   TRY(dalloc(&m->d_qsp, 1));
@@ -1935,12 +2071,22 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
   TRYH(hipMemcpy(m->cshared, cs.cshared.data(), ncp, hipMemcpyHostToDevice));
   if (cs.nmca.empty()) TRYH(hipMemset(m->nmca, 0, nn));
   else TRYH(hipMemcpy(m->nmca, cs.nmca.data(), nn, hipMemcpyHostToDevice));
+  {
+    std::vector<unsigned char> ek(ne, 0);
+    for (int e = 0; e < ne; e++)
+      for (int k = 0; k < 27; k++) {
+        const long long c = 3LL * conn[9 * e + k / 3] + k % 3;
+        ek[e] |= ctype[c] == 0 ? kNeedG : kNeedH;
+        if (cval[c] != 0.0) ek[e] |= ctype[c] == 0 ? kNeedH : kNeedG;
+      }
+    TRYH(hipMemcpy(m->ekind, ek.data(), ne, hipMemcpyHostToDevice));
+  }
   TRYH(hipMemset(m->err, 0, sizeof(int)));
   TRYH(hipMemset(m->counters, 0, 2 * sizeof(long long)));
   d.x = m->x; d.conn = m->conn; d.ctype = m->ctype; d.cval = m->cval; d.elem = m->elem;
   d.ps = m->ps; d.nfn = m->nfn; d.inc_ptr = m->inc_ptr; d.inc_e = m->inc_e; d.inc_k = m->inc_k;
   d.xc = m->xc; d.cxi = m->cxi; d.crow = m->crow; d.cel = m->cel; d.cshared = m->cshared;
-  d.nmca = m->nmca;
+  d.nmca = m->nmca; d.ekind = m->ekind;
 
   hipLaunchKernelGGL(k_elem_setup, dim3((ne + 63) / 64), dim3(64), 0, 0, d, m->elem);
   TRYH(hipGetLastError());
@@ -2132,7 +2278,7 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
   for (int k = 0; k < m->n_colors; k++) {
     if (!ts.cnt[k]) continue;
     if (events) m->last_regular_launches++;
-    hipLaunchKernelGGL((k_regular_tile<H>), dim3((unsigned)ts.cnt[k]), dim3(kTileThreads), 0, s, d,
+    hipLaunchKernelGGL((k_regular_tile<H>), dim3((unsigned)ts.cnt[k]), dim3(kWave), 0, s, d,
                        kpp, lists, ts.d + ts.off[k], A, lda, b);
   }
   if (events) MFB_HIP(hipEventRecord(m->ev[2], s));

@@ -607,76 +607,163 @@ __device__ inline void subdiv_l3(const double* X, const double* xs, double* Xs) 
 #pragma clang fp contract(fast)
 
 // ---------------------------------------------------------------------------------------------
-// E_0..E_6 of exp(z) (numerical.f90:1258-1330); only E_2..E_5 are consumed by the kernels
+// harmonic scalar factors at distance r (bem_harela3d.f90:660-682)
 // ---------------------------------------------------------------------------------------------
-__device__ inline void zexp_dec(zd z, zd* E2, zd* E3, zd* E4, zd* E5) {
-  double az = sqrt(z.re * z.re + z.im * z.im);   // |z| <~ 1e3 here: no overflow to guard
-  if (az <= 1.0) {
-    // E6 = z^6/6! (1 + z/7 (1 + z/8 (... (1 + z/21)))) by Horner: the smallest terms first, as
-    // the reference sums its terms (downwards from k = n + 6, n = round(10^(1.176 + 0.175
-    // log10|z|)) <= 15 on |z| <= 1, numerical.f90:1276); the terms it leaves out are below the
-    // last bit of E6 (|z|^22/22! < 1e-21 |z|^6/6! here), so every lane takes the same 15 steps
-    // (no divergent loop, compile-time 1/k)
-    zd h = mkz(1.0);
-#pragma unroll
-    for (int k = 21; k >= 7; k--) h = mkz(1.0) + h * (z * (1.0 / k));
-    const zd z2 = z * z, z3 = z2 * z, z4 = z3 * z, z5 = z4 * z, z6 = z5 * z;
-    *E5 = z6 * (1.0 / 720.0) * h + z5 * (1.0 / 120.0);
-    *E4 = *E5 + z4 * (1.0 / 24.0);
-    *E3 = *E4 + z3 * (1.0 / 6.0);
-    *E2 = *E3 + z2 * 0.5;
-  } else {
-    double ex = exp(z.re), s, c;
-    sincos(z.im, &s, &c);
-    zd ez = mkz(ex * c, ex * s);
-    zd z2 = z * z, z3 = z2 * z, z4 = z3 * z;
-    zd e1 = ez - mkz(1.0);
-    *E2 = e1 - z;
-    *E3 = *E2 - 0.5 * z2;
-    *E4 = *E3 - (1.0 / 6.0) * z3;
-    *E5 = *E4 - (1.0 / 24.0) * z4;
-  }
+// exp(-k r): both exponentials of a quadrature point run through these few instructions instead of
+// the library's exp and sincos (whose large-argument path and private-memory results the kernel
+// does not need: |k r| is the number of wavelengths across the boundary).  Cody-Waite reduction
+// with one fused step each, Taylor polynomials on |x| <= pi/4 and |x| <= ln(2)/2 to below half an
+// ulp.
+__host__ __device__ inline zd exp_minus(zd k, double r) {
+  const double a = -(k.re * r), b = -(k.im * r);
+  const double na = rint(a * 1.44269504088896340736);
+  double x = __builtin_fma(na, -6.93147180559945286227e-01, a);
+  x = __builtin_fma(na, -2.31904681384629955842e-17, x);
+  double e = 1.0 / 6227020800.0;
+  e = __builtin_fma(e, x, 1.0 / 479001600.0);
+  e = __builtin_fma(e, x, 1.0 / 39916800.0);
+  e = __builtin_fma(e, x, 1.0 / 3628800.0);
+  e = __builtin_fma(e, x, 1.0 / 362880.0);
+  e = __builtin_fma(e, x, 1.0 / 40320.0);
+  e = __builtin_fma(e, x, 1.0 / 5040.0);
+  e = __builtin_fma(e, x, 1.0 / 720.0);
+  e = __builtin_fma(e, x, 1.0 / 120.0);
+  e = __builtin_fma(e, x, 1.0 / 24.0);
+  e = __builtin_fma(e, x, 1.0 / 6.0);
+  e = __builtin_fma(e, x, 0.5);
+  e = __builtin_fma(e, x, 1.0);
+  e = __builtin_fma(e, x, 1.0);
+  e = ldexp(e, (int)na);
+  const double nb = rint(b * 6.36619772367581382433e-01);
+  double y = __builtin_fma(nb, -1.57079632679489655800e+00, b);
+  y = __builtin_fma(nb, -6.12323399573676603587e-17, y);
+  const double y2 = y * y;
+  double s = -1.0 / 1307674368000.0;
+  s = __builtin_fma(s, y2, 1.0 / 6227020800.0);
+  s = __builtin_fma(s, y2, -1.0 / 39916800.0);
+  s = __builtin_fma(s, y2, 1.0 / 362880.0);
+  s = __builtin_fma(s, y2, -1.0 / 5040.0);
+  s = __builtin_fma(s, y2, 1.0 / 120.0);
+  s = __builtin_fma(s, y2, -1.0 / 6.0);
+  s = __builtin_fma(s * y2, y, y);
+  double c = 1.0 / 20922789888000.0;
+  c = __builtin_fma(c, y2, -1.0 / 87178291200.0);
+  c = __builtin_fma(c, y2, 1.0 / 479001600.0);
+  c = __builtin_fma(c, y2, -1.0 / 3628800.0);
+  c = __builtin_fma(c, y2, 1.0 / 40320.0);
+  c = __builtin_fma(c, y2, -1.0 / 720.0);
+  c = __builtin_fma(c, y2, 1.0 / 24.0);
+  c = __builtin_fma(c, y2, -0.5);
+  c = __builtin_fma(c, y2, 1.0);
+  const int m = (int)nb;
+  const double ss = (m & 1) ? c : s, cc = (m & 1) ? s : c;
+  return mkz(e * ((m + 1) & 2 ? -cc : cc), e * (m & 2 ? -ss : ss));
 }
 
-// harmonic scalar factors at distance r (bem_harela3d.f90:660-682); full=false drops the 1/r^2
-// leading terms of TT1..TT3 (regular parts used by the singular integration)
-__device__ inline void har_factors(const HarParams& k, double r, bool full, zd& psi, zd& chi,
-                                   zd& TT1, zd& TT2, zd& TT3) {
-  double d1 = 1.0 / r, d2 = d1 * d1, d3 = d2 * d1, d4 = d3 * d1;
-  auto C = [](const double* v) { return mkz(v[0], v[1]); };
-  zd t1, t2, t3;
-  // z = -i k r; the terms of the first wave number are summed before the second one's E_n are
-  // formed (fewer values live at once)
-  {
-    const zd z1 = mkz(-(-k.k1[1] * r), -(k.k1[0] * r));
-    zd a2, a3, a4, a5;
-    zexp_dec(z1, &a2, &a3, &a4, &a5);
-    a2 *= d1; a3 *= d2; a4 *= d3; a5 *= d4;
-    psi = C(k.psi[0]) * d1 + C(k.psi[1]) + C(k.psi[2]) * a3 + C(k.psi[4]) * a4;
-    chi = C(k.chi[0]) * d1 + C(k.chi[1]) * a2 + C(k.chi[2]) * a3 + C(k.chi[4]) * a4;
-    t1 = C(k.T1[1]) + C(k.T1[2]) * a2 + C(k.T1[4]) * a3 + C(k.T1[6]) * a4 + C(k.T1[8]) * a5;
-    t2 = C(k.T2[1]) + C(k.T2[3]) * a3 + C(k.T2[5]) * a4 + C(k.T2[7]) * a5;
-    t3 = C(k.T3[1]) + C(k.T3[2]) * a2 + C(k.T3[3]) * a3 + C(k.T3[5]) * a4 + C(k.T3[7]) * a5;
+// r = |v| and s = 1/r from r2 = |v|^2: one reciprocal square root, r corrected once
+__device__ inline void dist_and_inverse(double r2, double& r, double& s) {
+  s = rsqrt(r2);
+  r = r2 * s;
+  r = __builtin_fma(__builtin_fma(-r, r, r2), 0.5 * s, r);
+}
+
+// G(z) = (e^z - 1 - z - z^2/2) / z^3 = sum_j z^j / (j + 3)! on |z| <= 1 (17 terms: the next is below
+// 1e-18): real coefficients at a complex argument by the recurrence b_j = c_j + 2 Re(z) b_{j+1} -
+// |z|^2 b_{j+2} (Knuth, The Art of Computer Programming 2, 4.6.4), two FMAs per term.
+__host__ __device__ inline zd exp_tail3(zd z) {
+  constexpr double c[17] = {
+      1.0 / 6.0,
+      1.0 / 24.0,
+      1.0 / 120.0,
+      1.0 / 720.0,
+      1.0 / 5040.0,
+      1.0 / 40320.0,
+      1.0 / 362880.0,
+      1.0 / 3628800.0,
+      1.0 / 39916800.0,
+      1.0 / 479001600.0,
+      1.0 / 6227020800.0,
+      1.0 / 87178291200.0,
+      1.0 / 1307674368000.0,
+      1.0 / 20922789888000.0,
+      1.0 / 355687428096000.0,
+      1.0 / 6402373705728000.0,
+      1.0 / 121645100408832000.0,
+  };
+  const double p = z.re + z.re, n = z.re * z.re + z.im * z.im;
+  double b1 = c[16], b2 = 0.0;
+#pragma unroll
+  for (int j = 15; j >= 1; j--) {
+    const double t = __builtin_fma(p, b1, c[j]) - n * b2;
+    b2 = b1;
+    b1 = t;
   }
-  {
-    const zd z2 = mkz(-(-k.k2[1] * r), -(k.k2[0] * r));
-    zd b2, b3, b4, b5;
-    zexp_dec(z2, &b2, &b3, &b4, &b5);
-    b2 *= d1; b3 *= d2; b4 *= d3; b5 *= d4;
-    psi = psi + b2 + C(k.psi[3]) * b3 + C(k.psi[5]) * b4;
-    chi = chi + b2 + C(k.chi[3]) * b3 + C(k.chi[5]) * b4;
-    t1 = t1 + C(k.T1[3]) * b2 + C(k.T1[5]) * b3 + C(k.T1[7]) * b4 + C(k.T1[9]) * b5;
-    t2 = t2 + C(k.T2[2]) * b2 + C(k.T2[4]) * b3 + C(k.T2[6]) * b4 + C(k.T2[8]) * b5;
-    t3 = t3 + C(k.T3[4]) * b3 + C(k.T3[6]) * b4 + C(k.T3[8]) * b5;
+  return mkz(c[0] + z.re * b1 - n * b2, z.im * b1);
+}
+
+// psi, chi (G) and TT1..TT3 (F) at distance r, s = 1/r; full = false drops the leading lead s^2 of
+// TT1..TT3 (regular parts used by the singular integration).  With z_j = -kappa_j r, w_j = s e^{z_j}:
+//   D = w2 (1/z2^2 - 1/z2) - w1 (1/z2^2 - z1/z2^2) = s (q H(z1) - H(z2)),  H(z) = (1 - (1-z) e^z)/z^2
+// and each factor is a short combination of w1, w2 and D.  From max |z_j| = 1 on the first form of
+// D is taken (its terms cancel by 1/z^2 at most); below, t = e^z - 1 and h = H - 1/2 are summed
+// without cancellation and the leading terms added in closed form.  No table and seven complex
+// constants, which stay in scalar registers: power series of the factors themselves take fewer
+// FMAs but read up to 170 constants per point, whose scalar-load latency cost more than it saved.
+template <bool F, bool G, class HP>
+__host__ __device__ inline void har_factors(HP k, double r, double s, bool full, zd& psi, zd& chi,
+                                            zd& TT1, zd& TT2, zd& TT3) {
+  const zd k1 = mkz(k->kap1[0], k->kap1[1]), k2 = mkz(k->kap2[0], k->kap2[1]);
+  const zd q = mkz(k->q[0], k->q[1]), qk1 = mkz(k->qk1[0], k->qk1[1]);
+  if (r < k->rser) {
+    const zd z1 = k1 * -r, z2 = k2 * -r;
+    const zd g1 = exp_tail3(z1), g2 = exp_tail3(z2);
+    const zd t1 = z1 * (mkz(1.0) + z1 * (mkz(0.5) + z1 * g1));
+    const zd t2 = z2 * (mkz(1.0) + z2 * (mkz(0.5) + z2 * g2));
+    const zd qt = q * t1;
+    const zd d = q * (z1 * (mkz(0.5) - g1 + z1 * g1)) - z2 * (mkz(0.5) - g2 + z2 * g2);
+    if (G) {
+      psi = (mkz(k->lead[0][0], k->lead[0][1]) + t2 + d) * s;
+      chi = (mkz(k->lead[1][0], k->lead[1][1]) + t2 - qt + 3.0 * d) * s;
+    }
+    if (F) {
+      const double s2 = s * s;
+      const zd A2 = k2 * ((t2 + mkz(1.0)) * s), w1 = (t1 + mkz(1.0)) * s;
+      const zd A1 = qk1 * w1, B1 = k1 * w1;
+      zd u1 = 12.0 * (t2 - qt) + 30.0 * d;
+      zd u2 = 2.0 * qt - 3.0 * t2 - 6.0 * d;
+      zd u3 = 4.0 * qt - 2.0 * t2 - t1 - 6.0 * d;
+      if (full) {
+        u1 += mkz(k->lead[2][0], k->lead[2][1]);
+        u2 = u2 - q;
+        u3 = u3 + q;
+      }
+      TT1 = 2.0 * (A2 - A1) + u1 * s2;
+      TT2 = u2 * s2 - A2;
+      TT3 = 2.0 * A1 - B1 + u3 * s2;
+    }
+    return;
   }
-  if (full) {
-    TT1 = C(k.T1[0]) * d2 + t1;
-    TT2 = C(k.T2[0]) * d2 + t2;
-    TT3 = C(k.T3[0]) * d2 + t3;
-  } else {
-    TT1 = t1;
-    TT2 = t2;
-    TT3 = t3;
+  const zd w1 = exp_minus(k1, r) * s, w2 = exp_minus(k2, r) * s;
+  const zd qw = q * w1, ik22 = mkz(k->ik22[0], k->ik22[1]);
+  const zd g2 = (mkz(k->v2[0], k->v2[1]) + ik22 * s) * s;
+  const zd g1 = (mkz(k->v1[0], k->v1[1]) + ik22 * s) * s;
+  const zd D = w2 * g2 - w1 * g1;
+  if (G) {
+    psi = w2 + D;
+    chi = w2 - qw + 3.0 * D;
+  }
+  if (F) {
+    const zd A2 = k2 * w2, A1 = qk1 * w1, B1 = k1 * w1;
+    const zd y2 = w2 * s, y1 = qw * s, yd = D * s;
+    TT1 = 2.0 * (A2 - A1) + 12.0 * (y2 - y1) + 30.0 * yd;
+    TT2 = 2.0 * y1 - 3.0 * y2 - A2 - 6.0 * yd;
+    TT3 = 2.0 * A1 - B1 + 4.0 * y1 - 2.0 * y2 - w1 * s - 6.0 * yd;
+    if (!full) {
+      const double s2 = s * s;
+      TT1 = TT1 - mkz(k->lead[2][0], k->lead[2][1]) * s2;
+      TT2 = TT2 + q * s2;
+      TT3 = TT3 - q * s2;
+    }
   }
 }
 

@@ -1,6 +1,7 @@
 // Host-side tables of libmfbem: Gauss-Legendre rules, quasi-singular estimator parameters and the
 // complex coefficients of the harmonic fundamental solution.  Computed once per call on the host
 // and handed to the kernels as plain data.
+#include <algorithm>
 #include <complex>
 #include <cmath>
 #include <cstdio>
@@ -153,36 +154,31 @@ void host_qsi_params(double relative_error, QsiParams* p) {
   }
 }
 
-// fbem_bem_harela3d_calculate_parameters (bem_harela3d.f90:143-287), the u* and t* coefficients.
+// Constants of the harmonic factors (fbem_bem_harela3d_calculate_parameters, bem_harela3d.f90:
+// 143-287, gives the same functions as sums of E_n terms), evaluated in extended precision and
+// rounded once.
 void host_har_params(double lam_re, double lam_im, double mu_re, double mu_im, double rho,
                      double omega, HarParams* p) {
-  typedef std::complex<double> z;
-  const z I(0.0, 1.0);
-  const double one_4pi = 0.07957747154594767280411105048;
-  z lambda(lam_re, lam_im), mu(mu_re, mu_im);
-  z c1 = std::sqrt((lambda + 2.0 * mu) / rho), c2 = std::sqrt(mu / rho);
-  z k1 = omega / c1, k2 = omega / c2;
-  z r = (c2 * c2) / (c1 * c1), ik1 = I * k1, ik2 = I * k2, c1s = c1 * c1, c2s = c2 * c2;
-  z psi[6] = {0.5 * (1.0 + r), -1.0 / 3.0 * (2.0 / c2 + c2s / (c1s * c1)) * I * omega,
-              I * k1 / (k2 * k2), 1.0 / ik2, 1.0 / (k2 * k2), -1.0 / (k2 * k2)};
-  z chi[6] = {-0.5 * (1.0 - r), -r, -3.0 * r / ik1, 3.0 / ik2, -3.0 * r / (ik1 * ik1),
-              3.0 / (ik2 * ik2)};
-  z T1[10] = {3.0 * (r - 1.0), -0.25 * (1.0 / c2s - c2s / (c1s * c1s)) * (omega * omega),
-              -2.0 * I * k1 * r, 2.0 * I * k2, -12.0 * r, 12.0, -r * 30.0 / ik1, 30.0 / ik2,
-              -r * 30.0 / (ik1 * ik1), 30.0 / (ik2 * ik2)};
-  z T2[9] = {-r, -0.25 * (1.0 / c2s + c2s / (c1s * c1s)) * (omega * omega), -I * k2, 2.0 * r,
-             -3.0, r * 6.0 / ik1, -6.0 / ik2, r * 6.0 / (ik1 * ik1), -6.0 / (ik2 * ik2)};
-  z T3[9] = {r, 0.25 * (3.0 * c2s / (c1s * c1s) - 2.0 / c1s + 1.0 / c2s) * (omega * omega),
-             (2.0 * r - 1.0) * I * k1, 4.0 * r - 1.0, -2.0, r * 6.0 / ik1, -6.0 / ik2,
-             r * 6.0 / (ik1 * ik1), -6.0 / (ik2 * ik2)};
-  auto put = [](double* d, z v) { d[0] = v.real(); d[1] = v.imag(); };
-  put(p->k1, k1);
-  put(p->k2, k2);
-  for (int i = 0; i < 6; i++) { put(p->psi[i], psi[i]); put(p->chi[i], chi[i]); }
-  for (int i = 0; i < 10; i++) put(p->T1[i], T1[i]);
-  for (int i = 0; i < 9; i++) { put(p->T2[i], T2[i]); put(p->T3[i], T3[i]); }
+  typedef std::complex<long double> z;
+  const z I(0.0L, 1.0L), one(1.0L, 0.0L);
+  const long double one_4pi = 0.07957747154594766788444188168625718L;
+  const z lambda(lam_re, lam_im), mu(mu_re, mu_im), om((long double)omega, 0.0L);
+  const long double rl = rho;
+  const z c1 = std::sqrt((lambda + 2.0L * mu) / rl), c2 = std::sqrt(mu / rl);
+  const z k1 = I * (om / c1), k2 = I * (om / c2), q = mu / (lambda + 2.0L * mu);
+  const z lead[5] = {0.5L * (one + q), -0.5L * (one - q), 3.0L * (q - one), -q, q};
+  auto put = [](double* d, z v) { d[0] = (double)v.real(); d[1] = (double)v.imag(); };
+  for (int a = 0; a < 5; a++) put(p->lead[a], lead[a]);
+  put(p->kap1, k1);
+  put(p->kap2, k2);
+  put(p->q, q);
+  put(p->qk1, q * k1);
+  put(p->v1, q / k1);
+  put(p->v2, one / k2);
+  put(p->ik22, one / (k2 * k2));
+  p->rser = (double)(1.0L / std::max(std::abs(k1), std::abs(k2)));
   put(p->cte_u, one_4pi / mu);
-  put(p->cte_t, z(one_4pi, 0.0));
+  put(p->cte_t, z(one_4pi, 0.0L));
 }
 
 }  // namespace mfb

@@ -10,12 +10,15 @@ struct QsiParams {
   double tdmin[3][8], tdmax[3][8], ta0[3][8], ta1[3][8], tb1[3][8];
 };
 
-// Complex coefficients of the harmonic fundamental solution, (re, im) pairs
-// (fbem_bem_harela3d_parameters, lib/fbem/src/bem_harela3d.f90:118-134; u* and t* parts only).
+// Constants of the harmonic fundamental solution, (re, im) pairs.  With kappa_j = i k_j (1: P, 2: S
+// waves), q = (c2/c1)^2 and s = 1/r, the factors of u* and t* (lib/fbem/src/bem_harela3d.f90:118-134,
+// 660-682) are finite sums of s^p exp(-kappa_j r).
 struct HarParams {
-  double k1[2], k2[2];
-  double psi[6][2], chi[6][2];
-  double T1[10][2], T2[9][2], T3[9][2];
+  double kap1[2], kap2[2];
+  double q[2], qk1[2];           // q, q kappa1
+  double v1[2], v2[2], ik22[2];  // q/kappa1, 1/kappa2, 1/kappa2^2
+  double rser;                   // r below which D is summed as a series (har_factors)
+  double lead[5][2];             // psi, chi: limit of r f; TT1, TT2, TT3: limit of r^2 f, r -> 0
   double cte_u[2], cte_t[2];
 };
 
