@@ -57,6 +57,11 @@ struct PolarSet {
   double thp[16];
 };
 __constant__ PolarSet c_polar[9];
+// Their quadrature points, (xi1, xi2, rho x weights) each: they depend on the node alone, so a
+// singular pair reads them instead of taking tan, atan, sine and cosine per point.
+constexpr int kPolarMax = 2400;  // 8 sub-triangles of at most 20 x 15 points
+__device__ double g_polar_pts[9][kPolarMax][3];
+__constant__ int c_polar_np[9];
 
 constexpr int kWave = 64;
 // adaptive subdivision: leaves integrated per batch, and the walk's stack (4 entries pushed per
@@ -143,11 +148,8 @@ __device__ inline zd scale_h(const KernelParams& k, zd v) { return mkz(k.h.cte_t
 __device__ inline zd scale_g(const KernelParams& k, zd v) { return mkz(k.h.cte_u[0], k.h.cte_u[1]) * v; }
 
 // Exterior kernel values at one point before the constants (bem_staela3d.f90:636-645;
-// bem_harela3d.f90:657-690) and the regularised values of the singular integration
-// (bem_staela3d.f90:1303-1322; bem_harela3d.f90:1418-1438):
-// h += ft*phi*jw + fc*(phi-phi_i)*jw, g += fu*phi*jw.
-// Same kernels, written component by component into an LDS row (keeps the 18-27 values out of
-// registers): row[c] = ft, row[9 + c] = fu, row[18 + c] = fc (entries `stride` apart).
+// bem_harela3d.f90:657-690), h += ft*phi*jw, g += fu*phi*jw, written component by component into an
+// LDS row: row[c] = ft, row[9 + c] = fu (entries `stride` apart).
 __device__ inline void ext_kernel_row(const KernelParams& k, const double* x, const double* n,
                                       const double* x_i, double* row, int stride = 1) {
   double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
@@ -179,73 +181,6 @@ __device__ inline void ext_kernel_row(const KernelParams& k, const double* x, co
       row[stride * (3 * il + ik)] = TT1 * dr[il] * dr[ik] * drdn +
                                     TT2 * (drdn * dk + dr[ik] * n[il]) + TT3 * dr[il] * n[ik];
     }
-}
-
-__device__ inline void sing_kernel_row(const KernelParams& k, const double* x, const double* n,
-                                       const double* x_i, double* row) {
-  double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
-  double r = sqrt(dot3(rv, rv)), d1r = 1.0 / r, d1r2 = d1r * d1r;
-  double dr[3] = {rv[0] * d1r, rv[1] * d1r, rv[2] * d1r};
-  double drdn = dot3(dr, n);
-  for (int il = 0; il < 3; il++)
-    for (int ik = 0; ik < 3; ik++) {
-      double dk = il == ik ? 1.0 : 0.0;
-      row[9 + 3 * il + ik] = d1r * (k.cteu2 * dk + dr[il] * dr[ik]);
-      row[3 * il + ik] = d1r2 * drdn * (k.ctet2 * dk + 3.0 * dr[il] * dr[ik]);
-      row[18 + 3 * il + ik] = d1r2 * k.ctet2 * (n[il] * dr[ik] - n[ik] * dr[il]);
-    }
-}
-
-__device__ inline void sing_kernel_row(const KernelParams& k, const double* x, const double* n,
-                                       const double* x_i, zd* row) {
-  double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
-  double r, d1r;
-  dist_and_inverse(dot3(rv, rv), r, d1r);
-  const double d1r2 = d1r * d1r;
-  double dr[3] = {rv[0] * d1r, rv[1] * d1r, rv[2] * d1r};
-  double drdn = dot3(dr, n);
-  zd psi, chi, TT1, TT2, TT3;
-  har_factors<true, true>(&k.h, r, d1r, false, psi, chi, TT1, TT2, TT3);
-  zd t1s = mkz(k.h.lead[2][0], k.h.lead[2][1]) * d1r2, t2s = mkz(k.h.lead[3][0], k.h.lead[3][1]) * d1r2;
-  for (int il = 0; il < 3; il++)
-    for (int ik = 0; ik < 3; ik++) {
-      double dk = il == ik ? 1.0 : 0.0;
-      row[9 + 3 * il + ik] = psi * dk - chi * dr[il] * dr[ik];
-      row[3 * il + ik] = (TT1 + t1s) * dr[il] * dr[ik] * drdn + (TT2 + t2s) * drdn * dk +
-                         TT2 * dr[ik] * n[il] + TT3 * dr[il] * n[ik];
-      row[18 + 3 * il + ik] = t2s * (n[il] * dr[ik] - n[ik] * dr[il]);
-    }
-}
-
-// Scatter of one (collocation node i, component il/ik, h|g) row of 9 node values (already
-// multiplied by the kernel constants) into A and b: BE ordinary boundary of
-// src/assemble_bem_staela_equation.f90:69-98 and src/assemble_bem_harela_equation.f90:78-113.
-template <typename T>
-__device__ inline void scatter_row(const DevMesh& m, const int* en, int i, int il, int ik,
-                                   bool is_g, const T* v, T* A, long long lda, T* b,
-                                   bool plain = false) {
-  long long row = 3LL * i + il;
-  T bs = zero_of(v[0]);
-  bool has_b = false;
-  for (int n = 0; n < 9; n++) {
-    int sn = en[n];
-    long long col = 3LL * sn + ik;
-    int ct = m.ctype[3 * sn + ik];
-    double cv = m.cval[3 * sn + ik];
-    if (!is_g) {
-      if (ct == 0) { bs = bs - v[n] * cv; has_b = true; }
-      else if (plain) A[row + lda * col] += v[n];
-      else atomic_add(&A[row + lda * col], v[n]);
-    } else {
-      if (ct == 0) {
-        if (plain) A[row + lda * col] += -v[n];
-        else atomic_add(&A[row + lda * col], -v[n]);
-      }
-      else if (ct == 1) { bs = bs + v[n] * cv; has_b = true; }
-      else { bs = bs + v[n] * (cv * m.nfn[3 * sn + ik]); has_b = true; }
-    }
-  }
-  if (has_b) atomic_add(&b[row], bs);
 }
 
 // Third output of the integration kernels: the displacement at interior points,
@@ -1174,20 +1109,17 @@ __global__ void __launch_bounds__(kWave) k_adaptive(DevMesh m, const QsiParams* 
 }
 
 // Line integral eps_ijk e_k . t / r over one line3 edge, adaptive Telles + bisection
-// (fbem_bem_staela3d_sbie_int_li, bem_staela3d.f90:2245-2376).  Returns the 3 independent
-// entries (1,2), (1,3), (2,3).
-__device__ __attribute__((noinline)) void line_integral(const double* Xl, const double* x_i, const QsiParams& q, int ns,
-                              double* out) {
+// (fbem_bem_staela3d_sbie_int_li, bem_staela3d.f90:2245-2376): the 3 independent entries (1,2),
+// (1,3), (2,3), by the 16 lanes of a quarter wave.  The lanes walk the bisection together (every
+// sub-interval is dyadic: level and index replace a stack) and share the points of a leaf.
+__device__ inline void line_integral(const double* Xl, const double* x_i, const QsiParams& q, int ns,
+                                     int sub_lane, double* out) {
   const GLTables& G = gl();
-  double stk[40][3];
-  int sp = 0;
-  stk[0][0] = -1.0; stk[0][1] = 1.0; stk[0][2] = 1;
-  sp = 1;
   out[0] = out[1] = out[2] = 0;
-  while (sp > 0) {
-    sp--;
-    double xs[2] = {stk[sp][0], stk[sp][1]};
-    int ks = (int)stk[sp][2];
+  int ks = 1, idx = 0;
+  for (;;) {
+    const double width = 2.0 / (double)(1 << (ks - 1));
+    const double xs[2] = {-1.0 + width * idx, -1.0 + width * (idx + 1)};
     double Xs[9];
     if (ks == 1) {
       for (int c = 0; c < 9; c++) Xs[c] = Xl[c];
@@ -1197,219 +1129,450 @@ __device__ __attribute__((noinline)) void line_integral(const double* Xl, const 
     double cl = length_l3(Xs, 1e-12), bx, rmin, d;
     nearest_l3(Xs, cl, x_i, &bx, &rmin, &d);
     int gln_near = qs_estimate(q, 1, 1, 1, d, &bx);
-    bool sub = false;
-    if (ks == ns) {
-      if (gln_near == 0) gln_near = 30;
-    } else if (gln_near == 0) {
-      sub = true;
+    if (gln_near == 0 && ks < ns) {
+      ks++;
+      idx *= 2;
+      continue;
     }
-    if (sub && sp + 2 <= 40) {
-      double mid = 0.5 * (xs[0] + xs[1]);
-      stk[sp][0] = mid; stk[sp][1] = xs[1]; stk[sp][2] = ks + 1; sp++;
-      stk[sp][0] = xs[0]; stk[sp][1] = mid; stk[sp][2] = ks + 1; sp++;
-    } else {
-      int gln = max(gln_near, 5);
-      double tp[4], t12 = 0, t13 = 0, t23 = 0;
-      telles11(bx, telles_barr(d), tp);
-      for (int kip = 0; kip < gln; kip++) {
-        double xip, jt;
-        telles_xj(tp, G.x11[gln][kip], &xip, &jt);
-        double xi = 0.5 * (1.0 - xip) * xs[0] + 0.5 * (1.0 + xip) * xs[1];
-        double js = 0.5 * (xs[1] - xs[0]);
-        double ph[3], dp[3], x[3] = {0, 0, 0}, T[3] = {0, 0, 0};
-        phi_l3(xi, ph);
-        dphi_l3(xi, dp);
-        for (int kk = 0; kk < 3; kk++)
-          for (int c = 0; c < 3; c++) {
-            x[c] += ph[kk] * Xl[3 * kk + c];
-            T[c] += dp[kk] * Xl[3 * kk + c];
-          }
-        double jg = sqrt(dot3(T, T));
-        double t[3] = {T[0] / jg, T[1] / jg, T[2] / jg};
-        double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
-        double dr1 = 1.0 / sqrt(dot3(rv, rv));
-        double jw = jg * js * jt * G.w11[gln][kip];
-        t12 = t12 - dr1 * t[2] * jw;
-        t13 = t13 + dr1 * t[1] * jw;
-        t23 = t23 - dr1 * t[0] * jw;
-      }
-      out[0] += t12;
-      out[1] += t13;
-      out[2] += t23;
+    if (gln_near == 0) gln_near = 30;
+    const int gln = max(gln_near, 5);
+    double tp[4];
+    telles11(bx, telles_barr(d), tp);
+    for (int kip = sub_lane; kip < gln; kip += 16) {
+      double xip, jt;
+      telles_xj(tp, G.x11[gln][kip], &xip, &jt);
+      double xi = 0.5 * (1.0 - xip) * xs[0] + 0.5 * (1.0 + xip) * xs[1];
+      double js = 0.5 * (xs[1] - xs[0]);
+      double ph[3], dp[3], x[3] = {0, 0, 0}, T[3] = {0, 0, 0};
+      phi_l3(xi, ph);
+      dphi_l3(xi, dp);
+      for (int kk = 0; kk < 3; kk++)
+        for (int c = 0; c < 3; c++) {
+          x[c] += ph[kk] * Xl[3 * kk + c];
+          T[c] += dp[kk] * Xl[3 * kk + c];
+        }
+      double jg = sqrt(dot3(T, T));
+      double t[3] = {T[0] / jg, T[1] / jg, T[2] / jg};
+      double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
+      double dr1 = 1.0 / sqrt(dot3(rv, rv));
+      double jw = jg * js * jt * G.w11[gln][kip];
+      out[0] -= dr1 * t[2] * jw;
+      out[1] += dr1 * t[1] * jw;
+      out[2] -= dr1 * t[0] * jw;
     }
+    // the next interval: out of right halves, then the right half beside
+    while (ks > 1 && (idx & 1)) { idx >>= 1; ks--; }
+    if (ks == 1) break;
+    idx++;
   }
+  for (int c = 0; c < 3; c++)
+    for (int mask = 1; mask < 16; mask *= 2) out[c] += __shfl_xor(out[c], mask);
 }
 
-// Singular pairs: fbem_bem_staela3d_sbie_int (bem_staela3d.f90:1100-1381) and
-// fbem_bem_harela3d_sbie_int (bem_harela3d.f90:1174-1472).
-template <bool H>
-__global__ void __launch_bounds__(kWave) k_singular(DevMesh m, const QsiParams* __restrict__ qsp_li_p,
-                                                    const KernelParams* __restrict__ kpp,
-                                                    const int* list, int count,
-                                                    typename Val<H>::T* A, long long lda,
-                                                    typename Val<H>::T* b, long long* counters,
-                                                    typename Val<H>::T* blocks, long long blk_base,
-                                                    VecOut<typename Val<H>::T> vec) {
-  typedef typename Val<H>::T T;
-  const QsiParams& qsp_li = *qsp_li_p;
-  const KernelParams& kp = *kpp;
-  const int lane = threadIdx.x;
-  const int pid = list[blockIdx.x];
-  const int e = pid / m.ncp, cp = pid % m.ncp;
-  __shared__ T sfs[kChunk * 27];     // ft, fu, fc
-  __shared__ double sw[kChunk * 18];  // phi*jw, (phi - phi_i)*jw
-  __shared__ double shli[4][3];
-  double X[27], el[8];
-  load_X(m, e, X);
-  for (int c = 0; c < 8; c++) el[c] = m.elem[8 * e + c];
-  const double xc[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
-  double xi_i[2], rmin, d;
+// local coordinates of the collocation point of a singular pair and, when it is one of the element's
+// nodes, that node (else -1)
+__device__ inline int singular_xi(const DevMesh& m, const double* X, int e, int cp, double* xi_i) {
   if (m.cel[cp] == e) {
     // an MCA point inside this element: its local coordinates are known exactly
     xi_i[0] = m.cxi[2 * cp];
     xi_i[1] = m.cxi[2 * cp + 1];
   } else {
-    nearest_q9(X, el[0], xc, xi_i, &rmin, &d);
+    double rmin, d;
+    const double xc[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
+    nearest_q9(X, m.elem[8 * e], xc, xi_i, &rmin, &d);
   }
-  double x_i[3], pf_i[9];
-  q9_x(X, xi_i[0], xi_i[1], x_i);
-  phi_q9(xi_i[0], xi_i[1], pf_i);
-  int st[8], ngt[8], base[9], nst = -1;
-  double th[16], thp[16];
   for (int k = 0; k < 9; k++)
-    if (xi_i[0] == kXiQ9[k][0] && xi_i[1] == kXiQ9[k][1]) {
-      const PolarSet& ps = c_polar[k];
-      nst = ps.n;
-      for (int s = 0; s < nst; s++) {
-        st[s] = ps.st[s];
-        ngt[s] = ps.ngt[s];
-        th[2 * s] = ps.th[2 * s];
-        th[2 * s + 1] = ps.th[2 * s + 1];
-        thp[2 * s] = ps.thp[2 * s];
-        thp[2 * s + 1] = ps.thp[2 * s + 1];
-      }
-      break;
-    }
-  if (nst < 0) {
+    if (xi_i[0] == kXiQ9[k][0] && xi_i[1] == kXiQ9[k][1]) return k;
+  return -1;
+}
+
+// What a singular pair's integration takes from the geometry alone: where its point lies on the
+// element, the polar sub-triangles when that is not a node, and the Stokes line integrals summed over
+// the edges that bound an integrated sub-triangle, (1,2), (1,3), (2,3).  Made once, with the lists:
+// inside the integration they were four lanes' serial walk, 300 of the 390 us that a launch over a
+// small mesh took.  One wave per pair, a quarter wave per edge.
+struct SingGeom {
+  double hli[3], xi[2], thp[16];
+  int node, np, st[8], base[9];   // node: element node at xi or -1; np: quadrature points
+};
+__global__ void __launch_bounds__(kWave) k_sing_geom(DevMesh m,
+                                                     const QsiParams* __restrict__ qsp_li,
+                                                     const int* __restrict__ list, SingGeom* geo) {
+  const int lane = threadIdx.x, edge = lane >> 4;
+  const int pid = list[blockIdx.x], e = pid / m.ncp, cp = pid % m.ncp;
+  double X[27], xi_i[2], x_i[3], o[3] = {0, 0, 0};
+  load_X(m, e, X);
+  const int k = singular_xi(m, X, e, cp, xi_i);
+  q9_x(X, xi_i[0], xi_i[1], x_i);
+  int st[8], nst;
+  SingGeom& out = geo[blockIdx.x];
+  if (k >= 0) {
+    nst = c_polar[k].n;
+    for (int s = 0; s < nst; s++) st[s] = c_polar[k].st[s];
+    if (lane == 0) out.np = c_polar_np[k];
+  } else {
+    double th[16], thp[16];
     nst = polar_setup_q(xi_i, st, th, thp);
-    for (int s = 0; s < nst; s++) ngt[s] = 5 + (int)round(25.0 * (th[2 * s + 1] - th[2 * s]) / kPi_2);
-  }
-  base[0] = 0;
-  for (int s = 0; s < nst; s++) base[s + 1] = base[s] + ngt[s] * 15;
-  const int P = base[nst];
-  const GLTables& G = gl();
-  T acc[3] = {zero_of(T()), zero_of(T()), zero_of(T())};
-  for (int start = 0; start < P; start += kChunk) {
-    int p = start + lane;
-    if (lane < kChunk && p < P) {
-      int s = 0;
-      while (p >= base[s + 1]) s++;
-      int q = p - base[s], kt = q / 15, kr = q % 15, nt = ngt[s];
-      double jtp = thp[2 * s + 1] - thp[2 * s];
-      double tpv = jtp * G.x01[nt][kt] + thp[2 * s];
-      double theta, rhoij;
-      polar_angular_q(xi_i, st[s], tpv, &theta, &rhoij);
-      double sn, cs;
-      sincos(theta, &sn, &cs);
-      double rho = rhoij * G.x01[15][kr];
-      double xi0 = xi_i[0] + rho * cs, xi1 = xi_i[1] + rho * sn;
-      double x[3], T1[3], T2[3], N[3], n[3], ph[9];
-      q9_geom(X, xi0, xi1, x, T1, T2);
-      cross3(T1, T2, N);
-      double jg = sqrt(dot3(N, N));
-      for (int c = 0; c < 3; c++) n[c] = N[c] / jg;
-      double jw = jg * rho * jtp * G.w01[nt][kt] * G.w01[15][kr];
-      phi_q9(xi0, xi1, ph);
-      sing_kernel_row(kp, x, n, x_i, &sfs[lane * 27]);
-      for (int c = 0; c < 9; c++) {
-        sw[lane * 18 + c] = ph[c] * jw;
-        sw[lane * 18 + 9 + c] = (ph[c] - pf_i[c]) * jw;
-      }
-    }
-    __syncthreads();
-    int np = min(kChunk, P - start);
-    for (int t = 0; t < 3; t++) {
-      int o = lane + kWave * t;
-      if (o < 162) {
-        int kind = o / 81, c = (o % 81) / 9, n = o % 9;
-        if (kind == 0) {
-          for (int pp = 0; pp < np; pp++)
-            acc[t] += sfs[pp * 27 + c] * sw[pp * 18 + n] + sfs[pp * 27 + 18 + c] * sw[pp * 18 + 9 + n];
-        } else {
-          for (int pp = 0; pp < np; pp++) acc[t] += sfs[pp * 27 + 9 + c] * sw[pp * 18 + n];
+    if (lane == 0) {
+      int base = 0;
+      for (int s = 0; s < 8; s++) {
+        out.base[s] = base;
+        if (s < nst) {
+          base += 15 * (5 + (int)round(25.0 * (th[2 * s + 1] - th[2 * s]) / kPi_2));
+          out.st[s] = st[s];
+          out.thp[2 * s] = thp[2 * s];
+          out.thp[2 * s + 1] = thp[2 * s + 1];
         }
       }
+      out.base[8] = base;
+      out.np = base;
+    }
+  }
+  bool integrate = false;
+  for (int s = 0; s < nst; s++)
+    if (st[s] == 2 * edge + 1 || st[s] == 2 * edge + 2) integrate = true;
+  if (integrate) {
+    double Xl[9];
+    for (int j = 0; j < 3; j++)
+      for (int c = 0; c < 3; c++) Xl[3 * j + c] = X[3 * kEdgeQ9[edge][j] + c];
+    line_integral(Xl, x_i, *qsp_li, 16, lane & 15, o);
+  }
+  for (int c = 0; c < 3; c++) {
+    o[c] += __shfl_xor(o[c], 16);
+    o[c] += __shfl_xor(o[c], 32);
+  }
+  if (lane == 0) {
+    for (int c = 0; c < 3; c++) out.hli[c] = o[c];
+    out.xi[0] = xi_i[0];
+    out.xi[1] = xi_i[1];
+    out.node = k;
+  }
+}
+
+// point (kt, kr) of a sub-triangle's rule at xi_i: local coordinates and rho x weights
+__device__ __attribute__((noinline)) void polar_point(const double* xi_i, int st, double thp0, double thp1, int nt,
+                                   int kt, int kr, double* xi, double* w) {
+  const GLTables& G = gl();
+  const double jtp = thp1 - thp0, tpv = jtp * G.x01[nt][kt] + thp0;
+  double theta, rhoij, sn, cs;
+  polar_angular_q(xi_i, st, tpv, &theta, &rhoij);
+  sincos(theta, &sn, &cs);
+  const double rho = rhoij * G.x01[15][kr];
+  xi[0] = xi_i[0] + rho * cs;
+  xi[1] = xi_i[1] + rho * sn;
+  *w = rho * jtp * G.w01[nt][kt] * G.w01[15][kr];
+}
+
+__global__ void k_polar_table() {
+  const int k = blockIdx.y, p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= c_polar_np[k]) return;
+  const PolarSet& ps = c_polar[k];
+  int s = 0, base = 0;
+  while (p >= base + ps.ngt[s] * 15) base += 15 * ps.ngt[s++];
+  const int q = p - base;
+  polar_point(kXiQ9[k], ps.st[s], ps.thp[2 * s], ps.thp[2 * s + 1], ps.ngt[s], q / 15, q % 15,
+              g_polar_pts[k][p], &g_polar_pts[k][p][2]);
+}
+
+// Kernel values of the singular integration (bem_staela3d.f90:1303-1322; bem_harela3d.f90:
+// 1418-1438), h += ft*phi*jw + fc*(phi-phi_i)*jw, g += fu*phi*jw, as rows of real numbers: ft first
+// (static: the 6 of a symmetric 3 x 3, harmonic: 9 complex), then the 6 of the symmetric fu, from
+// row fc0 on the 3 of the antisymmetric fc without its constant factor (ctet2, lead of TT2).
+template <bool H, int KIND>
+struct SingRows {
+  static constexpr int NH = KIND & kNeedH ? (H ? 18 : 6) : 0, NG = KIND & kNeedG ? (H ? 12 : 6) : 0;
+  static constexpr int fc0 = (NH + NG + 3) / 4 * 4;                // rows in groups of four
+  static constexpr int NR = fc0 + (KIND & kNeedH ? 4 : 0);
+};
+
+template <int KIND>
+__device__ inline void sing_rows(ConstKP k, const double* x, const double* n, const double* x_i,
+                                 double* v, double) {
+  typedef SingRows<false, KIND> R;
+  const double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
+  const double s = rsqrt(dot3(rv, rv)), s2 = s * s;
+  const double dr[3] = {rv[0] * s, rv[1] * s, rv[2] * s}, drdn = dot3(dr, n);
+  const double a = s2 * drdn, ac = a * k->ctet2, u = s * k->cteu2;
+  int c = 0;
+#pragma unroll
+  for (int l = 0; l < 3; l++)
+#pragma unroll
+    for (int q = l; q < 3; q++, c++) {
+      const double rr = dr[l] * dr[q];
+      if (KIND & kNeedH) v[c] = 3.0 * a * rr + (l == q ? ac : 0.0);
+      if (KIND & kNeedG) v[R::NH + c] = s * rr + (l == q ? u : 0.0);
+    }
+  if (KIND & kNeedH) {
+    v[R::fc0] = s2 * (n[0] * dr[1] - n[1] * dr[0]);
+    v[R::fc0 + 1] = s2 * (n[0] * dr[2] - n[2] * dr[0]);
+    v[R::fc0 + 2] = s2 * (n[1] * dr[2] - n[2] * dr[1]);
+  }
+}
+
+template <int KIND>
+__device__ inline void sing_rows(ConstKP k, const double* x, const double* n, const double* x_i,
+                                 double* v, zd) {
+  typedef SingRows<true, KIND> R;
+  const double rv[3] = {x[0] - x_i[0], x[1] - x_i[1], x[2] - x_i[2]};
+  double r, s;
+  dist_and_inverse(dot3(rv, rv), r, s);
+  const double dr[3] = {rv[0] * s, rv[1] * s, rv[2] * s}, drdn = dot3(dr, n), s2 = s * s;
+  zd psi, chi, TT1, TT2, TT3;
+  har_factors<(KIND & kNeedH) != 0, (KIND & kNeedG) != 0>(&k->h, r, s, false, psi, chi, TT1, TT2, TT3);
+  if (KIND & kNeedH) {
+    const zd a = (TT1 + mkz(k->h.lead[2][0], k->h.lead[2][1]) * s2) * drdn;
+    const zd d = (TT2 + mkz(k->h.lead[3][0], k->h.lead[3][1]) * s2) * drdn;
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+      const zd u = a * dr[l] + TT2 * n[l], w = TT3 * dr[l];
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        zd f = u * dr[q] + w * n[q];
+        if (l == q) f += d;
+        v[2 * (3 * l + q)] = f.re;
+        v[2 * (3 * l + q) + 1] = f.im;
+      }
+    }
+    v[R::fc0] = s2 * (n[0] * dr[1] - n[1] * dr[0]);
+    v[R::fc0 + 1] = s2 * (n[0] * dr[2] - n[2] * dr[0]);
+    v[R::fc0 + 2] = s2 * (n[1] * dr[2] - n[2] * dr[1]);
+  }
+  if (KIND & kNeedG) {
+    int c = 0;
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+      const zd u = -(chi * dr[l]);
+#pragma unroll
+      for (int q = l; q < 3; q++, c++) {
+        const zd f = l == q ? psi + u * dr[q] : u * dr[q];
+        v[R::NH + 2 * c] = f.re;
+        v[R::NH + 2 * c + 1] = f.im;
+      }
+    }
+  }
+}
+
+// LDS of one pair integrated by W waves: 12 rows of kernel values and phi, jw of a wave's 64 points
+// (rows 72 doubles apart: the matrix operands' loads meet no bank twice), then the waves' sums.
+constexpr int kRowStride = 72, kPassRows = 12;
+template <int W>
+struct PairLds {
+  union {
+    struct {
+      double f[W][kPassRows][kRowStride];
+      double ph[W][10][kRowStride];
+    };
+    double sum[W][36][9];
+  };
+};
+
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// acc[g][q] += sum over the wave's 64 points of (rows 4 g .. 4 g + 3) x (weights of nodes 4 q ..
+// 4 q + 3): the lane's values v of its point go through LDS, 12 rows at a time, into the layout of
+// the left operand; each of the four blocks of an instruction takes four of 16 points, so the result
+// is summed over lane bits 2, 3 at the end (rows_reduce).  From row FC on the weights are
+// (phi - phi_i) jw.  A point without weight carries jw = 0 and finite values.
+template <int NR, int FC>
+__device__ inline void rows_mfma(const double* v, const double* ph, double jw, const double* pf_i,
+                                 double (*f)[kRowStride], double (*sp)[kRowStride], int lane,
+                                 double (*acc)[3]) {
+  wave_lds_fence();
+#pragma unroll
+  for (int n = 0; n < 9; n++) sp[n][lane] = ph[n];
+  sp[9][lane] = jw;
+  const int i = lane & 3, at = 4 * (lane >> 4) + ((lane >> 2) & 3);
+#pragma unroll
+  for (int r0 = 0; r0 < NR; r0 += kPassRows) {
+    wave_lds_fence();
+#pragma unroll
+    for (int r = r0; r < r0 + kPassRows && r < NR; r++) f[r - r0][lane] = v[r];
+    wave_lds_fence();
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const double j = sp[9][16 * t + at], p0 = sp[i][16 * t + at], p1 = sp[4 + i][16 * t + at];
+      const double p2 = sp[8][16 * t + at];
+#pragma unroll
+      for (int r = r0; r < r0 + kPassRows && r < NR; r += 4) {
+        const double a = f[r - r0 + i][16 * t + at];
+        const bool fc = r >= FC;
+        acc[r / 4][0] = mfma4(a, (fc ? p0 - pf_i[0] : p0) * j, acc[r / 4][0]);
+        acc[r / 4][1] = mfma4(a, (fc ? p1 - pf_i[1] : p1) * j, acc[r / 4][1]);
+        acc[r / 4][2] = mfma4(a, i == 0 ? (fc ? p2 - pf_i[2] : p2) * j : 0.0, acc[r / 4][2]);
+      }
+    }
+  }
+}
+
+// sums of the workgroup's W waves: lds.sum[0][row][node] afterwards
+template <int NR, int W>
+__device__ inline void rows_reduce(double (*acc)[3], PairLds<W>& lds, int wave, int lane) {
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < NR / 4; g++)
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      double t = acc[g][q];
+      t += __shfl_xor(t, 4);
+      t += __shfl_xor(t, 8);
+      const int n = 4 * q + (lane & 3);
+      if (!(lane & 12) && n < 9) lds.sum[wave][4 * g + (lane >> 4)][n] = t;
+    }
+  __syncthreads();
+  if (W > 1) {
+    for (int o = threadIdx.x; o < NR * 9; o += W * kWave) {
+      double t = lds.sum[0][0][o];
+      for (int w = 1; w < W; w++) t += lds.sum[w][0][o];
+      lds.sum[0][0][o] = t;
     }
     __syncthreads();
   }
-  // Stokes line integrals over the edges that bound an integrated sub-triangle
-  if (lane < 4) {
-    bool integrate = false;
-    for (int s = 0; s < nst; s++)
-      if (st[s] == 2 * (lane + 1) - 1 || st[s] == 2 * (lane + 1)) integrate = true;
-    double o3[3] = {0, 0, 0};
-    if (integrate) {
-      double Xl[9];
-      for (int j = 0; j < 3; j++)
-        for (int c = 0; c < 3; c++) Xl[3 * j + c] = X[3 * kEdgeQ9[lane][j] + c];
-      line_integral(Xl, x_i, qsp_li, 16, o3);
-    }
-    shli[lane][0] = o3[0];
-    shli[lane][1] = o3[1];
-    shli[lane][2] = o3[2];
-  }
-  __syncthreads();
-  double h12 = 0, h13 = 0, h23 = 0;
-  for (int ke = 0; ke < 4; ke++) { h12 += shli[ke][0]; h13 += shli[ke][1]; h23 += shli[ke][2]; }
-  // hli(il,ik): antisymmetric with (1,2)=h12, (1,3)=h13, (2,3)=h23
-  const double hli[3][3] = {{0, h12, h13}, {-h12, 0, h23}, {-h13, -h23, 0}};
+}
+
+// Output of one pair: value(kind, l, k, n) -> h (0) or g (1) with the kernel constants.  Threads
+// t < 81 take (n, l, k) each: scatter into A and b (scatter of
+// src/assemble_bem_{staela,harela}_equation.f90), the pair's blocks, or the displacement of its point.
+template <bool H, int KIND, class Value>
+__device__ inline void pair_output(const DevMesh& m, int e, int cp, int t,
+                                   typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
+                                   typename Val<H>::T* block, const VecOut<typename Val<H>::T>& vec,
+                                   Value&& value) {
+  typedef typename Val<H>::T T;
+  __shared__ T red[3];
   if (vec.out) {
-    T fin[3];
-    for (int t = 0; t < 3; t++) {
-      const int o = lane + kWave * t;
-      fin[t] = acc[t];
-      if (o < 81) {
-        const int c = o / 9, n = o % 9;
-        const double f = pf_i[n] * hli[c / 3][c % 3];
-        if constexpr (H) fin[t] += mkz(kp.h.lead[3][0], kp.h.lead[3][1]) * f;
-        else fin[t] += kp.ctet2 * f;
-      }
-    }
-    vec_reduce(m, kp, e, cp, fin, vec, lane);
-    if (lane == 0) atomicAdd((unsigned long long*)&counters[0], (unsigned long long)P);
-    return;
+    if (t < 3) red[t] = zero_of(T());
+    __syncthreads();
   }
-  for (int t = 0; t < 3; t++) {
-    int o = lane + kWave * t;
-    if (o < 162) {
-      int kind = o / 81, c = (o % 81) / 9, n = o % 9;
-      int il = c / 3, ik = c % 3;
-      T v = acc[t];
-      if (kind == 0) {
-        double f = pf_i[n] * hli[il][ik];
-        if constexpr (H) v += mkz(kp.h.lead[3][0], kp.h.lead[3][1]) * f;
-        else v += kp.ctet2 * f;
-      }
-      v = kind ? scale_g(kp, v) : scale_h(kp, v);
-      if (blocks) {
-        blocks[162LL * (blk_base + blockIdx.x) + 81 * kind + n + 9 * il + 27 * ik] = v;
-        continue;
-      }
-      int sn = m.conn[9 * e + n];
-      long long row = 3LL * m.crow[cp] + il, col = 3LL * sn + ik;
-      int ct = m.ctype[3 * sn + ik];
-      double cv = m.cval[3 * sn + ik];
-      if (kind == 0) {
-        if (ct == 0) atomic_add(&b[row], -(v * cv));
-        else atomic_add(&A[row + lda * col], v);
-      } else {
-        if (ct == 0) atomic_add(&A[row + lda * col], -v);
-        else if (ct == 1) atomic_add(&b[row], v * cv);
-        else atomic_add(&b[row], v * (cv * m.nfn[3 * sn + ik]));
+  if (t < 81) {
+    const int il = t % 3, n = (t / 3) % 9, ik = t / 27;
+    const int sn = m.conn[9 * e + n];
+    const long long col = 3LL * sn + ik;
+    if (block) {
+      const int o = n + 9 * il + 27 * ik;
+      block[o] = value(0, il, ik, n);
+      block[81 + o] = value(1, il, ik, n);
+    } else if (vec.out) {
+      lds_add(&red[il], value(1, il, ik, n) * vec.t[col] - value(0, il, ik, n) * vec.u[col]);
+    } else {
+      const long long row = 3LL * m.crow[cp] + il;
+      const int ct = m.ctype[col];
+      const double cv = m.cval[col];
+      atomic_add(&A[row + lda * col], ct == 0 ? -value(1, il, ik, n) : value(0, il, ik, n));
+      if (KIND == (kNeedH | kNeedG) && cv != 0.0) {
+        if (ct == 0) atomic_add(&b[row], value(0, il, ik, n) * -cv);
+        else atomic_add(&b[row], value(1, il, ik, n) * (ct == 1 ? cv : cv * m.nfn[col]));
       }
     }
   }
-  if (lane == 0) atomicAdd((unsigned long long*)&counters[0], (unsigned long long)P);
+  if (vec.out) {
+    __syncthreads();
+    if (t < 3) atomic_add(&vec.out[3 * cp + t], red[t]);
+  }
+}
+
+// Singular pairs: fbem_bem_staela3d_sbie_int (bem_staela3d.f90:1100-1381) and
+// fbem_bem_harela3d_sbie_int (bem_harela3d.f90:1174-1472).
+constexpr int kSingWaves = 4;
+template <bool H, int KIND>
+__device__ inline void singular_body(const DevMesh& m, ConstKP kp, int e, int cp,
+                                     const SingGeom* __restrict__ geo, PairLds<kSingWaves>& lds,
+                                     typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
+                                     long long* counters, typename Val<H>::T* block,
+                                     const VecOut<typename Val<H>::T>& vec) {
+  typedef typename Val<H>::T T;
+  typedef SingRows<H, KIND> R;
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  double X[27], x_i[3], pf[9];
+  load_X(m, e, X);
+  const double xi_i[2] = {geo->xi[0], geo->xi[1]};
+  const int node = geo->node, P = geo->np;
+  q9_x(X, xi_i[0], xi_i[1], x_i);
+  phi_q9(xi_i[0], xi_i[1], pf);
+  double acc[R::NR / 4][3];
+#pragma unroll
+  for (int g = 0; g < R::NR / 4; g++) acc[g][0] = acc[g][1] = acc[g][2] = 0.0;
+  const int i = lane & 3;
+  const double pfi[3] = {pf[i], pf[4 + i], pf[8]};
+  for (int start = wave * kWave; start < P; start += kSingWaves * kWave) {
+    const int p = min(start + lane, P - 1);
+    double xi[2], w;
+    if (node >= 0) {
+      const double* q = g_polar_pts[node][p];
+      xi[0] = q[0];
+      xi[1] = q[1];
+      w = q[2];
+    } else {
+      int s = 0;
+      while (p >= geo->base[s + 1]) s++;
+      const int q = p - geo->base[s];
+      polar_point(xi_i, geo->st[s], geo->thp[2 * s], geo->thp[2 * s + 1],
+                  (geo->base[s + 1] - geo->base[s]) / 15, q / 15, q % 15, xi, &w);
+    }
+    double x[3], T1[3], T2[3], N[3], ph[9], v[R::NR];
+    q9_geom(X, xi[0], xi[1], x, T1, T2);
+    cross3(T1, T2, N);
+    const double jg = sqrt(dot3(N, N)), ij = 1.0 / jg;
+    const double n[3] = {N[0] * ij, N[1] * ij, N[2] * ij};
+    phi_q9(xi[0], xi[1], ph);
+#pragma unroll
+    for (int r = 0; r < R::NR; r++) v[r] = 0.0;
+    sing_rows<KIND>(kp, x, n, x_i, v, T());
+    rows_mfma<R::NR, (KIND & kNeedH) ? R::fc0 : R::NR>(
+        v, ph, start + lane < P ? jg * w : 0.0, pfi, lds.f[wave], lds.ph[wave], lane, acc);
+  }
+  rows_reduce<R::NR, kSingWaves>(acc, lds, wave, lane);
+  const double(*S)[9] = lds.sum[0];
+  pair_output<H, KIND>(
+      m, e, cp, (int)threadIdx.x, A, lda, b, block, vec, [&](int kind, int il, int ik, int n) {
+        const int c = il == ik ? -1 : il + ik - 1;   // (0,1) 0, (0,2) 1, (1,2) 2
+        if constexpr (H) {
+          const int r = kind ? R::NH + 2 * kSym[3 * il + ik] : 2 * (3 * il + ik);
+          T v = mkz(S[r][n], S[r + 1][n]);
+          if (kind) return mkz(kp->h.cte_u[0], kp->h.cte_u[1]) * v;
+          if (c >= 0) {
+            const double a = S[R::fc0 + c][n] + pf[n] * geo->hli[c];
+            v += mkz(kp->h.lead[3][0], kp->h.lead[3][1]) * (il < ik ? a : -a);
+          }
+          return mkz(kp->h.cte_t[0], kp->h.cte_t[1]) * v;
+        } else {
+          double v = S[(kind ? R::NH : 0) + kSym[3 * il + ik]][n];
+          if (kind) return v * kp->cteu1;
+          if (c >= 0) {
+            const double a = S[R::fc0 + c][n] + pf[n] * geo->hli[c];
+            v += kp->ctet2 * (il < ik ? a : -a);
+          }
+          return v * kp->ctet1;
+        }
+      });
+  if (threadIdx.x == 0) atomicAdd((unsigned long long*)&counters[0], (unsigned long long)P);
+}
+
+// One workgroup of four waves per pair, a wave 64 polar points at a time; per point the values are
+// few real rows (the antisymmetric part and u* by their distinct components), summed against the
+// nine weights on the FP64 matrix cores.
+template <bool H>
+__global__ void __launch_bounds__(kSingWaves* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    k_singular(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
+               const SingGeom* __restrict__ geo, typename Val<H>::T* A, long long lda,
+               typename Val<H>::T* b, long long* counters, typename Val<H>::T* blocks,
+               long long blk_base, VecOut<typename Val<H>::T> vec) {
+  __shared__ PairLds<kSingWaves> lds;
+  const int pid = list[blockIdx.x], e = pid / m.ncp, cp = pid % m.ncp;
+  const SingGeom* li = geo + blockIdx.x;
+  typename Val<H>::T* block = blocks ? blocks + 162LL * (blk_base + blockIdx.x) : nullptr;
+  const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e];
+  ConstKP kp = (ConstKP)kpp;
+  if (kind == kNeedH)
+    singular_body<H, kNeedH>(m, kp, e, cp, li, lds, A, lda, b, counters, block, vec);
+  else if (kind == kNeedG)
+    singular_body<H, kNeedG>(m, kp, e, cp, li, lds, A, lda, b, counters, block, vec);
+  else
+    singular_body<H, kNeedH | kNeedG>(m, kp, e, cp, li, lds, A, lda, b, counters, block, vec);
 }
 
 // err[q * nr + r] = max(max|h - h_ref| / max|h_ref|, max|g - g_ref| / max|g_ref|) of pair q
@@ -1619,21 +1782,8 @@ void set_error(const char* fmt, ...) {
   va_end(ap);
 }
 
-static int upload_polar_table() {
-  static const double xin[9][2] = {{-1, -1}, {1, -1}, {1, 1}, {-1, 1}, {0, -1},
-                                   {1, 0},   {0, 1},  {-1, 0}, {0, 0}};
-  PolarSet t[9];
-  std::memset(t, 0, sizeof t);
-  for (int k = 0; k < 9; k++) {
-    t[k].n = polar_setup_q(xin[k], t[k].st, t[k].th, t[k].thp);
-    for (int s = 0; s < t[k].n; s++)
-      t[k].ngt[s] = 5 + (int)std::round(25.0 * (t[k].th[2 * s + 1] - t[k].th[2 * s]) / kPi_2);
-  }
-  MFB_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_polar), t, sizeof t));
-  return MFB_OK;
-}
-
-static int upload_gl_tables() {
+// Constant tables of the current device: Gauss-Legendre rules, polar sub-triangles and their points.
+static int upload_tables() {
   static bool done = false;
   static int device = -1;
   int dev = 0;
@@ -1642,6 +1792,25 @@ static int upload_gl_tables() {
   static GLTables t;
   host_gl_tables(&t.x11[0][0], &t.w11[0][0], &t.x01[0][0], &t.w01[0][0]);
   MFB_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_gl), &t, sizeof t));
+  static const double xin[9][2] = {{-1, -1}, {1, -1}, {1, 1}, {-1, 1}, {0, -1},
+                                   {1, 0},   {0, 1},  {-1, 0}, {0, 0}};
+  PolarSet ps[9];
+  int np[9];
+  std::memset(ps, 0, sizeof ps);
+  for (int k = 0; k < 9; k++) {
+    ps[k].n = polar_setup_q(xin[k], ps[k].st, ps[k].th, ps[k].thp);
+    np[k] = 0;
+    for (int s = 0; s < ps[k].n; s++) {
+      ps[k].ngt[s] = 5 + (int)std::round(25.0 * (ps[k].th[2 * s + 1] - ps[k].th[2 * s]) / kPi_2);
+      np[k] += 15 * ps[k].ngt[s];
+    }
+    MFB_ARG(np[k] <= kPolarMax, "polar table overflow");
+  }
+  MFB_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_polar), ps, sizeof ps));
+  MFB_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_polar_np), np, sizeof np));
+  hipLaunchKernelGGL(k_polar_table, dim3((kPolarMax + 255) / 256, 9), dim3(256), 0, 0);
+  MFB_HIP(hipGetLastError());
+  MFB_HIP(hipStreamSynchronize(0));
   done = true;
   device = dev;
   return MFB_OK;
@@ -1711,6 +1880,7 @@ struct mfb_mesh_s {
   double *xc = nullptr, *cxi = nullptr;
   int *crow = nullptr, *cel = nullptr;
   unsigned char *cshared = nullptr, *nmca = nullptr, *ekind = nullptr;
+  mfb::SingGeom* sgeo = nullptr;   // of the singular pairs, in list order
   std::vector<int> h_crow, h_cel;
   std::vector<double> h_xc;
   int n_mca = 0;
@@ -1750,7 +1920,7 @@ static void mesh_release(mfb_mesh_s* m) {
                 m->qcls, m->lcls, m->llists, m->judge_counters, m->judge_err,
                 m->xc, m->cxi, m->crow, m->cel, m->cshared, m->nmca,
                 m->ws[0], m->ws[1], m->ws[2], m->ws[3], m->ws[4], m->ws[5], m->ws[6], m->ws[7],
-                m->tiles.d, m->ltiles.d, m->d_promo, m->ekind};
+                m->tiles.d, m->ltiles.d, m->d_promo, m->ekind, m->sgeo};
   for (void* p : ps)
     if (p) (void)hipFree(p);
 }
@@ -1767,6 +1937,17 @@ static int mesh_ws(mfb_mesh_s* m, int slot, size_t bytes, P** out) {
     m->ws_cap[slot] = bytes;
   }
   *out = reinterpret_cast<P*>(m->ws[slot]);
+  return MFB_OK;
+}
+
+// Geometry records of the singular pairs of the mesh's lists (null stream).
+static int make_sing_geom(mfb_mesh_t m) {
+  const long long n = m->cls_cnt[m->dm.n_ps + 1];
+  if (!n) return MFB_OK;
+  MFB_HIP(hipMalloc((void**)&m->sgeo, sizeof(SingGeom) * (size_t)n));
+  hipLaunchKernelGGL(k_sing_geom, dim3((unsigned)n), dim3(kWave), 0, 0, m->dm, m->d_qsp_li,
+                     m->lists + m->cls_off[m->dm.n_ps + 1], m->sgeo);
+  MFB_HIP(hipGetLastError());
   return MFB_OK;
 }
 
@@ -1934,8 +2115,7 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
   for (long long q = 0; q < 9LL * ne; q++) MFB_ARG(conn[q] >= 0 && conn[q] < nn, "connectivity out of range");
   for (long long q = 0; q < 3LL * nn; q++)
     MFB_ARG(ctype[q] == 0 || ctype[q] == 1 || ctype[q] == 10, "ctype must be 0, 1 or 10");
-  int rc = upload_gl_tables();
-  if (rc == MFB_OK) rc = upload_polar_table();
+  int rc = upload_tables();
   if (rc) return rc;
 
   // node -> (element, local node) incidences, in element order
@@ -2116,6 +2296,7 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
       (void)hipFree(counts);
       if (rc) return fail(rc);
     }
+    TRY(make_sing_geom(m));
     // decision checksum (host) and regular-rule quadrature points
     std::vector<unsigned char> hcls((size_t)ncp * ne);
     TRYH(hipMemcpy(hcls.data(), m->cls, hcls.size(), hipMemcpyDeviceToHost));
@@ -2288,9 +2469,9 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
                        m->counters, m->err, (T*)nullptr, cls_off[d.n_ps], VecOut<T>{});
   if (events) MFB_HIP(hipEventRecord(m->ev[3], s));
   if (cls_cnt[d.n_ps + 1])
-    hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]), dim3(kWave), 0, s, d,
-                       m->d_qsp_li, kpp, lists + cls_off[d.n_ps + 1], (int)cls_cnt[d.n_ps + 1], A,
-                       lda, b, m->counters, (T*)nullptr, cls_off[d.n_ps + 1], VecOut<T>{});
+    hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]),
+                       dim3(kSingWaves * kWave), 0, s, d, kpp, lists + cls_off[d.n_ps + 1], m->sgeo,
+                       A, lda, b, m->counters, (T*)nullptr, 0LL, VecOut<T>{});
   if (events) MFB_HIP(hipEventRecord(m->ev[4], s));
   hipLaunchKernelGGL(k_freeterm<T>, dim3((d.nn + 127) / 128), dim3(128), 0, s, d, nu, A, lda, b,
                      m->err);
@@ -2370,10 +2551,9 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
     }
     MFB_HIP(hipEventRecord(m->ev[3], s));
     if (cls_cnt[d.n_ps + 1]) {
-      hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]), dim3(kWave), 0, s, d,
-                         m->d_qsp_li, m->d_kp, lists + cls_off[d.n_ps + 1],
-                         (int)cls_cnt[d.n_ps + 1], A, lda, b, m->counters, blocks,
-                         cls_off[d.n_ps + 1], vec);
+      hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]),
+                         dim3(kSingWaves * kWave), 0, s, d, m->d_kp, lists + cls_off[d.n_ps + 1],
+                         m->sgeo, A, lda, b, m->counters, blocks, cls_off[d.n_ps + 1], vec);
     }
     MFB_HIP(hipEventRecord(m->ev[4], s));
     MFB_HIP(hipEventRecord(m->ev[5], s));
@@ -3184,6 +3364,8 @@ static int pair_blocks(int npairs, const double* X, const double* xc, double qsi
     set_error("pair_blocks: %s", hipGetErrorString(he));
     return done(MFB_ERR_HIP);
   }
+  rc = make_sing_geom(m);
+  if (rc) return done(rc);
   rc = harmonic ? assemble<true>(m, kp, 0.0, nullptr, 0, nullptr, nullptr, dblk)
                 : assemble<false>(m, kp, 0.0, nullptr, 0, nullptr, nullptr, dblk);
   if (rc == MFB_OK) {
