@@ -64,18 +64,12 @@ __device__ double g_polar_pts[9][kPolarMax][3];
 __constant__ int c_polar_np[9];
 
 constexpr int kWave = 64;
-// adaptive subdivision: leaves integrated per batch, and the walk's stack (4 entries pushed per
-// level: at most 3 ns_max + 1 live entries, so ns_max <= kMaxNs)
-constexpr int kMaxLeaves = 128;
-constexpr int kStack = 64;
+// deepest adaptive subdivision
 constexpr int kMaxNs = 20;
 // largest precalculated rule: g^2 points x 360 B of kernel values and weights (harmonic) within
 // the 160 KB of LDS a gfx950 workgroup may hold
 constexpr int kMaxPrecalGln = 21;
 constexpr size_t kMaxLds = 160 * 1024;
-// quadrature points staged in LDS per pass by the adaptive and singular kernels: one per lane
-// (their LDS stays under 40 KB)
-constexpr int kChunk = 64;
 constexpr int kMaxIncid = 24;
 
 // Collocation points: the reference's nodal SBIE puts one point on every node; a node on the open
@@ -880,234 +874,6 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2
   else tile_body<H, kNeedH | kNeedG>(m, *kpp, list, tile, e, A, lda, b);
 }
 
-// Interior-displacement contribution of one pair held as the per-lane outputs o = lane + 64 t
-// (o = kind 81 + c 9 + n, before the kernel constants) of the adaptive and singular kernels.
-template <typename T>
-__device__ void vec_reduce(const DevMesh& m, const KernelParams& kp, int e, int cp, const T* acc,
-                           const VecOut<T>& vec, int lane) {
-  __shared__ T red[3];
-  if (lane < 3) red[lane] = zero_of(T());
-  __syncthreads();
-  T part[3] = {zero_of(T()), zero_of(T()), zero_of(T())};
-  for (int t = 0; t < 3; t++) {
-    const int o = lane + kWave * t;
-    if (o >= 162) continue;
-    const int kind = o / 81, c = (o % 81) / 9, n = o % 9, il = c / 3, ik = c % 3;
-    const int sn = m.conn[9 * e + n];
-    if (kind == 0) part[il] = part[il] - scale_h(kp, acc[t]) * vec.u[3 * sn + ik];
-    else part[il] = part[il] + scale_g(kp, acc[t]) * vec.t[3 * sn + ik];
-  }
-  for (int il = 0; il < 3; il++) lds_add(&red[il], part[il]);
-  __syncthreads();
-  if (lane < 3) atomic_add(&vec.out[3 * cp + lane], red[lane]);
-}
-
-// Adaptive quasi-singular pairs: fbem_bem_staela3d_sbie_ext_adp (bem_staela3d.f90:973-1096,
-// bem_harela3d.f90:1050-1172) with ext_st leaves (:654-969, :702-1048).
-struct Leaf {
-  double xs[8];
-  double barxi[2];
-  double barr;
-  int gln;
-  int pad;
-};
-
-template <bool H>
-__global__ void __launch_bounds__(kWave) k_adaptive(DevMesh m, const QsiParams* __restrict__ qsp_p,
-                                                    const KernelParams* __restrict__ kpp,
-                                                    const int* list, int count,
-                                                    typename Val<H>::T* A, long long lda,
-                                                    typename Val<H>::T* b, long long* counters,
-                                                    int* err, typename Val<H>::T* blocks,
-                                                    long long blk_base,
-                                                    VecOut<typename Val<H>::T> vec) {
-  typedef typename Val<H>::T T;
-  const QsiParams& qsp = *qsp_p;
-  const KernelParams& kp = *kpp;
-  const int lane = threadIdx.x;
-  const int pid = list[blockIdx.x];
-  const int e = pid / m.ncp, cp = pid % m.ncp;
-  __shared__ Leaf leaves[kMaxLeaves];
-  __shared__ double stk[kStack][9];  // xs(8) + level
-  __shared__ int nleaves, sp_sh;
-  __shared__ bool ovf;
-  __shared__ T sfs[kChunk * 18];
-  __shared__ double sw[kChunk * 9];
-  double X[27], el[8];
-  load_X(m, e, X);
-  for (int c = 0; c < 8; c++) el[c] = m.elem[8 * e + c];
-  const double xi_c[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
-  const int gln_far = (int)el[5];
-  if (lane == 0) {
-    const double root[8] = {-1, -1, 1, -1, 1, 1, -1, 1};
-    for (int c = 0; c < 8; c++) stk[0][c] = root[c];
-    stk[0][8] = 1;
-    sp_sh = 1;
-    ovf = false;
-  }
-  const GLTables& G = gl();
-  // lane owns outputs o = lane + 64 t, o = kind*81 + c*9 + n
-  T acc[3] = {zero_of(T()), zero_of(T()), zero_of(T())};
-  long long npts = 0;
-  int nl_total = 0;
-  // The walk (lane 0) stops after kMaxLeaves leaves, all lanes integrate them, and the walk goes on
-  // from its stack: leaves are integrated in the recursion's order and their number is unbounded.
-  bool more = true;
-  while (more) {
-    __syncthreads();
-    if (lane == 0) {
-      int sp = sp_sh, nl = 0;
-      bool overflow = false;
-      while (sp > 0 && nl < kMaxLeaves) {
-        sp--;
-        double xs[8];
-        for (int c = 0; c < 8; c++) xs[c] = stk[sp][c];
-        int ks = (int)stk[sp][8];
-        double barxi[2], rmin, d;
-        if (ks == 1) {
-          nearest_q9(X, el[0], xi_c, barxi, &rmin, &d);
-        } else {
-          double Xs[27];
-          subdiv_q9(X, xs, Xs);
-          double cl = clen_q9(Xs, 1e-12);
-          nearest_q9(Xs, cl, xi_c, barxi, &rmin, &d);
-        }
-        int gln_near = qs_estimate(qsp, 1, 2, 5, d, barxi);
-        bool sub = false;
-        if (ks == m.ns_max) {
-          if (gln_near == 0) gln_near = 30;
-        } else if (gln_near == 0) {
-          sub = true;
-        }
-        if (sub) {
-          // the stack holds at most 3 ns_max + 1 entries (ns_max is bounded at mesh creation)
-          if (sp + 4 > kStack) { overflow = true; break; }
-          double c0 = 0.25 * (xs[0] + xs[2] + xs[4] + xs[6]), c1 = 0.25 * (xs[1] + xs[3] + xs[5] + xs[7]);
-          double m01[2] = {0.5 * (xs[0] + xs[2]), 0.5 * (xs[1] + xs[3])};
-          double m12[2] = {0.5 * (xs[2] + xs[4]), 0.5 * (xs[3] + xs[5])};
-          double m23[2] = {0.5 * (xs[4] + xs[6]), 0.5 * (xs[5] + xs[7])};
-          double m03[2] = {0.5 * (xs[0] + xs[6]), 0.5 * (xs[1] + xs[7])};
-          const double s1[8] = {xs[0], xs[1], m01[0], m01[1], c0, c1, m03[0], m03[1]};
-          const double s2[8] = {m01[0], m01[1], xs[2], xs[3], m12[0], m12[1], c0, c1};
-          const double s3[8] = {c0, c1, m12[0], m12[1], xs[4], xs[5], m23[0], m23[1]};
-          const double s4[8] = {m03[0], m03[1], c0, c1, m23[0], m23[1], xs[6], xs[7]};
-          // push in reverse so that sub-quad 1 is integrated first, as the recursion does
-          const double* sq[4] = {s4, s3, s2, s1};
-          for (int s = 0; s < 4; s++) {
-            for (int c = 0; c < 8; c++) stk[sp][c] = sq[s][c];
-            stk[sp][8] = ks + 1;
-            sp++;
-          }
-        } else {
-          Leaf& L = leaves[nl++];
-          for (int c = 0; c < 8; c++) L.xs[c] = xs[c];
-          L.barxi[0] = barxi[0];
-          L.barxi[1] = barxi[1];
-          L.barr = telles_barr(d);
-          L.gln = max(gln_near, gln_far);
-        }
-      }
-      if (overflow) {
-        atomicExch(err, MFB_ERR_LIMIT);
-        ovf = true;
-        sp = 0;
-        nl = 0;
-      }
-      sp_sh = sp;
-      nleaves = nl;
-    }
-    __syncthreads();
-    const int nl = nleaves;
-    more = sp_sh > 0;
-    nl_total += nl;
-    for (int l = 0; l < nl; l++) {
-      const Leaf L = leaves[l];
-      const int gln = L.gln, P = gln * gln;
-      double tp1[4], tp2[4];
-      telles11(L.barxi[0], L.barr, tp1);
-      telles11(L.barxi[1], L.barr, tp2);
-      npts += P;
-      for (int start = 0; start < P; start += kChunk) {
-        int p = start + lane;
-        if (lane < kChunk && p < P) {
-          int k1 = p / gln, k2 = p % gln;
-          double xp0, xp1, jt1, jt2;
-          telles_xj(tp1, G.x11[gln][k1], &xp0, &jt1);
-          telles_xj(tp2, G.x11[gln][k2], &xp1, &jt2);
-          double w1 = G.w11[gln][k1], w2 = G.w11[gln][k2];
-          // xip -> xi through the quad4 map of the sub-element
-          double gp[4] = {0.25 * (1.0 - xp0) * (1.0 - xp1), 0.25 * (1.0 + xp0) * (1.0 - xp1),
-                          0.25 * (1.0 + xp0) * (1.0 + xp1), 0.25 * (1.0 - xp0) * (1.0 + xp1)};
-          double b2 = 0.25 * xp1, b3 = 0.25, c2 = 0.25 * xp0;
-          double d1[4] = {b2 - b3, -(b2 - b3), b2 + b3, -(b2 + b3)};
-          double d2[4] = {c2 - b3, -c2 - b3, -(-c2 - b3), -(c2 - b3)};
-          double xi0 = 0, xi1 = 0, a0 = 0, a1 = 0, a2 = 0, a3 = 0;
-          for (int kk = 0; kk < 4; kk++) {
-            xi0 += gp[kk] * L.xs[2 * kk]; xi1 += gp[kk] * L.xs[2 * kk + 1];
-            a0 += d1[kk] * L.xs[2 * kk]; a1 += d1[kk] * L.xs[2 * kk + 1];
-            a2 += d2[kk] * L.xs[2 * kk]; a3 += d2[kk] * L.xs[2 * kk + 1];
-          }
-          double js = a0 * a3 - a1 * a2;
-          double x[3], T1[3], T2[3], N[3], n[3], ph[9];
-          q9_geom(X, xi0, xi1, x, T1, T2);
-          cross3(T1, T2, N);
-          double jg = sqrt(dot3(N, N));
-          for (int c = 0; c < 3; c++) n[c] = N[c] / jg;
-          double jw = jg * js * jt1 * jt2 * w1 * w2;
-          phi_q9(xi0, xi1, ph);
-          ext_kernel_row(kp, x, n, xi_c, &sfs[lane * 18]);
-          for (int c = 0; c < 9; c++) sw[lane * 9 + c] = ph[c] * jw;
-        }
-        __syncthreads();
-        int np = min(kChunk, P - start);
-        for (int t = 0; t < 3; t++) {
-          int o = lane + kWave * t;
-          if (o < 162) {
-            int kind = o / 81, c = (o % 81) / 9, n = o % 9;
-            for (int pp = 0; pp < np; pp++) acc[t] += sfs[pp * 18 + kind * 9 + c] * sw[pp * 9 + n];
-          }
-        }
-        __syncthreads();
-      }
-    }
-  }
-  const int nl = nl_total;
-  if (vec.out) {
-    vec_reduce(m, kp, e, cp, acc, vec, lane);
-  } else
-  // each lane scatters its outputs directly (single values)
-  for (int t = 0; t < 3; t++) {
-    int o = lane + kWave * t;
-    if (o < 162) {
-      int kind = o / 81, c = (o % 81) / 9, n = o % 9;
-      T v = kind ? scale_g(kp, acc[t]) : scale_h(kp, acc[t]);
-      int il = c / 3, ik = c % 3;
-      if (blocks) {
-        // a pair whose subdivision overflowed is marked (NaN) rather than given a wrong value
-        blocks[162LL * (blk_base + blockIdx.x) + 81 * kind + n + 9 * il + 27 * ik] =
-            ovf ? from_real<T>(__builtin_nan("")) : v;
-        continue;
-      }
-      int sn = m.conn[9 * e + n];
-      long long row = 3LL * m.crow[cp] + il, col = 3LL * sn + ik;
-      int ct = m.ctype[3 * sn + ik];
-      double cv = m.cval[3 * sn + ik];
-      if (kind == 0) {
-        if (ct == 0) atomic_add(&b[row], -(v * cv));
-        else atomic_add(&A[row + lda * col], v);
-      } else {
-        if (ct == 0) atomic_add(&A[row + lda * col], -v);
-        else if (ct == 1) atomic_add(&b[row], v * cv);
-        else atomic_add(&b[row], v * (cv * m.nfn[3 * sn + ik]));
-      }
-    }
-  }
-  if (lane == 0) {
-    atomicAdd((unsigned long long*)&counters[0], (unsigned long long)npts);
-    atomicAdd((unsigned long long*)&counters[1], (unsigned long long)nl);
-  }
-}
-
 // Line integral eps_ijk e_k . t / r over one line3 edge, adaptive Telles + bisection
 // (fbem_bem_staela3d_sbie_int_li, bem_staela3d.f90:2245-2376): the 3 independent entries (1,2),
 // (1,3), (2,3), by the 16 lanes of a quarter wave.  The lanes walk the bisection together (every
@@ -1433,20 +1199,17 @@ __device__ inline void rows_reduce(double (*acc)[3], PairLds<W>& lds, int wave, 
   }
 }
 
-// Output of one pair: value(kind, l, k, n) -> h (0) or g (1) with the kernel constants.  Threads
-// t < 81 take (n, l, k) each: scatter into A and b (scatter of
-// src/assemble_bem_{staela,harela}_equation.f90), the pair's blocks, or the displacement of its point.
+// Output of one pair: value(kind, l, k, n) -> h (0) or g (1) with the kernel constants.  Items
+// t < 81 are (n, l, k) each: scatter into A and b (scatter of
+// src/assemble_bem_{staela,harela}_equation.f90), the pair's blocks, or the displacement of its point
+// (summed over the calling wave's items).
 template <bool H, int KIND, class Value>
 __device__ inline void pair_output(const DevMesh& m, int e, int cp, int t,
                                    typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
                                    typename Val<H>::T* block, const VecOut<typename Val<H>::T>& vec,
                                    Value&& value) {
   typedef typename Val<H>::T T;
-  __shared__ T red[3];
-  if (vec.out) {
-    if (t < 3) red[t] = zero_of(T());
-    __syncthreads();
-  }
+  T part = zero_of(T());
   if (t < 81) {
     const int il = t % 3, n = (t / 3) % 9, ik = t / 27;
     const int sn = m.conn[9 * e + n];
@@ -1456,7 +1219,7 @@ __device__ inline void pair_output(const DevMesh& m, int e, int cp, int t,
       block[o] = value(0, il, ik, n);
       block[81 + o] = value(1, il, ik, n);
     } else if (vec.out) {
-      lds_add(&red[il], value(1, il, ik, n) * vec.t[col] - value(0, il, ik, n) * vec.u[col]);
+      part = value(1, il, ik, n) * vec.t[col] - value(0, il, ik, n) * vec.u[col];
     } else {
       const long long row = 3LL * m.crow[cp] + il;
       const int ct = m.ctype[col];
@@ -1469,8 +1232,11 @@ __device__ inline void pair_output(const DevMesh& m, int e, int cp, int t,
     }
   }
   if (vec.out) {
-    __syncthreads();
-    if (t < 3) atomic_add(&vec.out[3 * cp + t], red[t]);
+    for (int il = 0; il < 3; il++) {
+      T q = t < 81 && t % 3 == il ? part : zero_of(T());
+      for (int mask = 1; mask < kWave; mask *= 2) q = lane_xor_add(q, mask);
+      if (t % kWave == 0 && t < 81) atomic_add(&vec.out[3 * cp + il], q);
+    }
   }
 }
 
@@ -1573,6 +1339,277 @@ __global__ void __launch_bounds__(kSingWaves* kWave) __attribute__((amdgpu_waves
     singular_body<H, kNeedG>(m, kp, e, cp, li, lds, A, lda, b, counters, block, vec);
   else
     singular_body<H, kNeedH | kNeedG>(m, kp, e, cp, li, lds, A, lda, b, counters, block, vec);
+}
+
+// Adaptive quasi-singular pairs: fbem_bem_staela3d_sbie_ext_adp (bem_staela3d.f90:973-1096,
+// bem_harela3d.f90:1050-1172) with ext_st leaves (:654-969, :702-1048).
+//
+// Root of a pair's subdivision tree: nearest point and order of the whole element, gln = 0 where it
+// is to be subdivided.  96 % of the pairs are a single leaf: the search, a serial chain of double-
+// double Newton steps, is taken by four lanes per pair in a kernel of its own, 16 pairs a wave, when
+// the lists are made (a wave of the integration ran it in one lane).
+struct AdaptGeom {
+  double barxi[2], d;
+  int gln, pad;
+};
+
+// order of the sub-element (nodes X, size cl) at tree level ks, 0: subdivide
+__device__ inline int leaf_order(const QsiParams& qsp, const double* X, double cl,
+                                 const double* x_i, int sub, int ks, int ns_max, double* barxi,
+                                 double* d) {
+  double rmin;
+  nearest_q9_team(X, cl, x_i, sub, barxi, &rmin, d);
+  const int gln = qs_estimate(qsp, 1, 2, 5, *d, barxi);
+  return gln == 0 && ks == ns_max ? 30 : gln;
+}
+
+// Records of `count` listed pairs in one buffer; behind them the number of pairs to be subdivided and
+// their list positions.
+__host__ __device__ inline size_t adapt_geom_bytes(size_t count) {
+  return count * (sizeof(AdaptGeom) + sizeof(int)) + 4 * sizeof(int);
+}
+__host__ __device__ inline int* adapt_tree(AdaptGeom* geo, size_t count) { return (int*)(geo + count); }
+
+__global__ void __launch_bounds__(kWave) k_adapt_geom(DevMesh m, const QsiParams* __restrict__ qsp,
+                                                      const int* __restrict__ list, int count,
+                                                      AdaptGeom* geo) {
+  const int q = blockIdx.x * 16 + (threadIdx.x >> 2), sub = threadIdx.x & 3;
+  const int pid = list[min(q, count - 1)], e = pid / m.ncp, cp = pid % m.ncp;
+  double X[27], barxi[2], d;
+  load_X(m, e, X);
+  const double x_i[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
+  const int gln = leaf_order(*qsp, X, m.elem[8 * e], x_i, sub, 1, m.ns_max, barxi, &d);
+  if (q < count && sub == 0) {
+    AdaptGeom& g = geo[q];
+    g.barxi[0] = barxi[0];
+    g.barxi[1] = barxi[1];
+    g.d = d;
+    g.gln = gln;
+    g.pad = 0;
+    if (gln == 0) {
+      int* tree = adapt_tree(geo, count);
+      tree[4 + atomicAdd(tree, 1)] = q;
+    }
+  }
+}
+
+// A leaf: the square of centre c and half width h, the nearest point in its own coordinates.
+struct Leaf {
+  double c[2], h, barxi[2], d;
+  int gln, pad;
+};
+constexpr int kLeaves = 32, kWalkWidth = 8;
+// The walk takes the kWalkWidth deepest sub-elements at a time, so at most 3 kWalkWidth wait per level
+// and 4 kWalkWidth on the last.
+constexpr int kWalkStack = 3 * kWalkWidth * kMaxNs + 4 * kWalkWidth;
+struct WalkLds {
+  unsigned long long stk[kWalkStack];   // level << 48 | ix << 24 | iy of the 2^(level-1) grid
+  Leaf leaf[kLeaves];
+};
+
+// One step of the walk: the deepest sub-elements of the stack (a team of four lanes each) become
+// leaves or are replaced by their four parts.  sp, nl: entries on the stack, leaves.
+__device__ __attribute__((noinline)) void walk_step(const QsiParams& qsp, const double* X,
+                                                    const double* x_i, int ns_max, int gln_far,
+                                                    WalkLds& w, int& sp, int& nl) {
+  const int lane = threadIdx.x % kWave, team = lane >> 2, sub = lane & 3;
+  const int n = min(sp, kWalkWidth);
+  const unsigned long long node = w.stk[sp - 1 - min(team, n - 1)];
+  const int ks = (int)(node >> 48), ix = (int)(node >> 24) & 0xffffff, iy = (int)node & 0xffffff;
+  const double width = 2.0 / (double)(1 << (ks - 1));
+  const double a0 = -1.0 + width * ix, b0 = -1.0 + width * iy, a1 = a0 + width, b1 = b0 + width;
+  const double xs[8] = {a0, b0, a1, b0, a1, b1, a0, b1};
+  double Xs[27], barxi[2], d;
+  subdiv_q9(X, xs, Xs);
+  const double cl = clen_q9_team(Xs, 1e-12, sub);
+  const int gln = leaf_order(qsp, Xs, cl, x_i, sub, ks, ns_max, barxi, &d);
+  const bool mine = team < n && sub == 0;
+  const unsigned long long split = __ballot(mine && gln == 0), leaf = __ballot(mine && gln != 0);
+  const unsigned long long below = (1ull << lane) - 1ull;
+  wave_lds_fence();   // the step's stack entries are read
+  if (mine && gln == 0) {
+    unsigned long long* t = w.stk + (sp - n) + 4 * __popcll(split & below);
+    const unsigned long long up = (unsigned long long)(ks + 1) << 48;
+    for (int c = 0; c < 4; c++)
+      t[c] = up | (unsigned long long)(2 * ix + (c == 1 || c == 2)) << 24 |
+             (unsigned long long)(2 * iy + (c >= 2));
+  } else if (mine) {
+    Leaf& l = w.leaf[nl + __popcll(leaf & below)];
+    l.c[0] = 0.5 * (a0 + a1);
+    l.c[1] = 0.5 * (b0 + b1);
+    l.h = 0.5 * width;
+    l.barxi[0] = barxi[0];
+    l.barxi[1] = barxi[1];
+    l.d = d;
+    l.gln = max(gln, gln_far);
+  }
+  wave_lds_fence();
+  sp += 4 * __popcll(split) - n;
+  nl += __popcll(leaf);
+}
+
+template <bool H, int KIND>
+struct ExtRows {
+  static constexpr int RC = H ? 2 : 1;
+  static constexpr int NH = KIND & kNeedH ? 9 * RC : 0, NG = KIND & kNeedG ? 6 * RC : 0;
+  static constexpr int NR = (NH + NG + 3) / 4 * 4;
+};
+__device__ inline void put_row(double* v, int c, double x) { v[c] = x; }
+__device__ inline void put_row(double* v, int c, zd x) {
+  v[2 * c] = x.re;
+  v[2 * c + 1] = x.im;
+}
+
+// sums of one leaf: Telles rule of order gln on the square (c, h)
+template <bool H, int KIND>
+__device__ inline int leaf_sums(ConstKP kp, const double* X, const double* x_i, const double* c,
+                                double h, const double* barxi, double d, int gln,
+                                PairLds<1>& lds, int lane, double (*acc)[3]) {
+  typedef typename Val<H>::T T;
+  typedef ExtRows<H, KIND> R;
+  const GLTables& G = gl();
+  double tp1[4], tp2[4];
+  const double barr = telles_barr(d);
+  telles11(barxi[0], barr, tp1);
+  telles11(barxi[1], barr, tp2);
+  const int P = gln * gln;
+  for (int start = 0; start < P; start += kWave) {
+    const int p = min(start + lane, P - 1), k1 = p / gln, k2 = p % gln;
+    double xp0, xp1, jt1, jt2;
+    telles_xj(tp1, G.x11[gln][k1], &xp0, &jt1);
+    telles_xj(tp2, G.x11[gln][k2], &xp1, &jt2);
+    const double xi0 = c[0] + h * xp0, xi1 = c[1] + h * xp1;
+    double x[3], T1[3], T2[3], N[3], ph[9], v[R::NR];
+    q9_geom(X, xi0, xi1, x, T1, T2);
+    cross3(T1, T2, N);
+    const double jg = sqrt(dot3(N, N)), ij = 1.0 / jg;
+    const double n[3] = {N[0] * ij, N[1] * ij, N[2] * ij};
+    const double jw = jg * (h * h) * (jt1 * jt2) * (G.w11[gln][k1] * G.w11[gln][k2]);
+    phi_q9(xi0, xi1, ph);
+#pragma unroll
+    for (int r = R::NH + R::NG; r < R::NR; r++) v[r] = 0.0;
+    ext_point<(KIND & kNeedH) != 0, (KIND & kNeedG) != 0>(
+        kp, x, n, x_i, T(), [&](int q, T f) { put_row(v, q, f); },
+        [&](int q, T f) { put_row(v + R::NH, q, f); });
+    rows_mfma<R::NR, R::NR>(v, ph, start + lane < P ? jw : 0.0, nullptr, lds.f[0], lds.ph[0], lane,
+                            acc);
+  }
+  return P;
+}
+
+template <bool H, int KIND, bool TREE>
+__device__ inline void adaptive_body(const DevMesh& m, const QsiParams& qsp, ConstKP kp, int e,
+                                     int cp, const AdaptGeom& root, PairLds<1>& lds, WalkLds* walk,
+                                     typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
+                                     long long* counters, typename Val<H>::T* block,
+                                     const VecOut<typename Val<H>::T>& vec) {
+  typedef typename Val<H>::T T;
+  typedef ExtRows<H, KIND> R;
+  const int lane = threadIdx.x, gln_far = (int)m.elem[8 * e + 5];
+  double X[27];
+  load_X(m, e, X);
+  const double x_i[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
+  double acc[R::NR / 4][3];
+#pragma unroll
+  for (int g = 0; g < R::NR / 4; g++) acc[g][0] = acc[g][1] = acc[g][2] = 0.0;
+  int leaves = 1, npts = 0;
+  if (!TREE) {
+    const double c[2] = {0.0, 0.0};
+    npts = leaf_sums<H, KIND>(kp, X, x_i, c, 1.0, root.barxi, root.d, max(root.gln, gln_far), lds,
+                              lane, acc);
+  } else {
+    int sp = 4, nl = 0;
+    if (lane < 4)
+      walk->stk[lane] = 2ull << 48 | (unsigned long long)(lane == 1 || lane == 2) << 24 |
+                        (unsigned long long)(lane >= 2);
+    wave_lds_fence();
+    // leaves are integrated in batches; the walk goes on from its stack
+    for (leaves = 0;;) {
+      while (sp > 0 && nl + kWalkWidth <= kLeaves)
+        walk_step(qsp, X, x_i, m.ns_max, gln_far, *walk, sp, nl);
+      for (int l = 0; l < nl; l++) {
+        const Leaf& q = walk->leaf[l];
+        npts += leaf_sums<H, KIND>(kp, X, x_i, q.c, q.h, q.barxi, q.d,
+                                   __builtin_amdgcn_readfirstlane(q.gln), lds, lane, acc);
+      }
+      leaves += nl;
+      nl = 0;
+      if (sp == 0) break;
+      wave_lds_fence();
+    }
+  }
+  rows_reduce<R::NR, 1>(acc, lds, 0, lane);
+  const double(*S)[9] = lds.sum[0];
+  auto value = [&](int kind, int il, int ik, int n) {
+    const int c = kind ? R::NH + R::RC * kSym[3 * il + ik] : R::RC * (3 * il + ik);
+    if constexpr (H) {
+      const T v = mkz(S[c][n], S[c + 1][n]);
+      return kind ? mkz(kp->h.cte_u[0], kp->h.cte_u[1]) * v : mkz(kp->h.cte_t[0], kp->h.cte_t[1]) * v;
+    } else {
+      return S[c][n] * (kind ? kp->cteu1 : kp->ctet1);
+    }
+  };
+  pair_output<H, KIND>(m, e, cp, lane, A, lda, b, block, vec, value);
+  pair_output<H, KIND>(m, e, cp, lane + kWave, A, lda, b, block, vec, value);
+  if (lane == 0) {
+    atomicAdd((unsigned long long*)&counters[0], (unsigned long long)npts);
+    atomicAdd((unsigned long long*)&counters[1], (unsigned long long)leaves);
+  }
+}
+
+template <bool H, bool TREE>
+__device__ inline void adaptive_pair(const DevMesh& m, const QsiParams* __restrict__ qsp, ConstKP kp,
+                                     const int* __restrict__ list,
+                                     const AdaptGeom* __restrict__ geo, int q, PairLds<1>& lds,
+                                     WalkLds* walk, typename Val<H>::T* A, long long lda,
+                                     typename Val<H>::T* b, long long* counters,
+                                     typename Val<H>::T* blocks, long long blk_base,
+                                     const VecOut<typename Val<H>::T>& vec) {
+  const int pid = list[q], e = pid / m.ncp, cp = pid % m.ncp;
+  typename Val<H>::T* block = blocks ? blocks + 162LL * (blk_base + q) : nullptr;
+  const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e];
+  if (kind == kNeedH)
+    adaptive_body<H, kNeedH, TREE>(m, *qsp, kp, e, cp, geo[q], lds, walk, A, lda, b, counters,
+                                   block, vec);
+  else if (kind == kNeedG)
+    adaptive_body<H, kNeedG, TREE>(m, *qsp, kp, e, cp, geo[q], lds, walk, A, lda, b, counters,
+                                   block, vec);
+  else
+    adaptive_body<H, kNeedH | kNeedG, TREE>(m, *qsp, kp, e, cp, geo[q], lds, walk, A, lda, b,
+                                            counters, block, vec);
+}
+
+// One wave per pair that is a single leaf (the others return).
+template <bool H>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    k_adaptive(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
+               const AdaptGeom* __restrict__ geo, typename Val<H>::T* A, long long lda,
+               typename Val<H>::T* b, long long* counters, typename Val<H>::T* blocks,
+               long long blk_base, VecOut<typename Val<H>::T> vec) {
+  __shared__ PairLds<1> lds;
+  const int q = blockIdx.x;
+  if (geo[q].gln == 0) return;
+  adaptive_pair<H, false>(m, nullptr, (ConstKP)kpp, list, geo, q, lds, nullptr, A, lda, b, counters,
+                          blocks, blk_base, vec);
+}
+
+// One wave per pair that is subdivided, in turn over tree[4 .. 4 + tree[0]).
+template <bool H>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    k_adaptive_tree(DevMesh m, const QsiParams* __restrict__ qsp,
+                    const KernelParams* __restrict__ kpp, const int* __restrict__ list,
+                    const AdaptGeom* __restrict__ geo, const int* __restrict__ tree,
+                    typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
+                    long long* counters, typename Val<H>::T* blocks, long long blk_base,
+                    VecOut<typename Val<H>::T> vec) {
+  __shared__ PairLds<1> lds;
+  __shared__ WalkLds walk;
+  const int n = tree[0];
+  for (int t = blockIdx.x; t < n; t += gridDim.x) {
+    __syncthreads();
+    adaptive_pair<H, true>(m, qsp, (ConstKP)kpp, list, geo, tree[4 + t], lds, &walk, A, lda, b,
+                           counters, blocks, blk_base, vec);
+  }
 }
 
 // err[q * nr + r] = max(max|h - h_ref| / max|h_ref|, max|g - g_ref| / max|g_ref|) of pair q
@@ -1870,8 +1907,8 @@ struct mfb_mesh_s {
   int* judge_err = nullptr;
   // grow-only device workspaces of the per-assembly steps (lists, learned classes, judge): a
   // repeated assembly allocates and frees nothing
-  void* ws[8] = {};
-  size_t ws_cap[8] = {};
+  void* ws[10] = {};
+  size_t ws_cap[10] = {};
   double *x = nullptr, *cval = nullptr, *elem = nullptr, *ps = nullptr, *nfn = nullptr;
   int *conn = nullptr, *ctype = nullptr, *inc_ptr = nullptr, *inc_e = nullptr, *inc_k = nullptr;
   unsigned char* cls = nullptr;
@@ -1880,7 +1917,9 @@ struct mfb_mesh_s {
   double *xc = nullptr, *cxi = nullptr;
   int *crow = nullptr, *cel = nullptr;
   unsigned char *cshared = nullptr, *nmca = nullptr, *ekind = nullptr;
-  mfb::SingGeom* sgeo = nullptr;   // of the singular pairs, in list order
+  mfb::SingGeom* sgeo = nullptr;   // of the singular and the adaptive pairs, in list order
+  mfb::AdaptGeom* ageo = nullptr;
+  int n_tree = 0;                  // adaptive pairs of `lists` that are subdivided
   std::vector<int> h_crow, h_cel;
   std::vector<double> h_xc;
   int n_mca = 0;
@@ -1920,12 +1959,13 @@ static void mesh_release(mfb_mesh_s* m) {
                 m->qcls, m->lcls, m->llists, m->judge_counters, m->judge_err,
                 m->xc, m->cxi, m->crow, m->cel, m->cshared, m->nmca,
                 m->ws[0], m->ws[1], m->ws[2], m->ws[3], m->ws[4], m->ws[5], m->ws[6], m->ws[7],
+                m->ws[8], m->ws[9], m->ageo,
                 m->tiles.d, m->ltiles.d, m->d_promo, m->ekind, m->sgeo};
   for (void* p : ps)
     if (p) (void)hipFree(p);
 }
 
-enum MeshWs { MW_OFF, MW_COUNTS, MW_REF, MW_BLK, MW_POS, MW_SAMPLE, MW_ERR, MW_PC };
+enum MeshWs { MW_OFF, MW_COUNTS, MW_REF, MW_BLK, MW_POS, MW_SAMPLE, MW_ERR, MW_PC, MW_AGEO, MW_JGEO };
 
 template <typename P>
 static int mesh_ws(mfb_mesh_s* m, int slot, size_t bytes, P** out) {
@@ -1940,14 +1980,46 @@ static int mesh_ws(mfb_mesh_s* m, int slot, size_t bytes, P** out) {
   return MFB_OK;
 }
 
-// Geometry records of the singular pairs of the mesh's lists (null stream).
-static int make_sing_geom(mfb_mesh_t m) {
-  const long long n = m->cls_cnt[m->dm.n_ps + 1];
-  if (!n) return MFB_OK;
-  MFB_HIP(hipMalloc((void**)&m->sgeo, sizeof(SingGeom) * (size_t)n));
-  hipLaunchKernelGGL(k_sing_geom, dim3((unsigned)n), dim3(kWave), 0, 0, m->dm, m->d_qsp_li,
-                     m->lists + m->cls_off[m->dm.n_ps + 1], m->sgeo);
+// The integration of `count` adaptive pairs; n_tree: how many of them are subdivided, -1 unknown on the
+// host.
+template <bool H>
+static void launch_adaptive(const DevMesh& d, const QsiParams* qsp, const KernelParams* kpp,
+                            const int* list, AdaptGeom* geo, int count, int n_tree,
+                            typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
+                            long long* counters, typename Val<H>::T* blocks, long long blk_base,
+                            VecOut<typename Val<H>::T> vec, hipStream_t s) {
+  if (!count) return;
+  if (n_tree)
+    hipLaunchKernelGGL(k_adaptive_tree<H>, dim3(std::min(n_tree < 0 ? count : n_tree, 2048)),
+                       dim3(kWave), 0, s, d, qsp, kpp, list, geo, adapt_tree(geo, count), A, lda, b,
+                       counters, blocks, blk_base, vec);
+  hipLaunchKernelGGL(k_adaptive<H>, dim3((unsigned)count), dim3(kWave), 0, s, d, kpp, list, geo, A,
+                     lda, b, counters, blocks, blk_base, vec);
+}
+
+// Records of `count` listed adaptive pairs at the tolerance of qsp into geo (adapt_geom_bytes).
+static void launch_adapt_geom(const DevMesh& d, const QsiParams* qsp, const int* list, int count,
+                              AdaptGeom* geo, hipStream_t s) {
+  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s, adapt_tree(geo, count), 4, 0);
+  hipLaunchKernelGGL(k_adapt_geom, dim3((unsigned)((count + 15) / 16)), dim3(kWave), 0, s, d, qsp,
+                     list, count, geo);
+}
+
+// Geometry records of the singular and the adaptive pairs of the mesh's lists (null stream).
+static int make_pair_geom(mfb_mesh_t m) {
+  const DevMesh& d = m->dm;
+  const long long ns = m->cls_cnt[d.n_ps + 1], na = m->cls_cnt[d.n_ps];
+  if (ns) {
+    MFB_HIP(hipMalloc((void**)&m->sgeo, sizeof(SingGeom) * (size_t)ns));
+    hipLaunchKernelGGL(k_sing_geom, dim3((unsigned)ns), dim3(kWave), 0, 0, d, m->d_qsp_li,
+                       m->lists + m->cls_off[d.n_ps + 1], m->sgeo);
+  }
+  if (na) {
+    MFB_HIP(hipMalloc((void**)&m->ageo, adapt_geom_bytes((size_t)na)));
+    launch_adapt_geom(d, m->d_qsp, m->lists + m->cls_off[d.n_ps], (int)na, m->ageo, 0);
+  }
   MFB_HIP(hipGetLastError());
+  if (na) MFB_HIP(hipMemcpy(&m->n_tree, adapt_tree(m->ageo, na), sizeof(int), hipMemcpyDeviceToHost));
   return MFB_OK;
 }
 
@@ -2296,7 +2368,7 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
       (void)hipFree(counts);
       if (rc) return fail(rc);
     }
-    TRY(make_sing_geom(m));
+    TRY(make_pair_geom(m));
     // decision checksum (host) and regular-rule quadrature points
     std::vector<unsigned char> hcls((size_t)ncp * ne);
     TRYH(hipMemcpy(hcls.data(), m->cls, hcls.size(), hipMemcpyDeviceToHost));
@@ -2415,8 +2487,17 @@ static int learned_lists(mfb_mesh_t m, double kw, hipStream_t s) {
     set_error("k_learned_map: %s", hipGetErrorString(he));
     return MFB_ERR_HIP;
   }
-  return build_lists(m, m->lcls, counts, m->llists, m->lcls_off, m->lcls_cnt, m->ltiles,
-                     m->l_regular_points, s);
+  rc = build_lists(m, m->lcls, counts, m->llists, m->lcls_off, m->lcls_cnt, m->ltiles,
+                   m->l_regular_points, s);
+  const long long na = rc ? 0 : m->lcls_cnt[d.n_ps];
+  if (na) {
+    AdaptGeom* geo = nullptr;
+    rc = mesh_ws(m, MW_AGEO, adapt_geom_bytes((size_t)na), &geo);
+    if (rc) return rc;
+    launch_adapt_geom(d, m->d_qsp, m->llists + m->lcls_off[d.n_ps], (int)na, geo, s);
+    MFB_HIP(hipGetLastError());
+  }
+  return rc;
 }
 
 // The kernels of one whole-boundary assembly into A, b (scatter mode) on stream s, reading the
@@ -2463,10 +2544,9 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
                        kpp, lists, ts.d + ts.off[k], A, lda, b);
   }
   if (events) MFB_HIP(hipEventRecord(m->ev[2], s));
-  if (cls_cnt[d.n_ps])
-    hipLaunchKernelGGL(k_adaptive<H>, dim3((unsigned)cls_cnt[d.n_ps]), dim3(kWave), 0, s, d,
-                       m->d_qsp, kpp, lists + cls_off[d.n_ps], (int)cls_cnt[d.n_ps], A, lda, b,
-                       m->counters, m->err, (T*)nullptr, cls_off[d.n_ps], VecOut<T>{});
+  launch_adaptive<H>(d, m->d_qsp, kpp, lists + cls_off[d.n_ps],
+                     learned ? (AdaptGeom*)m->ws[MW_AGEO] : m->ageo, (int)cls_cnt[d.n_ps],
+                     learned ? -1 : m->n_tree, A, lda, b, m->counters, nullptr, 0LL, VecOut<T>{}, s);
   if (events) MFB_HIP(hipEventRecord(m->ev[3], s));
   if (cls_cnt[d.n_ps + 1])
     hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]),
@@ -2544,11 +2624,9 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
                            m->d_kp, lists + o, (int)cnt, r, blocks, o, vec);
     }
     MFB_HIP(hipEventRecord(m->ev[2], s));
-    if (cls_cnt[d.n_ps]) {
-      hipLaunchKernelGGL(k_adaptive<H>, dim3((unsigned)cls_cnt[d.n_ps]), dim3(kWave), 0, s, d,
-                         m->d_qsp, m->d_kp, lists + cls_off[d.n_ps], (int)cls_cnt[d.n_ps], A, lda,
-                         b, m->counters, m->err, blocks, cls_off[d.n_ps], vec);
-    }
+    launch_adaptive<H>(d, m->d_qsp, m->d_kp, lists + cls_off[d.n_ps], m->ageo,
+                       (int)cls_cnt[d.n_ps], m->n_tree, A, lda, b, m->counters, blocks,
+                       cls_off[d.n_ps], vec, s);
     MFB_HIP(hipEventRecord(m->ev[3], s));
     if (cls_cnt[d.n_ps + 1]) {
       hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]),
@@ -2844,14 +2922,16 @@ static int rule_errors(mfb_mesh_t m, const KernelParams& kp, const int* dlist, i
   T *ref = nullptr, *blk = nullptr;
   int rc = mesh_ws(m, MW_REF, sizeof(T) * 162 * (size_t)np, &ref);
   if (!rc) rc = mesh_ws(m, MW_BLK, sizeof(T) * 162 * (size_t)np, &blk);
+  AdaptGeom* geo = nullptr;
+  if (!rc) rc = mesh_ws(m, MW_JGEO, adapt_geom_bytes((size_t)np), &geo);
   if (rc) return rc;
   hipError_t he = hipMemcpyAsync(m->d_kp, &kp, sizeof(KernelParams), hipMemcpyHostToDevice, s);
   if (he == hipSuccess) he = hipStreamSynchronize(s);
   if (he == hipSuccess) {
     hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, counters, errflag);
-    hipLaunchKernelGGL(k_adaptive<H>, dim3((unsigned)np), dim3(kWave), 0, s, d, d_qsp_ref, m->d_kp,
-                       dlist, np, (T*)nullptr, 0LL, (T*)nullptr, counters, errflag, ref, 0LL,
-                       VecOut<T>{});
+    launch_adapt_geom(d, d_qsp_ref, dlist, np, geo, s);
+    launch_adaptive<H>(d, d_qsp_ref, m->d_kp, dlist, geo, np, -1, nullptr, 0LL, nullptr, counters,
+                       ref, 0LL, VecOut<T>{}, s);
     for (int r = 0; r < d.n_ps; r++) {
       const int P = d.ps_gln[r] * d.ps_gln[r], B = P >= kWave ? 1 : kWave / P;
       hipLaunchKernelGGL((k_regular<H, kBlocks>), dim3((unsigned)((np + B - 1) / B)), dim3(kWave),
@@ -3364,7 +3444,7 @@ static int pair_blocks(int npairs, const double* X, const double* xc, double qsi
     set_error("pair_blocks: %s", hipGetErrorString(he));
     return done(MFB_ERR_HIP);
   }
-  rc = make_sing_geom(m);
+  rc = make_pair_geom(m);
   if (rc) return done(rc);
   rc = harmonic ? assemble<true>(m, kp, 0.0, nullptr, 0, nullptr, nullptr, dblk)
                 : assemble<false>(m, kp, 0.0, nullptr, 0, nullptr, nullptr, dblk);

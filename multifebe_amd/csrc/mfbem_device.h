@@ -481,16 +481,12 @@ __device__ inline void nearest_l3_local(const double* X, double cl, const double
   *d = *rmin / cl;
 }
 
-// Newton minimisation of |x(xi) - x_i| (geometry.f90:5289-5408).  The reference carries the
-// iteration in real128; here the element is first recentred on x_i (Y_k = X_k - x_i, exact to one
-// rounding of the small differences) so that FP64 reaches the same 1e-14 convergence test even on
-// small sub-elements far from the coordinate origin.
-__device__ inline int minimize_q9(const double* X, const double* x_i, double* barxi,
-                                  double* rmin) {
-  double Y[27];
-  for (int k = 0; k < 9; k++)
-    for (int c = 0; c < 3; c++) Y[3 * k + c] = X[3 * k + c] - x_i[c];
-  const double zero[3] = {0.0, 0.0, 0.0};
+// Newton minimisation of |x(xi) - x_i| (geometry.f90:5289-5408) from barxi; Y: the element's nodes
+// less x_i.  The reference carries the iteration in real128; here the element is first recentred on
+// x_i (Y_k = X_k - x_i, exact to one rounding of the small differences) so that FP64 reaches the same
+// 1e-14 convergence test even on small sub-elements far from the coordinate origin.  Returns 1 when
+// it converged.
+__device__ inline int newton_q9(const double* Y, double* barxi) {
   double prev[2];
   if (!check_xi_q(barxi)) { prev[0] = 0; prev[1] = 0; }
   else { prev[0] = barxi[0]; prev[1] = barxi[1]; }
@@ -524,6 +520,17 @@ __device__ inline int minimize_q9(const double* X, const double* x_i, double* ba
     prev[0] = n0;
     prev[1] = n1;
   }
+  return info;
+}
+
+// the minimiser, on the element's edges where the interior search leaves the element
+__device__ inline int minimize_q9(const double* X, const double* x_i, double* barxi,
+                                  double* rmin) {
+  double Y[27];
+  for (int k = 0; k < 9; k++)
+    for (int c = 0; c < 3; c++) Y[3 * k + c] = X[3 * k + c] - x_i[c];
+  const double zero[3] = {0.0, 0.0, 0.0};
+  const int info = newton_q9(Y, barxi);
   if (info == 1) {
     if (!check_xi_q(barxi)) {
       double best_r = 0, best_x = 0;
@@ -572,6 +579,74 @@ __device__ inline void nearest_q9(const double* X, double cl, const double* x_i,
     if (minimize_q9(X, x_i, barxi, rmin) != 1) sample_q9(X, x_i, barxi, rmin);
     *d = *rmin / cl;
   }
+}
+
+// nearest_q9 by a team of four lanes (lane bits 0, 1 = sub) that hold the same arguments and return the
+// same results, identical to nearest_q9's: every lane runs the interior search, each one edge of the
+// search along the edges.
+__device__ inline void nearest_q9_team(const double* X, double cl, const double* x_i, int sub,
+                                       double* barxi, double* rmin, double* d) {
+  double Y[27];
+  for (int k = 0; k < 9; k++)
+    for (int c = 0; c < 3; c++) Y[3 * k + c] = X[3 * k + c] - x_i[c];
+  const double zero[3] = {0.0, 0.0, 0.0};
+  int node = 0;
+  *rmin = sqrt(dot3(Y, Y));
+  for (int k = 1; k < 9; k++) {
+    const double t = sqrt(dot3(Y + 3 * k, Y + 3 * k));
+    if (t < *rmin) { *rmin = t; node = k; }
+  }
+  barxi[0] = kXiQ9[node][0];
+  barxi[1] = kXiQ9[node][1];
+  *d = *rmin / cl;
+  if (*rmin == 0.0 || !(*d < 1.0)) return;
+  const int info = newton_q9(Y, barxi);
+  if (info != 1) {
+    sample_q9(X, x_i, barxi, rmin);
+  } else {
+    if (!check_xi_q(barxi)) {
+      double ye[9], bx, rr, dd;
+      for (int j = 0; j < 3; j++) {
+        const int n = kEdgeQ9[0][j];
+        for (int c = 0; c < 3; c++) {
+          double v = Y[3 * n + c];
+          for (int q = 1; q < 4; q++) v = sub == q ? Y[3 * kEdgeQ9[q][j] + c] : v;
+          ye[3 * j + c] = v;
+        }
+      }
+      nearest_l3(ye, length_l3(ye, 1e-12), zero, &bx, &rr, &dd);
+      int kb = sub;   // the smallest distance, the first edge of equal ones
+      for (int mask = 1; mask < 4; mask *= 2) {
+        const double r2 = __shfl_xor(rr, mask), b2 = __shfl_xor(bx, mask);
+        const int k2 = __shfl_xor(kb, mask);
+        if (r2 < rr || (r2 == rr && k2 < kb)) { rr = r2; bx = b2; kb = k2; }
+      }
+      double ph[3];
+      phi_l3(bx, ph);
+      barxi[0] = 0;
+      barxi[1] = 0;
+      for (int j = 0; j < 3; j++) {
+        barxi[0] += ph[j] * kXiQ9[kEdgeQ9[kb][j]][0];
+        barxi[1] += ph[j] * kXiQ9[kEdgeQ9[kb][j]][1];
+      }
+    }
+    *rmin = dist_q9(Y, zero, barxi);
+  }
+  *d = *rmin / cl;
+}
+
+// clen_q9 by such a team: one edge per lane
+__device__ inline double clen_q9_team(const double* X, double tol, int sub) {
+  double xe[9];
+  for (int j = 0; j < 3; j++)
+    for (int c = 0; c < 3; c++) {
+      double v = X[3 * kEdgeQ9[0][j] + c];
+      for (int q = 1; q < 4; q++) v = sub == q ? X[3 * kEdgeQ9[q][j] + c] : v;
+      xe[3 * j + c] = v;
+    }
+  double l = length_l3(xe, tol);
+  for (int mask = 1; mask < 4; mask *= 2) l = fmax(l, __shfl_xor(l, mask));
+  return l;
 }
 
 // fbem_obtain_element_subdivision_coordinates (geometry.f90:2591-2697), quad9 and line3
