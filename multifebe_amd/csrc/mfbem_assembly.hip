@@ -346,16 +346,14 @@ __global__ void k_node_normals(DevMesh m, double* nfn) {
 
 // Integration class of pair (i, e): the decision sequence of fbem_bem_staela3d_sbie_auto
 // (bem_staela3d.f90:549-587), which the harmonic version repeats (bem_harela3d.f90:1498-1536).
+// (all lanes of the wave call; the result of an inactive one is not used)
 __device__ int classify_pair(const DevMesh& m, const QsiParams& qsp, const double* X,
-                             const double* el, const double* x_i) {
+                             const double* el, const double* x_i, bool active) {
   double rr[3] = {el[2] - x_i[0], el[3] - x_i[1], el[4] - x_i[2]};
-  double rmin = sqrt(dot3(rr, rr)) - el[1], barxi[2] = {0, 0}, d;
-  if (rmin > 4.0 * el[1]) {
-    d = rmin / el[0];
-  } else {
-    nearest_q9(X, el[0], x_i, barxi, &rmin, &d);
-    if (d <= 1e-12) return m.n_ps + 1;
-  }
+  double rmin = sqrt(dot3(rr, rr)) - el[1], barxi[2] = {0, 0}, d = rmin / el[0];
+  const bool near = !(rmin > 4.0 * el[1]);
+  nearest_q9_wave<false>(active && near, X, el[0], x_i, barxi, &rmin, &d);
+  if (near && d <= 1e-12) return m.n_ps + 1;
   int gln_near = qs_estimate(qsp, 0, 2, 5, d, barxi);
   int gln = max((int)el[5], gln_near);
   int gmax = m.ps_gln[m.n_ps - 1];
@@ -370,11 +368,11 @@ __device__ int classify_pair(const DevMesh& m, const QsiParams& qsp, const doubl
 //   log10(d) / 2 with d as sbie_auto defines it (ball distance over cl for far pairs, nearest
 //   point distance over cl otherwise), log2(aspect), curvature, k cl / 4, max(|barxi_1|, |barxi_2|)
 __device__ void pair_features(const double* X, const double* el, const double* x_i, double kw,
-                              float* f) {
+                              bool active, float* f) {
   double rr[3] = {el[2] - x_i[0], el[3] - x_i[1], el[4] - x_i[2]};
-  double rmin = sqrt(dot3(rr, rr)) - el[1], barxi[2] = {0, 0}, d;
-  if (rmin > 4.0 * el[1]) d = rmin / el[0];
-  else nearest_q9(X, el[0], x_i, barxi, &rmin, &d);
+  double rmin = sqrt(dot3(rr, rr)) - el[1], barxi[2] = {0, 0}, d = rmin / el[0];
+  nearest_q9_wave<false>(active && !(rmin > 4.0 * el[1]), X, el[0], x_i, barxi, &rmin, &d);
+  if (!active) return;
   f[0] = (float)(0.5 * log10(fmax(d, 1e-12)));
   f[1] = (float)log2(el[6]);
   f[2] = (float)el[7];
@@ -382,25 +380,24 @@ __device__ void pair_features(const double* X, const double* el, const double* x
   f[4] = (float)fmax(fabs(barxi[0]), fabs(barxi[1]));
 }
 
-__global__ void k_pair_features(DevMesh m, const int* pairs, int np, double kw, float* feats) {
+__global__ void __launch_bounds__(256) k_pair_features(DevMesh m, const int* pairs, int np, double kw, float* feats) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= np) return;
-  const int pid = pairs[q], e = pid / m.ncp, cp = pid % m.ncp;
+  const int pid = pairs[min(q, np - 1)], e = pid / m.ncp, cp = pid % m.ncp;
   double X[27], el[8];
   load_X(m, e, X);
   for (int c = 0; c < 8; c++) el[c] = m.elem[8 * e + c];
-  pair_features(X, el, m.xc + 3 * cp, kw, feats + (long long)q * MFB_QNET_INPUTS);
+  pair_features(X, el, m.xc + 3 * cp, kw, q < np, feats + (long long)q * MFB_QNET_INPUTS);
 }
 
 // features of every pair (pair id = e * ncp + cp), k h left at 0 (set per assembly by k_set_kh)
-__global__ void k_all_features(DevMesh m, float* feats) {
-  const long long pid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (pid >= (long long)m.ne * m.ncp) return;
+__global__ void __launch_bounds__(256) k_all_features(DevMesh m, float* feats) {
+  const long long own = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long last = (long long)m.ne * m.ncp - 1, pid = own < last ? own : last;
   const int e = (int)(pid / m.ncp), cp = (int)(pid % m.ncp);
   double X[27], el[8];
   load_X(m, e, X);
   for (int c = 0; c < 8; c++) el[c] = m.elem[8 * e + c];
-  pair_features(X, el, m.xc + 3 * cp, 0.0, feats + pid * MFB_QNET_INPUTS);
+  pair_features(X, el, m.xc + 3 * cp, 0.0, own <= last, feats + pid * MFB_QNET_INPUTS);
 }
 
 __global__ void k_set_kh(DevMesh m, float* feats, double kw) {
@@ -453,8 +450,10 @@ __global__ void __launch_bounds__(256) k_classify(DevMesh m, const QsiParams* __
   double X[27], el[8];
   load_X(m, e, X);
   for (int c = 0; c < 8; c++) el[c] = m.elem[8 * e + c];
-  for (int cp = threadIdx.x; cp < m.ncp; cp += blockDim.x) {
-    int c = classify_pair(m, qsp, X, el, m.xc + 3 * cp);
+  for (int c0 = 0; c0 < m.ncp; c0 += blockDim.x) {
+    const int cp = c0 + threadIdx.x;
+    const int c = classify_pair(m, qsp, X, el, m.xc + 3 * min(cp, m.ncp - 1), cp < m.ncp);
+    if (cp >= m.ncp) continue;
     cls[(long long)e * m.ncp + cp] = (unsigned char)c;
     atomicAdd(&hist[c], 1);
   }
@@ -517,15 +516,15 @@ __global__ void k_fill_tiles(DevMesh m, const int* counts, const long long* offs
 }
 
 // classes of listed pairs only (a batch of independent pairs)
-__global__ void k_classify_listed(DevMesh m, const QsiParams* __restrict__ qsp_p, const int* pids,
+__global__ void __launch_bounds__(128) k_classify_listed(DevMesh m, const QsiParams* __restrict__ qsp_p, const int* pids,
                                   int np, unsigned char* cls) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= np) return;
-  const int pid = pids[q], e = pid / m.ncp, cp = pid % m.ncp;
+  const int pid = pids[min(q, np - 1)], e = pid / m.ncp, cp = pid % m.ncp;
   double X[27], el[8];
   load_X(m, e, X);
   for (int c = 0; c < 8; c++) el[c] = m.elem[8 * e + c];
-  cls[q] = (unsigned char)classify_pair(m, *qsp_p, X, el, m.xc + 3 * cp);
+  const int c = classify_pair(m, *qsp_p, X, el, m.xc + 3 * cp, q < np);
+  if (q < np) cls[q] = (unsigned char)c;
 }
 
 #pragma clang fp contract(fast)
@@ -1355,10 +1354,9 @@ struct AdaptGeom {
 
 // order of the sub-element (nodes X, size cl) at tree level ks, 0: subdivide
 __device__ inline int leaf_order(const QsiParams& qsp, const double* X, double cl,
-                                 const double* x_i, int sub, int ks, int ns_max, double* barxi,
-                                 double* d) {
+                                 const double* x_i, int ks, int ns_max, double* barxi, double* d) {
   double rmin;
-  nearest_q9_team(X, cl, x_i, sub, barxi, &rmin, d);
+  nearest_q9_wave<true>(true, X, cl, x_i, barxi, &rmin, d);
   const int gln = qs_estimate(qsp, 1, 2, 5, *d, barxi);
   return gln == 0 && ks == ns_max ? 30 : gln;
 }
@@ -1378,7 +1376,7 @@ __global__ void __launch_bounds__(kWave) k_adapt_geom(DevMesh m, const QsiParams
   double X[27], barxi[2], d;
   load_X(m, e, X);
   const double x_i[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
-  const int gln = leaf_order(*qsp, X, m.elem[8 * e], x_i, sub, 1, m.ns_max, barxi, &d);
+  const int gln = leaf_order(*qsp, X, m.elem[8 * e], x_i, 1, m.ns_max, barxi, &d);
   if (q < count && sub == 0) {
     AdaptGeom& g = geo[q];
     g.barxi[0] = barxi[0];
@@ -1422,7 +1420,7 @@ __device__ __attribute__((noinline)) void walk_step(const QsiParams& qsp, const 
   double Xs[27], barxi[2], d;
   subdiv_q9(X, xs, Xs);
   const double cl = clen_q9_team(Xs, 1e-12, sub);
-  const int gln = leaf_order(qsp, Xs, cl, x_i, sub, ks, ns_max, barxi, &d);
+  const int gln = leaf_order(qsp, Xs, cl, x_i, ks, ns_max, barxi, &d);
   const bool mine = team < n && sub == 0;
   const unsigned long long split = __ballot(mine && gln == 0), leaf = __ballot(mine && gln != 0);
   const unsigned long long below = (1ull << lane) - 1ull;

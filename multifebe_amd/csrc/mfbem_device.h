@@ -581,58 +581,135 @@ __device__ inline void nearest_q9(const double* X, double cl, const double* x_i,
   }
 }
 
-// nearest_q9 by a team of four lanes (lane bits 0, 1 = sub) that hold the same arguments and return the
-// same results, identical to nearest_q9's: every lane runs the interior search, each one edge of the
-// search along the edges.
-__device__ inline void nearest_q9_team(const double* X, double cl, const double* x_i, int sub,
-                                       double* barxi, double* rmin, double* d) {
-  double Y[27];
-  for (int k = 0; k < 9; k++)
-    for (int c = 0; c < 3; c++) Y[3 * k + c] = X[3 * k + c] - x_i[c];
-  const double zero[3] = {0.0, 0.0, 0.0};
-  int node = 0;
-  *rmin = sqrt(dot3(Y, Y));
-  for (int k = 1; k < 9; k++) {
-    const double t = sqrt(dot3(Y + 3 * k, Y + 3 * k));
-    if (t < *rmin) { *rmin = t; node = k; }
+__device__ inline double lane_value(double v, int lane) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+  return __hiloint2double(hi, lo);
+}
+
+// sample_q9 of the element X and point p of lane `src`, its samples shared by the wave's 64 lanes (all
+// of them call): the same samples, distances and choice -- the smallest distance, the first sample
+// of equal ones.
+__device__ inline void sample_q9_wave(const double* X, const double* p, int src, double* xi_out,
+                                      double* r_out) {
+  const int ns = 25, nr = 14, lane = threadIdx.x % 64;
+  double Xs[27], ps[3];
+  for (int c = 0; c < 27; c++) Xs[c] = lane_value(X[c], src);
+  for (int c = 0; c < 3; c++) ps[c] = lane_value(p[c], src);
+  double xm[2] = {0, 0}, rmin = 0, width = 2.0 / (double)(ns + 1), xo[2] = {0, 0};
+  for (int l = 0; l < 3; l++) {
+    const int side = l == 0 ? ns + 2 : nr;
+    auto at = [&](int q, double* xi) {
+      const int k[2] = {q / side, q % side};
+      for (int c = 0; c < 2; c++)
+        xi[c] = l == 0 ? -1.0 + 2.0 * (double)k[c] / (double)(ns + 1)
+                       : xo[c] + 2.0 * ((double)(k[c] + 1) - (double)(nr + 1) / 2.0) /
+                                     (double)(nr + 1) * width;
+    };
+    double best = __builtin_inf();
+    int arg = side * side;
+    for (int q = lane; q < side * side; q += 64) {
+      double xi[2];
+      at(q, xi);
+      if (l > 0 && !(xi[0] > -1.0 && xi[0] < 1.0 && xi[1] > -1.0 && xi[1] < 1.0)) continue;
+      const double r = dist_q9(Xs, ps, xi);
+      if (r < best) { best = r; arg = q; }
+    }
+    for (int mask = 1; mask < 64; mask *= 2) {
+      const double r2 = __shfl_xor(best, mask);
+      const int a2 = __shfl_xor(arg, mask);
+      if (r2 < best || (r2 == best && a2 < arg)) { best = r2; arg = a2; }
+    }
+    if (arg < side * side && (l == 0 || best < rmin)) {
+      rmin = best;
+      at(arg, xm);
+    }
+    if (l > 0) {
+      width = width / (double)(nr + 1);
+      width = 2.0 * width / (double)(nr + 1);
+    }
+    xo[0] = xm[0];
+    xo[1] = xm[1];
   }
-  barxi[0] = kXiQ9[node][0];
-  barxi[1] = kXiQ9[node][1];
-  *d = *rmin / cl;
-  if (*rmin == 0.0 || !(*d < 1.0)) return;
-  const int info = newton_q9(Y, barxi);
-  if (info != 1) {
-    sample_q9(X, x_i, barxi, rmin);
-  } else {
-    if (!check_xi_q(barxi)) {
-      double ye[9], bx, rr, dd;
-      for (int j = 0; j < 3; j++) {
-        const int n = kEdgeQ9[0][j];
-        for (int c = 0; c < 3; c++) {
-          double v = Y[3 * n + c];
-          for (int q = 1; q < 4; q++) v = sub == q ? Y[3 * kEdgeQ9[q][j] + c] : v;
-          ye[3 * j + c] = v;
+  xi_out[0] = xm[0];
+  xi_out[1] = xm[1];
+  *r_out = rmin;
+}
+
+// nearest_q9 for a whole wave at once (all lanes call, those with active = false take part in the
+// shared steps only): one pair per lane, or (TEAM) per team of four lanes (lane bits 0, 1) that hold
+// the same arguments, each searching one edge where the interior search leaves the element.  The
+// fallback sampling, 1,100 distances, is shared by the wave's lanes, pair after pair.  Same result
+// as nearest_q9.
+template <bool TEAM>
+__device__ inline void nearest_q9_wave(bool active, const double* X, double cl, const double* x_i,
+                                       double* barxi, double* rmin, double* d) {
+  const int sub = threadIdx.x & 3;
+  bool sample = false;
+  if (active) {
+    double Y[27];
+    for (int k = 0; k < 9; k++)
+      for (int c = 0; c < 3; c++) Y[3 * k + c] = X[3 * k + c] - x_i[c];
+    const double zero[3] = {0.0, 0.0, 0.0};
+    int node = 0;
+    *rmin = sqrt(dot3(Y, Y));
+    for (int k = 1; k < 9; k++) {
+      const double t = sqrt(dot3(Y + 3 * k, Y + 3 * k));
+      if (t < *rmin) { *rmin = t; node = k; }
+    }
+    barxi[0] = kXiQ9[node][0];
+    barxi[1] = kXiQ9[node][1];
+    *d = *rmin / cl;
+    if (*rmin != 0.0 && *d < 1.0) {
+      if (!TEAM) {
+        sample = minimize_q9(X, x_i, barxi, rmin) != 1;
+      } else {
+        sample = newton_q9(Y, barxi) != 1;
+        if (!sample) {
+          if (!check_xi_q(barxi)) {
+            double ye[9], bx, rr, dd;
+            for (int j = 0; j < 3; j++)
+              for (int c = 0; c < 3; c++) {
+                double v = Y[3 * kEdgeQ9[0][j] + c];
+                for (int q = 1; q < 4; q++) v = sub == q ? Y[3 * kEdgeQ9[q][j] + c] : v;
+                ye[3 * j + c] = v;
+              }
+            nearest_l3(ye, length_l3(ye, 1e-12), zero, &bx, &rr, &dd);
+            int kb = sub;   // the smallest distance, the first edge of equal ones
+            for (int mask = 1; mask < 4; mask *= 2) {
+              const double r2 = __shfl_xor(rr, mask), b2 = __shfl_xor(bx, mask);
+              const int k2 = __shfl_xor(kb, mask);
+              if (r2 < rr || (r2 == rr && k2 < kb)) { rr = r2; bx = b2; kb = k2; }
+            }
+            double ph[3];
+            phi_l3(bx, ph);
+            barxi[0] = 0;
+            barxi[1] = 0;
+            for (int j = 0; j < 3; j++) {
+              barxi[0] += ph[j] * kXiQ9[kEdgeQ9[kb][j]][0];
+              barxi[1] += ph[j] * kXiQ9[kEdgeQ9[kb][j]][1];
+            }
+          }
+          *rmin = dist_q9(Y, zero, barxi);
         }
       }
-      nearest_l3(ye, length_l3(ye, 1e-12), zero, &bx, &rr, &dd);
-      int kb = sub;   // the smallest distance, the first edge of equal ones
-      for (int mask = 1; mask < 4; mask *= 2) {
-        const double r2 = __shfl_xor(rr, mask), b2 = __shfl_xor(bx, mask);
-        const int k2 = __shfl_xor(kb, mask);
-        if (r2 < rr || (r2 == rr && k2 < kb)) { rr = r2; bx = b2; kb = k2; }
-      }
-      double ph[3];
-      phi_l3(bx, ph);
-      barxi[0] = 0;
-      barxi[1] = 0;
-      for (int j = 0; j < 3; j++) {
-        barxi[0] += ph[j] * kXiQ9[kEdgeQ9[kb][j]][0];
-        barxi[1] += ph[j] * kXiQ9[kEdgeQ9[kb][j]][1];
-      }
+      *d = *rmin / cl;
     }
-    *rmin = dist_q9(Y, zero, barxi);
   }
-  *d = *rmin / cl;
+  unsigned long long todo = __ballot(sample && (!TEAM || sub == 0));
+  while (todo) {
+    const int src = __ffsll(todo) - 1;
+    todo &= todo - 1;
+    double xi[2], r;
+    sample_q9_wave(X, x_i, src, xi, &r);
+    const int lane = threadIdx.x % 64;
+    if ((TEAM ? lane & ~3 : lane) == src) {
+      barxi[0] = xi[0];
+      barxi[1] = xi[1];
+      *rmin = r;
+      *d = r / cl;
+    }
+  }
 }
 
 // clen_q9 by such a team: one edge per lane
