@@ -1246,7 +1246,7 @@ template <bool H, int KIND>
 __device__ inline void singular_body(const DevMesh& m, ConstKP kp, int e, int cp,
                                      const SingGeom* __restrict__ geo, PairLds<kSingWaves>& lds,
                                      typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
-                                     long long* counters, typename Val<H>::T* block,
+                                     typename Val<H>::T* block,
                                      const VecOut<typename Val<H>::T>& vec) {
   typedef typename Val<H>::T T;
   typedef SingRows<H, KIND> R;
@@ -1314,7 +1314,6 @@ __device__ inline void singular_body(const DevMesh& m, ConstKP kp, int e, int cp
           return v * kp->ctet1;
         }
       });
-  if (threadIdx.x == 0) atomicAdd((unsigned long long*)&counters[0], (unsigned long long)P);
 }
 
 // One workgroup of four waves per pair, a wave 64 polar points at a time; per point the values are
@@ -1324,8 +1323,8 @@ template <bool H>
 __global__ void __launch_bounds__(kSingWaves* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
     k_singular(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
                const SingGeom* __restrict__ geo, typename Val<H>::T* A, long long lda,
-               typename Val<H>::T* b, long long* counters, typename Val<H>::T* blocks,
-               long long blk_base, VecOut<typename Val<H>::T> vec) {
+               typename Val<H>::T* b, typename Val<H>::T* blocks, long long blk_base,
+               VecOut<typename Val<H>::T> vec) {
   __shared__ PairLds<kSingWaves> lds;
   const int pid = list[blockIdx.x], e = pid / m.ncp, cp = pid % m.ncp;
   const SingGeom* li = geo + blockIdx.x;
@@ -1333,18 +1332,18 @@ __global__ void __launch_bounds__(kSingWaves* kWave) __attribute__((amdgpu_waves
   const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e];
   ConstKP kp = (ConstKP)kpp;
   if (kind == kNeedH)
-    singular_body<H, kNeedH>(m, kp, e, cp, li, lds, A, lda, b, counters, block, vec);
+    singular_body<H, kNeedH>(m, kp, e, cp, li, lds, A, lda, b, block, vec);
   else if (kind == kNeedG)
-    singular_body<H, kNeedG>(m, kp, e, cp, li, lds, A, lda, b, counters, block, vec);
+    singular_body<H, kNeedG>(m, kp, e, cp, li, lds, A, lda, b, block, vec);
   else
-    singular_body<H, kNeedH | kNeedG>(m, kp, e, cp, li, lds, A, lda, b, counters, block, vec);
+    singular_body<H, kNeedH | kNeedG>(m, kp, e, cp, li, lds, A, lda, b, block, vec);
 }
 
 // Adaptive quasi-singular pairs: fbem_bem_staela3d_sbie_ext_adp (bem_staela3d.f90:973-1096,
 // bem_harela3d.f90:1050-1172) with ext_st leaves (:654-969, :702-1048).
 //
-// Root of a pair's subdivision tree: nearest point and order of the whole element, gln = 0 where it
-// is to be subdivided.  96 % of the pairs are a single leaf: the search, a serial chain of double-
+// Root of a pair's subdivision tree: nearest point and rule order of the whole element, gln = 0 where
+// it is to be subdivided.  96 % of the pairs are a single leaf: the search, a serial chain of double-
 // double Newton steps, is taken by four lanes per pair in a kernel of its own, 16 pairs a wave, when
 // the lists are made (a wave of the integration ran it in one lane).
 struct AdaptGeom {
@@ -1382,7 +1381,7 @@ __global__ void __launch_bounds__(kWave) k_adapt_geom(DevMesh m, const QsiParams
     g.barxi[0] = barxi[0];
     g.barxi[1] = barxi[1];
     g.d = d;
-    g.gln = gln;
+    g.gln = gln ? max(gln, (int)m.elem[8 * e + 5]) : 0;
     g.pad = 0;
     if (gln == 0) {
       int* tree = adapt_tree(geo, count);
@@ -1444,6 +1443,27 @@ __device__ __attribute__((noinline)) void walk_step(const QsiParams& qsp, const 
   wave_lds_fence();
   sp += 4 * __popcll(split) - n;
   nl += __popcll(leaf);
+}
+
+// sums[0]: points of the singular and the single-leaf adaptive pairs, sums[1]: those leaves (one
+// workgroup; the integration kernels would have to add to one address per pair: at 24,000 pairs
+// that took longer than the integration)
+__global__ void __launch_bounds__(1024) k_count_points(const SingGeom* sg, long long ns,
+                                                       const AdaptGeom* ag, long long na,
+                                                       long long* sums) {
+  __shared__ unsigned long long t[2];
+  if (threadIdx.x < 2) t[threadIdx.x] = 0;
+  __syncthreads();
+  unsigned long long p = 0, l = 0;
+  for (long long q = threadIdx.x; q < ns; q += blockDim.x) p += sg[q].np;
+  for (long long q = threadIdx.x; q < na; q += blockDim.x) {
+    p += ag[q].gln * ag[q].gln;
+    l += ag[q].gln != 0;
+  }
+  atomicAdd(&t[0], p);
+  atomicAdd(&t[1], l);
+  __syncthreads();
+  if (threadIdx.x < 2) sums[threadIdx.x] = t[threadIdx.x];
 }
 
 template <bool H, int KIND>
@@ -1513,7 +1533,7 @@ __device__ inline void adaptive_body(const DevMesh& m, const QsiParams& qsp, Con
   int leaves = 1, npts = 0;
   if (!TREE) {
     const double c[2] = {0.0, 0.0};
-    npts = leaf_sums<H, KIND>(kp, X, x_i, c, 1.0, root.barxi, root.d, max(root.gln, gln_far), lds,
+    npts = leaf_sums<H, KIND>(kp, X, x_i, c, 1.0, root.barxi, root.d, root.gln, lds,
                               lane, acc);
   } else {
     int sp = 4, nl = 0;
@@ -1549,7 +1569,7 @@ __device__ inline void adaptive_body(const DevMesh& m, const QsiParams& qsp, Con
   };
   pair_output<H, KIND>(m, e, cp, lane, A, lda, b, block, vec, value);
   pair_output<H, KIND>(m, e, cp, lane + kWave, A, lda, b, block, vec, value);
-  if (lane == 0) {
+  if (TREE && lane == 0) {
     atomicAdd((unsigned long long*)&counters[0], (unsigned long long)npts);
     atomicAdd((unsigned long long*)&counters[1], (unsigned long long)leaves);
   }
@@ -1582,12 +1602,12 @@ template <bool H>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
     k_adaptive(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
                const AdaptGeom* __restrict__ geo, typename Val<H>::T* A, long long lda,
-               typename Val<H>::T* b, long long* counters, typename Val<H>::T* blocks,
-               long long blk_base, VecOut<typename Val<H>::T> vec) {
+               typename Val<H>::T* b, typename Val<H>::T* blocks, long long blk_base,
+               VecOut<typename Val<H>::T> vec) {
   __shared__ PairLds<1> lds;
   const int q = blockIdx.x;
   if (geo[q].gln == 0) return;
-  adaptive_pair<H, false>(m, nullptr, (ConstKP)kpp, list, geo, q, lds, nullptr, A, lda, b, counters,
+  adaptive_pair<H, false>(m, nullptr, (ConstKP)kpp, list, geo, q, lds, nullptr, A, lda, b, nullptr,
                           blocks, blk_base, vec);
 }
 
@@ -1926,7 +1946,8 @@ struct mfb_mesh_s {
   std::vector<int> h_conn, h_ctype, h_ps;
   double h_tol = 1e-6;
   int* err = nullptr;
-  long long* counters = nullptr;  // points, leaves of adaptive + singular kernels
+  long long* counters = nullptr;  // points, leaves of the subdivided pairs; of the others (stats)
+  bool integrated = false;        // an assembly has run
   mfb::QsiParams* d_qsp = nullptr;     // estimator tables and kernel constants live in device memory:
   mfb::QsiParams* d_qsp_li = nullptr;  // they are too large to travel as kernel arguments
   mfb::KernelParams* d_kp = nullptr;
@@ -1992,7 +2013,7 @@ static void launch_adaptive(const DevMesh& d, const QsiParams* qsp, const Kernel
                        dim3(kWave), 0, s, d, qsp, kpp, list, geo, adapt_tree(geo, count), A, lda, b,
                        counters, blocks, blk_base, vec);
   hipLaunchKernelGGL(k_adaptive<H>, dim3((unsigned)count), dim3(kWave), 0, s, d, kpp, list, geo, A,
-                     lda, b, counters, blocks, blk_base, vec);
+                     lda, b, blocks, blk_base, vec);
 }
 
 // Records of `count` listed adaptive pairs at the tolerance of qsp into geo (adapt_geom_bytes).
@@ -2300,7 +2321,7 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
   TRY(dalloc(&m->nmca, nn));
   TRY(dalloc(&m->ekind, ne));
   TRY(dalloc(&m->err, 1));
-  TRY(dalloc(&m->counters, 2));
+  TRY(dalloc(&m->counters, 4));
   TRY(dalloc(&m->d_qsp, 1));
   TRY(dalloc(&m->d_qsp_li, 1));
   TRY(dalloc(&m->d_kp, 1));
@@ -2427,19 +2448,24 @@ extern "C" int mfb_mesh_learned_classes(mfb_mesh_t m, unsigned char* classes) {
 
 extern "C" int mfb_mesh_stats(mfb_mesh_t m, mfb_assembly_stats* s) {
   MFB_ARG(m && s, "null argument");
-  long long c[2];
-  MFB_HIP(hipMemcpy(c, m->counters, sizeof c, hipMemcpyDeviceToHost));
   const int np = m->dm.n_ps;
   const bool L = m->learned_last;
   const std::vector<long long>& cnt = L ? m->lcls_cnt : m->cls_cnt;
+  long long c[4] = {0, 0, 0, 0};
+  if (m->integrated) {
+    hipLaunchKernelGGL(k_count_points, dim3(1), dim3(1024), 0, 0, m->sgeo, cnt[np + 1],
+                       L ? (const AdaptGeom*)m->ws[MW_AGEO] : m->ageo, cnt[np], m->counters + 2);
+    MFB_HIP(hipGetLastError());
+    MFB_HIP(hipMemcpy(c, m->counters, sizeof c, hipMemcpyDeviceToHost));
+  }
   const long long rp = L ? m->l_regular_points : m->regular_points;
   s->pairs = (long long)m->dm.ncp * m->dm.ne;
   s->singular = cnt[np + 1];
   s->adaptive = cnt[np];
   s->pre = 0;
   for (int r = 0; r < np; r++) s->pre += cnt[r];
-  s->points = rp + c[0];
-  s->leaves = c[1];
+  s->points = rp + c[0] + c[2];
+  s->leaves = c[1] + c[3];
   s->decisions = m->decisions;
   s->regular_points = rp;
   s->learned = L ? 1 : 0;
@@ -2549,7 +2575,7 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
   if (cls_cnt[d.n_ps + 1])
     hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]),
                        dim3(kSingWaves * kWave), 0, s, d, kpp, lists + cls_off[d.n_ps + 1], m->sgeo,
-                       A, lda, b, m->counters, (T*)nullptr, 0LL, VecOut<T>{});
+                       A, lda, b, (T*)nullptr, 0LL, VecOut<T>{});
   if (events) MFB_HIP(hipEventRecord(m->ev[4], s));
   hipLaunchKernelGGL(k_freeterm<T>, dim3((d.nn + 127) / 128), dim3(128), 0, s, d, nu, A, lda, b,
                      m->err);
@@ -2585,6 +2611,7 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
   // rule choice: the reference's estimator (classes fixed at mesh creation) or the network
   const bool learned = m->qnet && !blocks && !vmode;
   m->learned_last = learned;
+  m->integrated = true;
   if (learned) {
     int rc = learned_lists(m, kw, s);
     if (rc) return rc;
@@ -2629,7 +2656,7 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
     if (cls_cnt[d.n_ps + 1]) {
       hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]),
                          dim3(kSingWaves * kWave), 0, s, d, m->d_kp, lists + cls_off[d.n_ps + 1],
-                         m->sgeo, A, lda, b, m->counters, blocks, cls_off[d.n_ps + 1], vec);
+                         m->sgeo, A, lda, b, blocks, cls_off[d.n_ps + 1], vec);
     }
     MFB_HIP(hipEventRecord(m->ev[4], s));
     MFB_HIP(hipEventRecord(m->ev[5], s));
@@ -2739,6 +2766,7 @@ static int enqueue_batch(int njobs, const mfb_assembly_job* jobs, const KernelPa
     mfb_mesh_t m = jobs[q].mesh;
     if (std::find(seen.begin(), seen.end(), m) != seen.end()) continue;
     seen.push_back(m);
+    m->integrated = true;
     hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, m->counters, m->err);
   }
   for (int q = 0; q < njobs; q++) {
