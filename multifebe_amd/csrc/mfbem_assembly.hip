@@ -95,17 +95,24 @@ struct DevMesh {
   const int* inc_k;
   const double* xc;             // (ncp, 3) collocation point coordinates
   const int* crow;              // (ncp) node whose equations (rows 3 crow + l) the point adds to
-  const unsigned char* cshared; // (ncp) 1 when other points add to the same rows (MCA)
+  // (ncp) MCA points that share their node's rows with an earlier point have rows of their own, 3 cx ..
+  // 3 cx + 2 of an extra matrix of 3 nx rows (TileOut::X); -1: the rows of A
+  const int* cx;
+  const int* xnode;             // (nx) node of each extra point, ascending
+  int nx;
   const int* cel;               // (ncp) element holding an MCA point, -1 for a nodal point
   const double* cxi;            // (ncp, 2) local coordinates of an MCA point in cel
   const unsigned char* nmca;    // (nn) 1 for a node collocated by MCA points
   const unsigned char* ekind;   // (ne) kNeedH | kNeedG: kernels that element's conditions need
+  const int* enode;             // (ne, 9) node; ~node where an element of a lower colour holds it
+  const int2* emask;            // (ne) bit 3 n + k of node n, direction k: u prescribed; value not zero
 };
 
 // What an element contributes: with h (t*) to columns of unknown u and, where u is prescribed and not
 // zero, to b; with g (u*) to columns of unknown t and, where t is prescribed and not zero, to b.  A
 // traction-free element needs h alone, one held at zero g alone.
-constexpr int kNeedH = 1, kNeedG = 2;
+// kTwice: the element holds a node more than once (its columns then meet in one instruction).
+constexpr int kNeedH = 1, kNeedG = 2, kTwice = 4;
 
 // ------------------------------------------------------------------------------------------------
 // small helpers
@@ -499,10 +506,10 @@ __global__ void __launch_bounds__(256) k_fill_lists(DevMesh m, const unsigned ch
 
 // Tiles of the scatter kernel (k_regular_tile): element e's run of precalculated rule c is cut
 // into tiles of at most kTileP consecutive list entries; toff[e*(kMaxPrecalsets+2)+c] is the
-// run's first tile.  A tile is (first list entry, count | rule << 8).
+// run's first tile.  A tile is (first list entry, count, rule, element).
 constexpr int kTileP = 16;
 __global__ void k_fill_tiles(DevMesh m, const int* counts, const long long* offsets,
-                             const long long* toff, int2* tiles) {
+                             const long long* toff, int4* tiles) {
   constexpr int S = kMaxPrecalsets + 2;
   const int e = blockIdx.x;
   for (int c = 0; c < m.n_ps; c++) {
@@ -510,8 +517,7 @@ __global__ void k_fill_tiles(DevMesh m, const int* counts, const long long* offs
     const int cnt = counts[k];
     const long long o = offsets[k], t0 = toff[k];
     for (int j = threadIdx.x; j * kTileP < cnt; j += blockDim.x)
-      tiles[t0 + j] = make_int2((int)(o + (long long)j * kTileP),
-                                min(kTileP, cnt - j * kTileP) | (c << 8));
+      tiles[t0 + j] = make_int4((int)(o + (long long)j * kTileP), min(kTileP, cnt - j * kTileP), c, e);
   }
 }
 
@@ -538,7 +544,7 @@ __global__ void k_reset(long long* counters, int* err) {
 }
 
 template <typename T>
-__global__ void k_zero(T* A, long long lda, int n, T* b) {
+__global__ void k_zero(T* A, long long lda, int n) {
   long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   long long total = (long long)n * n;
   if (lda == n) {   // contiguous: a flat fill, no index division
@@ -549,8 +555,6 @@ __global__ void k_zero(T* A, long long lda, int n, T* b) {
       A[row + lda * col] = zero_of(T());
     }
   }
-  t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) b[t] = zero_of(T());
 }
 
 template <typename T>
@@ -718,6 +722,13 @@ __device__ inline void ext_point(ConstKP k, const double* x, const double* n,
 
 __device__ constexpr int kSym[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};
 
+// a wave's own LDS stores are seen by its lanes
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Sums over the points of one rule of one element for 16 collocation points, one wave, on the FP64
 // matrix cores (v_mfma_f64_4x4x4_4b).  A lane evaluates the kernel of pair lane % 16 at point
 // p0 + lane / 16: its values are, as they stand, the 16 x 4 left operand, and the weights
@@ -784,71 +795,110 @@ __device__ inline zd lane_xor_add(zd v, int mask) {
   return mkz(v.re + __shfl_xor(v.re, mask), v.im + __shfl_xor(v.im, mask));
 }
 
+// Launches of fewer tiles spread them one by one (runs would leave XCDs without work at the end).
+constexpr int kRunTiles = 16384;
+
+// Columns of four nodes for a tile's 48 rows, on their way to A.
+template <typename T>
+struct TileLds {
+  T v[12][3 * kTileP + 1];
+};
+typedef const __attribute__((address_space(4))) int* ConstInt;
+
+// where tiles store: A, and the extra points' rows (column stride 3 nx)
+template <typename T>
+struct TileOut {
+  T* A;
+  long long lda;
+  T* b;
+  T* X;
+};
+
+// One kind of values (KIND: kNeedH or kNeedG) of a tile: h goes to the columns of unknown u, -g to
+// those of unknown t, so the two kinds of an element that needs both store different columns.
 template <bool H, int KIND>
 __device__ inline void tile_body(const DevMesh& m, const KernelParams& kp,
-                                 const int* __restrict__ list, int2 tile, int e,
-                                 typename Val<H>::T* A, long long lda, typename Val<H>::T* b) {
+                                 const int* __restrict__ list, int4 tile, bool twice,
+                                 TileLds<typename Val<H>::T>& lds,
+                                 const TileOut<typename Val<H>::T>& out) {
   typedef typename Val<H>::T T;
-  const int cnt = tile.y & 0xff, rule = tile.y >> 8, lane = threadIdx.x;
+  constexpr bool kH = KIND == kNeedH;
+  const int cnt = tile.y, rule = tile.z, e = tile.w, lane = threadIdx.x;
   const int P = m.ps_gln[rule] * m.ps_gln[rule], first = e * m.ncp;
   const double* pe = m.ps + ((long long)e * m.npts + m.ps_off[rule]) * kPsStride;
   // a slot past the tile's pairs repeats the first one; its rows of the result are not stored
   const int slot = lane & 15, cpi = list[tile.x + (slot < cnt ? slot : 0)] - first;
   const double xi[3] = {m.xc[3 * cpi], m.xc[3 * cpi + 1], m.xc[3 * cpi + 2]};
+  // lane = row of the tile: three rows per pair
+  const int cpr = list[tile.x + (lane < 3 * cnt ? lane / 3 : 0)] - first;
+  const int xr = m.cx[cpr];
+  T* const arow = (xr < 0 ? out.A + 3LL * m.crow[cpr] : out.X + 3LL * xr) + lane % 3;
+  const long long ld = xr < 0 ? out.lda : 3LL * m.nx;
+  const bool live = lane < 3 * cnt;
+  int code[9];
+#pragma unroll
+  for (int k = 0; k < 9; k++) code[k] = ((ConstInt)(m.enode + 9LL * e))[k];
+  const int fixed = ((ConstInt)(m.emask + e))[0], value = ((ConstInt)(m.emask + e))[1];
+  const int to_a = kH ? ~fixed : fixed, to_b = (kH ? fixed : ~fixed) & value;
   TileAcc<H, KIND> acc;
   acc.clear();
   tile_points<H, KIND>((ConstKP)&kp, pe, P, xi, lane, acc);
   const int po = 4 * ((lane >> 2) & 3) + (lane >> 4), j = lane & 3;
-  const bool live = po < cnt;
-  const int cp = list[tile.x + (live ? po : 0)] - first;
-  const long long row = 3LL * m.crow[cp];
-  const bool shared = m.cshared[cp] != 0;
-  T bs[3] = {zero_of(T()), zero_of(T()), zero_of(T())};
+  // the lane's value for row component il, node group q, direction ik
+  auto val = [&](int il, int ik, int q) {
+    if constexpr (kH) return scale_h(kp, tile_value(acc.f, 3 * il + ik, q, T()));
+    else return -scale_g(kp, tile_value(acc.g, kSym[3 * il + ik], q, T()));
+  };
+  constexpr int kNodes[3] = {4, 4, 1};
+  // what the columns hold already (nodes that an earlier colour stored): all loads are on their way
+  // before the first is waited for
+  T w[27];
+#pragma unroll
+  for (int c = 0; c < 27; c++) {
+    w[c] = zero_of(T());
+    if (code[c / 3] < 0 && (to_a >> c & 1) && live) w[c] = arow[ld * (3LL * ~code[c / 3] + c % 3)];
+  }
 #pragma unroll
   for (int q = 0; q < 3; q++) {
-    const int n = 4 * q + j;
-    if (!live || n >= 9) continue;
-    const int sn = m.conn[9 * e + n];
+    wave_lds_fence();
+    if (j < kNodes[q]) {
 #pragma unroll
-    for (int ik = 0; ik < 3; ik++) {
-      const long long col = 3LL * sn + ik;
-      T v[3];
-      if (KIND == kNeedH) {
+      for (int ik = 0; ik < 3; ik++)
 #pragma unroll
-        for (int il = 0; il < 3; il++)
-          v[il] = scale_h(kp, tile_value(acc.f, 3 * il + ik, q, T()));
-      } else if (KIND == kNeedG) {
+        for (int il = 0; il < 3; il++) lds.v[3 * j + ik][3 * po + il] = val(il, ik, q);
+    }
+    wave_lds_fence();
 #pragma unroll
-        for (int il = 0; il < 3; il++)
-          v[il] = -scale_g(kp, tile_value(acc.g, kSym[3 * il + ik], q, T()));
-      } else {
-        const int ct = m.ctype[col];
-        const double cv = m.cval[col];
-        const double cb = ct == 0 ? -cv : ct == 1 ? cv : cv == 0.0 ? 0.0 : cv * m.nfn[col];
-#pragma unroll
-        for (int il = 0; il < 3; il++) {
-          const T h = scale_h(kp, tile_value(acc.f, 3 * il + ik, q, T()));
-          const T g = scale_g(kp, tile_value(acc.g, kSym[3 * il + ik], q, T()));
-          v[il] = ct == 0 ? -g : h;
-          if (cv != 0.0) bs[il] = bs[il] + (ct == 0 ? h : g) * cb;
-        }
-      }
-      T* a = A + row + lda * col;
-      if (shared) {
-        for (int il = 0; il < 3; il++) atomic_add(a + il, v[il]);
-      } else {
-        const T a0 = a[0], a1 = a[1], a2 = a[2];
-        a[0] = a0 + v[0];
-        a[1] = a1 + v[1];
-        a[2] = a2 + v[2];
-      }
+    for (int i = 0; i < 3 * kNodes[q]; i++) {
+      const int c = 12 * q + i, node = code[c / 3] < 0 ? ~code[c / 3] : code[c / 3];
+      if (!(to_a >> c & 1) || !live) continue;
+      T* a = arow + ld * (3LL * node + c % 3);
+      const T v = lds.v[i][lane];
+      if (!twice) *a = w[c] + v;
+      else atomic_add(a, v);
     }
   }
-  if (KIND == (kNeedH | kNeedG)) {
+  if (to_b & 0x7ffffff) {
+    T bs[3] = {zero_of(T()), zero_of(T()), zero_of(T())};
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      if (j >= kNodes[q]) continue;
+      const int col0 = 3 * m.conn[9 * e + 4 * q + j];
+#pragma unroll
+      for (int ik = 0; ik < 3; ik++) {
+        if (!(to_b >> (3 * (4 * q + j) + ik) & 1)) continue;
+        const int col = col0 + ik;
+        const double f = m.ctype[col] == 10 ? m.cval[col] * m.nfn[col] : m.cval[col];
+#pragma unroll
+        for (int il = 0; il < 3; il++) bs[il] = bs[il] - val(il, ik, q) * f;
+      }
+    }
+    const int cp = list[tile.x + (po < cnt ? po : 0)] - first;
+    const long long row = 3LL * m.crow[cp];
 #pragma unroll
     for (int il = 0; il < 3; il++) {
       bs[il] = lane_xor_add(lane_xor_add(bs[il], 1), 2);
-      if (live && j == 0) atomic_add(&b[row + il], bs[il]);
+      if (po < cnt && j == 0) atomic_add(&out.b[row + il], bs[il]);
     }
   }
 }
@@ -857,20 +907,70 @@ __device__ inline void tile_body(const DevMesh& m, const KernelParams& kp,
 // bem_harela3d.f90:628-700; scatter: src/assemble_bem_staela_equation.f90,
 // src/assemble_bem_harela_equation.f90), one tile per wave: up to 16 pairs of one element and one
 // rule, consecutive entries of the class list (ascending collocation points, so mostly consecutive
-// matrix rows).  The tiles of one launch belong to elements of one colour (no shared node): two of
-// them touch the same entry only if their points share rows (MCA points of one node), which add
-// atomically.
+// matrix rows).  The tiles of one launch belong to elements of one colour (no shared node) and no two
+// points share a row (DevMesh::cx), so no two waves touch the same entry.  The element of the lowest colour that holds a node stores its columns, the others add
+// to them: no reset of A and 5 reads instead of 9 per element on a structured surface.  The columns
+// go through LDS so that a lane holds a row: a store covers 768 consecutive bytes.  t* (tiles h0 .. h0 +
+// n_h) and u* (0 .. n_g) are summed by waves of their own, also for elements that need both: together
+// their sums do not fit the registers of two waves per SIMD (61 spilled).
 template <bool H>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2)))
     k_regular_tile(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
-                   const int2* __restrict__ tiles, typename Val<H>::T* A, long long lda,
-                   typename Val<H>::T* b) {
-  const int2 tile = tiles[blockIdx.x];
-  const int e = __builtin_amdgcn_readfirstlane(list[tile.x] / m.ncp);
-  const int kind = __builtin_amdgcn_readfirstlane(m.ekind[e]);
-  if (kind == kNeedH) tile_body<H, kNeedH>(m, *kpp, list, tile, e, A, lda, b);
-  else if (kind == kNeedG) tile_body<H, kNeedG>(m, *kpp, list, tile, e, A, lda, b);
-  else tile_body<H, kNeedH | kNeedG>(m, *kpp, list, tile, e, A, lda, b);
+                   const int4* __restrict__ tiles, int h0, int n_h, int n_g, int run,
+                   TileOut<typename Val<H>::T> out) {
+  __shared__ TileLds<typename Val<H>::T> lds;
+  // workgroups go to the eight XCDs in turn: `run` consecutive tiles, neighbours in A, to each
+  const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
+  const int t = ((i / run) * 8 + x) * run + i % run;
+  if (t >= n_h + n_g) return;
+  const bool is_h = t < n_h;
+  const int4 tile = tiles[is_h ? h0 + t : t - n_h];
+  const bool twice = m.ekind[tile.w] & kTwice;
+  if (is_h) tile_body<H, kNeedH>(m, *kpp, list, tile, twice, lds, out);
+  else tile_body<H, kNeedG>(m, *kpp, list, tile, twice, lds, out);
+}
+
+// First kernel of an assembly: b := 0, counters (if given) and error flag cleared and, of A and the
+// extra rows, what no tile stores: the entries of adaptive and singular pairs (list[0 .. count)) in
+// columns that their element would store.  Workgroups: 4 pairs each, then 256 entries of b each.
+template <typename T>
+__global__ void __launch_bounds__(256) k_begin(DevMesh m, const int* __restrict__ list, int count,
+                                               TileOut<T> out, long long* counters, int* err) {
+  if (blockIdx.x == 0 && counters) {
+    if (threadIdx.x < 2) counters[threadIdx.x] = 0;
+    if (threadIdx.x == 0) *err = 0;
+  }
+  const int pair_blocks = (count + 3) / 4, blk = blockIdx.x;
+  if (blk < pair_blocks) {
+    const int q = 4 * blk + threadIdx.x / kWave;
+    if (q >= count) return;
+    const int pid = list[q], e = pid / m.ncp, cp = pid % m.ncp, x = m.cx[cp];
+    T* row = x < 0 ? out.A + 3LL * m.crow[cp] : out.X + 3LL * x;
+    const long long ld = x < 0 ? out.lda : 3LL * m.nx;
+    for (int t = threadIdx.x % kWave; t < 81; t += kWave) {
+      const int col = t / 3, node = m.enode[9 * e + col / 3];
+      if (node >= 0) row[t % 3 + ld * (3LL * node + col % 3)] = zero_of(T());
+    }
+    return;
+  }
+  const int i = 256 * (blk - pair_blocks) + threadIdx.x;
+  if (i < 3 * m.nn) out.b[i] = zero_of(T());
+}
+
+// rows of the extra points added to their nodes' rows (one thread per component and column of the
+// first extra point of a node)
+template <typename T>
+__global__ void __launch_bounds__(256) k_fold_extra(DevMesh m, TileOut<T> out) {
+  const int r = blockIdx.x * 256 + threadIdx.x, x0 = r / 3, il = r % 3;
+  if (x0 >= m.nx || (x0 > 0 && m.xnode[x0] == m.xnode[x0 - 1])) return;
+  const long long ldx = 3LL * m.nx;
+  const int node = m.xnode[x0];
+  for (int col = blockIdx.y; col < 3 * m.nn; col += gridDim.y) {
+    T v = zero_of(T());
+    for (int x = x0; x < m.nx && m.xnode[x] == node; x++) v = v + out.X[3LL * x + il + ldx * col];
+    T* a = out.A + 3LL * node + il + out.lda * col;
+    *a = *a + v;
+  }
 }
 
 // Line integral eps_ijk e_k . t / r over one line3 edge, adaptive Telles + bisection
@@ -1131,12 +1231,6 @@ struct PairLds {
   };
 };
 
-__device__ inline void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // acc[g][q] += sum over the wave's 64 points of (rows 4 g .. 4 g + 3) x (weights of nodes 4 q ..
 // 4 q + 3): the lane's values v of its point go through LDS, 12 rows at a time, into the layout of
 // the left operand; each of the four blocks of an instruction takes four of 16 points, so the result
@@ -1320,7 +1414,7 @@ __device__ inline void singular_body(const DevMesh& m, ConstKP kp, int e, int cp
 // few real rows (the antisymmetric part and u* by their distinct components), summed against the
 // nine weights on the FP64 matrix cores.
 template <bool H>
-__global__ void __launch_bounds__(kSingWaves* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(kSingWaves* kWave) __attribute__((amdgpu_waves_per_eu(2)))
     k_singular(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
                const SingGeom* __restrict__ geo, typename Val<H>::T* A, long long lda,
                typename Val<H>::T* b, typename Val<H>::T* blocks, long long blk_base,
@@ -1329,7 +1423,7 @@ __global__ void __launch_bounds__(kSingWaves* kWave) __attribute__((amdgpu_waves
   const int pid = list[blockIdx.x], e = pid / m.ncp, cp = pid % m.ncp;
   const SingGeom* li = geo + blockIdx.x;
   typename Val<H>::T* block = blocks ? blocks + 162LL * (blk_base + blockIdx.x) : nullptr;
-  const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e];
+  const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e] & (kNeedH | kNeedG);
   ConstKP kp = (ConstKP)kpp;
   if (kind == kNeedH)
     singular_body<H, kNeedH>(m, kp, e, cp, li, lds, A, lda, b, block, vec);
@@ -1585,7 +1679,7 @@ __device__ inline void adaptive_pair(const DevMesh& m, const QsiParams* __restri
                                      const VecOut<typename Val<H>::T>& vec) {
   const int pid = list[q], e = pid / m.ncp, cp = pid % m.ncp;
   typename Val<H>::T* block = blocks ? blocks + 162LL * (blk_base + q) : nullptr;
-  const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e];
+  const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e] & (kNeedH | kNeedG);
   if (kind == kNeedH)
     adaptive_body<H, kNeedH, TREE>(m, *qsp, kp, e, cp, geo[q], lds, walk, A, lda, b, counters,
                                    block, vec);
@@ -1599,7 +1693,7 @@ __device__ inline void adaptive_pair(const DevMesh& m, const QsiParams* __restri
 
 // One wave per pair that is a single leaf (the others return).
 template <bool H>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2)))
     k_adaptive(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
                const AdaptGeom* __restrict__ geo, typename Val<H>::T* A, long long lda,
                typename Val<H>::T* b, typename Val<H>::T* blocks, long long blk_base,
@@ -1613,7 +1707,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2
 
 // One wave per pair that is subdivided, in turn over tree[4 .. 4 + tree[0]).
 template <bool H>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2)))
     k_adaptive_tree(DevMesh m, const QsiParams* __restrict__ qsp,
                     const KernelParams* __restrict__ kpp, const int* __restrict__ list,
                     const AdaptGeom* __restrict__ geo, const int* __restrict__ tree,
@@ -1876,9 +1970,11 @@ static int upload_tables() {
 namespace mfb {
 // scatter tiles of the precalculated classes (k_regular_tile), launched per element colour
 struct TileSet {
-  int2* d = nullptr;
+  int4* d = nullptr;
   size_t cap = 0;                  // tiles the device buffer holds
-  std::vector<long long> off, cnt;  // per colour: first tile, tiles
+  // per colour: first tile, tiles; of these the ones that need g alone, and both (in this order, those
+  // that need h alone last)
+  std::vector<long long> off, cnt, g_only, both;
 };
 }  // namespace mfb
 
@@ -1925,8 +2021,8 @@ struct mfb_mesh_s {
   int* judge_err = nullptr;
   // grow-only device workspaces of the per-assembly steps (lists, learned classes, judge): a
   // repeated assembly allocates and frees nothing
-  void* ws[10] = {};
-  size_t ws_cap[10] = {};
+  void* ws[11] = {};
+  size_t ws_cap[11] = {};
   double *x = nullptr, *cval = nullptr, *elem = nullptr, *ps = nullptr, *nfn = nullptr;
   int *conn = nullptr, *ctype = nullptr, *inc_ptr = nullptr, *inc_e = nullptr, *inc_k = nullptr;
   unsigned char* cls = nullptr;
@@ -1934,7 +2030,11 @@ struct mfb_mesh_s {
   // collocation points (device) and host copies of their rows / elements / coordinates
   double *xc = nullptr, *cxi = nullptr;
   int *crow = nullptr, *cel = nullptr;
-  unsigned char *cshared = nullptr, *nmca = nullptr, *ekind = nullptr;
+  unsigned char *nmca = nullptr, *ekind = nullptr;
+  int *enode = nullptr, *cx = nullptr, *xnode = nullptr;
+  int2* emask = nullptr;
+  std::vector<unsigned char> h_kind;   // kNeedH | kNeedG of each element
+  bool prezero = false;            // A is reset before the tiles (enode is then ~node throughout)
   mfb::SingGeom* sgeo = nullptr;   // of the singular and the adaptive pairs, in list order
   mfb::AdaptGeom* ageo = nullptr;
   int n_tree = 0;                  // adaptive pairs of `lists` that are subdivided
@@ -1976,15 +2076,15 @@ static void mesh_release(mfb_mesh_s* m) {
                 m->ctype, m->inc_ptr, m->inc_e, m->inc_k, m->cls,  m->lists, m->err,
                 m->counters, m->d_qsp, m->d_qsp_li, m->d_kp, m->d_qsp_judge, m->feats,
                 m->qcls, m->lcls, m->llists, m->judge_counters, m->judge_err,
-                m->xc, m->cxi, m->crow, m->cel, m->cshared, m->nmca,
+                m->xc, m->cxi, m->crow, m->cel, m->cx, m->xnode, m->nmca,
                 m->ws[0], m->ws[1], m->ws[2], m->ws[3], m->ws[4], m->ws[5], m->ws[6], m->ws[7],
-                m->ws[8], m->ws[9], m->ageo,
-                m->tiles.d, m->ltiles.d, m->d_promo, m->ekind, m->sgeo};
+                m->ws[8], m->ws[9], m->ws[10], m->ageo,
+                m->tiles.d, m->ltiles.d, m->d_promo, m->ekind, m->enode, m->emask, m->sgeo};
   for (void* p : ps)
     if (p) (void)hipFree(p);
 }
 
-enum MeshWs { MW_OFF, MW_COUNTS, MW_REF, MW_BLK, MW_POS, MW_SAMPLE, MW_ERR, MW_PC, MW_AGEO, MW_JGEO };
+enum MeshWs { MW_OFF, MW_COUNTS, MW_REF, MW_BLK, MW_POS, MW_SAMPLE, MW_ERR, MW_PC, MW_AGEO, MW_JGEO, MW_EXTRA };
 
 template <typename P>
 static int mesh_ws(mfb_mesh_s* m, int slot, size_t bytes, P** out) {
@@ -2076,22 +2176,29 @@ static int build_lists(mfb_mesh_t m, const unsigned char* cls, const int* counts
   ts.off.assign(nc, 0);
   ts.cnt.assign(nc, 0);
   long long nt = 0;
+  ts.g_only.assign(nc, 0);
+  ts.both.assign(nc, 0);
   for (int k = 0; k < nc; k++) {
     ts.off[k] = nt;
-    for (int r : rorder)
-      for (int q = 0; q < ne; q++) {
-        const int e = m->eorder[q];
-        if (m->ecol[e] != k) continue;
-        toff[(size_t)e * S + r] = nt;
-        nt += (hc[(size_t)e * S + r] + kTileP - 1) / kTileP;
-      }
+    for (int kind : {kNeedG, kNeedG | kNeedH, kNeedH}) {
+      const long long n0 = nt;
+      for (int r : rorder)
+        for (int q = 0; q < ne; q++) {
+          const int e = m->eorder[q];
+          if (m->ecol[e] != k || m->h_kind[e] != kind) continue;
+          toff[(size_t)e * S + r] = nt;
+          nt += (hc[(size_t)e * S + r] + kTileP - 1) / kTileP;
+        }
+      if (kind == kNeedG) ts.g_only[k] = nt - n0;
+      else if (kind != kNeedH) ts.both[k] = nt - n0;
+    }
     ts.cnt[k] = nt - ts.off[k];
   }
   if ((size_t)nt > ts.cap) {
     if (ts.d) (void)hipFree(ts.d);
     ts.d = nullptr;
     ts.cap = 0;
-    MFB_HIP(hipMalloc(&ts.d, sizeof(int2) * (size_t)nt));
+    MFB_HIP(hipMalloc(&ts.d, sizeof(int4) * (size_t)nt));
     ts.cap = (size_t)nt;
   }
   long long* doff = nullptr;
@@ -2120,7 +2227,7 @@ struct CollocSet {
   int ncp = 0;
   std::vector<double> xc, cxi;
   std::vector<int> crow, cel;
-  std::vector<unsigned char> cshared, nmca;
+  std::vector<unsigned char> nmca;
 };
 
 static const double kXiQ9H[9][2] = {{-1, -1}, {1, -1}, {1, 1}, {-1, 1}, {0, -1},
@@ -2160,7 +2267,6 @@ static void default_collocation(int nn, int ne, const double* x, const int* conn
       cs.cxi.push_back(0.0);
       cs.crow.push_back(i);
       cs.cel.push_back(-1);
-      cs.cshared.push_back(0);
       cs.ncp++;
       continue;
     }
@@ -2176,7 +2282,6 @@ static void default_collocation(int nn, int ne, const double* x, const int* conn
       cs.cxi.push_back(xi2);
       cs.crow.push_back(i);
       cs.cel.push_back(e);
-      cs.cshared.push_back(1);
       cs.ncp++;
     }
   }
@@ -2317,7 +2422,7 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
   TRY(dalloc(&m->cxi, 2LL * ncp));
   TRY(dalloc(&m->crow, ncp));
   TRY(dalloc(&m->cel, ncp));
-  TRY(dalloc(&m->cshared, ncp));
+  TRY(dalloc(&m->cx, ncp));
   TRY(dalloc(&m->nmca, nn));
   TRY(dalloc(&m->ekind, ne));
   TRY(dalloc(&m->err, 1));
@@ -2339,25 +2444,60 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
   TRYH(hipMemcpy(m->cxi, cs.cxi.data(), sizeof(double) * 2 * ncp, hipMemcpyHostToDevice));
   TRYH(hipMemcpy(m->crow, cs.crow.data(), sizeof(int) * ncp, hipMemcpyHostToDevice));
   TRYH(hipMemcpy(m->cel, cs.cel.data(), sizeof(int) * ncp, hipMemcpyHostToDevice));
-  TRYH(hipMemcpy(m->cshared, cs.cshared.data(), ncp, hipMemcpyHostToDevice));
+  {
+    std::vector<int> cx(ncp, -1), xnode;
+    for (int c = 1; c < ncp && !explicit_cs; c++)
+      if (cs.crow[c] == cs.crow[c - 1]) {
+        cx[c] = (int)xnode.size();
+        xnode.push_back(cs.crow[c]);
+      }
+    d.nx = (int)xnode.size();
+    TRYH(hipMemcpy(m->cx, cx.data(), sizeof(int) * ncp, hipMemcpyHostToDevice));
+    TRY(dalloc(&m->xnode, xnode.size()));
+    if (d.nx)
+      TRYH(hipMemcpy(m->xnode, xnode.data(), sizeof(int) * xnode.size(), hipMemcpyHostToDevice));
+  }
   if (cs.nmca.empty()) TRYH(hipMemset(m->nmca, 0, nn));
   else TRYH(hipMemcpy(m->nmca, cs.nmca.data(), nn, hipMemcpyHostToDevice));
   {
     std::vector<unsigned char> ek(ne, 0);
-    for (int e = 0; e < ne; e++)
+    std::vector<int2> em(ne, make_int2(0, 0));
+    for (int e = 0; e < ne; e++) {
       for (int k = 0; k < 27; k++) {
         const long long c = 3LL * conn[9 * e + k / 3] + k % 3;
         ek[e] |= ctype[c] == 0 ? kNeedG : kNeedH;
         if (cval[c] != 0.0) ek[e] |= ctype[c] == 0 ? kNeedH : kNeedG;
+        em[e].x |= (ctype[c] == 0) << k;
+        em[e].y |= (cval[c] != 0.0) << k;
       }
+    }
+    m->h_kind = ek;
+    TRY(dalloc(&m->emask, ne));
+    TRYH(hipMemcpy(m->emask, em.data(), sizeof(int2) * ne, hipMemcpyHostToDevice));
+    // the element that stores a node's columns: the one of the lowest colour.  Without one per node, or
+    // with a node twice in an element, A is reset and every element adds.
+    std::vector<int> en(9LL * ne), owner(nn, -1);
+    for (int e = 0; e < ne; e++)
+      for (int k = 0; k < 9; k++) {
+        for (int l = 0; l < k; l++)
+          if (conn[9 * e + k] == conn[9 * e + l]) ek[e] |= kTwice;
+        if (ek[e] & kTwice) m->prezero = true;
+        int& o = owner[conn[9 * e + k]];
+        if (o < 0 || ecol[e] < ecol[o]) o = e;
+      }
+    for (int i = 0; i < nn; i++) m->prezero = m->prezero || owner[i] < 0;
+    for (long long q = 0; q < 9LL * ne; q++)
+      en[q] = m->prezero || owner[conn[q]] != q / 9 ? ~conn[q] : conn[q];
+    TRY(dalloc(&m->enode, en.size()));
+    TRYH(hipMemcpy(m->enode, en.data(), sizeof(int) * en.size(), hipMemcpyHostToDevice));
     TRYH(hipMemcpy(m->ekind, ek.data(), ne, hipMemcpyHostToDevice));
   }
   TRYH(hipMemset(m->err, 0, sizeof(int)));
   TRYH(hipMemset(m->counters, 0, 2 * sizeof(long long)));
   d.x = m->x; d.conn = m->conn; d.ctype = m->ctype; d.cval = m->cval; d.elem = m->elem;
   d.ps = m->ps; d.nfn = m->nfn; d.inc_ptr = m->inc_ptr; d.inc_e = m->inc_e; d.inc_k = m->inc_k;
-  d.xc = m->xc; d.cxi = m->cxi; d.crow = m->crow; d.cel = m->cel; d.cshared = m->cshared;
-  d.nmca = m->nmca; d.ekind = m->ekind;
+  d.xc = m->xc; d.cxi = m->cxi; d.crow = m->crow; d.cel = m->cel; d.cx = m->cx; d.xnode = m->xnode;
+  d.nmca = m->nmca; d.ekind = m->ekind; d.enode = m->enode; d.emask = m->emask;
 
   hipLaunchKernelGGL(k_elem_setup, dim3((ne + 63) / 64), dim3(64), 0, 0, d, m->elem);
   TRYH(hipGetLastError());
@@ -2524,15 +2664,20 @@ static int learned_lists(mfb_mesh_t m, double kw, hipStream_t s) {
   return rc;
 }
 
+// bytes of the extra points' rows
+static size_t extra_bytes(mfb_mesh_t m, bool harmonic) {
+  return (harmonic ? sizeof(zd) : sizeof(double)) * 9 * (size_t)m->dm.nx * m->dm.nn;
+}
+
 // The kernels of one whole-boundary assembly into A, b (scatter mode) on stream s, reading the
 // kernel constants at kpp (device): zeroing, the precalculated-rule tiles (one launch per element
 // colour), adaptive and singular pairs, free terms.  No host synchronisation and no memset: the
-// sequence can be captured into a graph.  events: record the mesh's timing events around the
-// kernel groups (not while capturing).
+// sequence can be captured into a graph.  extra: workspace of extra_bytes.  events: record the mesh's
+// timing events around the kernel groups (not while capturing).
 template <bool H>
 static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, double nu,
                            typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
-                           hipStream_t s, bool events) {
+                           void* extra, hipStream_t s, bool events) {
   typedef typename Val<H>::T T;
   const DevMesh& d = m->dm;
   const int n = 3 * d.nn;
@@ -2541,20 +2686,18 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
   const std::vector<long long>& cls_cnt = learned ? m->lcls_cnt : m->cls_cnt;
   const TileSet& ts = learned ? m->ltiles : m->tiles;
   if (events) MFB_HIP(hipEventRecord(m->ev[0], s));
+  const TileOut<T> out{A, lda, b, (T*)extra};
+  if (m->prezero) {
+    const long long tot = (long long)n * n, nx = 3LL * d.nx * n;
+    const long long nblk = std::min<long long>((tot + 255) / 256, 1 << 14);   // 5.6 TB/s; 1 << 16: 5.1
+    hipLaunchKernelGGL(k_zero<T>, dim3((unsigned)nblk), dim3(256), 0, s, A, lda, n);
+    if (nx) hipLaunchKernelGGL(k_fill_zero<T>, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, s, out.X, nx);
+  }
   {
-    // A, b := 0: the runtime's fill (6.1 TB/s at 30k) on a stream that is not being captured;
-    // under capture (the batch graphs) a kernel, since memset nodes are kept out of graphs
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    MFB_HIP(hipStreamIsCapturing(s, &cap));
-    if (cap == hipStreamCaptureStatusNone && lda == n) {
-      MFB_HIP(hipMemsetAsync(A, 0, sizeof(T) * (size_t)n * n, s));
-      MFB_HIP(hipMemsetAsync(b, 0, sizeof(T) * (size_t)n, s));
-    } else {
-      long long tot = (long long)n * n;
-      long long nblk = std::min<long long>((tot + 255) / 256, 1 << 14);   // 5.6 TB/s; 1 << 16: 5.1
-      nblk = std::max<long long>(nblk, (n + 255) / 256);
-      hipLaunchKernelGGL(k_zero<T>, dim3((unsigned)nblk), dim3(256), 0, s, A, lda, n, b);
-    }
+    // adaptive and singular pairs are consecutive in the lists
+    const int np = m->prezero ? 0 : (int)(cls_cnt[d.n_ps] + cls_cnt[d.n_ps + 1]);
+    hipLaunchKernelGGL(k_begin<T>, dim3((unsigned)((np + 3) / 4 + (n + 255) / 256)), dim3(256), 0, s,
+                       d, lists + cls_off[d.n_ps], np, out, events ? m->counters : nullptr, m->err);
   }
   if (events) MFB_HIP(hipEventRecord(m->ev[1], s));
   // precalculated rules: one launch per element colour over its tiles (elements of one colour
@@ -2564,9 +2707,15 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
   for (int k = 0; k < m->n_colors; k++) {
     if (!ts.cnt[k]) continue;
     if (events) m->last_regular_launches++;
-    hipLaunchKernelGGL((k_regular_tile<H>), dim3((unsigned)ts.cnt[k]), dim3(kWave), 0, s, d,
-                       kpp, lists, ts.d + ts.off[k], A, lda, b);
+    const int ng = (int)(ts.g_only[k] + ts.both[k]), nh = (int)(ts.cnt[k] - ts.g_only[k]);
+    const int run = ng + nh < kRunTiles ? 1 : 32;
+    hipLaunchKernelGGL((k_regular_tile<H>), dim3((unsigned)((ng + nh + 8 * run - 1) / (8 * run) * 8 * run)),
+                       dim3(kWave), 0, s, d, kpp, lists, ts.d + ts.off[k], (int)ts.g_only[k], nh, ng,
+                       run, out);
   }
+  if (d.nx)
+    hipLaunchKernelGGL(k_fold_extra<T>, dim3((3 * d.nx + 255) / 256, std::min(n, 4096)), dim3(256), 0,
+                       s, d, out);
   if (events) MFB_HIP(hipEventRecord(m->ev[2], s));
   launch_adaptive<H>(d, m->d_qsp, kpp, lists + cls_off[d.n_ps],
                      learned ? (AdaptGeom*)m->ws[MW_AGEO] : m->ageo, (int)cls_cnt[d.n_ps],
@@ -2621,8 +2770,9 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
   const std::vector<long long>& cls_cnt = learned ? m->lcls_cnt : m->cls_cnt;
   // counters and error flag are cleared by a kernel (no memset nodes if the caller captures)
   if (!blocks && !vmode) {
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, m->counters, m->err);
-    const int rc = enqueue_scatter<H>(m, m->d_kp, learned, nu, A, lda, b, s, true);
+    void* extra = nullptr;
+    int rc = d.nx ? mesh_ws(m, MW_EXTRA, extra_bytes(m, H), &extra) : MFB_OK;
+    if (rc == MFB_OK) rc = enqueue_scatter<H>(m, m->d_kp, learned, nu, A, lda, b, extra, s, true);
     if (rc) return rc;
   } else {
     MFB_HIP(hipEventRecord(m->ev[0], s));
@@ -2758,8 +2908,16 @@ static int job_params(const mfb_assembly_job& j, KernelParams* kp) {
 
 // the jobs' kernels on s: one parameter upload (host_kp pinned), a counter / error reset per
 // distinct mesh, then every job's sequence
+// bytes of the extra points' rows of a batch (its jobs run one after the other)
+static size_t batch_extra_bytes(int njobs, const mfb_assembly_job* jobs) {
+  size_t n = 0;
+  for (int q = 0; q < njobs; q++)
+    if (jobs[q].mesh) n = std::max(n, extra_bytes(jobs[q].mesh, jobs[q].harmonic != 0));
+  return n;
+}
+
 static int enqueue_batch(int njobs, const mfb_assembly_job* jobs, const KernelParams* host_kp,
-                         KernelParams* dev_kp, hipStream_t s) {
+                         KernelParams* dev_kp, void* extra, hipStream_t s) {
   MFB_HIP(hipMemcpyAsync(dev_kp, host_kp, sizeof(KernelParams) * njobs, hipMemcpyHostToDevice, s));
   std::vector<mfb_mesh_t> seen;
   for (int q = 0; q < njobs; q++) {
@@ -2772,8 +2930,10 @@ static int enqueue_batch(int njobs, const mfb_assembly_job* jobs, const KernelPa
   for (int q = 0; q < njobs; q++) {
     const mfb_assembly_job& j = jobs[q];
     const int rc = j.harmonic
-        ? enqueue_scatter<true>(j.mesh, dev_kp + q, false, j.nu, (zd*)j.A, j.lda, (zd*)j.b, s, false)
-        : enqueue_scatter<false>(j.mesh, dev_kp + q, false, j.nu, j.A, j.lda, j.b, s, false);
+        ? enqueue_scatter<true>(j.mesh, dev_kp + q, false, j.nu, (zd*)j.A, j.lda, (zd*)j.b,
+                                extra, s, false)
+        : enqueue_scatter<false>(j.mesh, dev_kp + q, false, j.nu, j.A, j.lda, j.b, extra,
+                                 s, false);
     if (rc) return rc;
   }
   return MFB_OK;
@@ -2800,6 +2960,7 @@ struct mfb_batch_graph_s {
   std::vector<mfb_assembly_job> jobs;
   KernelParams* host_kp = nullptr;   // pinned: the graph's copy node reads it at every launch
   KernelParams* dev_kp = nullptr;
+  void* extra = nullptr;             // rows of the extra collocation points
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipStream_t cap = nullptr;
@@ -2811,6 +2972,7 @@ static void batch_graph_release(mfb_batch_graph_s* g) {
   if (g->cap) (void)hipStreamDestroy(g->cap);
   if (g->host_kp) (void)hipHostFree(g->host_kp);
   if (g->dev_kp) (void)hipFree(g->dev_kp);
+  if (g->extra) (void)hipFree(g->extra);
   delete g;
 }
 
@@ -2821,15 +2983,18 @@ extern "C" int mfb_assemble_batch(int njobs, const mfb_assembly_job* jobs, void*
   MFB_HIP(hipHostMalloc((void**)&hk, sizeof(KernelParams) * njobs));
   struct Free {
     KernelParams *h, *d;
-    ~Free() { if (h) (void)hipHostFree(h); if (d) (void)hipFree(d); }
-  } fr{hk, nullptr};
+    void* x;
+    ~Free() { if (h) (void)hipHostFree(h); if (d) (void)hipFree(d); if (x) (void)hipFree(x); }
+  } fr{hk, nullptr, nullptr};
   for (int q = 0; q < njobs; q++) {
     const int rc = job_params(jobs[q], hk + q);
     if (rc) return rc;
   }
   MFB_HIP(hipMalloc(&dk, sizeof(KernelParams) * njobs));
   fr.d = dk;
-  int rc = enqueue_batch(njobs, jobs, hk, dk, s);
+  const size_t xb = batch_extra_bytes(njobs, jobs);
+  if (xb) MFB_HIP(hipMalloc(&fr.x, xb));
+  int rc = enqueue_batch(njobs, jobs, hk, dk, fr.x, s);
   if (rc) return rc;
   MFB_HIP(hipStreamSynchronize(s));
   return batch_errors(njobs, jobs);
@@ -2851,12 +3016,17 @@ extern "C" int mfb_batch_graph_create(int njobs, const mfb_assembly_job* jobs,
     const int rc = job_params(jobs[q], g->host_kp + q);
     if (rc) return fail(rc);
   }
+  const size_t xb = batch_extra_bytes(njobs, jobs);
+  if (xb && hipMalloc(&g->extra, xb) != hipSuccess) {
+    set_error("mfb_batch_graph_create: allocation failed");
+    return fail(MFB_ERR_HIP);
+  }
   hipError_t he = hipStreamBeginCapture(g->cap, hipStreamCaptureModeThreadLocal);
   if (he != hipSuccess) {
     set_error("hipStreamBeginCapture: %s", hipGetErrorString(he));
     return fail(MFB_ERR_HIP);
   }
-  const int rc = enqueue_batch(njobs, jobs, g->host_kp, g->dev_kp, g->cap);
+  const int rc = enqueue_batch(njobs, jobs, g->host_kp, g->dev_kp, g->extra, g->cap);
   he = hipStreamEndCapture(g->cap, &g->graph);
   if (rc) return fail(rc);
   if (he == hipSuccess) he = hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0);
@@ -3417,7 +3587,6 @@ static int pair_blocks(int npairs, const double* X, const double* xc, double qsi
     cs.cxi.push_back(0.0);
     cs.crow.push_back(0);
     cs.cel.push_back(-1);
-    cs.cshared.push_back(0);
   }
   mfb_mesh_t m = nullptr;
   int rc = mesh_create_impl(nn, ne, x.data(), conn.data(), ctype.data(), cval.data(), qsi_re, ns,
@@ -3554,7 +3723,6 @@ extern "C" int mfb_points_create(mfb_mesh_t mesh, int npts, const double* x, mfb
   cs.cxi.assign(2LL * npts, 0.0);
   cs.crow.assign(npts, 0);
   cs.cel.assign(npts, -1);
-  cs.cshared.assign(npts, 0);
   const DevMesh& d = mesh->dm;
   mfb_mesh_t pm = nullptr;
   int rc = mesh_create_impl(d.nn, d.ne, mesh->h_x.data(), mesh->h_conn.data(),
