@@ -1267,10 +1267,11 @@ __device__ inline void rows_mfma(const double* v, const double* ph, double jw, c
   }
 }
 
-// sums of the workgroup's W waves: lds.sum[0][row][node] afterwards
+// sums of the workgroup's W waves (W = 1: of the calling wave alone): lds.sum[0][row][node] afterwards
 template <int NR, int W>
 __device__ inline void rows_reduce(double (*acc)[3], PairLds<W>& lds, int wave, int lane) {
-  __syncthreads();
+  if (W > 1) __syncthreads();
+  else wave_lds_fence();
 #pragma unroll
   for (int g = 0; g < NR / 4; g++)
 #pragma unroll
@@ -1281,7 +1282,8 @@ __device__ inline void rows_reduce(double (*acc)[3], PairLds<W>& lds, int wave, 
       const int n = 4 * q + (lane & 3);
       if (!(lane & 12) && n < 9) lds.sum[wave][4 * g + (lane >> 4)][n] = t;
     }
-  __syncthreads();
+  if (W > 1) __syncthreads();
+  else wave_lds_fence();
   if (W > 1) {
     for (int o = threadIdx.x; o < NR * 9; o += W * kWave) {
       double t = lds.sum[0][0][o];
@@ -1414,23 +1416,16 @@ __device__ inline void singular_body(const DevMesh& m, ConstKP kp, int e, int cp
 // few real rows (the antisymmetric part and u* by their distinct components), summed against the
 // nine weights on the FP64 matrix cores.
 template <bool H>
-__global__ void __launch_bounds__(kSingWaves* kWave) __attribute__((amdgpu_waves_per_eu(2)))
-    k_singular(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
-               const SingGeom* __restrict__ geo, typename Val<H>::T* A, long long lda,
-               typename Val<H>::T* b, typename Val<H>::T* blocks, long long blk_base,
-               VecOut<typename Val<H>::T> vec) {
-  __shared__ PairLds<kSingWaves> lds;
-  const int pid = list[blockIdx.x], e = pid / m.ncp, cp = pid % m.ncp;
-  const SingGeom* li = geo + blockIdx.x;
-  typename Val<H>::T* block = blocks ? blocks + 162LL * (blk_base + blockIdx.x) : nullptr;
+__device__ inline void singular_pair(const DevMesh& m, ConstKP kp, int pid,
+                                     const SingGeom* __restrict__ geo, PairLds<kSingWaves>& lds,
+                                     typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
+                                     typename Val<H>::T* block,
+                                     const VecOut<typename Val<H>::T>& vec) {
+  const int e = pid / m.ncp, cp = pid % m.ncp;
   const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e] & (kNeedH | kNeedG);
-  ConstKP kp = (ConstKP)kpp;
-  if (kind == kNeedH)
-    singular_body<H, kNeedH>(m, kp, e, cp, li, lds, A, lda, b, block, vec);
-  else if (kind == kNeedG)
-    singular_body<H, kNeedG>(m, kp, e, cp, li, lds, A, lda, b, block, vec);
-  else
-    singular_body<H, kNeedH | kNeedG>(m, kp, e, cp, li, lds, A, lda, b, block, vec);
+  if (kind == kNeedH) singular_body<H, kNeedH>(m, kp, e, cp, geo, lds, A, lda, b, block, vec);
+  else if (kind == kNeedG) singular_body<H, kNeedG>(m, kp, e, cp, geo, lds, A, lda, b, block, vec);
+  else singular_body<H, kNeedH | kNeedG>(m, kp, e, cp, geo, lds, A, lda, b, block, vec);
 }
 
 // Adaptive quasi-singular pairs: fbem_bem_staela3d_sbie_ext_adp (bem_staela3d.f90:973-1096,
@@ -1617,7 +1612,7 @@ __device__ inline void adaptive_body(const DevMesh& m, const QsiParams& qsp, Con
                                      const VecOut<typename Val<H>::T>& vec) {
   typedef typename Val<H>::T T;
   typedef ExtRows<H, KIND> R;
-  const int lane = threadIdx.x, gln_far = (int)m.elem[8 * e + 5];
+  const int lane = threadIdx.x % kWave, gln_far = (int)m.elem[8 * e + 5];
   double X[27];
   load_X(m, e, X);
   const double x_i[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
@@ -1675,10 +1670,10 @@ __device__ inline void adaptive_pair(const DevMesh& m, const QsiParams* __restri
                                      const AdaptGeom* __restrict__ geo, int q, PairLds<1>& lds,
                                      WalkLds* walk, typename Val<H>::T* A, long long lda,
                                      typename Val<H>::T* b, long long* counters,
-                                     typename Val<H>::T* blocks, long long blk_base,
+                                     typename Val<H>::T* blocks,
                                      const VecOut<typename Val<H>::T>& vec) {
   const int pid = list[q], e = pid / m.ncp, cp = pid % m.ncp;
-  typename Val<H>::T* block = blocks ? blocks + 162LL * (blk_base + q) : nullptr;
+  typename Val<H>::T* block = blocks ? blocks + 162LL * q : nullptr;
   const int kind = block || vec.out ? kNeedH | kNeedG : m.ekind[e] & (kNeedH | kNeedG);
   if (kind == kNeedH)
     adaptive_body<H, kNeedH, TREE>(m, *qsp, kp, e, cp, geo[q], lds, walk, A, lda, b, counters,
@@ -1689,39 +1684,6 @@ __device__ inline void adaptive_pair(const DevMesh& m, const QsiParams* __restri
   else
     adaptive_body<H, kNeedH | kNeedG, TREE>(m, *qsp, kp, e, cp, geo[q], lds, walk, A, lda, b,
                                             counters, block, vec);
-}
-
-// One wave per pair that is a single leaf (the others return).
-template <bool H>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2)))
-    k_adaptive(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
-               const AdaptGeom* __restrict__ geo, typename Val<H>::T* A, long long lda,
-               typename Val<H>::T* b, typename Val<H>::T* blocks, long long blk_base,
-               VecOut<typename Val<H>::T> vec) {
-  __shared__ PairLds<1> lds;
-  const int q = blockIdx.x;
-  if (geo[q].gln == 0) return;
-  adaptive_pair<H, false>(m, nullptr, (ConstKP)kpp, list, geo, q, lds, nullptr, A, lda, b, nullptr,
-                          blocks, blk_base, vec);
-}
-
-// One wave per pair that is subdivided, in turn over tree[4 .. 4 + tree[0]).
-template <bool H>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2)))
-    k_adaptive_tree(DevMesh m, const QsiParams* __restrict__ qsp,
-                    const KernelParams* __restrict__ kpp, const int* __restrict__ list,
-                    const AdaptGeom* __restrict__ geo, const int* __restrict__ tree,
-                    typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
-                    long long* counters, typename Val<H>::T* blocks, long long blk_base,
-                    VecOut<typename Val<H>::T> vec) {
-  __shared__ PairLds<1> lds;
-  __shared__ WalkLds walk;
-  const int n = tree[0];
-  for (int t = blockIdx.x; t < n; t += gridDim.x) {
-    __syncthreads();
-    adaptive_pair<H, true>(m, qsp, (ConstKP)kpp, list, geo, tree[4 + t], lds, &walk, A, lda, b,
-                           counters, blocks, blk_base, vec);
-  }
 }
 
 // err[q * nr + r] = max(max|h - h_ref| / max|h_ref|, max|g - g_ref| / max|g_ref|) of pair q
@@ -1849,8 +1811,8 @@ __device__ bool mantic(int m_, double (*ln)[3], double (*lt)[3], double tol, dou
 }
 
 template <typename T>
-__global__ void k_freeterm(DevMesh m, double nu, T* A, long long lda, T* b, int* err) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ inline void free_term(const DevMesh& m, int i, double nu, T* A, long long lda, T* b,
+                                 int* err) {
   if (i >= m.nn) return;
   int q0 = m.inc_ptr[i], q1 = m.inc_ptr[i + 1];
   if (q1 == q0 || m.nmca[i]) return;
@@ -1894,8 +1856,7 @@ __global__ void k_freeterm(DevMesh m, double nu, T* A, long long lda, T* b, int*
 // phi_n(xi_i) I on the element's nodes (src/build_lse_mechanics_bem_staela.f90:444-457), scattered by
 // the BE-ordinary rule.
 template <typename T>
-__global__ void k_freeterm_mca(DevMesh m, T* A, long long lda, T* b) {
-  const int cp = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ inline void free_term_mca(const DevMesh& m, int cp, T* A, long long lda, T* b) {
   if (cp >= m.ncp) return;
   const int e = m.cel[cp];
   if (e < 0) return;
@@ -1914,6 +1875,82 @@ __global__ void k_freeterm_mca(DevMesh m, T* A, long long lda, T* b) {
 }
 
 #pragma clang fp contract(fast)
+
+// ------------------------------------------------------------------------------------------------
+// Everything that adds to what the tiles have stored, in one launch: subdivided adaptive pairs (a wave
+// each, in turn), singular pairs (a workgroup each), the other adaptive pairs (a wave each), free
+// terms (a thread each).  The parts are independent (atomic additions), each is a chain of a few
+// dependent loads and reductions and none fills the chip on a small mesh: one after the other they
+// took 150 of 480 us of a 1,158-DOF assembly.  The longest come first.
+// ------------------------------------------------------------------------------------------------
+template <typename T>
+struct NearArgs {
+  const int *alist, *slist;     // adaptive, singular pairs
+  const AdaptGeom* ageo;
+  const SingGeom* sgeo;
+  int na, ns;
+  int tree_wgs;                 // workgroups that take the subdivided pairs
+  int nfree, nfree_mca;         // nodes, collocation points whose free terms are added
+  double nu;
+  T* A;
+  long long lda;
+  T* b;
+  long long* counters;          // points, leaves of the subdivided pairs
+  int* err;
+  T *ablocks, *sblocks;         // blocks of the pairs (162 values each) instead of A, b
+  VecOut<T> vec;                // displacements of their points instead of A, b
+};
+constexpr int kNearWaves = 4;
+static_assert(kNearWaves == kSingWaves, "one workgroup shape");
+template <bool H>
+struct NearLds {
+  union {
+    PairLds<kSingWaves> sing;
+    struct {
+      PairLds<1> pair[kNearWaves];
+      WalkLds walk[kNearWaves];
+    };
+  };
+};
+template <bool H>
+__global__ void __launch_bounds__(kNearWaves* kWave) __attribute__((amdgpu_waves_per_eu(2)))
+    k_near(DevMesh m, const QsiParams* __restrict__ qsp, const KernelParams* __restrict__ kpp,
+           NearArgs<typename Val<H>::T> a) {
+  typedef typename Val<H>::T T;
+  __shared__ NearLds<H> lds;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const ConstKP kp = (ConstKP)kpp;
+  int wg = blockIdx.x;
+  if (wg < a.tree_wgs) {
+    const int* tree = adapt_tree((AdaptGeom*)a.ageo, a.na);
+    const int n = tree[0];
+    for (int t = kNearWaves * wg + wave; t < n; t += kNearWaves * a.tree_wgs) {
+      wave_lds_fence();
+      adaptive_pair<H, true>(m, qsp, kp, a.alist, a.ageo, tree[4 + t], lds.pair[wave],
+                             &lds.walk[wave], a.A, a.lda, a.b, a.counters, a.ablocks, a.vec);
+    }
+    return;
+  }
+  wg -= a.tree_wgs;
+  if (wg < a.ns) {
+    singular_pair<H>(m, kp, a.slist[wg], a.sgeo + wg, lds.sing, a.A, a.lda, a.b,
+                     a.sblocks ? a.sblocks + 162LL * wg : (T*)nullptr, a.vec);
+    return;
+  }
+  wg -= a.ns;
+  const int adapt_wgs = (a.na + kNearWaves - 1) / kNearWaves;
+  if (wg < adapt_wgs) {
+    const int q = kNearWaves * wg + wave;
+    if (q < a.na && a.ageo[q].gln)
+      adaptive_pair<H, false>(m, qsp, kp, a.alist, a.ageo, q, lds.pair[wave], nullptr, a.A, a.lda,
+                              a.b, nullptr, a.ablocks, a.vec);
+    return;
+  }
+  wg -= adapt_wgs;
+  const int free_wgs = (a.nfree + 255) / 256, i = threadIdx.x;
+  if (wg < free_wgs) free_term<T>(m, 256 * wg + i, a.nu, a.A, a.lda, a.b, a.err);
+  else free_term_mca<T>(m, 256 * (wg - free_wgs) + i, a.A, a.lda, a.b);
+}
 
 }  // namespace mfb
 
@@ -2099,21 +2136,16 @@ static int mesh_ws(mfb_mesh_s* m, int slot, size_t bytes, P** out) {
   return MFB_OK;
 }
 
-// The integration of `count` adaptive pairs; n_tree: how many of them are subdivided, -1 unknown on the
-// host.
+// k_near; n_tree: how many of the adaptive pairs are subdivided, -1 unknown on the host
 template <bool H>
-static void launch_adaptive(const DevMesh& d, const QsiParams* qsp, const KernelParams* kpp,
-                            const int* list, AdaptGeom* geo, int count, int n_tree,
-                            typename Val<H>::T* A, long long lda, typename Val<H>::T* b,
-                            long long* counters, typename Val<H>::T* blocks, long long blk_base,
-                            VecOut<typename Val<H>::T> vec, hipStream_t s) {
-  if (!count) return;
-  if (n_tree)
-    hipLaunchKernelGGL(k_adaptive_tree<H>, dim3(std::min(n_tree < 0 ? count : n_tree, 2048)),
-                       dim3(kWave), 0, s, d, qsp, kpp, list, geo, adapt_tree(geo, count), A, lda, b,
-                       counters, blocks, blk_base, vec);
-  hipLaunchKernelGGL(k_adaptive<H>, dim3((unsigned)count), dim3(kWave), 0, s, d, kpp, list, geo, A,
-                     lda, b, blocks, blk_base, vec);
+static void launch_near(const DevMesh& d, const QsiParams* qsp, const KernelParams* kpp,
+                        NearArgs<typename Val<H>::T> a, int n_tree, hipStream_t s) {
+  const int most = n_tree < 0 ? a.na : n_tree;
+  a.tree_wgs = std::min((most + kNearWaves - 1) / kNearWaves, 512);
+  const long long wgs = (long long)a.tree_wgs + a.ns + (a.na + kNearWaves - 1) / kNearWaves +
+                        (a.nfree + 255) / 256 + (a.nfree_mca + 255) / 256;
+  if (wgs)
+    hipLaunchKernelGGL(k_near<H>, dim3((unsigned)wgs), dim3(kNearWaves * kWave), 0, s, d, qsp, kpp, a);
 }
 
 // Records of `count` listed adaptive pairs at the tolerance of qsp into geo (adapt_geom_bytes).
@@ -2717,19 +2749,26 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
     hipLaunchKernelGGL(k_fold_extra<T>, dim3((3 * d.nx + 255) / 256, std::min(n, 4096)), dim3(256), 0,
                        s, d, out);
   if (events) MFB_HIP(hipEventRecord(m->ev[2], s));
-  launch_adaptive<H>(d, m->d_qsp, kpp, lists + cls_off[d.n_ps],
-                     learned ? (AdaptGeom*)m->ws[MW_AGEO] : m->ageo, (int)cls_cnt[d.n_ps],
-                     learned ? -1 : m->n_tree, A, lda, b, m->counters, nullptr, 0LL, VecOut<T>{}, s);
-  if (events) MFB_HIP(hipEventRecord(m->ev[3], s));
-  if (cls_cnt[d.n_ps + 1])
-    hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]),
-                       dim3(kSingWaves * kWave), 0, s, d, kpp, lists + cls_off[d.n_ps + 1], m->sgeo,
-                       A, lda, b, (T*)nullptr, 0LL, VecOut<T>{});
-  if (events) MFB_HIP(hipEventRecord(m->ev[4], s));
-  hipLaunchKernelGGL(k_freeterm<T>, dim3((d.nn + 127) / 128), dim3(128), 0, s, d, nu, A, lda, b,
-                     m->err);
-  if (m->n_mca)
-    hipLaunchKernelGGL(k_freeterm_mca<T>, dim3((d.ncp + 127) / 128), dim3(128), 0, s, d, A, lda, b);
+  NearArgs<T> a{};
+  a.alist = lists + cls_off[d.n_ps];
+  a.slist = lists + cls_off[d.n_ps + 1];
+  a.ageo = learned ? (AdaptGeom*)m->ws[MW_AGEO] : m->ageo;
+  a.sgeo = m->sgeo;
+  a.na = (int)cls_cnt[d.n_ps];
+  a.ns = (int)cls_cnt[d.n_ps + 1];
+  a.nfree = d.nn;
+  a.nfree_mca = m->n_mca ? d.ncp : 0;
+  a.nu = nu;
+  a.A = A;
+  a.lda = lda;
+  a.b = b;
+  a.counters = m->counters;
+  a.err = m->err;
+  launch_near<H>(d, m->d_qsp, kpp, a, learned ? -1 : m->n_tree, s);
+  if (events) {
+    MFB_HIP(hipEventRecord(m->ev[3], s));
+    MFB_HIP(hipEventRecord(m->ev[4], s));
+  }
   if (events) MFB_HIP(hipEventRecord(m->ev[5], s));
   MFB_HIP(hipGetLastError());
   return MFB_OK;
@@ -2799,15 +2838,19 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
                            m->d_kp, lists + o, (int)cnt, r, blocks, o, vec);
     }
     MFB_HIP(hipEventRecord(m->ev[2], s));
-    launch_adaptive<H>(d, m->d_qsp, m->d_kp, lists + cls_off[d.n_ps], m->ageo,
-                       (int)cls_cnt[d.n_ps], m->n_tree, A, lda, b, m->counters, blocks,
-                       cls_off[d.n_ps], vec, s);
+    NearArgs<T> a{};
+    a.alist = lists + cls_off[d.n_ps];
+    a.slist = lists + cls_off[d.n_ps + 1];
+    a.ageo = m->ageo;
+    a.sgeo = m->sgeo;
+    a.na = (int)cls_cnt[d.n_ps];
+    a.ns = (int)cls_cnt[d.n_ps + 1];
+    a.counters = m->counters;
+    a.ablocks = blocks ? blocks + 162 * cls_off[d.n_ps] : nullptr;
+    a.sblocks = blocks ? blocks + 162 * cls_off[d.n_ps + 1] : nullptr;
+    a.vec = vec;
+    launch_near<H>(d, m->d_qsp, m->d_kp, a, m->n_tree, s);
     MFB_HIP(hipEventRecord(m->ev[3], s));
-    if (cls_cnt[d.n_ps + 1]) {
-      hipLaunchKernelGGL(k_singular<H>, dim3((unsigned)cls_cnt[d.n_ps + 1]),
-                         dim3(kSingWaves * kWave), 0, s, d, m->d_kp, lists + cls_off[d.n_ps + 1],
-                         m->sgeo, A, lda, b, blocks, cls_off[d.n_ps + 1], vec);
-    }
     MFB_HIP(hipEventRecord(m->ev[4], s));
     MFB_HIP(hipEventRecord(m->ev[5], s));
   }
@@ -3126,8 +3169,13 @@ static int rule_errors(mfb_mesh_t m, const KernelParams& kp, const int* dlist, i
   if (he == hipSuccess) {
     hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, counters, errflag);
     launch_adapt_geom(d, d_qsp_ref, dlist, np, geo, s);
-    launch_adaptive<H>(d, d_qsp_ref, m->d_kp, dlist, geo, np, -1, nullptr, 0LL, nullptr, counters,
-                       ref, 0LL, VecOut<T>{}, s);
+    NearArgs<T> a{};
+    a.alist = dlist;
+    a.ageo = geo;
+    a.na = np;
+    a.counters = counters;
+    a.ablocks = ref;
+    launch_near<H>(d, d_qsp_ref, m->d_kp, a, -1, s);
     for (int r = 0; r < d.n_ps; r++) {
       const int P = d.ps_gln[r] * d.ps_gln[r], B = P >= kWave ? 1 : kWave / P;
       hipLaunchKernelGGL((k_regular<H, kBlocks>), dim3((unsigned)((np + B - 1) / B)), dim3(kWave),
