@@ -2319,6 +2319,57 @@ static void default_collocation(int nn, int ne, const double* x, const int* conn
   }
 }
 
+// Colours of the elements (no two of a colour share a node), greedily in index order, and where that
+// takes more than the four of a structured surface (closed ones: six) once more by saturation
+// degree (Brelaz), which is kept if it needs fewer: every colour is a launch, and on a small mesh a
+// launch takes its latency.
+constexpr int kMaxColors = 64;
+static int color_elements(int ne, const int* conn, const std::vector<int>& ip,
+                          const std::vector<int>& ie, std::vector<int>& col) {
+  auto pick = [&](const std::vector<int>& c, int e) {
+    unsigned long long used = 0;
+    for (int k = 0; k < 9; k++)
+      for (int q = ip[conn[9LL * e + k]]; q < ip[conn[9LL * e + k] + 1]; q++)
+        if (c[ie[q]] >= 0) used |= 1ull << c[ie[q]];
+    return ~used ? __builtin_ctzll(~used) : kMaxColors;
+  };
+  int n = 0;
+  col.assign(ne, -1);
+  for (int e = 0; e < ne; e++) {
+    const int c = pick(col, e);
+    n = std::max(n, c + 1);
+    if (n > kMaxColors) return n;
+    col[e] = c;
+  }
+  if (n <= 4 || ne > 4096) return n;
+  std::vector<int> c2(ne, -1), sat(ne, 0);
+  std::vector<unsigned long long> seen(ne, 0ull);
+  std::vector<std::vector<int>> heap(kMaxColors + 1);   // elements by saturation, stale ones included
+  for (int e = ne - 1; e >= 0; e--) heap[0].push_back(e);
+  int n2 = 0, top = 0;
+  for (int left = ne; left > 0;) {
+    while (top > 0 && heap[top].empty()) top--;
+    const int e = heap[top].back();
+    heap[top].pop_back();
+    if (c2[e] >= 0 || sat[e] != top) continue;
+    const int c = pick(c2, e);
+    n2 = std::max(n2, c + 1);
+    if (n2 >= n) return n;
+    c2[e] = c;
+    left--;
+    for (int k = 0; k < 9; k++)
+      for (int q = ip[conn[9LL * e + k]]; q < ip[conn[9LL * e + k] + 1]; q++) {
+        const int f = ie[q];
+        if (c2[f] >= 0 || (seen[f] >> c & 1)) continue;
+        seen[f] |= 1ull << c;
+        heap[++sat[f]].push_back(f);
+        top = std::max(top, sat[f]);
+      }
+  }
+  col.swap(c2);
+  return n2;
+}
+
 // explicit: a caller-given collocation set (batches of independent pairs); otherwise the
 // reference's default formulation with MCA parameter mca_delta.  classify_all = false leaves
 // classification and lists to the caller.
@@ -2395,25 +2446,10 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
   m->n_mca = 0;
   for (unsigned char f : cs.nmca) m->n_mca += f;
 
-  // greedy colouring over shared nodes, elements in index order
-  std::vector<int> ecol(ne, -1);
-  bool color_overflow = false;
-  {
-    constexpr int kMaxColors = 64;
-    std::vector<int> seen(kMaxColors, -1);
-    for (int e = 0; e < ne; e++) {
-      for (int k = 0; k < 9; k++) {
-        const int j = conn[9 * e + k];
-        for (int q = ip[j]; q < ip[j + 1]; q++)
-          if (ecol[ie[q]] >= 0) seen[ecol[ie[q]]] = e;
-      }
-      int c = 0;
-      while (c < kMaxColors && seen[c] == e) c++;
-      if (c == kMaxColors) { color_overflow = true; c = 0; }
-      ecol[e] = c;
-      m->n_colors = std::max(m->n_colors, c + 1);
-    }
-  }
+  std::vector<int> ecol;
+  const int n_colors = color_elements(ne, conn, ip, ie, ecol);
+  const bool color_overflow = n_colors > kMaxColors;
+  m->n_colors = n_colors;
   std::vector<int> eorder(ne);
   for (int e = 0; e < ne; e++) eorder[e] = e;
   std::stable_sort(eorder.begin(), eorder.end(), [&](int a, int b) { return ecol[a] < ecol[b]; });
