@@ -322,8 +322,8 @@ class Points:
         torch = _torch()
         harm = omega is not None
         dt = torch.complex128 if harm else torch.float64
-        ub = torch.as_tensor(np.asarray(u.cpu() if hasattr(u, "cpu") else u), device="cuda").to(dt).contiguous()
-        tb = torch.as_tensor(np.asarray(t.cpu() if hasattr(t, "cpu") else t), device="cuda").to(dt).contiguous()
+        ub, tb = (torch.as_tensor(v if hasattr(v, "cpu") else np.asarray(v), device="cuda")
+                  .to(dt).contiguous() for v in (u, t))
         out = torch.empty((self.npts, 3), dtype=dt, device="cuda")
         if harm:
             rc = lib().mfb_points_displacement_harela(self._h, omega, lam.real, lam.imag, mu_c.real,

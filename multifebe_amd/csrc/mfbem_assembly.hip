@@ -571,18 +571,13 @@ inline size_t kreg_lds_bytes(int items) {
 
 // Precalculated-rule pairs (ext_pre: bem_staela3d.f90:592-650, bem_harela3d.f90:628-700) of one
 // rule, 64/P pairs per wave: lanes evaluate the kernel at the (pair, point) items into LDS, then each
-// lane sums one (pair, kind, c = 3 l + k) row over the rule's points for three element nodes.
-// MODE kBlocks: write each pair's 9x3x3 h and g blocks to blocks[162 (blk_base + position) ...];
-// MODE kVector: add the pair's contribution to the interior displacement of its point (vec).
-constexpr int kBlocks = 1, kVector = 2;
-template <bool H, int MODE>
+// lane sums one (pair, kind, c = 3 l + k) row over the rule's points for three element nodes and writes
+// it to the pair's 9x3x3 h and g blocks, blocks[162 (blk_base + position) ...].
+template <bool H>
 __global__ void __launch_bounds__(kWave) k_regular(DevMesh m, const KernelParams* __restrict__ kpp,
                                                    const int* list, int count, int rule,
-                                                   typename Val<H>::T* blocks, long long blk_base,
-                                                   VecOut<typename Val<H>::T> vec) {
+                                                   typename Val<H>::T* blocks, long long blk_base) {
   typedef typename Val<H>::T T;
-  constexpr bool VEC = MODE == kVector;
-  __shared__ T vred[kWave * 3];  // MODE kVector: per (pair of the batch, l) sums
   const KernelParams& kp = *kpp;
   const int g = m.ps_gln[rule], P = g * g, B = P >= kWave ? 1 : kWave / P;
   const int base = blockIdx.x * B;
@@ -604,15 +599,11 @@ __global__ void __launch_bounds__(kWave) k_regular(DevMesh m, const KernelParams
     ext_kernel_row(kp, x, n, xi, &sfs[it * 18]);
     for (int c = 0; c < 9; c++) sw[it * 9 + c] = q[6 + c];
   }
-  if (VEC)
-    for (int q = lane; q < 3 * nb; q += kWave) vred[q] = zero_of(T());
   __syncthreads();
   // one lane per (pair, kind, c = 3 l + k, three element nodes): sums over the rule's points, each
   // kernel value read once and used for the three nodes
   for (int it = lane; it < nb * 54; it += kWave) {
     const int bb = it / 54, o = it % 54, kind = o / 27, c = (o % 27) / 3, n0 = 3 * (o % 3);
-    const int pid = list[base + bb];
-    const int e = pid / m.ncp, cp = pid % m.ncp;
     const T* f = &sfs[bb * P * 18 + kind * 9 + c];
     const double* wq = &sw[bb * P * 9 + n0];
     T acc[3] = {zero_of(T()), zero_of(T()), zero_of(T())};
@@ -623,28 +614,10 @@ __global__ void __launch_bounds__(kWave) k_regular(DevMesh m, const KernelParams
       acc[2] += fv * wq[p * 9 + 2];
     }
     const int il = c / 3, ik = c % 3;
-    if (VEC) {
-      T sum = zero_of(T());
-#pragma unroll
-      for (int q = 0; q < 3; q++) {
-        const int sn = m.conn[9 * e + n0 + q];
-        if (kind == 0) sum = sum - scale_h(kp, acc[q]) * vec.u[3 * sn + ik];
-        else sum = sum + scale_g(kp, acc[q]) * vec.t[3 * sn + ik];
-      }
-      lds_add(&vred[3 * bb + il], sum);
-      continue;
-    }
 #pragma unroll
     for (int q = 0; q < 3; q++) {
       const T v = kind ? scale_g(kp, acc[q]) : scale_h(kp, acc[q]);
       blocks[162LL * (blk_base + base + bb) + 81 * kind + n0 + q + 9 * il + 27 * ik] = v;
-    }
-  }
-  if (VEC) {
-    __syncthreads();
-    for (int q = lane; q < 3 * nb; q += kWave) {
-      const int cp = list[base + q / 3] % m.ncp;
-      atomic_add(&vec.out[3 * cp + q % 3], vred[q]);
     }
   }
 }
@@ -970,6 +943,108 @@ __global__ void __launch_bounds__(256) k_fold_extra(DevMesh m, TileOut<T> out) {
     for (int x = x0; x < m.nx && m.xnode[x] == node; x++) v = v + out.X[3LL * x + il + ldx * col];
     T* a = out.A + 3LL * node + il + out.lda * col;
     *a = *a + v;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Interior displacements of the precalculated pairs
+// ------------------------------------------------------------------------------------------------
+// Boundary fields at the precalculated points, with weights and constants: (t, -u) phi J w summed over
+// the element's nodes, so that a pair needs 3 products with u* and t* per point instead of their
+// 162 integrals over the 9 nodes.
+template <typename T>
+__global__ void __launch_bounds__(256) k_field(DevMesh m, const KernelParams* __restrict__ kpp,
+                                               VecOut<T> vec, T* field) {
+  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (q >= (long long)m.ne * m.npts) return;
+  const int e = (int)(q / m.npts);
+  const double* w = m.ps + q * kPsStride + 6;
+  T f[6];
+  for (int c = 0; c < 6; c++) f[c] = zero_of(T());
+  for (int n = 0; n < 9; n++) {
+    const int sn = m.conn[9 * e + n];
+    for (int k = 0; k < 3; k++) {
+      f[k] = f[k] + vec.t[3 * sn + k] * w[n];
+      f[3 + k] = f[3 + k] - vec.u[3 * sn + k] * w[n];
+    }
+  }
+  for (int k = 0; k < 3; k++) {
+    field[6 * q + k] = scale_g(*kpp, f[k]);
+    field[6 * q + 3 + k] = scale_h(*kpp, f[3 + k]);
+  }
+}
+
+// u_l += u*_lk t_k - t*_lk u_k of one point; f: (t, -u) there (the values of ext_point)
+__device__ inline void point_values(ConstKP k, const double* rv, const double* n, bool on,
+                                    const double* f, double* u) {
+  const double s = on ? rsqrt(dot3(rv, rv)) : 0.0;
+  const double dr[3] = {rv[0] * s, rv[1] * s, rv[2] * s};
+  const double rn = dot3(dr, n), s2 = s * s, dt = dot3(dr, f), du = dot3(dr, f + 3), nu = dot3(n, f + 3);
+  const double c = s2 * k->ctet2, a = s * dt + 3.0 * s2 * rn * du - c * nu;
+  const double ct = s * k->cteu2, cu = c * rn, cn = c * du;
+#pragma unroll
+  for (int l = 0; l < 3; l++) u[l] += ct * f[l] + cu * f[3 + l] + dr[l] * a + n[l] * cn;
+}
+
+__device__ inline void point_values(ConstKP k, const double* rv, const double* n, bool on,
+                                    const zd* f, zd* u) {
+  double r, s;
+  dist_and_inverse(dot3(rv, rv), r, s);
+  if (!on) {
+    r = 1.0;
+    s = 0.0;
+  }
+  const double dr[3] = {rv[0] * s, rv[1] * s, rv[2] * s}, rn = dot3(dr, n);
+  zd psi, chi, TT1, TT2, TT3;
+  har_factors<true, true>(&k->h, r, s, true, psi, chi, TT1, TT2, TT3);
+  const zd dt = f[0] * dr[0] + f[1] * dr[1] + f[2] * dr[2];
+  const zd du = f[3] * dr[0] + f[4] * dr[1] + f[5] * dr[2];
+  const zd nu = f[3] * n[0] + f[4] * n[1] + f[5] * n[2];
+  const zd a = TT1 * (du * rn) + TT3 * nu - chi * dt, cu = TT2 * rn, cn = TT2 * du;
+#pragma unroll
+  for (int l = 0; l < 3; l++) u[l] += psi * f[l] + cu * f[3 + l] + a * dr[l] + cn * n[l];
+}
+
+// One wave per 16 points and `chunk` elements, the sums in registers over the elements.  Four lanes
+// share the quadrature points of a pair's own rule, the wave takes as many as the longest of its 16:
+// order, the points along a space-filling curve, keeps that close to what each needs, and lanes of one
+// rule load one address.  10,000 harmonic points, 216 elements: 0.83 ms; a lane per pair, 64 pairs a
+// wave, 1.2 ms; 64 pairs a wave by one rule after the other, its records as scalars, 2.9 ms.
+template <bool H>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(3)))
+    k_points(DevMesh m, const KernelParams* __restrict__ kpp, const unsigned char* __restrict__ cls,
+             const int* __restrict__ order, const typename Val<H>::T* __restrict__ field, int chunk,
+             typename Val<H>::T* out) {
+  typedef typename Val<H>::T T;
+  const ConstKP kp = (ConstKP)kpp;
+  const int i = blockIdx.x * 16 + (threadIdx.x & 15), part = threadIdx.x >> 4;
+  const bool live = i < m.ncp;
+  const int cp = order[live ? i : m.ncp - 1];
+  const double xi[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
+  T u[3] = {zero_of(T()), zero_of(T()), zero_of(T())};
+  const int e0 = blockIdx.y * chunk, e1 = min(m.ne, e0 + chunk);
+  int c = live ? cls[(long long)e0 * m.ncp + cp] : 255;
+  for (int e = e0; e < e1; e++) {
+    const int next = live ? cls[(long long)min(e + 1, e1 - 1) * m.ncp + cp] : 255;
+    const int rule = c < m.n_ps ? c : 0, P = c < m.n_ps ? m.ps_gln[rule] * m.ps_gln[rule] : 0;
+    int most = P;
+    for (int mask = 1; mask < 16; mask *= 2) most = max(most, __shfl_xor(most, mask));
+    const long long q0 = (long long)e * m.npts + m.ps_off[rule];
+    for (int p0 = 0; p0 < most; p0 += 4) {
+      const int p = p0 + part;
+      const long long at = q0 + min(p, max(P - 1, 0));
+      const double* q = m.ps + at * kPsStride;
+      const double rv[3] = {q[0] - xi[0], q[1] - xi[1], q[2] - xi[2]}, n[3] = {q[3], q[4], q[5]};
+      T f[6];
+#pragma unroll
+      for (int k = 0; k < 6; k++) f[k] = field[6 * at + k];
+      point_values(kp, rv, n, p < P, f, u);
+    }
+    c = next;
+  }
+  for (int l = 0; l < 3; l++) {
+    u[l] = lane_xor_add(lane_xor_add(u[l], 16), 32);
+    if (live && part == 0) atomic_add(&out[3 * cp + l], u[l]);
   }
 }
 
@@ -2058,8 +2133,8 @@ struct mfb_mesh_s {
   int* judge_err = nullptr;
   // grow-only device workspaces of the per-assembly steps (lists, learned classes, judge): a
   // repeated assembly allocates and frees nothing
-  void* ws[11] = {};
-  size_t ws_cap[11] = {};
+  void* ws[12] = {};
+  size_t ws_cap[12] = {};
   double *x = nullptr, *cval = nullptr, *elem = nullptr, *ps = nullptr, *nfn = nullptr;
   int *conn = nullptr, *ctype = nullptr, *inc_ptr = nullptr, *inc_e = nullptr, *inc_k = nullptr;
   unsigned char* cls = nullptr;
@@ -2070,6 +2145,8 @@ struct mfb_mesh_s {
   unsigned char *nmca = nullptr, *ekind = nullptr;
   int *enode = nullptr, *cx = nullptr, *xnode = nullptr;
   int2* emask = nullptr;
+  // interior point sets: the points along a space-filling curve; the node each lies on, -1 none
+  int *order = nullptr, *snap = nullptr;
   std::vector<unsigned char> h_kind;   // kNeedH | kNeedG of each element
   bool prezero = false;            // A is reset before the tiles (enode is then ~node throughout)
   mfb::SingGeom* sgeo = nullptr;   // of the singular and the adaptive pairs, in list order
@@ -2115,13 +2192,13 @@ static void mesh_release(mfb_mesh_s* m) {
                 m->qcls, m->lcls, m->llists, m->judge_counters, m->judge_err,
                 m->xc, m->cxi, m->crow, m->cel, m->cx, m->xnode, m->nmca,
                 m->ws[0], m->ws[1], m->ws[2], m->ws[3], m->ws[4], m->ws[5], m->ws[6], m->ws[7],
-                m->ws[8], m->ws[9], m->ws[10], m->ageo,
+                m->ws[8], m->ws[9], m->ws[10], m->ws[11], m->order, m->snap, m->ageo,
                 m->tiles.d, m->ltiles.d, m->d_promo, m->ekind, m->enode, m->emask, m->sgeo};
   for (void* p : ps)
     if (p) (void)hipFree(p);
 }
 
-enum MeshWs { MW_OFF, MW_COUNTS, MW_REF, MW_BLK, MW_POS, MW_SAMPLE, MW_ERR, MW_PC, MW_AGEO, MW_JGEO, MW_EXTRA };
+enum MeshWs { MW_OFF, MW_COUNTS, MW_REF, MW_BLK, MW_POS, MW_SAMPLE, MW_ERR, MW_PC, MW_AGEO, MW_JGEO, MW_EXTRA, MW_FIELD };
 
 template <typename P>
 static int mesh_ws(mfb_mesh_s* m, int slot, size_t bytes, P** out) {
@@ -2694,11 +2771,8 @@ static int run_judge(mfb_mesh_t m, const KernelParams& kp, hipStream_t s);
 // workgroup's dynamic LDS limit (up to the 160 KB of a gfx950 CU)
 template <bool H>
 static hipError_t set_kreg_lds(size_t lds) {
-  hipError_t e = hipFuncSetAttribute((const void*)k_regular<H, kBlocks>,
+  hipError_t e = hipFuncSetAttribute((const void*)k_regular<H>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_regular<H, kVector>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   return e;
 }
 
@@ -2857,8 +2931,22 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
                          3LL * d.ncp);
     MFB_HIP(hipEventRecord(m->ev[1], s));
     m->last_regular_launches = 0;
-    // per-pair blocks and interior displacements have no shared entries: one launch per rule
-    for (int r = 0; r < d.n_ps; r++) {
+    if (vmode) {
+      T* field = nullptr;
+      const long long nq = (long long)d.ne * d.npts;
+      const int rc = mesh_ws(m, MW_FIELD, sizeof(T) * 6 * (size_t)nq, &field);
+      if (rc) return rc;
+      hipLaunchKernelGGL(k_field<T>, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, d, m->d_kp,
+                         vec, field);
+      // about 8,192 waves; fewer elements per wave would add more sums to the same points
+      const long long wv = (d.ncp + 15) / 16;
+      const int chunk = (int)std::max<long long>(1, std::max<long long>(wv * d.ne / 8192, (d.ne + 65534) / 65535));
+      hipLaunchKernelGGL(k_points<H>, dim3((unsigned)wv, (unsigned)((d.ne + chunk - 1) / chunk)),
+                         dim3(kWave), 0, s, d, m->d_kp, m->cls, m->order, field, chunk, vec.out);
+      m->last_regular_launches = 1;
+    }
+    // per-pair blocks: one launch per rule
+    for (int r = 0; r < d.n_ps && !vmode; r++) {
       const long long cnt = cls_cnt[r], o = cls_off[r];
       if (!cnt) continue;
       m->last_regular_launches++;
@@ -2866,12 +2954,8 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
       long long grid = (cnt + B - 1) / B;
       const size_t lds = kreg_lds_bytes<H>(B * P);
       if (lds > 64 * 1024) MFB_HIP(set_kreg_lds<H>(lds));
-      if (vmode)
-        hipLaunchKernelGGL((k_regular<H, kVector>), dim3((unsigned)grid), dim3(kWave), lds, s, d,
-                           m->d_kp, lists + o, (int)cnt, r, blocks, o, vec);
-      else
-        hipLaunchKernelGGL((k_regular<H, kBlocks>), dim3((unsigned)grid), dim3(kWave), lds, s, d,
-                           m->d_kp, lists + o, (int)cnt, r, blocks, o, vec);
+      hipLaunchKernelGGL(k_regular<H>, dim3((unsigned)grid), dim3(kWave), lds, s, d, m->d_kp,
+                         lists + o, (int)cnt, r, blocks, o);
     }
     MFB_HIP(hipEventRecord(m->ev[2], s));
     NearArgs<T> a{};
@@ -3214,9 +3298,8 @@ static int rule_errors(mfb_mesh_t m, const KernelParams& kp, const int* dlist, i
     launch_near<H>(d, d_qsp_ref, m->d_kp, a, -1, s);
     for (int r = 0; r < d.n_ps; r++) {
       const int P = d.ps_gln[r] * d.ps_gln[r], B = P >= kWave ? 1 : kWave / P;
-      hipLaunchKernelGGL((k_regular<H, kBlocks>), dim3((unsigned)((np + B - 1) / B)), dim3(kWave),
-                         kreg_lds_bytes<H>(B * P), s, d, m->d_kp, dlist, np, r, blk, 0LL,
-                         VecOut<T>{});
+      hipLaunchKernelGGL(k_regular<H>, dim3((unsigned)((np + B - 1) / B)), dim3(kWave),
+                         kreg_lds_bytes<H>(B * P), s, d, m->d_kp, dlist, np, r, blk, 0LL);
       hipLaunchKernelGGL(k_block_err<T>, dim3((unsigned)np), dim3(kWave), 0, s, ref, blk, d.n_ps,
                          r, err);
     }
@@ -3785,18 +3868,54 @@ struct mfb_points_s {
 // A point that coincides with a boundary node (distance below 1e-12 of the characteristic length
 // of the node's first element) takes the node's displacement, as the reference does
 // (src/calculate_internal_points_mechanics_bem_harela.f90:197-210).
-template <typename T>
-__global__ void k_snap_nodes(DevMesh m, const T* ub, T* out) {
+// (found when the set is made: blockIdx.y runs over parts of the nodes; of several the last one)
+__global__ void __launch_bounds__(128) k_snap_find(DevMesh m, int* snap) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= m.ncp) return;
   const double* xp = m.xc + 3 * p;
-  for (int i = 0; i < m.nn; i++) {
+  int found = -1;
+  for (int i = blockIdx.y; i < m.nn; i += gridDim.y) {
     if (m.inc_ptr[i + 1] == m.inc_ptr[i]) continue;
     const double cl = m.elem[8 * m.inc_e[m.inc_ptr[i]]];
     const double dx = xp[0] - m.x[3 * i], dy = xp[1] - m.x[3 * i + 1], dz = xp[2] - m.x[3 * i + 2];
-    if (sqrt(dx * dx + dy * dy + dz * dz) / cl < 1e-12)
-      for (int k = 0; k < 3; k++) out[3 * p + k] = ub[3 * i + k];
+    if (sqrt(dx * dx + dy * dy + dz * dz) / cl < 1e-12) found = i;
   }
+  if (found >= 0) atomicMax(&snap[p], found);
+}
+
+template <typename T>
+__global__ void k_snap_nodes(DevMesh m, const int* __restrict__ snap, const T* ub, T* out) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= m.ncp || snap[p] < 0) return;
+  for (int k = 0; k < 3; k++) out[3 * p + k] = ub[3 * snap[p] + k];
+}
+
+// the points in Morton order of a 1024^3 grid over their bounding box
+static std::vector<int> morton_order(int n, const double* x) {
+  double lo[3], hi[3];
+  for (int c = 0; c < 3; c++) {
+    lo[c] = hi[c] = x[c];
+    for (int i = 1; i < n; i++) {
+      lo[c] = std::min(lo[c], x[3LL * i + c]);
+      hi[c] = std::max(hi[c], x[3LL * i + c]);
+    }
+  }
+  const double side = std::max(std::max(hi[0] - lo[0], hi[1] - lo[1]), hi[2] - lo[2]);
+  const double f = side > 0 ? 1023.0 / side : 0.0;
+  std::vector<std::pair<unsigned, int>> key(n);
+  for (int i = 0; i < n; i++) {
+    unsigned k = 0;
+    for (int c = 0; c < 3; c++) {
+      const double t = (x[3LL * i + c] - lo[c]) * f;
+      const unsigned v = t > 0 ? (unsigned)std::min(t, 1023.0) : 0u;   // (NaN: 0)
+      for (int b = 0; b < 10; b++) k |= (v >> b & 1u) << (3 * b + c);
+    }
+    key[i] = {k, i};
+  }
+  std::sort(key.begin(), key.end());
+  std::vector<int> o(n);
+  for (int i = 0; i < n; i++) o[i] = key[i].second;
+  return o;
 }
 
 extern "C" int mfb_points_create(mfb_mesh_t mesh, int npts, const double* x, mfb_points_t* out) {
@@ -3813,6 +3932,23 @@ extern "C" int mfb_points_create(mfb_mesh_t mesh, int npts, const double* x, mfb
                             mesh->h_ctype.data(), mesh->h_cval.data(), d.qsi_re, d.ns_max, d.n_ps,
                             mesh->h_ps.data(), mesh->h_tol, &cs, 0.0, true, &pm);
   if (rc) return rc;
+  const std::vector<int> order = morton_order(npts, x);
+  hipError_t he = hipMalloc((void**)&pm->order, sizeof(int) * (size_t)npts);
+  if (he == hipSuccess) he = hipMalloc((void**)&pm->snap, sizeof(int) * (size_t)npts);
+  if (he == hipSuccess)
+    he = hipMemcpy(pm->order, order.data(), sizeof(int) * (size_t)npts, hipMemcpyHostToDevice);
+  if (he == hipSuccess) {
+    hipLaunchKernelGGL(k_fill_int, dim3((npts + 255) / 256), dim3(256), 0, 0, pm->snap, npts, -1);
+    hipLaunchKernelGGL(k_snap_find, dim3((npts + 127) / 128, std::min(64, d.nn)), dim3(128), 0, 0,
+                       pm->dm, pm->snap);
+    he = hipGetLastError();
+  }
+  if (he == hipSuccess) he = hipStreamSynchronize(0);
+  if (he != hipSuccess) {
+    mfb_mesh_destroy(pm);
+    set_error("mfb_points_create: %s", hipGetErrorString(he));
+    return MFB_ERR_HIP;
+  }
   mfb_points_s* p = new mfb_points_s();
   p->pm = pm;
   p->npts = npts;
@@ -3847,7 +3983,7 @@ static int points_eval(mfb_points_t p, const KernelParams& kp, const double* ub,
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(k_snap_nodes<T>, dim3((p->npts + 127) / 128), dim3(128), 0, s, p->pm->dm,
-                     (const T*)ub, (T*)out);
+                     p->pm->snap, (const T*)ub, (T*)out);
   MFB_HIP(hipGetLastError());
   MFB_HIP(hipStreamSynchronize(s));
   return MFB_OK;
