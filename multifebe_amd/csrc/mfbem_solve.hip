@@ -261,26 +261,24 @@ __global__ void __launch_bounds__(ROWS) k_col_step(T* B, long long ld, int m, in
 // (LAPACK i?amax order), the owner of the pivot row takes row j's content, row j takes the pivot
 // row, and the rows below are scaled and updated.  The arithmetic is that of k_col_step.
 //
-// Synchronisation without a shared counter: a workgroup's post is a record (tag, |a|_1) plus the
-// candidate row, written with relaxed agent-scope atomics (coherent across XCDs without cache
-// write-back or invalidation); the data is written first, the workgroup waits until it is
-// performed (s_waitcnt), and then writes the tag = (launch epoch, column, row).  Readers poll the
-// tags (one thread per workgroup slot) and read the data after seeing the tag.  Posts alternate
-// between two halves by column parity: a workgroup posts into half (j & 1) again only at column
-// j + 2, after it has seen every post of column j + 1, and each workgroup posts column j + 1 only
-// after its reads of column j.  Every spin-wait is bounded: on expiry the thread sets *err and
+// Synchronisation without a shared counter or a tag: everything posted travels in 64-bit words, a
+// 32-bit half of a value (or the row index) with a 32-bit stamp (launch epoch x 32 + column), by
+// relaxed agent-scope atomics (coherent across XCDs without cache write-back or invalidation).  A
+// reader that sees the stamp has the value, so no store has to be performed before another.  Posts
+// alternate between two halves by column parity: a workgroup posts into half (j & 1) again only at
+// column j + 2, after it has seen every post of column j + 1, and each workgroup posts column j + 1
+// only after its reads of column j.  Every spin-wait is bounded: on expiry the thread sets *err and
 // goes on, so the grid always drains (the host reports the error).
 constexpr int PANEL_GMAX = 256;   // workgroups of the persistent panel (rows <= 65,536)
 
 // Every workgroup's record sits on its own 256-byte line: posts and polls of different
 // workgroups never touch the same line.
-constexpr int REC = 32;   // record stride in 8-byte words: tag, |a|_1, padding
+constexpr int REC = 32;   // record stride in 8-byte words: |a|_1 (1 or 2 words), row, padding
 
 struct PanelSync {
-  unsigned long long* rec;   // [2][PANEL_GMAX][REC]: word 0 = epoch << 32 | column << 16 | row,
-                             // word 1 = candidate |a|_1 (double bits)
-  void* crow;                // [2][PANEL_GMAX][IB] candidate rows (T; FP32 types: stamped words)
-  void* rowj;                // [2][IB] row j (T; FP32 types: stamped words)
+  unsigned long long* rec;   // [2][PANEL_GMAX][REC] candidate records
+  unsigned long long* crow;  // [2][PANEL_GMAX][RW] candidate rows, RW words of IB entries
+  unsigned long long* rowj;  // [2][RW] row j
   unsigned* err;             // time-out flag
   unsigned spin;             // spin limit of a wait (MFB_SPIN_LIMIT; expiry sets *err)
 };
@@ -368,146 +366,44 @@ struct PanelCtx {
   T* stage;   // LDS [2 * IB]: candidate row, row J (posted one element per lane)
 };
 
-// Column J of the persistent panel for FP32 / complex FP32 entries: every posted 32-bit value
-// travels in one 64-bit word with a 32-bit stamp (launch epoch x 32 + J; a slot set is reused two
-// columns later, and only after every reader has left it), so a reader that sees the stamp has the
-// value: no store has to be performed before another (no s_waitcnt round trip between the data
-// and a tag).  Records: word 0 = stamp | |a|_1 bits, word 1 = stamp | candidate row; candidate
-// rows and row J as stamped floats.  Pivot order and arithmetic are those of the FP64 protocol.
-template <typename T, int J>
-__device__ __attribute__((always_inline)) inline void panel_col_s(T (&x)[IB], const PanelCtx<T>& k) {
-  constexpr int NW = ROWS / 64;
-  constexpr int par = J & 1;
-  constexpr int NF = sizeof(T) / sizeof(float);   // floats per entry
-  constexpr int RW = IB * NF;                      // stamped words per row
-  static_assert(64 + RW <= 128 && RW <= 64, "posting lanes");
-  const int tid = k.tid, g = k.g, r = k.r, m = k.m;
-  // bit 31 set: never equal to the upper word of the FP64 protocol's tags (the epoch itself)
-  const unsigned long long st =
-      (unsigned long long)(0x80000000u | ((k.epoch * 32u + (unsigned)J) & 0x7fffffffu)) << 32;
-  unsigned long long* crow = (unsigned long long*)k.ps.crow;   // [2][PANEL_GMAX][RW]
-  unsigned long long* rowj = (unsigned long long*)k.ps.rowj;   // [2][RW]
-  auto put = [](unsigned long long* a, unsigned long long v) {
-    __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  // a stamped word of this column (bounded spin; on expiry the flag is set and the word used)
-  auto take = [&](const unsigned long long* a) {
-    unsigned long long w = __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    unsigned spins = 0;
-    while ((w & 0xffffffff00000000ull) != st) {
-      if (++spins > k.ps.spin) {
-        atomicOr(k.ps.err, 1u);
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-      w = __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    return w;
-  };
-  // local candidate of column J among rows J .. m-1
-  float v = -1.0f;
-  int vi = 0x7fffffff;
-  if (r < m && r >= J) {
-    v = tabs1(x[J]);
-    vi = r;
-  }
-  wave_cand_max_t(v, vi);
-  if ((tid & 63) == 0) {
-    k.wv[tid >> 6] = v;
-    k.wi[tid >> 6] = vi;
-  }
-  __syncthreads();
-  float bv = k.wv[0];
-  int bi = k.wi[0];
-#pragma unroll
-  for (int q = 1; q < NW; q++) cand_max_t(bv, bi, k.wv[q], k.wi[q]);
-  if (r == bi) {
-#pragma unroll
-    for (int c = 0; c < IB; c++) k.stage[c] = x[c];
-  }
-  if (r == J) {   // workgroup 0
-#pragma unroll
-    for (int c = 0; c < IB; c++) k.stage[IB + c] = x[c];
-  }
-  __syncthreads();
-  const float* sf = (const float*)k.stage;
-  if (tid < RW)
-    put(crow + ((size_t)par * PANEL_GMAX + g) * RW + tid, st | __float_as_uint(sf[tid]));
-  if (g == 0 && tid >= 64 && tid < 64 + RW)
-    put(rowj + par * RW + (tid - 64), st | __float_as_uint(sf[RW + tid - 64]));
-  unsigned long long* myrec = k.ps.rec + ((size_t)par * PANEL_GMAX + g) * REC;
-  if (tid == 128) {
-    put(myrec, st | __float_as_uint(bv));
-    put(myrec + 1, st | (unsigned)bi);
-  }
-  // every workgroup's record of column J (thread t reads slot t), then the winner
-  v = -1.0f;
-  vi = 0x7fffffff;
-  if (tid < k.G) {
-    const unsigned long long* rt = k.ps.rec + ((size_t)par * PANEL_GMAX + tid) * REC;
-    const unsigned long long a = take(rt), b = take(rt + 1);
-    v = __uint_as_float((unsigned)a);
-    vi = (int)(unsigned)b;
-    if (v < 0.0f) vi = 0x7fffffff;   // a workgroup without rows at or below J
-  }
-  wave_cand_max_t(v, vi);
-  if ((tid & 63) == 0) {
-    k.wv[tid >> 6] = v;
-    k.wi[tid >> 6] = vi;
-  }
-  __syncthreads();
-  float pv = k.wv[0];
-  int p = k.wi[0];
-#pragma unroll
-  for (int q = 1; q < NW; q++) cand_max_t(pv, p, k.wv[q], k.wi[q]);
-  if (p < J || p >= m) p = J;   // no candidate (or data of a timed-out wait)
-  if (g == 0 && tid == 0) {
-    k.ipiv[J] = p;
-    if (pv == 0.0f && *k.info == 0) *k.info = k.gcol0 + J + 1;
-  }
-  // the pivot row and row J, one stamped word per lane
-  if (tid < RW) {
-    float* pf = (float*)k.prow;
-    pf[tid] = __uint_as_float((unsigned)take(crow + ((size_t)par * PANEL_GMAX + p / ROWS) * RW + tid));
-    if (p / ROWS == g && p != J)
-      ((float*)k.srowj)[tid] = __uint_as_float((unsigned)take(rowj + par * RW + tid));
-  }
-  __syncthreads();
-  if (r == p && p != J) {
-#pragma unroll
-    for (int c = 0; c < IB; c++) x[c] = k.srowj[c];
-  }
-  if (r == J) {
-#pragma unroll
-    for (int c = 0; c < IB; c++) x[c] = k.prow[c];
-  }
-  if (r < m && r > J) {
-    const T piv = k.prow[J];
-    if (!tiszero(piv)) {
-      const T l = tmul(x[J], trcp(piv));
-      x[J] = l;
-#pragma unroll
-      for (int c = J + 1; c < IB; c++) x[c] = tsub(x[c], tmul(l, k.prow[c]));
-    }
-  }
-}
-
 // Column J of the persistent panel (J a compile-time constant, so every register index of the
-// thread's row x is one too).
+// thread's row x is one too).  The pivot row is fetched when the pivot is known: reading the rows of
+// all workgroups while waiting for the records saves that round trip but its polls slow the posts
+// (1,707 rows: 140 against 108 us a panel).
 template <typename T, int J>
 __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], const PanelCtx<T>& k) {
   typedef typename Tr<T>::R R;
   constexpr int NW = ROWS / 64;
   constexpr int par = J & 1;
+  constexpr int NV = sizeof(R) / 4;              // words of |a|_1
+  constexpr int RW = IB * (int)(sizeof(T) / 4);  // words of a row
+  static_assert(2 * RW <= ROWS && ROWS % RW == 0, "posting threads");
   if (J >= k.w) return;   // uniform: the whole grid skips the same columns
-  if constexpr (std::is_same<R, float>::value) {
-    panel_col_s<T, J>(x, k);
-    return;
-  }
   const int tid = k.tid, g = k.g, r = k.r, m = k.m;
-  const unsigned long long stamp = ((unsigned long long)k.epoch << 32) | ((unsigned)J << 16);
-  T* crow = (T*)k.ps.crow;
-  T* rowj = (T*)k.ps.rowj;
+  // bit 31 set: never the upper word of a cleared buffer
+  const unsigned long long st =
+      (unsigned long long)(0x80000000u | ((k.epoch * 32u + (unsigned)J) & 0x7fffffffu)) << 32;
+  auto put = [](unsigned long long* a, unsigned long long v) {
+    __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto load = [](const unsigned long long* a) {
+    return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto fresh = [&](unsigned long long w) { return (w & 0xffffffff00000000ull) == st; };
+  // a stamped word of this column (bounded spin; on expiry the flag is set and the word used)
+  auto take = [&](const unsigned long long* a) {
+    unsigned long long w = load(a);
+    unsigned spins = 0;
+    while (!fresh(w)) {
+      if (++spins > k.ps.spin) {
+        atomicOr(k.ps.err, 1u);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      w = load(a);
+    }
+    return w;
+  };
   // local candidate of column J among rows J .. m-1
   R v = (R)-1;
   int vi = 0x7fffffff;
@@ -526,8 +422,7 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], cons
   int bi = k.wi[0];
 #pragma unroll
   for (int q = 1; q < NW; q++) cand_max_t(bv, bi, k.wv[q], k.wi[q]);
-  // post the data (whole rows: columns beyond w are zeros), staged through LDS so that every
-  // lane stores one element; wait until it is performed, then the tag
+  // post whole rows (columns beyond w are zeros), staged through LDS so that a lane posts one word
   if (r == bi) {
 #pragma unroll
     for (int c = 0; c < IB; c++) k.stage[c] = x[c];
@@ -537,34 +432,33 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], cons
     for (int c = 0; c < IB; c++) k.stage[IB + c] = x[c];
   }
   __syncthreads();
-  if (tid < IB && bi != 0x7fffffff)
-    post_val(crow + ((size_t)par * PANEL_GMAX + g) * IB + tid, k.stage[tid]);
-  if (g == 0 && tid >= 64 && tid < 64 + IB)
-    post_val(rowj + par * IB + (tid - 64), k.stage[IB + tid - 64]);
-  unsigned long long* myrec = k.ps.rec + ((size_t)par * PANEL_GMAX + g) * REC;
-  if (tid == 128) post_val((double*)(myrec + 1), (double)bv);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (tid == 0)
-    __hip_atomic_store(myrec, stamp | (unsigned)(bi & 0xffff), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  // wait for every workgroup's post of column J (thread t watches slot t), then the winner
+  const unsigned* sw = (const unsigned*)k.stage;
+  unsigned long long* crow = k.ps.crow + (size_t)par * PANEL_GMAX * RW;
+  unsigned long long* rowj = k.ps.rowj + par * RW;
+  unsigned long long* rec = k.ps.rec + (size_t)par * PANEL_GMAX * REC;
+  if (tid >= ROWS - 1 - NV) {   // the record: halves of |a|_1, row
+    const int q = tid - (ROWS - 1 - NV);
+    const unsigned long long vb = key_bits(bv);
+    put(rec + (size_t)g * REC + q, st | (q == NV ? (unsigned)bi : (unsigned)(vb >> (32 * q))));
+  }
+  if (tid < RW) put(crow + (size_t)g * RW + tid, st | sw[tid]);
+  if (g == 0 && tid >= ROWS - RW) put(rowj + (tid - (ROWS - RW)), st | sw[tid - (ROWS - RW) + RW]);
+  // every workgroup's record of column J (thread t reads slot t), then the winner
+  unsigned long long a[NV + 1];
+  if (tid < k.G) {
+#pragma unroll
+    for (int q = 0; q <= NV; q++) a[q] = load(rec + (size_t)tid * REC + q);   // on their way together
+#pragma unroll
+    for (int q = 0; q <= NV; q++)
+      if (!fresh(a[q])) a[q] = take(rec + (size_t)tid * REC + q);
+  }
   v = (R)-1;
   vi = 0x7fffffff;
   if (tid < k.G) {
-    const unsigned long long* rt = k.ps.rec + ((size_t)par * PANEL_GMAX + tid) * REC;
-    unsigned long long tg = 0;
-    unsigned spins = 0;
-    while (((tg = __hip_atomic_load(rt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 16) !=
-           (stamp >> 16)) {
-      if (++spins > k.ps.spin) {
-        atomicOr(k.ps.err, 1u);
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-    v = (R)fetch_val((const double*)(rt + 1));
-    vi = (int)(tg & 0xffff);
+    unsigned long long vb = (unsigned)a[0];
+    if (NV == 2) vb |= (a[NV - 1] & 0xffffffffull) << 32;
+    from_key(vb, v);
+    vi = (int)(unsigned)a[NV];
     if (v < (R)0) vi = 0x7fffffff;   // a workgroup without rows at or below J
   }
   wave_cand_max_t(v, vi);
@@ -583,11 +477,11 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], cons
     k.ipiv[J] = p;
     if (pv == (R)0 && *k.info == 0) *k.info = k.gcol0 + J + 1;
   }
-  // the pivot row and row J, one element per lane (both loads in flight together)
-  if (tid < IB) {
-    k.prow[tid] = fetch_val(crow + ((size_t)par * PANEL_GMAX + p / ROWS) * IB + tid);
-    if (p / ROWS == g && p != J) k.srowj[tid] = fetch_val(rowj + par * IB + tid);
-  }
+  // the pivot row and row J, one word per lane
+  const int pg = p / ROWS;
+  if (tid < RW) ((unsigned*)k.prow)[tid] = (unsigned)take(crow + (size_t)pg * RW + tid);
+  if (tid >= ROWS - RW && pg == g && p != J)
+    ((unsigned*)k.srowj)[tid - (ROWS - RW)] = (unsigned)take(rowj + (tid - (ROWS - RW)));
   __syncthreads();
   if (r == p && p != J) {
 #pragma unroll
@@ -1695,10 +1589,12 @@ static int ensure_ctx(hipStream_t s, int n) {
     const size_t rb = sizeof(unsigned long long) * 2 * PANEL_GMAX * REC;
     MFB_HIP(hipMalloc(&c.pan.rec, rb));
     MFB_HIP(hipMalloc(&c.pan.err, sizeof(unsigned)));
-    MFB_HIP(hipMalloc(&c.pan.crow, sizeof(cz) * 2 * PANEL_GMAX * IB));
-    MFB_HIP(hipMalloc(&c.pan.rowj, sizeof(cz) * 2 * IB));
-    MFB_HIP(hipMemset(c.pan.crow, 0, sizeof(cz) * 2 * PANEL_GMAX * IB));
-    MFB_HIP(hipMemset(c.pan.rowj, 0, sizeof(cz) * 2 * IB));
+    // rows of complex128, four words per entry
+    const size_t rowb = sizeof(unsigned long long) * 4 * IB;
+    MFB_HIP(hipMalloc(&c.pan.crow, rowb * 2 * PANEL_GMAX));
+    MFB_HIP(hipMalloc(&c.pan.rowj, rowb * 2));
+    MFB_HIP(hipMemset(c.pan.crow, 0, rowb * 2 * PANEL_GMAX));
+    MFB_HIP(hipMemset(c.pan.rowj, 0, rowb * 2));
     MFB_HIP(hipMemset(c.pan.rec, 0, rb));
     MFB_HIP(hipMemset(c.pan.err, 0, sizeof(unsigned)));
     MFB_HIP(hipDeviceSynchronize());
