@@ -546,6 +546,129 @@ __global__ void __launch_bounds__(ROWS) k_panel(T* B, long long ld, int m, int w
   }
 }
 
+// The same narrow block by one workgroup: ONE_THREADS threads hold RPT rows each (row tid +
+// ONE_THREADS q), and the column's arg-max goes through LDS and two barriers instead of two round
+// trips to the coherence point (3 us a column, the whole of k_panel's time): blocks of at most
+// panel_one_rows() rows, what the registers of a CU hold beside the temporaries.  Same pivots and
+// arithmetic.  Measured a block of 32 columns: up to 512 rows 55 us in double and 61 in complex float
+// (k_panel 97 and 107), 77 in complex double (141); up to 1536 rows 86 and 97.  Complex double keeps
+// to one row a thread: two did not fit the registers.
+constexpr int ONE_THREADS = 512;
+// Products with the roundings k_panel has, written out: which of the two products of an imaginary part
+// is rounded first would else be the compiler's choice in each kernel, and the factors of a block
+// would depend in the last bit on the kernel that takes it.
+__device__ inline double pmul(double a, double b) { return a * b; }
+__device__ inline float pmul(float a, float b) { return a * b; }
+__device__ inline cz pmul(cz a, cz b) {
+  return cz{__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im)};
+}
+__device__ inline cf pmul(cf a, cf b) {
+  return cf{__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.im, b.re, a.re * b.im)};
+}
+template <typename T>
+constexpr int panel_one_rpt() { return sizeof(T) <= 8 ? 3 : 1; }
+template <typename T>
+constexpr int panel_one_rows() { return panel_one_rpt<T>() * ONE_THREADS; }
+
+template <typename T, int RPT, int J>
+__device__ __attribute__((always_inline)) inline void panel_one_col(
+    T (&x)[RPT][IB], int m, int w, int tid, int gcol0, int* ipiv, int* info, T* prow, T* srowj,
+    typename Tr<T>::R* wv, int* wi) {
+  typedef typename Tr<T>::R R;
+  constexpr int NW = ONE_THREADS / 64;
+  if (J >= w) return;   // uniform
+  R v = (R)-1;
+  int vi = 0x7fffffff;
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = tid + ONE_THREADS * q;
+    if (r < m && r >= J) cand_max_t(v, vi, tabs1(x[q][J]), r);
+  }
+  wave_cand_max_t(v, vi);
+  if ((tid & 63) == 0) {
+    wv[tid >> 6] = v;
+    wi[tid >> 6] = vi;
+  }
+  __syncthreads();
+  R pv = wv[0];
+  int p = wi[0];
+#pragma unroll
+  for (int q = 1; q < NW; q++) cand_max_t(pv, p, wv[q], wi[q]);
+  if (p < J || p >= m) p = J;   // no candidate (every entry NaN)
+  if (tid == 0) {
+    ipiv[J] = p;
+    if (pv == (R)0 && *info == 0) *info = gcol0 + J + 1;
+  }
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = tid + ONE_THREADS * q;
+    if (r == p) {
+#pragma unroll
+      for (int c = 0; c < IB; c++) prow[c] = x[q][c];
+    }
+    if (r == J) {
+#pragma unroll
+      for (int c = 0; c < IB; c++) srowj[c] = x[q][c];
+    }
+  }
+  __syncthreads();
+  // prow, srowj and wv are written again only behind the next column's first barrier
+  const T piv = prow[J];
+  const bool zero = tiszero(piv);
+  const T inv = zero ? tzero<T>() : trcp(piv);
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = tid + ONE_THREADS * q;
+    if (r == p && p != J) {
+#pragma unroll
+      for (int c = 0; c < IB; c++) x[q][c] = srowj[c];
+    }
+    if (r == J) {
+#pragma unroll
+      for (int c = 0; c < IB; c++) x[q][c] = prow[c];
+    }
+    if (r < m && r > J && !zero) {
+      const T l = pmul(x[q][J], inv);
+      x[q][J] = l;
+#pragma unroll
+      for (int c = J + 1; c < IB; c++) x[q][c] = tsub(x[q][c], pmul(l, prow[c]));
+    }
+  }
+}
+
+template <typename T, int RPT, int... Js>
+__device__ __attribute__((always_inline)) inline void panel_one_cols(
+    T (&x)[RPT][IB], int m, int w, int tid, int gcol0, int* ipiv, int* info, T* prow, T* srowj,
+    typename Tr<T>::R* wv, int* wi, std::integer_sequence<int, Js...>) {
+  (panel_one_col<T, RPT, Js>(x, m, w, tid, gcol0, ipiv, info, prow, srowj, wv, wi), ...);
+}
+
+template <typename T, int RPT>
+__global__ void __launch_bounds__(ONE_THREADS) k_panel_one(T* B, long long ld, int m, int w,
+                                                           int* ipiv, int* info, int gcol0) {
+  typedef typename Tr<T>::R R;
+  __shared__ T prow[IB], srowj[IB];
+  __shared__ R wv[ONE_THREADS / 64];
+  __shared__ int wi[ONE_THREADS / 64];
+  const int tid = threadIdx.x;
+  T x[RPT][IB];
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = tid + ONE_THREADS * q;
+#pragma unroll
+    for (int c = 0; c < IB; c++) x[q][c] = (r < m && c < w) ? B[r + ld * c] : tzero<T>();
+  }
+  panel_one_cols<T, RPT>(x, m, w, tid, gcol0, ipiv, info, prow, srowj, wv, wi,
+                         std::make_integer_sequence<int, IB>{});
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = tid + ONE_THREADS * q;
+#pragma unroll
+    for (int c = 0; c < IB; c++)
+      if (r < m && c < w) B[r + ld * c] = x[q][c];
+  }
+}
+
 // Row interchanges.  A run of LAPACK-order swaps (row R <-> row piv(R), R = r0 .. r0+cnt-1, in
 // increasing order; piv(R) = floor(R / IB) * IB + ipiv[R] because each narrow block stores its
 // pivots relative to its first row) is turned into the net row moves it produces, dst <- src.
@@ -1873,7 +1996,15 @@ static int getrf(LU<T>& f, T* A, long long lda, int n, hipStream_t s) {
         T* Bk = P + jj + lda * (long long)jj;
         int* piv = f.ipiv + k1 + jj;
         const int grid = (mm + ROWS - 1) / ROWS;
-        if (c.panel_mode == 1 && grid <= c.panel_grid[sizeof(typename Tr<T>::R) == 8 ? 1 : 0]) {
+        if (c.panel_mode == 1 && mm <= panel_one_rows<T>()) {
+          constexpr int RPT = panel_one_rpt<T>();
+          if (mm <= ONE_THREADS)
+            hipLaunchKernelGGL((k_panel_one<T, 1>), dim3(1), dim3(ONE_THREADS), 0, s, Bk, lda, mm,
+                               w, piv, c.ps.info, k1 + jj);
+          else
+            hipLaunchKernelGGL((k_panel_one<T, RPT>), dim3(1), dim3(ONE_THREADS), 0, s, Bk, lda,
+                               mm, w, piv, c.ps.info, k1 + jj);
+        } else if (c.panel_mode == 1 && grid <= c.panel_grid[sizeof(typename Tr<T>::R) == 8 ? 1 : 0]) {
           long long ld_ = lda;
           int mm_ = mm, w_ = w, g0_ = k1 + jj;
           int* info_ = c.ps.info;
