@@ -255,14 +255,20 @@ __global__ void __launch_bounds__(ROWS) k_col_step(T* B, long long ld, int m, in
 }
 
 // Persistent narrow-block factorisation: the whole m x w block (w <= IB) in one launch (grid
-// within the co-resident capacity), one thread per row holding its row in registers for all w columns.  Column j: every
-// workgroup posts its pivot candidate (|a|_1, row) with the candidate's whole row, and workgroup
-// 0 posts row j; every workgroup then waits for all posts of column j, picks the same winner
-// (LAPACK i?amax order), the owner of the pivot row takes row j's content, row j takes the pivot
-// row, and the rows below are scaled and updated.  The arithmetic is that of k_col_step.
+// within the co-resident capacity), one thread per row holding its row in registers for all w
+// columns.  Rows are not exchanged: a thread keeps the row that it has read and the position that the
+// row has got by the interchanges so far (LAPACK's row index, what ties are broken by), and stores it
+// there in the end.  Column j: every workgroup posts its pivot candidate (|a|_1, position, workgroup)
+// with the candidate's columns from j on; every workgroup then waits for all posts of column j, picks
+// the same winner (LAPACK i?amax order), the winner and the holder of position j trade positions, and
+// the rows below are scaled and updated.  The arithmetic is that of k_col_step.  No row is stored
+// before all are read: a workgroup ends after every other one's post of the last column.  Exchanging
+// the rows themselves, staged in LDS by single lanes and posted by workgroup 0, took 144 us a block of
+// up to 4,614 complex double rows, 108 of 10,374 complex float and 100 of 1,707 double ones; positions
+// take 130, 105 and 97.
 //
 // Synchronisation without a shared counter or a tag: everything posted travels in 64-bit words, a
-// 32-bit half of a value (or the row index) with a 32-bit stamp (launch epoch x 32 + column), by
+// 32-bit half of a value (or position << 8 | workgroup) with a 32-bit stamp (launch epoch x 32 + column), by
 // relaxed agent-scope atomics (coherent across XCDs without cache write-back or invalidation).  A
 // reader that sees the stamp has the value, so no store has to be performed before another.  Posts
 // alternate between two halves by column parity: a workgroup posts into half (j & 1) again only at
@@ -270,15 +276,16 @@ __global__ void __launch_bounds__(ROWS) k_col_step(T* B, long long ld, int m, in
 // only after its reads of column j.  Every spin-wait is bounded: on expiry the thread sets *err and
 // goes on, so the grid always drains (the host reports the error).
 constexpr int PANEL_GMAX = 256;   // workgroups of the persistent panel (rows <= 65,536)
+static_assert(PANEL_GMAX <= 256, "a record holds position << 8 | workgroup");
 
 // Every workgroup's record sits on its own 256-byte line: posts and polls of different
 // workgroups never touch the same line.
-constexpr int REC = 32;   // record stride in 8-byte words: |a|_1 (1 or 2 words), row, padding
+constexpr int REC = 32;   // record stride in 8-byte words: |a|_1 (1 or 2 words), position and
+                          // workgroup, padding
 
 struct PanelSync {
   unsigned long long* rec;   // [2][PANEL_GMAX][REC] candidate records
   unsigned long long* crow;  // [2][PANEL_GMAX][RW] candidate rows, RW words of IB entries
-  unsigned long long* rowj;  // [2][RW] row j
   unsigned* err;             // time-out flag
   unsigned spin;             // spin limit of a wait (MFB_SPIN_LIMIT; expiry sets *err)
 };
@@ -354,32 +361,45 @@ __device__ inline void wave_cand_max_t(R& v, int& i) {
 template <typename T>
 struct PanelCtx {
   typedef typename Tr<T>::R R;
-  int tid, g, G, r, m, w, gcol0;
+  int tid, g, G, m, w, gcol0;
   unsigned epoch;
   int* ipiv;
   int* info;
   PanelSync ps;
   T* prow;    // LDS [IB]
-  T* srowj;   // LDS [IB]
   R* wv;      // LDS [ROWS / 64]
   int* wi;    // LDS [ROWS / 64]
-  T* stage;   // LDS [2 * IB]: candidate row, row J (posted one element per lane)
+  T* stage;   // LDS [IB]: candidate row (posted one word per lane)
 };
+
+// Products with their roundings written out: which of the two products of an imaginary part is
+// rounded first would else be the compiler's choice in each kernel, and the factors of a block
+// would depend in the last bit on the kernel that takes it.
+__device__ inline double pmul(double a, double b) { return a * b; }
+__device__ inline float pmul(float a, float b) { return a * b; }
+__device__ inline cz pmul(cz a, cz b) {
+  return cz{__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im)};
+}
+__device__ inline cf pmul(cf a, cf b) {
+  return cf{__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.im, b.re, a.re * b.im)};
+}
 
 // Column J of the persistent panel (J a compile-time constant, so every register index of the
 // thread's row x is one too).  The pivot row is fetched when the pivot is known: reading the rows of
 // all workgroups while waiting for the records saves that round trip but its polls slow the posts
 // (1,707 rows: 140 against 108 us a panel).
 template <typename T, int J>
-__device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], const PanelCtx<T>& k) {
+__device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int& pos,
+                                                                const PanelCtx<T>& k) {
   typedef typename Tr<T>::R R;
   constexpr int NW = ROWS / 64;
   constexpr int par = J & 1;
   constexpr int NV = sizeof(R) / 4;              // words of |a|_1
   constexpr int RW = IB * (int)(sizeof(T) / 4);  // words of a row
-  static_assert(2 * RW <= ROWS && ROWS % RW == 0, "posting threads");
+  constexpr int J0 = J * (int)(sizeof(T) / 4);   // first word of column J
+  static_assert(RW + NV < ROWS, "posting threads");
   if (J >= k.w) return;   // uniform: the whole grid skips the same columns
-  const int tid = k.tid, g = k.g, r = k.r, m = k.m;
+  const int tid = k.tid, g = k.g, m = k.m;
   // bit 31 set: never the upper word of a cleared buffer
   const unsigned long long st =
       (unsigned long long)(0x80000000u | ((k.epoch * 32u + (unsigned)J) & 0x7fffffffu)) << 32;
@@ -404,12 +424,12 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], cons
     }
     return w;
   };
-  // local candidate of column J among rows J .. m-1
+  // local candidate of column J among positions J .. m-1
   R v = (R)-1;
   int vi = 0x7fffffff;
-  if (r < m && r >= J) {
+  if (pos < m && pos >= J) {
     v = tabs1(x[J]);
-    vi = r;
+    vi = pos;
   }
   wave_cand_max_t(v, vi);
   if ((tid & 63) == 0) {
@@ -422,27 +442,23 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], cons
   int bi = k.wi[0];
 #pragma unroll
   for (int q = 1; q < NW; q++) cand_max_t(bv, bi, k.wv[q], k.wi[q]);
-  // post whole rows (columns beyond w are zeros), staged through LDS so that a lane posts one word
-  if (r == bi) {
+  // post the row from column J on (columns beyond w are zeros), staged through LDS so that a lane
+  // posts one word
+  if (pos == bi) {
 #pragma unroll
-    for (int c = 0; c < IB; c++) k.stage[c] = x[c];
-  }
-  if (r == J) {   // workgroup 0
-#pragma unroll
-    for (int c = 0; c < IB; c++) k.stage[IB + c] = x[c];
+    for (int c = J; c < IB; c++) k.stage[c] = x[c];
   }
   __syncthreads();
   const unsigned* sw = (const unsigned*)k.stage;
   unsigned long long* crow = k.ps.crow + (size_t)par * PANEL_GMAX * RW;
-  unsigned long long* rowj = k.ps.rowj + par * RW;
   unsigned long long* rec = k.ps.rec + (size_t)par * PANEL_GMAX * REC;
-  if (tid >= ROWS - 1 - NV) {   // the record: halves of |a|_1, row
+  if (tid >= ROWS - 1 - NV) {   // the record: halves of |a|_1, position and workgroup
     const int q = tid - (ROWS - 1 - NV);
     const unsigned long long vb = key_bits(bv);
-    put(rec + (size_t)g * REC + q, st | (q == NV ? (unsigned)bi : (unsigned)(vb >> (32 * q))));
+    const int code = bi == 0x7fffffff ? bi : bi << 8 | g;
+    put(rec + (size_t)g * REC + q, st | (q == NV ? (unsigned)code : (unsigned)(vb >> (32 * q))));
   }
-  if (tid < RW) put(crow + (size_t)g * RW + tid, st | sw[tid]);
-  if (g == 0 && tid >= ROWS - RW) put(rowj + (tid - (ROWS - RW)), st | sw[tid - (ROWS - RW) + RW]);
+  if (tid >= J0 && tid < RW) put(crow + (size_t)g * RW + tid, st | sw[tid]);
   // every workgroup's record of column J (thread t reads slot t), then the winner
   unsigned long long a[NV + 1];
   if (tid < k.G) {
@@ -469,43 +485,37 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], cons
   __syncthreads();
   // every thread picks the same winner (no second barrier)
   R pv = k.wv[0];
-  int p = k.wi[0];
+  int code = k.wi[0];
 #pragma unroll
-  for (int q = 1; q < NW; q++) cand_max_t(pv, p, k.wv[q], k.wi[q]);
-  if (p < J || p >= m) p = J;   // no candidate (or data of a timed-out wait)
+  for (int q = 1; q < NW; q++) cand_max_t(pv, code, k.wv[q], k.wi[q]);
+  int p = code >> 8, pg = code & 255;
+  if (p < J || p >= m || pg >= k.G) p = J, pg = 0;   // no candidate (or data of a timed-out wait)
   if (g == 0 && tid == 0) {
     k.ipiv[J] = p;
     if (pv == (R)0 && *k.info == 0) *k.info = k.gcol0 + J + 1;
   }
-  // the pivot row and row J, one word per lane
-  const int pg = p / ROWS;
-  if (tid < RW) ((unsigned*)k.prow)[tid] = (unsigned)take(crow + (size_t)pg * RW + tid);
-  if (tid >= ROWS - RW && pg == g && p != J)
-    ((unsigned*)k.srowj)[tid - (ROWS - RW)] = (unsigned)take(rowj + (tid - (ROWS - RW)));
+  // the pivot row, one word per lane
+  if (tid >= J0 && tid < RW)
+    ((unsigned*)k.prow)[tid] = (unsigned)take(crow + (size_t)pg * RW + tid);
   __syncthreads();
-  if (r == p && p != J) {
-#pragma unroll
-    for (int c = 0; c < IB; c++) x[c] = k.srowj[c];
-  }
-  if (r == J) {
-#pragma unroll
-    for (int c = 0; c < IB; c++) x[c] = k.prow[c];
-  }
-  if (r < m && r > J) {
+  if (pos == p) pos = J;
+  else if (pos == J) pos = p;
+  if (pos < m && pos > J) {
     const T piv = k.prow[J];
     if (!tiszero(piv)) {
-      const T l = tmul(x[J], trcp(piv));
+      const T l = pmul(x[J], trcp(piv));
       x[J] = l;
 #pragma unroll
-      for (int c = J + 1; c < IB; c++) x[c] = tsub(x[c], tmul(l, k.prow[c]));
+      for (int c = J + 1; c < IB; c++) x[c] = tsub(x[c], pmul(l, k.prow[c]));
     }
   }
 }
 
 template <typename T, int... Js>
-__device__ __attribute__((always_inline)) inline void panel_cols(T (&x)[IB], const PanelCtx<T>& k,
+__device__ __attribute__((always_inline)) inline void panel_cols(T (&x)[IB], int& pos,
+                                                                 const PanelCtx<T>& k,
                                                                  std::integer_sequence<int, Js...>) {
-  (panel_col<T, Js>(x, k), ...);
+  (panel_col<T, Js>(x, pos, k), ...);
 }
 
 template <typename T>
@@ -513,14 +523,13 @@ __global__ void __launch_bounds__(ROWS) k_panel(T* B, long long ld, int m, int w
                                                 PanelSync ps, int* info, int gcol0,
                                                 unsigned epoch) {
   typedef typename Tr<T>::R R;
-  __shared__ T prow[IB], srowj[IB], stage[2 * IB];
+  __shared__ T prow[IB], stage[IB];
   __shared__ R wv[ROWS / 64];
   __shared__ int wi[ROWS / 64];
   PanelCtx<T> k;
   k.tid = threadIdx.x;
   k.g = blockIdx.x;
   k.G = gridDim.x;
-  k.r = k.g * ROWS + k.tid;
   k.m = m;
   k.w = w;
   k.gcol0 = gcol0;
@@ -529,20 +538,20 @@ __global__ void __launch_bounds__(ROWS) k_panel(T* B, long long ld, int m, int w
   k.info = info;
   k.ps = ps;
   k.prow = prow;
-  k.srowj = srowj;
   k.wv = wv;
   k.wi = wi;
   k.stage = stage;
-  const int r = k.r;
+  const int r = k.g * ROWS + k.tid;
   // the thread's row, zero beyond column w (the updates run unmasked over IB columns)
   T x[IB];
 #pragma unroll
   for (int c = 0; c < IB; c++) x[c] = (r < m && c < w) ? B[r + ld * c] : tzero<T>();
-  panel_cols<T>(x, k, std::make_integer_sequence<int, IB>{});
+  int pos = r;
+  panel_cols<T>(x, pos, k, std::make_integer_sequence<int, IB>{});
   if (r < m) {
 #pragma unroll
     for (int c = 0; c < IB; c++)
-      if (c < w) B[r + ld * c] = x[c];
+      if (c < w) B[pos + ld * c] = x[c];
   }
 }
 
@@ -550,21 +559,11 @@ __global__ void __launch_bounds__(ROWS) k_panel(T* B, long long ld, int m, int w
 // ONE_THREADS q), and the column's arg-max goes through LDS and two barriers instead of two round
 // trips to the coherence point (3 us a column, the whole of k_panel's time): blocks of at most
 // panel_one_rows() rows, what the registers of a CU hold beside the temporaries.  Same pivots and
-// arithmetic.  Measured a block of 32 columns: up to 512 rows 55 us in double and 61 in complex float
-// (k_panel 97 and 107), 77 in complex double (141); up to 1536 rows 86 and 97.  Complex double keeps
-// to one row a thread: two did not fit the registers.
+// arithmetic.  Measured a block of 32 columns: up to 512 rows 46 us in double, 52 in complex float and
+// 59 in complex double (k_panel 97, 105 and 130), up to 1536 rows 72 and 82 (55, 61, 77, 86 and 97 with
+// the rows exchanged instead of their positions).  Complex double keeps to one row a thread: two did
+// not fit the registers.
 constexpr int ONE_THREADS = 512;
-// Products with the roundings k_panel has, written out: which of the two products of an imaginary part
-// is rounded first would else be the compiler's choice in each kernel, and the factors of a block
-// would depend in the last bit on the kernel that takes it.
-__device__ inline double pmul(double a, double b) { return a * b; }
-__device__ inline float pmul(float a, float b) { return a * b; }
-__device__ inline cz pmul(cz a, cz b) {
-  return cz{__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im)};
-}
-__device__ inline cf pmul(cf a, cf b) {
-  return cf{__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.im, b.re, a.re * b.im)};
-}
 template <typename T>
 constexpr int panel_one_rpt() { return sizeof(T) <= 8 ? 3 : 1; }
 template <typename T>
@@ -572,18 +571,16 @@ constexpr int panel_one_rows() { return panel_one_rpt<T>() * ONE_THREADS; }
 
 template <typename T, int RPT, int J>
 __device__ __attribute__((always_inline)) inline void panel_one_col(
-    T (&x)[RPT][IB], int m, int w, int tid, int gcol0, int* ipiv, int* info, T* prow, T* srowj,
-    typename Tr<T>::R* wv, int* wi) {
+    T (&x)[RPT][IB], int (&pos)[RPT], int m, int w, int tid, int gcol0, int* ipiv, int* info,
+    T* prow, typename Tr<T>::R* wv, int* wi) {
   typedef typename Tr<T>::R R;
   constexpr int NW = ONE_THREADS / 64;
   if (J >= w) return;   // uniform
   R v = (R)-1;
   int vi = 0x7fffffff;
 #pragma unroll
-  for (int q = 0; q < RPT; q++) {
-    const int r = tid + ONE_THREADS * q;
-    if (r < m && r >= J) cand_max_t(v, vi, tabs1(x[q][J]), r);
-  }
+  for (int q = 0; q < RPT; q++)
+    if (pos[q] < m && pos[q] >= J) cand_max_t(v, vi, tabs1(x[q][J]), pos[q]);
   wave_cand_max_t(v, vi);
   if ((tid & 63) == 0) {
     wv[tid >> 6] = v;
@@ -601,72 +598,59 @@ __device__ __attribute__((always_inline)) inline void panel_one_col(
   }
 #pragma unroll
   for (int q = 0; q < RPT; q++) {
-    const int r = tid + ONE_THREADS * q;
-    if (r == p) {
+    if (pos[q] == p) {
+      pos[q] = J;
 #pragma unroll
-      for (int c = 0; c < IB; c++) prow[c] = x[q][c];
-    }
-    if (r == J) {
-#pragma unroll
-      for (int c = 0; c < IB; c++) srowj[c] = x[q][c];
+      for (int c = J; c < IB; c++) prow[c] = x[q][c];
+    } else if (pos[q] == J) {
+      pos[q] = p;
     }
   }
   __syncthreads();
-  // prow, srowj and wv are written again only behind the next column's first barrier
+  // prow and wv are written again only behind the next column's first barrier
   const T piv = prow[J];
   const bool zero = tiszero(piv);
   const T inv = zero ? tzero<T>() : trcp(piv);
 #pragma unroll
-  for (int q = 0; q < RPT; q++) {
-    const int r = tid + ONE_THREADS * q;
-    if (r == p && p != J) {
-#pragma unroll
-      for (int c = 0; c < IB; c++) x[q][c] = srowj[c];
-    }
-    if (r == J) {
-#pragma unroll
-      for (int c = 0; c < IB; c++) x[q][c] = prow[c];
-    }
-    if (r < m && r > J && !zero) {
+  for (int q = 0; q < RPT; q++)
+    if (pos[q] < m && pos[q] > J && !zero) {
       const T l = pmul(x[q][J], inv);
       x[q][J] = l;
 #pragma unroll
       for (int c = J + 1; c < IB; c++) x[q][c] = tsub(x[q][c], pmul(l, prow[c]));
     }
-  }
 }
 
 template <typename T, int RPT, int... Js>
 __device__ __attribute__((always_inline)) inline void panel_one_cols(
-    T (&x)[RPT][IB], int m, int w, int tid, int gcol0, int* ipiv, int* info, T* prow, T* srowj,
-    typename Tr<T>::R* wv, int* wi, std::integer_sequence<int, Js...>) {
-  (panel_one_col<T, RPT, Js>(x, m, w, tid, gcol0, ipiv, info, prow, srowj, wv, wi), ...);
+    T (&x)[RPT][IB], int (&pos)[RPT], int m, int w, int tid, int gcol0, int* ipiv, int* info,
+    T* prow, typename Tr<T>::R* wv, int* wi, std::integer_sequence<int, Js...>) {
+  (panel_one_col<T, RPT, Js>(x, pos, m, w, tid, gcol0, ipiv, info, prow, wv, wi), ...);
 }
 
 template <typename T, int RPT>
 __global__ void __launch_bounds__(ONE_THREADS) k_panel_one(T* B, long long ld, int m, int w,
                                                            int* ipiv, int* info, int gcol0) {
   typedef typename Tr<T>::R R;
-  __shared__ T prow[IB], srowj[IB];
+  __shared__ T prow[IB];
   __shared__ R wv[ONE_THREADS / 64];
   __shared__ int wi[ONE_THREADS / 64];
   const int tid = threadIdx.x;
   T x[RPT][IB];
+  int pos[RPT];
 #pragma unroll
   for (int q = 0; q < RPT; q++) {
-    const int r = tid + ONE_THREADS * q;
+    const int r = pos[q] = tid + ONE_THREADS * q;
 #pragma unroll
     for (int c = 0; c < IB; c++) x[q][c] = (r < m && c < w) ? B[r + ld * c] : tzero<T>();
   }
-  panel_one_cols<T, RPT>(x, m, w, tid, gcol0, ipiv, info, prow, srowj, wv, wi,
+  panel_one_cols<T, RPT>(x, pos, m, w, tid, gcol0, ipiv, info, prow, wv, wi,
                          std::make_integer_sequence<int, IB>{});
 #pragma unroll
-  for (int q = 0; q < RPT; q++) {
-    const int r = tid + ONE_THREADS * q;
+  for (int q = 0; q < RPT; q++)
 #pragma unroll
     for (int c = 0; c < IB; c++)
-      if (r < m && c < w) B[r + ld * c] = x[q][c];
-  }
+      if (pos[q] < m && c < w) B[pos[q] + ld * c] = x[q][c];
 }
 
 // Row interchanges.  A run of LAPACK-order swaps (row R <-> row piv(R), R = r0 .. r0+cnt-1, in
@@ -1715,9 +1699,7 @@ static int ensure_ctx(hipStream_t s, int n) {
     // rows of complex128, four words per entry
     const size_t rowb = sizeof(unsigned long long) * 4 * IB;
     MFB_HIP(hipMalloc(&c.pan.crow, rowb * 2 * PANEL_GMAX));
-    MFB_HIP(hipMalloc(&c.pan.rowj, rowb * 2));
     MFB_HIP(hipMemset(c.pan.crow, 0, rowb * 2 * PANEL_GMAX));
-    MFB_HIP(hipMemset(c.pan.rowj, 0, rowb * 2));
     MFB_HIP(hipMemset(c.pan.rec, 0, rb));
     MFB_HIP(hipMemset(c.pan.err, 0, sizeof(unsigned)));
     MFB_HIP(hipDeviceSynchronize());
@@ -3346,7 +3328,7 @@ static void shutdown_solver() {
   if (c.ev_fork) (void)hipEventDestroy(c.ev_fork);
   if (c.ev_join) (void)hipEventDestroy(c.ev_join);
   void* bufs[] = {c.ps.val, c.ps.idx, c.ps.counter, c.ps.info, c.moves, c.nmoves, c.pan.rec,
-                  c.pan.err, c.pan.crow, c.pan.rowj, c.sol.rec, c.sol.err};
+                  c.pan.err, c.pan.crow, c.sol.rec, c.sol.err};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (int k = 0; k < WS_COUNT; k++)
