@@ -332,30 +332,66 @@ __device__ inline void cand_max_t(R& v, int& i, R v2, int i2) {
     i = i2;
   }
 }
-// Wave arg-max in pivot order through the wave-reduction library (DPP, no LDS round trips):
-// the largest |a|_1 (non-negative, so its IEEE bits order like the values), then the lowest row
-// among the lanes that hold it.  v < 0 marks a lane without a candidate; a wave without any
-// candidate returns v = -1, i = INT_MAX.
-extern "C" __device__ __attribute__((const)) unsigned long long __ockl_wfred_max_u64(
-    unsigned long long);
+// Wave arg-max in pivot order through the wave-reduction library (DPP, no LDS round trips): the
+// largest |a|_1 (non-negative, so its IEEE bits order like the values), then the lowest row.  The
+// upper 32 bits of a double decide mostly: a step on 32 bits is one instruction, on 64 a chain of
+// five, and the row needs a reduction of its own only where two lanes hold the same.  A column has one
+// such arg-max in k_panel_one and two in k_panel: 46 -> 39 us a block of 512 double rows, 105 -> 95
+// of 10,374 complex float ones, with the waves' results compared pairwise instead of one by one.  v < 0 marks a
+// lane without a candidate; a wave without any candidate returns v = -1, i = INT_MAX.
+extern "C" __device__ __attribute__((const)) unsigned __ockl_wfred_max_u32(unsigned);
 extern "C" __device__ __attribute__((const)) int __ockl_wfred_min_i32(int);
-__device__ inline unsigned long long key_bits(float v) { return __float_as_uint(v); }
-__device__ inline unsigned long long key_bits(double v) { return (unsigned long long)__double_as_longlong(v); }
-__device__ inline void from_key(unsigned long long k, float& v) { v = __uint_as_float((unsigned)k); }
-__device__ inline void from_key(unsigned long long k, double& v) { v = __longlong_as_double((long long)k); }
+__device__ inline unsigned upper_bits(float v) { return __float_as_uint(v); }
+__device__ inline unsigned upper_bits(double v) { return (unsigned)__double2hiint(v); }
+__device__ inline unsigned lower_bits(float) { return 0u; }
+__device__ inline unsigned lower_bits(double v) { return (unsigned)__double2loint(v); }
+__device__ inline void from_bits(unsigned hi, unsigned, float& v) { v = __uint_as_float(hi); }
+__device__ inline void from_bits(unsigned hi, unsigned lo, double& v) {
+  v = __hiloint2double((int)hi, (int)lo);
+}
 
 template <typename R>
 __device__ inline void wave_cand_max_t(R& v, int& i) {
-  const bool has = v >= (R)0;
-  const unsigned long long key = has ? key_bits(v) : 0ull;
-  const unsigned long long kmax = __ockl_wfred_max_u64(key);
-  const int imin = __ockl_wfred_min_i32(has && key == kmax ? i : 0x7fffffff);
-  if (imin == 0x7fffffff) {
+  bool has = v >= (R)0;
+  const unsigned hi = upper_bits(v), lo = lower_bits(v);
+  const unsigned hmax = __ockl_wfred_max_u32(has ? hi : 0u);
+  has = has && hi == hmax;
+  unsigned long long lanes = __ballot(has);
+  if (!lanes) {
     v = (R)-1;
-  } else {
-    from_key(kmax, v);
+    i = 0x7fffffff;
+    return;
   }
-  i = imin;
+  if (lanes & (lanes - 1)) {
+    if (sizeof(R) == 8) {
+      const unsigned lmax = __ockl_wfred_max_u32(has ? lo : 0u);   // by all lanes
+      has = has && lo == lmax;
+    }
+    const int imin = __ockl_wfred_min_i32(has ? i : 0x7fffffff);
+    lanes = __ballot(has && i == imin);
+  }
+  const int l = __builtin_ctzll(lanes);
+  from_bits(hmax, (unsigned)__builtin_amdgcn_readlane((int)lo, l), v);
+  i = __builtin_amdgcn_readlane(i, l);
+}
+
+// the same over the N waves' candidates in LDS (read by every thread), pairwise
+template <int N, typename R>
+__device__ __attribute__((always_inline)) inline void block_cand_max_t(const R* wv, const int* wi,
+                                                                       R& v, int& i) {
+  R a[N];
+  int b[N];
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    a[q] = wv[q];
+    b[q] = wi[q];
+  }
+#pragma unroll
+  for (int d = N / 2; d > 0; d /= 2)
+#pragma unroll
+    for (int q = 0; q < d; q++) cand_max_t(a[q], b[q], a[q + d], b[q + d]);
+  v = a[0];
+  i = b[0];
 }
 
 template <typename T>
@@ -438,10 +474,9 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   }
   __syncthreads();
   // every thread combines the waves' candidates (no second barrier)
-  R bv = k.wv[0];
-  int bi = k.wi[0];
-#pragma unroll
-  for (int q = 1; q < NW; q++) cand_max_t(bv, bi, k.wv[q], k.wi[q]);
+  R bv;
+  int bi;
+  block_cand_max_t<NW>(k.wv, k.wi, bv, bi);
   // post the row from column J on (columns beyond w are zeros), staged through LDS so that a lane
   // posts one word
   if (pos == bi) {
@@ -454,9 +489,8 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   unsigned long long* rec = k.ps.rec + (size_t)par * PANEL_GMAX * REC;
   if (tid >= ROWS - 1 - NV) {   // the record: halves of |a|_1, position and workgroup
     const int q = tid - (ROWS - 1 - NV);
-    const unsigned long long vb = key_bits(bv);
     const int code = bi == 0x7fffffff ? bi : bi << 8 | g;
-    put(rec + (size_t)g * REC + q, st | (q == NV ? (unsigned)code : (unsigned)(vb >> (32 * q))));
+    put(rec + (size_t)g * REC + q, st | (q == NV ? (unsigned)code : q ? lower_bits(bv) : upper_bits(bv)));
   }
   if (tid >= J0 && tid < RW) put(crow + (size_t)g * RW + tid, st | sw[tid]);
   // every workgroup's record of column J (thread t reads slot t), then the winner
@@ -471,9 +505,7 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   v = (R)-1;
   vi = 0x7fffffff;
   if (tid < k.G) {
-    unsigned long long vb = (unsigned)a[0];
-    if (NV == 2) vb |= (a[NV - 1] & 0xffffffffull) << 32;
-    from_key(vb, v);
+    from_bits((unsigned)a[0], (unsigned)a[NV - 1], v);
     vi = (int)(unsigned)a[NV];
     if (v < (R)0) vi = 0x7fffffff;   // a workgroup without rows at or below J
   }
@@ -484,10 +516,9 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   }
   __syncthreads();
   // every thread picks the same winner (no second barrier)
-  R pv = k.wv[0];
-  int code = k.wi[0];
-#pragma unroll
-  for (int q = 1; q < NW; q++) cand_max_t(pv, code, k.wv[q], k.wi[q]);
+  R pv;
+  int code;
+  block_cand_max_t<NW>(k.wv, k.wi, pv, code);
   int p = code >> 8, pg = code & 255;
   if (p < J || p >= m || pg >= k.G) p = J, pg = 0;   // no candidate (or data of a timed-out wait)
   if (g == 0 && tid == 0) {
@@ -559,10 +590,10 @@ __global__ void __launch_bounds__(ROWS) k_panel(T* B, long long ld, int m, int w
 // ONE_THREADS q), and the column's arg-max goes through LDS and two barriers instead of two round
 // trips to the coherence point (3 us a column, the whole of k_panel's time): blocks of at most
 // panel_one_rows() rows, what the registers of a CU hold beside the temporaries.  Same pivots and
-// arithmetic.  Measured a block of 32 columns: up to 512 rows 46 us in double, 52 in complex float and
-// 59 in complex double (k_panel 97, 105 and 130), up to 1536 rows 72 and 82 (55, 61, 77, 86 and 97 with
-// the rows exchanged instead of their positions).  Complex double keeps to one row a thread: two did
-// not fit the registers.
+// arithmetic.  Measured a block of 32 columns: up to 512 rows 39 us in double, 44 in complex float and
+// 53 in complex double (k_panel 97, 95 and 130), up to 1536 rows 66 and 74 (55, 61, 77, 86 and 97 with
+// the rows exchanged instead of their positions and the arg-max on 64 bits).  Complex double keeps to
+// one row a thread: two did not fit the registers.
 constexpr int ONE_THREADS = 512;
 template <typename T>
 constexpr int panel_one_rpt() { return sizeof(T) <= 8 ? 3 : 1; }
@@ -587,10 +618,9 @@ __device__ __attribute__((always_inline)) inline void panel_one_col(
     wi[tid >> 6] = vi;
   }
   __syncthreads();
-  R pv = wv[0];
-  int p = wi[0];
-#pragma unroll
-  for (int q = 1; q < NW; q++) cand_max_t(pv, p, wv[q], wi[q]);
+  R pv;
+  int p;
+  block_cand_max_t<NW>(wv, wi, pv, p);
   if (p < J || p >= m) p = J;   // no candidate (every entry NaN)
   if (tid == 0) {
     ipiv[J] = p;
