@@ -259,13 +259,15 @@ __global__ void __launch_bounds__(ROWS) k_col_step(T* B, long long ld, int m, in
 // columns.  Rows are not exchanged: a thread keeps the row that it has read and the position that the
 // row has got by the interchanges so far (LAPACK's row index, what ties are broken by), and stores it
 // there in the end.  Column j: every workgroup posts its pivot candidate (|a|_1, position, workgroup)
-// with the candidate's columns from j on; every workgroup then waits for all posts of column j, picks
+// with the candidate's columns from j on, and behind them the candidate's reciprocal, which is formed
+// while the records travel; every workgroup then waits for all posts of column j, picks
 // the same winner (LAPACK i?amax order), the winner and the holder of position j trade positions, and
 // the rows below are scaled and updated.  The arithmetic is that of k_col_step.  No row is stored
 // before all are read: a workgroup ends after every other one's post of the last column.  Exchanging
 // the rows themselves, staged in LDS by single lanes and posted by workgroup 0, took 144 us a block of
 // up to 4,614 complex double rows, 108 of 10,374 complex float and 100 of 1,707 double ones; positions
-// take 130, 105 and 97.
+// took 130, 105 and 97, and 123, 90 and 89 with the reciprocal posted instead of formed by every thread
+// once it has the pivot (and the arg-max below).
 //
 // Synchronisation without a shared counter or a tag: everything posted travels in 64-bit words, a
 // 32-bit half of a value (or position << 8 | workgroup) with a 32-bit stamp (launch epoch x 32 + column), by
@@ -285,7 +287,7 @@ constexpr int REC = 32;   // record stride in 8-byte words: |a|_1 (1 or 2 words)
 
 struct PanelSync {
   unsigned long long* rec;   // [2][PANEL_GMAX][REC] candidate records
-  unsigned long long* crow;  // [2][PANEL_GMAX][RW] candidate rows, RW words of IB entries
+  unsigned long long* crow;  // [2][PANEL_GMAX][CW] candidate rows: words of IB entries, reciprocal
   unsigned* err;             // time-out flag
   unsigned spin;             // spin limit of a wait (MFB_SPIN_LIMIT; expiry sets *err)
 };
@@ -337,8 +339,8 @@ __device__ inline void cand_max_t(R& v, int& i, R v2, int i2) {
 // upper 32 bits of a double decide mostly: a step on 32 bits is one instruction, on 64 a chain of
 // five, and the row needs a reduction of its own only where two lanes hold the same.  A column has one
 // such arg-max in k_panel_one and two in k_panel: 46 -> 39 us a block of 512 double rows, 105 -> 95
-// of 10,374 complex float ones, with the waves' results compared pairwise instead of one by one.  v < 0 marks a
-// lane without a candidate; a wave without any candidate returns v = -1, i = INT_MAX.
+// of 10,374 complex float ones, with the waves' results compared pairwise instead of one by one.
+// v < 0 marks a lane without a candidate; a wave without any candidate returns v = -1, i = INT_MAX.
 extern "C" __device__ __attribute__((const)) unsigned __ockl_wfred_max_u32(unsigned);
 extern "C" __device__ __attribute__((const)) int __ockl_wfred_min_i32(int);
 __device__ inline unsigned upper_bits(float v) { return __float_as_uint(v); }
@@ -402,7 +404,7 @@ struct PanelCtx {
   int* ipiv;
   int* info;
   PanelSync ps;
-  T* prow;    // LDS [IB]
+  T* prow;    // LDS [IB + 1]: pivot row, reciprocal of the pivot
   R* wv;      // LDS [ROWS / 64]
   int* wi;    // LDS [ROWS / 64]
   T* stage;   // LDS [IB]: candidate row (posted one word per lane)
@@ -431,9 +433,10 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   constexpr int NW = ROWS / 64;
   constexpr int par = J & 1;
   constexpr int NV = sizeof(R) / 4;              // words of |a|_1
-  constexpr int RW = IB * (int)(sizeof(T) / 4);  // words of a row
-  constexpr int J0 = J * (int)(sizeof(T) / 4);   // first word of column J
-  static_assert(RW + NV < ROWS, "posting threads");
+  constexpr int WE = (int)(sizeof(T) / 4);       // words of an entry
+  constexpr int RW = IB * WE, CW = RW + WE;      // words of a row, with the reciprocal
+  constexpr int J0 = J * WE;                     // first word of column J
+  static_assert(CW + NV < ROWS, "posting threads");
   if (J >= k.w) return;   // uniform: the whole grid skips the same columns
   const int tid = k.tid, g = k.g, m = k.m;
   // bit 31 set: never the upper word of a cleared buffer
@@ -485,14 +488,21 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   }
   __syncthreads();
   const unsigned* sw = (const unsigned*)k.stage;
-  unsigned long long* crow = k.ps.crow + (size_t)par * PANEL_GMAX * RW;
+  unsigned long long* crow = k.ps.crow + ((size_t)par * PANEL_GMAX + g) * CW;
   unsigned long long* rec = k.ps.rec + (size_t)par * PANEL_GMAX * REC;
   if (tid >= ROWS - 1 - NV) {   // the record: halves of |a|_1, position and workgroup
     const int q = tid - (ROWS - 1 - NV);
     const int code = bi == 0x7fffffff ? bi : bi << 8 | g;
     put(rec + (size_t)g * REC + q, st | (q == NV ? (unsigned)code : q ? lower_bits(bv) : upper_bits(bv)));
   }
-  if (tid >= J0 && tid < RW) put(crow + (size_t)g * RW + tid, st | sw[tid]);
+  if (tid >= J0 && tid < RW) put(crow + tid, st | sw[tid]);
+  if (bi == 0x7fffffff ? tid == 0 : pos == bi) {
+    const T inv = bi == 0x7fffffff || tiszero(x[J]) ? tzero<T>() : trcp(x[J]);
+    unsigned iw[WE];
+    __builtin_memcpy(iw, &inv, sizeof(T));
+#pragma unroll
+    for (int q = 0; q < WE; q++) put(crow + RW + q, st | iw[q]);
+  }
   // every workgroup's record of column J (thread t reads slot t), then the winner
   unsigned long long a[NV + 1];
   if (tid < k.G) {
@@ -525,16 +535,15 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
     k.ipiv[J] = p;
     if (pv == (R)0 && *k.info == 0) *k.info = k.gcol0 + J + 1;
   }
-  // the pivot row, one word per lane
-  if (tid >= J0 && tid < RW)
-    ((unsigned*)k.prow)[tid] = (unsigned)take(crow + (size_t)pg * RW + tid);
+  // the pivot row and the reciprocal, one word per lane
+  if (tid >= J0 && tid < CW)
+    ((unsigned*)k.prow)[tid] = (unsigned)take(crow + (long long)(pg - g) * CW + tid);
   __syncthreads();
   if (pos == p) pos = J;
   else if (pos == J) pos = p;
   if (pos < m && pos > J) {
-    const T piv = k.prow[J];
-    if (!tiszero(piv)) {
-      const T l = pmul(x[J], trcp(piv));
+    if (!tiszero(k.prow[J])) {
+      const T l = pmul(x[J], k.prow[IB]);
       x[J] = l;
 #pragma unroll
       for (int c = J + 1; c < IB; c++) x[c] = tsub(x[c], pmul(l, k.prow[c]));
@@ -554,7 +563,7 @@ __global__ void __launch_bounds__(ROWS) k_panel(T* B, long long ld, int m, int w
                                                 PanelSync ps, int* info, int gcol0,
                                                 unsigned epoch) {
   typedef typename Tr<T>::R R;
-  __shared__ T prow[IB], stage[IB];
+  __shared__ T prow[IB + 1], stage[IB];
   __shared__ R wv[ROWS / 64];
   __shared__ int wi[ROWS / 64];
   PanelCtx<T> k;
@@ -591,7 +600,7 @@ __global__ void __launch_bounds__(ROWS) k_panel(T* B, long long ld, int m, int w
 // trips to the coherence point (3 us a column, the whole of k_panel's time): blocks of at most
 // panel_one_rows() rows, what the registers of a CU hold beside the temporaries.  Same pivots and
 // arithmetic.  Measured a block of 32 columns: up to 512 rows 39 us in double, 44 in complex float and
-// 53 in complex double (k_panel 97, 95 and 130), up to 1536 rows 66 and 74 (55, 61, 77, 86 and 97 with
+// 53 in complex double (k_panel 89, 90 and 123), up to 1536 rows 66 and 74 (55, 61, 77, 86 and 97 with
 // the rows exchanged instead of their positions and the arg-max on 64 bits).  Complex double keeps to
 // one row a thread: two did not fit the registers.
 constexpr int ONE_THREADS = 512;
@@ -1727,7 +1736,7 @@ static int ensure_ctx(hipStream_t s, int n) {
     MFB_HIP(hipMalloc(&c.pan.rec, rb));
     MFB_HIP(hipMalloc(&c.pan.err, sizeof(unsigned)));
     // rows of complex128, four words per entry
-    const size_t rowb = sizeof(unsigned long long) * 4 * IB;
+    const size_t rowb = sizeof(unsigned long long) * 4 * (IB + 1);
     MFB_HIP(hipMalloc(&c.pan.crow, rowb * 2 * PANEL_GMAX));
     MFB_HIP(hipMemset(c.pan.crow, 0, rowb * 2 * PANEL_GMAX));
     MFB_HIP(hipMemset(c.pan.rec, 0, rb));
