@@ -267,7 +267,9 @@ __global__ void __launch_bounds__(ROWS) k_col_step(T* B, long long ld, int m, in
 // the rows themselves, staged in LDS by single lanes and posted by workgroup 0, took 144 us a block of
 // up to 4,614 complex double rows, 108 of 10,374 complex float and 100 of 1,707 double ones; positions
 // took 130, 105 and 97, and 123, 90 and 89 with the reciprocal posted instead of formed by every thread
-// once it has the pivot (and the arg-max below).
+// once it has the pivot (and the arg-max below).  The record goes out before the row is staged for its
+// post, 115, 85 and 86, and a column's update of all but the next one waits until the next one's record
+// is out: 113, 84 and 84.
 //
 // Synchronisation without a shared counter or a tag: everything posted travels in 64-bit words, a
 // 32-bit half of a value (or position << 8 | workgroup) with a 32-bit stamp (launch epoch x 32 + column), by
@@ -427,7 +429,8 @@ __device__ inline cf pmul(cf a, cf b) {
 // all workgroups while waiting for the records saves that round trip but its polls slow the posts
 // (1,707 rows: 140 against 108 us a panel).
 template <typename T, int J>
-__device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int& pos,
+__device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int& pos, T& l,
+                                                                bool& below,
                                                                 const PanelCtx<T>& k) {
   typedef typename Tr<T>::R R;
   constexpr int NW = ROWS / 64;
@@ -480,6 +483,17 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   R bv;
   int bi;
   block_cand_max_t<NW>(k.wv, k.wi, bv, bi);
+  unsigned long long* rec = k.ps.rec + (size_t)par * PANEL_GMAX * REC;
+  if (tid >= ROWS - 1 - NV) {   // the record: halves of |a|_1, position and workgroup
+    const int q = tid - (ROWS - 1 - NV);
+    const int code = bi == 0x7fffffff ? bi : bi << 8 | g;
+    put(rec + (size_t)g * REC + q, st | (q == NV ? (unsigned)code : q ? lower_bits(bv) : upper_bits(bv)));
+  }
+  // column J - 1's update of the columns behind J, while the records travel
+  if (J > 0 && below) {
+#pragma unroll
+    for (int c = J + 1; c < IB; c++) x[c] = tsub(x[c], pmul(l, k.prow[c]));
+  }
   // post the row from column J on (columns beyond w are zeros), staged through LDS so that a lane
   // posts one word
   if (pos == bi) {
@@ -489,12 +503,6 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   __syncthreads();
   const unsigned* sw = (const unsigned*)k.stage;
   unsigned long long* crow = k.ps.crow + ((size_t)par * PANEL_GMAX + g) * CW;
-  unsigned long long* rec = k.ps.rec + (size_t)par * PANEL_GMAX * REC;
-  if (tid >= ROWS - 1 - NV) {   // the record: halves of |a|_1, position and workgroup
-    const int q = tid - (ROWS - 1 - NV);
-    const int code = bi == 0x7fffffff ? bi : bi << 8 | g;
-    put(rec + (size_t)g * REC + q, st | (q == NV ? (unsigned)code : q ? lower_bits(bv) : upper_bits(bv)));
-  }
   if (tid >= J0 && tid < RW) put(crow + tid, st | sw[tid]);
   if (bi == 0x7fffffff ? tid == 0 : pos == bi) {
     const T inv = bi == 0x7fffffff || tiszero(x[J]) ? tzero<T>() : trcp(x[J]);
@@ -541,13 +549,10 @@ __device__ __attribute__((always_inline)) inline void panel_col(T (&x)[IB], int&
   __syncthreads();
   if (pos == p) pos = J;
   else if (pos == J) pos = p;
-  if (pos < m && pos > J) {
-    if (!tiszero(k.prow[J])) {
-      const T l = pmul(x[J], k.prow[IB]);
-      x[J] = l;
-#pragma unroll
-      for (int c = J + 1; c < IB; c++) x[c] = tsub(x[c], pmul(l, k.prow[c]));
-    }
+  below = pos < m && pos > J && !tiszero(k.prow[J]);
+  if (below) {
+    x[J] = l = pmul(x[J], k.prow[IB]);
+    if constexpr (J + 1 < IB) x[J + 1] = tsub(x[J + 1], pmul(l, k.prow[J + 1]));
   }
 }
 
@@ -555,7 +560,9 @@ template <typename T, int... Js>
 __device__ __attribute__((always_inline)) inline void panel_cols(T (&x)[IB], int& pos,
                                                                  const PanelCtx<T>& k,
                                                                  std::integer_sequence<int, Js...>) {
-  (panel_col<T, Js>(x, pos, k), ...);
+  T l = tzero<T>();
+  bool below = false;
+  (panel_col<T, Js>(x, pos, l, below, k), ...);
 }
 
 template <typename T>
@@ -600,7 +607,7 @@ __global__ void __launch_bounds__(ROWS) k_panel(T* B, long long ld, int m, int w
 // trips to the coherence point (3 us a column, the whole of k_panel's time): blocks of at most
 // panel_one_rows() rows, what the registers of a CU hold beside the temporaries.  Same pivots and
 // arithmetic.  Measured a block of 32 columns: up to 512 rows 39 us in double, 44 in complex float and
-// 53 in complex double (k_panel 89, 90 and 123), up to 1536 rows 66 and 74 (55, 61, 77, 86 and 97 with
+// 53 in complex double (k_panel 84, 84 and 113), up to 1536 rows 66 and 74 (55, 61, 77, 86 and 97 with
 // the rows exchanged instead of their positions and the arg-max on 64 bits).  Complex double keeps to
 // one row a thread: two did not fit the registers.
 constexpr int ONE_THREADS = 512;
