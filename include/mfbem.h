@@ -96,8 +96,9 @@ int mfb_mesh_create(int nn, int ne, const double *x, const int *conn, const int 
 int mfb_mesh_destroy(mfb_mesh_t mesh);
 int mfb_mesh_stats(mfb_mesh_t mesh, mfb_assembly_stats *stats);
 /* Durations (ms, HIP events on the assembly stream) of the kernel groups of the last assembly:
- * ms[0] precalculated-rule pairs, ms[1] adaptive pairs, ms[2] singular pairs, ms[3] zeroing and
- * free terms; regular_launches: kernel launches behind ms[0].  No counterpart in the reference
+ * ms[0] precalculated-rule pairs, ms[1] adaptive pairs, singular pairs and free terms (one launch),
+ * ms[2] 0 (singular pairs, when they were launched by themselves), ms[3] zeroing;
+ * regular_launches: kernel launches behind ms[0].  No counterpart in the reference
  * (instrumentation of this build). */
 int mfb_mesh_timings(mfb_mesh_t mesh, double *ms, int *regular_launches);
 /* integration class of every (collocation point, element) pair, host array of ncp*ne bytes,

@@ -8,19 +8,17 @@
 //     k_classify       per element block x collocation nodes: integration class of every pair
 //     k_fill_lists     pair ids grouped by class (precalculated rule r, adaptive, singular),
 //                      each class list ordered by element so that batches share element data
+//     k_sing_geom, k_adapt_geom  what the singular and the adaptive pairs take from the geometry
 //   every assembly (material / frequency dependent):
-//     k_zero           A, b := 0
-//     k_regular_tile<H> one workgroup per tile of up to 14 pairs of one element and one
-//                      precalculated rule, one launch per element colour: threads evaluate the
-//                      kernel at (pair, point) items into LDS, then each thread contracts one
-//                      (pair, h|g, component) row against the element's 9 weights and adds the
-//                      row to A (or b)
-//     k_regular<H,MODE> per-rule variant writing per-pair blocks or interior displacements
-//     k_adaptive<H>    one wave per quasi-singular pair: lane 0 walks the reference's 4-way
-//                      subdivision tree, all lanes integrate the Telles leaves
-//     k_singular<H>    one wave per pair with the collocation node on the element: polar
-//                      sub-triangles, CPV regularisation, Stokes line integrals on the edges
-//     k_freeterm<H>    per node: Mantic free term (or I/2 at element-interior nodes)
+//     k_begin<T>       b := 0 and the few entries of A that no tile stores
+//     k_regular_tile<H> one wave per tile of up to 16 pairs of one element and one precalculated
+//                      rule, one launch per element colour: kernel values straight into the FP64
+//                      matrix cores, the first colour of a node stores, the others add
+//     k_fold_extra<T>  rows of the second points of edge nodes added to their nodes' rows
+//     k_near<H>        adaptive pairs (a wave each), singular pairs (a workgroup each) and free
+//                      terms (a thread each) in one launch, added atomically
+//   k_regular<H>       per-rule variant writing per-pair blocks
+//   k_field, k_points  interior displacements of the precalculated pairs
 // Scatter follows the BE-ordinary rule of src/assemble_bem_{staela,harela}_equation.f90: the
 // unknown of node j, direction k is column 3j+k; u-known directions move h to b and put -g in A.
 #include <hip/hip_runtime.h>
@@ -195,11 +193,6 @@ struct VecOut {
   T* out;      // (ncp, 3) interior displacements (accumulated)
 };
 
-__device__ inline void lds_add(double* a, double v) { atomicAdd(a, v); }
-__device__ inline void lds_add(zd* a, zd v) {
-  atomicAdd(&a->re, v.re);
-  atomicAdd(&a->im, v.im);
-}
 
 // mesh setup and classification decide rules: plain FP64 rounding, as in the geometry helpers
 #pragma clang fp contract(off)
@@ -769,6 +762,9 @@ __device__ inline zd lane_xor_add(zd v, int mask) {
 }
 
 // Launches of fewer tiles spread them one by one (runs would leave XCDs without work at the end).
+// Runs of 32 keep a rule's neighbouring rows in one L2: 139 us against 188 for the stores alone of a
+// launch over 26 x 26 elements.  One eighth of the tiles to each XCD: 847 us against 685, the long
+// rules come first and two XCDs take them all.
 constexpr int kRunTiles = 16384;
 
 // Columns of four nodes for a tile's 48 rows, on their way to A.
@@ -881,11 +877,20 @@ __device__ inline void tile_body(const DevMesh& m, const KernelParams& kp,
 // src/assemble_bem_harela_equation.f90), one tile per wave: up to 16 pairs of one element and one
 // rule, consecutive entries of the class list (ascending collocation points, so mostly consecutive
 // matrix rows).  The tiles of one launch belong to elements of one colour (no shared node) and no two
-// points share a row (DevMesh::cx), so no two waves touch the same entry.  The element of the lowest colour that holds a node stores its columns, the others add
-// to them: no reset of A and 5 reads instead of 9 per element on a structured surface.  The columns
-// go through LDS so that a lane holds a row: a store covers 768 consecutive bytes.  t* (tiles h0 .. h0 +
-// n_h) and u* (0 .. n_g) are summed by waves of their own, also for elements that need both: together
-// their sums do not fit the registers of two waves per SIMD (61 spilled).
+// points share a row (DevMesh::cx), so no two waves touch the same entry.  The element of the lowest
+// colour that holds a node stores its columns, the others add to them: no reset of A and 5 reads
+// instead of 9 per element on a structured surface.  The columns go through LDS so that a lane holds
+// a row: a store covers 768 consecutive bytes.  t* (tiles h0 .. h0 + n_h) and u* (0 .. n_g) are summed
+// by waves of their own, also for elements that need both: together their sums do not fit the
+// registers of two waves per SIMD (61 spilled).
+// Bound by its FP64 instructions: the 4x4x4 matrix instruction and the vector FMA share one pipe, and
+// the sums over the element's nodes are contractions that the former does with a third of the issue
+// slots and no LDS traffic for the values.  An open harmonic surface of 26 x 26 elements: 410
+// us a launch, 1340 with kernel values staged in LDS by workgroups of 256 and A cleared first; one of
+// 50 x 50: 5.1 ms a launch and 13.6 GB, 16.3 ms and 25.8 GB before; a static box of 454 elements 88
+// and 157 us.
+// One launch over all colours with atomic additions needs no colours, but the chip does 27e9 of them a
+// second: 11.8 ms against 4 x 0.695 (26 x 26, this kernel before it stored).
 template <bool H>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2)))
     k_regular_tile(DevMesh m, const KernelParams* __restrict__ kpp, const int* __restrict__ list,
@@ -1411,7 +1416,11 @@ __device__ inline void pair_output(const DevMesh& m, int e, int cp, int t,
 }
 
 // Singular pairs: fbem_bem_staela3d_sbie_int (bem_staela3d.f90:1100-1381) and
-// fbem_bem_harela3d_sbie_int (bem_harela3d.f90:1174-1472).
+// fbem_bem_harela3d_sbie_int (bem_harela3d.f90:1174-1472).  A pair's points are spread over four waves
+// and the rows summed over them by the FP64 matrix cores, which leaves a lane's share of the sums in
+// registers: as one wave per pair with tables and line integrals made inside, a launch of its own took
+// 391 us on a cube of 24 static elements (23 now), 550 on a sphere of 96 (69), 2112 on an open surface
+// of 26 x 26 (351).
 constexpr int kSingWaves = 4;
 template <bool H, int KIND>
 __device__ inline void singular_body(const DevMesh& m, ConstKP kp, int e, int cp,
@@ -1782,7 +1791,7 @@ __global__ void __launch_bounds__(kWave) k_block_err(const T* ref, const T* blk,
   }
   if (lane == 0) {
     const double r0 = mag(ref[162 * q]);
-    // a reference marked NaN (overflowed subdivision) gives a NaN error
+    // a reference that is not a number gives a NaN error
     err[q * nr + r] = r0 != r0 ? r0 : fmax(mh > 0 ? dh / mh : dh, mg > 0 ? dg / mg : dg);
   }
 }
@@ -1796,7 +1805,7 @@ __global__ void k_rule_labels(const double* err, int np, int nr, DevMesh m, doub
   int lab = MFB_QNET_CLASSES - 1;
   const double e0 = err[(long long)q * nr];
   if (e0 != e0) {
-    lab = -1;  // no reference (subdivision overflow): no label
+    lab = -1;  // no reference: no label
   } else {
     for (int r = 0; r < nr; r++)
       if (err[(long long)q * nr + r] <= tau) {
@@ -1956,7 +1965,9 @@ __device__ inline void free_term_mca(const DevMesh& m, int cp, T* A, long long l
 // each, in turn), singular pairs (a workgroup each), the other adaptive pairs (a wave each), free
 // terms (a thread each).  The parts are independent (atomic additions), each is a chain of a few
 // dependent loads and reductions and none fills the chip on a small mesh: one after the other they
-// took 150 of 480 us of a 1,158-DOF assembly.  The longest come first.
+// took 150 of 480 us of a 1,158-DOF assembly (29 us against 61 on a cube of 24 elements,
+// 80 against 125 on a sphere of 96, 689 against 930 on an open surface of 26 x 26).  The longest come
+// first.
 // ------------------------------------------------------------------------------------------------
 template <typename T>
 struct NearArgs {
@@ -2399,7 +2410,8 @@ static void default_collocation(int nn, int ne, const double* x, const int* conn
 // Colours of the elements (no two of a colour share a node), greedily in index order, and where that
 // takes more than the four of a structured surface (closed ones: six) once more by saturation
 // degree (Brelaz), which is kept if it needs fewer: every colour is a launch, and on a small mesh a
-// launch takes its latency.
+// launch takes its latency (15 us on a cube of 24 elements, 44 on a sphere of 96 elements, each of two
+// launches fewer; the assemblies take 167 and 349 us).
 constexpr int kMaxColors = 64;
 static int color_elements(int ne, const int* conn, const std::vector<int>& ip,
                           const std::vector<int>& ie, std::vector<int>& col) {
@@ -3275,7 +3287,7 @@ __global__ void k_fill_double(double* a, long long n, double v) {
 template <bool H>
 static int rule_errors(mfb_mesh_t m, const KernelParams& kp, const int* dlist, int np,
                        const QsiParams* d_qsp_ref, double* err, long long* counters, int* errflag,
-                       hipStream_t s, bool keep_overflow = false) {
+                       hipStream_t s) {
   typedef typename Val<H>::T T;
   const DevMesh& d = m->dm;
   T *ref = nullptr, *blk = nullptr;
@@ -3305,15 +3317,10 @@ static int rule_errors(mfb_mesh_t m, const KernelParams& kp, const int* dlist, i
     }
     he = hipGetLastError();
   }
-  int herr = 0;
-  if (he == hipSuccess) he = hipMemcpyAsync(&herr, errflag, sizeof(int), hipMemcpyDeviceToHost, s);
   if (he == hipSuccess) he = hipStreamSynchronize(s);
   if (he != hipSuccess) {
     set_error("rule_errors: %s", hipGetErrorString(he));
     rc = MFB_ERR_HIP;
-  } else if (herr && !keep_overflow) {
-    set_error("rule_errors: adaptive subdivision stack exceeded");
-    rc = MFB_ERR_LIMIT;
   }
   return rc;
 }
@@ -3351,8 +3358,8 @@ static int run_judge(mfb_mesh_t m, const KernelParams& kp, hipStream_t s) {
   if (he == hipSuccess) {
     hipLaunchKernelGGL(k_gather_list, dim3((K + 255) / 256), dim3(256), 0, s, m->llists, dpos, K,
                        dsample);
-    rc = rule_errors<H>(m, kp, dsample, K, m->d_qsp_judge, err, m->judge_counters, m->judge_err, s,
-                        true);
+    rc = rule_errors<H>(m, kp, dsample, K, m->d_qsp_judge, err, m->judge_counters, m->judge_err,
+                        s);
   } else {
     set_error("run_judge: %s", hipGetErrorString(he));
     rc = MFB_ERR_HIP;
@@ -3384,7 +3391,7 @@ static int run_judge(mfb_mesh_t m, const KernelParams& kp, hipStream_t s) {
       long long pn = 0, nk = 0;
       for (int k = 0; k < K; k++) {
         const double e = he_[(size_t)k * d.n_ps + rk[k]];
-        if (e != e) continue;  // no reference for this pair (subdivision overflow)
+        if (e != e) continue;  // no reference for this pair
         nk++;
         mx = std::max(mx, e);
         sum += e;
@@ -3525,7 +3532,7 @@ static int pair_labels(mfb_mesh_t m, const KernelParams& kp, const int* pairs, i
   MFB_HIP(hipMalloc(&err, sizeof(double) * (size_t)nf * nr));
   MFB_HIP(hipMemcpyAsync(dl, flist.data(), sizeof(int) * nf, hipMemcpyHostToDevice, s));
   MFB_HIP(hipMemcpyAsync(di, fidx.data(), sizeof(int) * nf, hipMemcpyHostToDevice, s));
-  int rc = rule_errors<H>(m, kp, dl, nf, m->d_qsp, err, m->counters, m->err, s, true);
+  int rc = rule_errors<H>(m, kp, dl, nf, m->d_qsp, err, m->counters, m->err, s);
   if (rc == MFB_OK) {
     hipLaunchKernelGGL(k_rule_labels, dim3((nf + 255) / 256), dim3(256), 0, s, err, nf, nr, d, tau,
                        di, labels);
