@@ -40,11 +40,13 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP64 = 78.6e12          # MI355X FP64 vector (AMD public spec)
-FLOPS_PER_POINT_HARM = 1500  # harmonic kernel with precalculated data: flops per quadrature point
+# flops per quadrature point of the direct formulation (complex exponentials, nine components of t* and
+# of u*, 9 weights each); the kernel sums the symmetric u* as six and executes about 950
+FLOPS_PER_POINT_HARM = 1500
 QNET_DEFAULT = os.path.join(ROOT, "multifebe_amd", "data", "qnet_tau1e-10.npz")
 # HBM bytes per launch of k_regular_tile<harmonic> (mean over one assembly's launches), from
 # rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE scaled by a 1 GiB copy; None where not measured
-TRAFFIC_PER_LAUNCH = {"sphere": None, "soil": 25.78e9}
+TRAFFIC_PER_LAUNCH = {"sphere": None, "soil": 13.62e9}
 
 
 def workload(name: str):
