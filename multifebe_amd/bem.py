@@ -281,6 +281,18 @@ class BemSystem:
         return lab, err
 
 
+def _device_field(torch, v):
+    """v (numpy, list or tensor) on the GPU.  A plain real or complex tensor that is there stays there;
+    anything else goes through the host and numpy, which resolves lazy conjugation and negation and
+    refuses tensors that require gradients, bfloat16 and sparse layouts."""
+    plain = (isinstance(v, torch.Tensor) and v.layout == torch.strided
+             and v.dtype in (torch.float32, torch.float64, torch.complex64, torch.complex128)
+             and not (v.requires_grad or v.is_conj() or v.is_neg()))
+    if not plain:
+        v = np.asarray(v.cpu() if hasattr(v, "cpu") else v)
+    return torch.as_tensor(v, device="cuda")
+
+
 class Points:
     """Interior points of a BEM region (src/calculate_internal_points_mechanics_*.f90): every
     (point, element) pair classified once, displacements from boundary fields on the GPU."""
@@ -322,8 +334,7 @@ class Points:
         torch = _torch()
         harm = omega is not None
         dt = torch.complex128 if harm else torch.float64
-        ub, tb = (torch.as_tensor(v if hasattr(v, "cpu") else np.asarray(v), device="cuda")
-                  .to(dt).contiguous() for v in (u, t))
+        ub, tb = (_device_field(torch, v).to(dt).contiguous() for v in (u, t))
         out = torch.empty((self.npts, 3), dtype=dt, device="cuda")
         if harm:
             rc = lib().mfb_points_displacement_harela(self._h, omega, lam.real, lam.imag, mu_c.real,

@@ -38,3 +38,25 @@ def test_points_sets(harmonic):
     for n in (1, 15, 16, 17, 63, 64, 65, 130):
         assert np.abs(field(x[:n]) - ref[:n]).max() <= tol, n
     assert np.abs(field(x[::-1]) - ref[::-1]).max() <= tol
+
+
+def test_boundary_fields_on_the_gpu():
+    """Device tensors give what numpy arrays of the same values give, in any plain type and stride;
+    lazily conjugated ones give their values, tensors that require gradients are refused."""
+    import torch
+    from multifebe_amd import bem
+    m = M.pressure_hemisphere_bcs(M.sphere(4))
+    mu, mu_c, lam_c = M.elastic_constants(1e9, 0.3, 0.05)
+    kw = dict(omega=2.0 * np.sqrt(mu / 2000.0), lam=lam_c, mu_c=mu_c, rho=2000.0)
+    p = bem.BemSystem(m).points(M.points_off_surface(m, 20, 0.02, 0.8, seed=4, outward=False))
+    rng = np.random.default_rng(5)
+    u, t = (rng.standard_normal((m.nn, 3)) * (1 + 0.5j) for _ in range(2))
+    ref = p.displacement(u, t, **kw)
+    ud, td = torch.from_numpy(u).cuda(), torch.from_numpy(t).cuda()
+    assert torch.allclose(p.displacement(ud, td, **kw), ref, rtol=0, atol=1e-13 * ref.abs().max())
+    ut = ud.T.contiguous().T
+    assert torch.allclose(p.displacement(ut, td, **kw), ref, rtol=0, atol=1e-13 * ref.abs().max())
+    lazy = p.displacement(torch.from_numpy(u.conj()).cuda().conj(), td, **kw)
+    assert torch.allclose(lazy, ref, rtol=0, atol=1e-13 * ref.abs().max())
+    with pytest.raises(RuntimeError):
+        p.displacement(ud.clone().requires_grad_(), td, **kw)
