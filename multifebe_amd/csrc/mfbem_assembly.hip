@@ -995,13 +995,14 @@ __device__ inline void point_values(ConstKP k, const double* rv, const double* n
                                     const zd* f, zd* u) {
   double r, s;
   dist_and_inverse(dot3(rv, rv), r, s);
-  if (!on) {
-    r = 1.0;
+  if (!on) {   // its own r keeps the lane on the branch of its neighbours
+    r = r > 0.0 ? r : 1.0;
     s = 0.0;
   }
   const double dr[3] = {rv[0] * s, rv[1] * s, rv[2] * s}, rn = dot3(dr, n);
   zd psi, chi, TT1, TT2, TT3;
   har_factors<true, true>(&k->h, r, s, true, psi, chi, TT1, TT2, TT3);
+  if (!on) psi = mkz(0.0);   // the other factors meet dr = 0
   const zd dt = f[0] * dr[0] + f[1] * dr[1] + f[2] * dr[2];
   const zd du = f[3] * dr[0] + f[4] * dr[1] + f[5] * dr[2];
   const zd nu = f[3] * n[0] + f[4] * n[1] + f[5] * n[2];

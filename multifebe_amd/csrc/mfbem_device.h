@@ -819,11 +819,26 @@ __device__ inline void dist_and_inverse(double r2, double& r, double& s) {
   r = __builtin_fma(__builtin_fma(-r, r, r2), 0.5 * s, r);
 }
 
-// G(z) = (e^z - 1 - z - z^2/2) / z^3 = sum_j z^j / (j + 3)! on |z| <= 1 (17 terms: the next is below
-// 1e-18): real coefficients at a complex argument by the recurrence b_j = c_j + 2 Re(z) b_{j+1} -
-// |z|^2 b_{j+2} (Knuth, The Art of Computer Programming 2, 4.6.4), two FMAs per term.
-__host__ __device__ inline zd exp_tail3(zd z) {
-  constexpr double c[17] = {
+// sum_j z^j / (j + B)! at two arguments: real coefficients at a complex argument by the recurrence
+// b_j = c_j + 2 Re(z) b_{j+1} - |z|^2 b_{j+2} (Knuth, The Art of Computer Programming 2, 4.6.4), two
+// FMAs per term.  large = false: |z| <= 1, the terms up to z^19/19!; true: |z| <= 2, up to z^23/23!
+// (the next is below 1e-17 of the factors in either case).
+struct ExpSeries {
+  double p, n, b1, b2;
+  __host__ __device__ inline ExpSeries(zd z, double c)
+      : p(z.re + z.re), n(z.re * z.re + z.im * z.im), b1(c), b2(0.0) {}
+  __host__ __device__ inline void term(double c) {
+    const double t = __builtin_fma(p, b1, __builtin_fma(-n, b2, c));
+    b2 = b1;
+    b1 = t;
+  }
+  __host__ __device__ inline zd sum(double c, zd z) const {
+    return mkz(__builtin_fma(z.re, b1, __builtin_fma(-n, b2, c)), z.im * b1);
+  }
+};
+template <int B>
+__host__ __device__ inline void exp_tails(zd z1, zd z2, bool large, zd& g1, zd& g2) {
+  constexpr double f[21] = {   // 1 / 3!, 1 / 4!, ..
       1.0 / 6.0,
       1.0 / 24.0,
       1.0 / 120.0,
@@ -841,78 +856,114 @@ __host__ __device__ inline zd exp_tail3(zd z) {
       1.0 / 355687428096000.0,
       1.0 / 6402373705728000.0,
       1.0 / 121645100408832000.0,
+      1.0 / 2432902008176640000.0,
+      1.0 / 51090942171709440000.0,
+      1.0 / 1124000727777607680000.0,
+      1.0 / 25852016738884976640000.0,
   };
-  const double p = z.re + z.re, n = z.re * z.re + z.im * z.im;
-  double b1 = c[16], b2 = 0.0;
+  constexpr int kSmall = 19 - B, kLarge = 23 - B;
+  ExpSeries a(z1, f[kSmall + B - 3]), b(z2, f[kSmall + B - 3]);
+  if (large) {
+    a.b1 = b.b1 = f[kLarge + B - 3];
 #pragma unroll
-  for (int j = 15; j >= 1; j--) {
-    const double t = __builtin_fma(p, b1, c[j]) - n * b2;
-    b2 = b1;
-    b1 = t;
+    for (int j = kLarge - 1; j >= kSmall; j--) { a.term(f[j + B - 3]); b.term(f[j + B - 3]); }
   }
-  return mkz(c[0] + z.re * b1 - n * b2, z.im * b1);
+#pragma unroll
+  for (int j = kSmall - 1; j >= 1; j--) { a.term(f[j + B - 3]); b.term(f[j + B - 3]); }
+  g1 = a.sum(f[B - 3], z1);
+  g2 = b.sum(f[B - 3], z2);
+}
+
+// What the factors below |z| = 2 are made of, summed from the first power that does not cancel; g5 =
+// sum_j z^j / (j + 5)!:
+//   e = (e^z - 1 - z) / z^2 = 1/2 + ..,  P = sum_{n>=2} 2 (n-1) / ((n+2) n!) z^{n-2} = 1/4 + ..,
+//   R = (z e^z - e^z + 1) / z^2 - P = 1/4 + ..
+__host__ __device__ inline void exp_sums(zd z, zd g5, zd& e, zd& P, zd& R) {
+  const zd g4 = mkz(1.0 / 24.0) + z * g5, g3 = mkz(1.0 / 6.0) + z * g4;
+  const zd h = 6.0 * (g4 - g5);
+  e = mkz(0.5) + z * g3;
+  P = mkz(0.25) + z * (2.0 * g3 - h);
+  R = mkz(0.25) + z * (e - 3.0 * g3 + h);
 }
 
 // psi, chi (G) and TT1..TT3 (F) at distance r, s = 1/r; full = false drops the leading lead s^2 of
-// TT1..TT3 (regular parts used by the singular integration).  With z_j = -kappa_j r, w_j = s e^{z_j}:
-//   D = w2 (1/z2^2 - 1/z2) - w1 (1/z2^2 - z1/z2^2) = s (q H(z1) - H(z2)),  H(z) = (1 - (1-z) e^z)/z^2
-// and each factor is a short combination of w1, w2 and D.  From max |z_j| = 1 on the first form of
-// D is taken (its terms cancel by 1/z^2 at most); below, t = e^z - 1 and h = H - 1/2 are summed
-// without cancellation and the leading terms added in closed form.  No table and seven complex
-// constants, which stay in scalar registers: power series of the factors themselves take fewer
-// FMAs but read up to 170 constants per point, whose scalar-load latency cost more than it saved.
+// TT1..TT3 (regular parts used by the singular integration).  With z_j = -kappa_j r, w_j = s e^{z_j},
+// B_j = w_j (kappa_j + s), q = (kappa1/kappa2)^2:
+//   chi = d/2,  d = 2 (w2 - q w1) + 6 s / kappa2^2 (B2 - B1),  psi = d/6 + (2 w2 + q w1)/3,
+//   TT1 = 5 s d + 2 (B2 - q B1),  TT2 = -s d - B2,  TT3 = -s d + (2 q - 1) B1.
+// Below max |z_j| = 2, where d's terms cancel by 1/z^2, the exponentials are expanded, and what is
+// linear in z, which cancels in every factor but psi, is left out beforehand:
+//   r chi = lead1 + A/2,  A = Q2 - q Q1,  Q = z^2 P,  r psi = lead0 + (2 t2 + q t1)/3 + A/6,  t = z + z^2 e,
+//   r^2 TT1 = lead2 + 3 A - 2 (V2 - q V1),  r^2 TT2 = lead3 + V2 + q Q1,  V = z^2 R,
+//   r^2 TT3 = lead4 + V1 + Q1 - 2 q V1 - q Q1 - Q2.
+// Largest error of TT1..TT3 (of the largest of them; nu 0.05..0.49, damping to 0.1) for |z| to 1, 2, 3
+// and 120: 5.3e-16, 1.2e-15, 2.9e-15, 4.3e-14.  The reference's E_n terms: 6.5e-16, 3.9e-15, 5.2e-15,
+// 1.4e-9; series of H = (1 - (1-z) e^z)/z^2 and e^z - 1 below |z| = 1, linear terms and all: 2.4e-15,
+// 9.4e-15, 2.8e-15, 4.3e-14, in about the same time (tiles of an open surface of 26 x 26 elements 1657
+// us, 1612 now; of a sphere of 96 185 and 155, of a cylinder of 384 545 and 548; 10,000 points 1.17 and
+// 1.16 ms).
+// Five complex constants, which stay in scalar registers: the same with kappa^2, q kappa, 6/kappa as
+// constants of their own takes 10 % fewer FMAs and 3 % more time, power series of the factors themselves
+// read up to 170 constants per point, whose scalar-load latency costs more than they save.
 template <bool F, bool G, class HP>
 __host__ __device__ inline void har_factors(HP k, double r, double s, bool full, zd& psi, zd& chi,
                                             zd& TT1, zd& TT2, zd& TT3) {
   const zd k1 = mkz(k->kap1[0], k->kap1[1]), k2 = mkz(k->kap2[0], k->kap2[1]);
-  const zd q = mkz(k->q[0], k->q[1]), qk1 = mkz(k->qk1[0], k->qk1[1]);
+  const zd q = mkz(k->q[0], k->q[1]), lead = mkz(k->lead[1][0], k->lead[1][1]);
   if (r < k->rser) {
-    const zd z1 = k1 * -r, z2 = k2 * -r;
-    const zd g1 = exp_tail3(z1), g2 = exp_tail3(z2);
-    const zd t1 = z1 * (mkz(1.0) + z1 * (mkz(0.5) + z1 * g1));
-    const zd t2 = z2 * (mkz(1.0) + z2 * (mkz(0.5) + z2 * g2));
-    const zd qt = q * t1;
-    const zd d = q * (z1 * (mkz(0.5) - g1 + z1 * g1)) - z2 * (mkz(0.5) - g2 + z2 * g2);
+    const zd z1 = k1 * -r, z2 = k2 * -r, qz = q * z1;
+    const bool large = r + r > k->rser;
+    zd g1, g2;
+    if (!F) {   // psi, chi alone: h = (H - 1/2) / z - 1/3 instead of P, with fewer products
+      exp_tails<3>(z1, z2, large, g1, g2);
+      const zd zg1 = z1 * g1, zg2 = z2 * g2;
+      const zd t2 = z2 * (z2 * (mkz(0.5) + zg2)), qt = qz * (z1 * (mkz(0.5) + zg1));
+      const zd d = qz * (mkz(1.0 / 6.0) - g1 + zg1) - z2 * (mkz(1.0 / 6.0) - g2 + zg2);
+      psi = (mkz(1.0) + lead + (t2 + d + (2.0 * z2 + qz) * (1.0 / 3.0))) * s;
+      chi = (lead + (t2 - qt + 3.0 * d)) * s;
+      return;
+    }
+    zd e1, P1, R1, e2, P2, R2;
+    exp_tails<5>(z1, z2, large, g1, g2);
+    exp_sums(z1, g1, e1, P1, R1);
+    exp_sums(z2, g2, e2, P2, R2);
+    const zd zz = z2 * z2, qzz = qz * z1;
+    const zd Q2 = zz * P2, qQ = qzz * P1, A = Q2 - qQ;
     if (G) {
-      psi = (mkz(k->lead[0][0], k->lead[0][1]) + t2 + d) * s;
-      chi = (mkz(k->lead[1][0], k->lead[1][1]) + t2 - qt + 3.0 * d) * s;
+      const zd t = z2 + zz * e2, qt = qz + qzz * e1;
+      psi = (mkz(1.0) + lead + ((2.0 * t + qt) * (1.0 / 3.0) + A * (1.0 / 6.0))) * s;
+      chi = (lead + 0.5 * A) * s;
     }
-    if (F) {
-      const double s2 = s * s;
-      const zd A2 = k2 * ((t2 + mkz(1.0)) * s), w1 = (t1 + mkz(1.0)) * s;
-      const zd A1 = qk1 * w1, B1 = k1 * w1;
-      zd u1 = 12.0 * (t2 - qt) + 30.0 * d;
-      zd u2 = 2.0 * qt - 3.0 * t2 - 6.0 * d;
-      zd u3 = 4.0 * qt - 2.0 * t2 - t1 - 6.0 * d;
-      if (full) {
-        u1 += mkz(k->lead[2][0], k->lead[2][1]);
-        u2 = u2 - q;
-        u3 = u3 + q;
-      }
-      TT1 = 2.0 * (A2 - A1) + u1 * s2;
-      TT2 = u2 * s2 - A2;
-      TT3 = 2.0 * A1 - B1 + u3 * s2;
+    const double s2 = s * s;
+    const zd V2 = zz * R2, qV = qzz * R1;
+    TT1 = 3.0 * A - 2.0 * (V2 - qV);
+    TT2 = V2 + qQ;
+    TT3 = (z1 * z1) * (P1 + R1) - 2.0 * qV - qQ - Q2;
+    if (full) {
+      TT1 += 6.0 * lead;
+      TT2 = TT2 - q;
+      TT3 = TT3 + q;
     }
+    TT1 = TT1 * s2;
+    TT2 = TT2 * s2;
+    TT3 = TT3 * s2;
     return;
   }
-  const zd w1 = exp_minus(k1, r) * s, w2 = exp_minus(k2, r) * s;
-  const zd qw = q * w1, ik22 = mkz(k->ik22[0], k->ik22[1]);
-  const zd g2 = (mkz(k->v2[0], k->v2[1]) + ik22 * s) * s;
-  const zd g1 = (mkz(k->v1[0], k->v1[1]) + ik22 * s) * s;
-  const zd D = w2 * g2 - w1 * g1;
+  const zd w1 = exp_minus(k1, r) * s, w2 = exp_minus(k2, r) * s, qw = q * w1;
+  const zd B2 = w2 * (k2 + mkz(s)), B1 = w1 * (k1 + mkz(s));
+  const zd d = 2.0 * (w2 - qw) + (mkz(k->ik22[0], k->ik22[1]) * s) * (B2 - B1);
   if (G) {
-    psi = w2 + D;
-    chi = w2 - qw + 3.0 * D;
+    psi = d * (1.0 / 6.0) + (2.0 * w2 + qw) * (1.0 / 3.0);
+    chi = 0.5 * d;
   }
   if (F) {
-    const zd A2 = k2 * w2, A1 = qk1 * w1, B1 = k1 * w1;
-    const zd y2 = w2 * s, y1 = qw * s, yd = D * s;
-    TT1 = 2.0 * (A2 - A1) + 12.0 * (y2 - y1) + 30.0 * yd;
-    TT2 = 2.0 * y1 - 3.0 * y2 - A2 - 6.0 * yd;
-    TT3 = 2.0 * A1 - B1 + 4.0 * y1 - 2.0 * y2 - w1 * s - 6.0 * yd;
+    const zd e = d * s, qB = q * B1;
+    TT1 = 5.0 * e + 2.0 * (B2 - qB);
+    TT2 = -(e + B2);
+    TT3 = 2.0 * qB - B1 - e;
     if (!full) {
       const double s2 = s * s;
-      TT1 = TT1 - mkz(k->lead[2][0], k->lead[2][1]) * s2;
+      TT1 = TT1 - 6.0 * lead * s2;
       TT2 = TT2 + q * s2;
       TT3 = TT3 - q * s2;
     }

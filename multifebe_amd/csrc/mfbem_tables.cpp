@@ -172,11 +172,8 @@ void host_har_params(double lam_re, double lam_im, double mu_re, double mu_im, d
   put(p->kap1, k1);
   put(p->kap2, k2);
   put(p->q, q);
-  put(p->qk1, q * k1);
-  put(p->v1, q / k1);
-  put(p->v2, one / k2);
-  put(p->ik22, one / (k2 * k2));
-  p->rser = (double)(1.0L / std::max(std::abs(k1), std::abs(k2)));
+  put(p->ik22, 6.0L / (k2 * k2));
+  p->rser = (double)(2.0L / std::max(std::abs(k1), std::abs(k2)));
   put(p->cte_u, one_4pi / mu);
   put(p->cte_t, z(one_4pi, 0.0L));
 }

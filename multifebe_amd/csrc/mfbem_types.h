@@ -15,10 +15,9 @@ struct QsiParams {
 // 660-682) are finite sums of s^p exp(-kappa_j r).
 struct HarParams {
   double kap1[2], kap2[2];
-  double q[2], qk1[2];           // q, q kappa1
-  double v1[2], v2[2], ik22[2];  // q/kappa1, 1/kappa2, 1/kappa2^2
-  double rser;                   // r below which D is summed as a series (har_factors)
-  double lead[5][2];             // psi, chi: limit of r f; TT1, TT2, TT3: limit of r^2 f, r -> 0
+  double q[2], ik22[2];            // q, 6 / kappa2^2
+  double rser;                     // r below which the factors are summed as series (har_factors)
+  double lead[5][2];               // psi, chi: limit of r f; TT1, TT2, TT3: limit of r^2 f, r -> 0
   double cte_u[2], cte_t[2];
 };
 
