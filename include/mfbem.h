@@ -38,8 +38,9 @@ typedef struct {
   long long singular;   /* pairs integrated by the polar (singular) rule                   */
   long long pre;        /* pairs integrated with a precalculated Gauss-Legendre dataset     */
   long long adaptive;   /* pairs integrated by Telles + adaptive subdivision               */
-  long long points;     /* quadrature points evaluated by the last assembly                */
-  long long leaves;     /* adaptive sub-elements integrated by the last assembly           */
+  long long points;     /* quadrature points evaluated by the last assembly; after a batch */
+                        /* regular_points + those of the near pairs of every job of the mesh */
+  long long leaves;     /* adaptive sub-elements integrated by the last assembly (or batch) */
   long long decisions;  /* class histogram checksum: sum over pairs of (class+1)*(pair%97+1) */
   long long regular_points; /* quadrature points of the precalculated-rule pairs (per assembly) */
   long long learned;        /* 1 when the last assembly chose the rules with the network     */

@@ -1141,9 +1141,11 @@ struct SingGeom {
   double hli[3], xi[2], thp[16];
   int node, np, st[8], base[9];   // node: element node at xi or -1; np: quadrature points
 };
+constexpr int kSingCounts = 64;   // the points are counted in that many places
 __global__ void __launch_bounds__(kWave) k_sing_geom(DevMesh m,
                                                      const QsiParams* __restrict__ qsp_li,
-                                                     const int* __restrict__ list, SingGeom* geo) {
+                                                     const int* __restrict__ list, SingGeom* geo,
+                                                     unsigned long long* np) {
   const int lane = threadIdx.x, edge = lane >> 4;
   const int pid = list[blockIdx.x], e = pid / m.ncp, cp = pid % m.ncp;
   double X[27], xi_i[2], x_i[3], o[3] = {0, 0, 0};
@@ -1192,6 +1194,7 @@ __global__ void __launch_bounds__(kWave) k_sing_geom(DevMesh m,
     out.xi[0] = xi_i[0];
     out.xi[1] = xi_i[1];
     out.node = k;
+    atomicAdd(&np[blockIdx.x % kSingCounts], (unsigned long long)out.np);
   }
 }
 
@@ -1534,12 +1537,19 @@ __device__ inline int leaf_order(const QsiParams& qsp, const double* X, double c
   return gln == 0 && ks == ns_max ? 30 : gln;
 }
 
-// Records of `count` listed pairs in one buffer; behind them the number of pairs to be subdivided and
-// their list positions.
+// Records of `count` listed pairs in one buffer; behind them what is to be subdivided and what the
+// others, single leaves, hold.
+struct AdaptSum {
+  unsigned long long points;   // quadrature points and number of the single leaves
+  int leaves, n_tree;          // pairs to be subdivided
+  __host__ __device__ int* tree() { return (int*)(this + 1); }   // their list positions
+};
 __host__ __device__ inline size_t adapt_geom_bytes(size_t count) {
-  return count * (sizeof(AdaptGeom) + sizeof(int)) + 4 * sizeof(int);
+  return count * (sizeof(AdaptGeom) + sizeof(int)) + sizeof(AdaptSum);
 }
-__host__ __device__ inline int* adapt_tree(AdaptGeom* geo, size_t count) { return (int*)(geo + count); }
+__host__ __device__ inline AdaptSum* adapt_sum(AdaptGeom* geo, size_t count) {
+  return (AdaptSum*)(geo + count);
+}
 
 __global__ void __launch_bounds__(kWave) k_adapt_geom(DevMesh m, const QsiParams* __restrict__ qsp,
                                                       const int* __restrict__ list, int count,
@@ -1550,17 +1560,24 @@ __global__ void __launch_bounds__(kWave) k_adapt_geom(DevMesh m, const QsiParams
   load_X(m, e, X);
   const double x_i[3] = {m.xc[3 * cp], m.xc[3 * cp + 1], m.xc[3 * cp + 2]};
   const int gln = leaf_order(*qsp, X, m.elem[8 * e], x_i, 1, m.ns_max, barxi, &d);
-  if (q < count && sub == 0) {
+  AdaptSum* sum = adapt_sum(geo, count);
+  const bool mine = q < count && sub == 0;
+  const int order = gln ? max(gln, (int)m.elem[8 * e + 5]) : 0;
+  if (mine) {
     AdaptGeom& g = geo[q];
     g.barxi[0] = barxi[0];
     g.barxi[1] = barxi[1];
     g.d = d;
-    g.gln = gln ? max(gln, (int)m.elem[8 * e + 5]) : 0;
+    g.gln = order;
     g.pad = 0;
-    if (gln == 0) {
-      int* tree = adapt_tree(geo, count);
-      tree[4 + atomicAdd(tree, 1)] = q;
-    }
+    if (gln == 0) sum->tree()[atomicAdd(&sum->n_tree, 1)] = q;
+  }
+  int points = mine ? order * order : 0;
+  for (int mask = 4; mask < kWave; mask *= 2) points += __shfl_xor(points, mask);
+  const int leaves = __popcll(__ballot(mine && order));
+  if (threadIdx.x == 0) {
+    atomicAdd(&sum->points, (unsigned long long)points);
+    atomicAdd(&sum->leaves, leaves);
   }
 }
 
@@ -1617,27 +1634,6 @@ __device__ __attribute__((noinline)) void walk_step(const QsiParams& qsp, const 
   wave_lds_fence();
   sp += 4 * __popcll(split) - n;
   nl += __popcll(leaf);
-}
-
-// sums[0]: points of the singular and the single-leaf adaptive pairs, sums[1]: those leaves (one
-// workgroup; the integration kernels would have to add to one address per pair: at 24,000 pairs
-// that took longer than the integration)
-__global__ void __launch_bounds__(1024) k_count_points(const SingGeom* sg, long long ns,
-                                                       const AdaptGeom* ag, long long na,
-                                                       long long* sums) {
-  __shared__ unsigned long long t[2];
-  if (threadIdx.x < 2) t[threadIdx.x] = 0;
-  __syncthreads();
-  unsigned long long p = 0, l = 0;
-  for (long long q = threadIdx.x; q < ns; q += blockDim.x) p += sg[q].np;
-  for (long long q = threadIdx.x; q < na; q += blockDim.x) {
-    p += ag[q].gln * ag[q].gln;
-    l += ag[q].gln != 0;
-  }
-  atomicAdd(&t[0], p);
-  atomicAdd(&t[1], l);
-  __syncthreads();
-  if (threadIdx.x < 2) sums[threadIdx.x] = t[threadIdx.x];
 }
 
 template <bool H, int KIND>
@@ -1982,7 +1978,8 @@ struct NearArgs {
   T* A;
   long long lda;
   T* b;
-  long long* counters;          // points, leaves of the subdivided pairs
+  long long* counters;          // quadrature points and leaves of all these pairs are added
+  long long sing_points;        // of the singular pairs
   int* err;
   T *ablocks, *sblocks;         // blocks of the pairs (162 values each) instead of A, b
   VecOut<T> vec;                // displacements of their points instead of A, b
@@ -2008,12 +2005,18 @@ __global__ void __launch_bounds__(kNearWaves* kWave) __attribute__((amdgpu_waves
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const ConstKP kp = (ConstKP)kpp;
   int wg = blockIdx.x;
+  AdaptSum* sum = adapt_sum((AdaptGeom*)a.ageo, a.na);
+  // what the records hold already; the subdivided pairs add their own (an addition per pair to one
+  // address took longer than the integration at 24,000 pairs)
+  if (wg == gridDim.x - 1 && threadIdx.x == 0) {
+    atomicAdd((unsigned long long*)&a.counters[0], a.sing_points + (a.na ? sum->points : 0ull));
+    if (a.na) atomicAdd((unsigned long long*)&a.counters[1], (unsigned long long)sum->leaves);
+  }
   if (wg < a.tree_wgs) {
-    const int* tree = adapt_tree((AdaptGeom*)a.ageo, a.na);
-    const int n = tree[0];
+    const int n = sum->n_tree;
     for (int t = kNearWaves * wg + wave; t < n; t += kNearWaves * a.tree_wgs) {
       wave_lds_fence();
-      adaptive_pair<H, true>(m, qsp, kp, a.alist, a.ageo, tree[4 + t], lds.pair[wave],
+      adaptive_pair<H, true>(m, qsp, kp, a.alist, a.ageo, sum->tree()[t], lds.pair[wave],
                              &lds.walk[wave], a.A, a.lda, a.b, a.counters, a.ablocks, a.vec);
     }
     return;
@@ -2164,6 +2167,7 @@ struct mfb_mesh_s {
   mfb::SingGeom* sgeo = nullptr;   // of the singular and the adaptive pairs, in list order
   mfb::AdaptGeom* ageo = nullptr;
   int n_tree = 0;                  // adaptive pairs of `lists` that are subdivided
+  long long sing_points = 0;       // quadrature points of the singular pairs
   std::vector<int> h_crow, h_cel;
   std::vector<double> h_xc;
   int n_mca = 0;
@@ -2172,8 +2176,7 @@ struct mfb_mesh_s {
   std::vector<int> h_conn, h_ctype, h_ps;
   double h_tol = 1e-6;
   int* err = nullptr;
-  long long* counters = nullptr;  // points, leaves of the subdivided pairs; of the others (stats)
-  bool integrated = false;        // an assembly has run
+  long long* counters = nullptr;  // points, leaves of the adaptive and singular pairs
   mfb::QsiParams* d_qsp = nullptr;     // estimator tables and kernel constants live in device memory:
   mfb::QsiParams* d_qsp_li = nullptr;  // they are too large to travel as kernel arguments
   mfb::KernelParams* d_kp = nullptr;
@@ -2240,7 +2243,8 @@ static void launch_near(const DevMesh& d, const QsiParams* qsp, const KernelPara
 // Records of `count` listed adaptive pairs at the tolerance of qsp into geo (adapt_geom_bytes).
 static void launch_adapt_geom(const DevMesh& d, const QsiParams* qsp, const int* list, int count,
                               AdaptGeom* geo, hipStream_t s) {
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s, adapt_tree(geo, count), 4, 0);
+  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s, (int*)adapt_sum(geo, count),
+                     (int)(sizeof(AdaptSum) / sizeof(int)), 0);
   hipLaunchKernelGGL(k_adapt_geom, dim3((unsigned)((count + 15) / 16)), dim3(kWave), 0, s, d, qsp,
                      list, count, geo);
 }
@@ -2250,16 +2254,24 @@ static int make_pair_geom(mfb_mesh_t m) {
   const DevMesh& d = m->dm;
   const long long ns = m->cls_cnt[d.n_ps + 1], na = m->cls_cnt[d.n_ps];
   if (ns) {
-    MFB_HIP(hipMalloc((void**)&m->sgeo, sizeof(SingGeom) * (size_t)ns));
+    MFB_HIP(hipMalloc((void**)&m->sgeo, sizeof(SingGeom) * (size_t)ns + sizeof(long long) * kSingCounts));
+    unsigned long long* np = (unsigned long long*)(m->sgeo + ns);
+    MFB_HIP(hipMemset(np, 0, sizeof(long long) * kSingCounts));
     hipLaunchKernelGGL(k_sing_geom, dim3((unsigned)ns), dim3(kWave), 0, 0, d, m->d_qsp_li,
-                       m->lists + m->cls_off[d.n_ps + 1], m->sgeo);
+                       m->lists + m->cls_off[d.n_ps + 1], m->sgeo, np);
   }
   if (na) {
     MFB_HIP(hipMalloc((void**)&m->ageo, adapt_geom_bytes((size_t)na)));
     launch_adapt_geom(d, m->d_qsp, m->lists + m->cls_off[d.n_ps], (int)na, m->ageo, 0);
   }
   MFB_HIP(hipGetLastError());
-  if (na) MFB_HIP(hipMemcpy(&m->n_tree, adapt_tree(m->ageo, na), sizeof(int), hipMemcpyDeviceToHost));
+  if (ns) {
+    long long np[kSingCounts];
+    MFB_HIP(hipMemcpy(np, m->sgeo + ns, sizeof np, hipMemcpyDeviceToHost));
+    for (long long n : np) m->sing_points += n;
+  }
+  if (na)
+    MFB_HIP(hipMemcpy(&m->n_tree, &adapt_sum(m->ageo, na)->n_tree, sizeof(int), hipMemcpyDeviceToHost));
   return MFB_OK;
 }
 
@@ -2584,7 +2596,7 @@ static int mesh_create_impl(int nn, int ne, const double* x, const int* conn, co
   TRY(dalloc(&m->nmca, nn));
   TRY(dalloc(&m->ekind, ne));
   TRY(dalloc(&m->err, 1));
-  TRY(dalloc(&m->counters, 4));
+  TRY(dalloc(&m->counters, 2));
   TRY(dalloc(&m->d_qsp, 1));
   TRY(dalloc(&m->d_qsp_li, 1));
   TRY(dalloc(&m->d_kp, 1));
@@ -2749,21 +2761,16 @@ extern "C" int mfb_mesh_stats(mfb_mesh_t m, mfb_assembly_stats* s) {
   const int np = m->dm.n_ps;
   const bool L = m->learned_last;
   const std::vector<long long>& cnt = L ? m->lcls_cnt : m->cls_cnt;
-  long long c[4] = {0, 0, 0, 0};
-  if (m->integrated) {
-    hipLaunchKernelGGL(k_count_points, dim3(1), dim3(1024), 0, 0, m->sgeo, cnt[np + 1],
-                       L ? (const AdaptGeom*)m->ws[MW_AGEO] : m->ageo, cnt[np], m->counters + 2);
-    MFB_HIP(hipGetLastError());
-    MFB_HIP(hipMemcpy(c, m->counters, sizeof c, hipMemcpyDeviceToHost));
-  }
+  long long c[2];
+  MFB_HIP(hipMemcpy(c, m->counters, sizeof c, hipMemcpyDeviceToHost));
   const long long rp = L ? m->l_regular_points : m->regular_points;
   s->pairs = (long long)m->dm.ncp * m->dm.ne;
   s->singular = cnt[np + 1];
   s->adaptive = cnt[np];
   s->pre = 0;
   for (int r = 0; r < np; r++) s->pre += cnt[r];
-  s->points = rp + c[0] + c[2];
-  s->leaves = c[1] + c[3];
+  s->points = rp + c[0];
+  s->leaves = c[1];
   s->decisions = m->decisions;
   s->regular_points = rp;
   s->learned = L ? 1 : 0;
@@ -2886,6 +2893,7 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
   a.lda = lda;
   a.b = b;
   a.counters = m->counters;
+  a.sing_points = m->sing_points;
   a.err = m->err;
   launch_near<H>(d, m->d_qsp, kpp, a, learned ? -1 : m->n_tree, s);
   if (events) {
@@ -2922,7 +2930,6 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
   // rule choice: the reference's estimator (classes fixed at mesh creation) or the network
   const bool learned = m->qnet && !blocks && !vmode;
   m->learned_last = learned;
-  m->integrated = true;
   if (learned) {
     int rc = learned_lists(m, kw, s);
     if (rc) return rc;
@@ -2979,6 +2986,7 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
     a.na = (int)cls_cnt[d.n_ps];
     a.ns = (int)cls_cnt[d.n_ps + 1];
     a.counters = m->counters;
+    a.sing_points = m->sing_points;
     a.ablocks = blocks ? blocks + 162 * cls_off[d.n_ps] : nullptr;
     a.sblocks = blocks ? blocks + 162 * cls_off[d.n_ps + 1] : nullptr;
     a.vec = vec;
@@ -3100,7 +3108,6 @@ static int enqueue_batch(int njobs, const mfb_assembly_job* jobs, const KernelPa
     mfb_mesh_t m = jobs[q].mesh;
     if (std::find(seen.begin(), seen.end(), m) != seen.end()) continue;
     seen.push_back(m);
-    m->integrated = true;
     hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, m->counters, m->err);
   }
   for (int q = 0; q < njobs; q++) {
