@@ -97,11 +97,14 @@ int mfb_mesh_create(int nn, int ne, const double *x, const int *conn, const int 
 int mfb_mesh_destroy(mfb_mesh_t mesh);
 int mfb_mesh_stats(mfb_mesh_t mesh, mfb_assembly_stats *stats);
 /* Durations (ms, HIP events on the assembly stream) of the kernel groups of the last assembly:
- * ms[0] precalculated-rule pairs, ms[1] adaptive pairs, singular pairs and free terms (one launch),
- * ms[2] 0 (singular pairs, when they were launched by themselves), ms[3] zeroing;
- * regular_launches: kernel launches behind ms[0].  No counterpart in the reference
+ * ms[0] precalculated-rule pairs, ms[1] adaptive pairs, singular pairs and free terms, which share one
+ * launch, ms[2] 0, ms[3] zeroing; regular_launches: kernel launches behind ms[0].
+ * mfb_mesh_time_groups(mesh, 1): the following assemblies of this mesh launch them one after the other,
+ * which takes longer, and ms[1] is the adaptive pairs, ms[2] the singular pairs, ms[3] zeroing and free
+ * terms; 0: one launch again.  Results are the same.  No counterpart in the reference
  * (instrumentation of this build). */
 int mfb_mesh_timings(mfb_mesh_t mesh, double *ms, int *regular_launches);
+int mfb_mesh_time_groups(mfb_mesh_t mesh, int on);
 /* integration class of every (collocation point, element) pair, host array of ncp*ne bytes,
  * index e*ncp + cp: 0..n_ps-1 precalculated dataset, n_ps adaptive, n_ps+1 singular.  (ncp = nn
  * on a closed surface, point cp = node cp.)  Pair ids taken or returned by the functions below are

@@ -66,6 +66,7 @@ _SIGS = {
     "mfb_mesh_collocation": (I, [P, P, P, P, P]),
     "mfb_mesh_node_normals": (I, [P, P]),
     "mfb_mesh_timings": (I, [P, P, P]),
+    "mfb_mesh_time_groups": (I, [P, I]),
     "mfb_assemble_staela": (I, [P, D, D, P, LL, P, P]),
     "mfb_assemble_harela": (I, [P, D, D, D, D, D, D, D, P, LL, P, P]),
     "mfb_assemble_batch": (I, [I, C.POINTER(AssemblyJob), P]),

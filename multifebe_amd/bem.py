@@ -98,12 +98,19 @@ class BemSystem:
         return st.as_dict()
 
     def timings(self) -> dict:
-        """HIP-event durations (ms) of the kernel groups of the last assembly."""
+        """HIP-event durations (ms) of the kernel groups of the last assembly.  Adaptive pairs, singular
+        pairs and free terms share a launch, whose time is adaptive_ms (singular_ms 0), unless
+        time_groups() asked for one launch each."""
         ms = np.zeros(4)
         nl = C.c_int()
         check(lib().mfb_mesh_timings(self._h, _ptr(ms), C.byref(nl)), "mfb_mesh_timings")
         return {"regular_ms": ms[0], "adaptive_ms": ms[1], "singular_ms": ms[2],
                 "freeterm_zero_ms": ms[3], "regular_launches": nl.value}
+
+    def time_groups(self, on: bool = True):
+        """mfb_mesh_time_groups: launch (and time) the groups of timings() one by one in the following
+        assemblies; same results, slower."""
+        check(lib().mfb_mesh_time_groups(self._h, int(bool(on))), "mfb_mesh_time_groups")
 
     def collocation(self):
         """Collocation points: (xc (ncp, 3), crow (node of each point's equations), cel (element

@@ -2184,7 +2184,8 @@ struct mfb_mesh_s {
   long long regular_points = 0;
   // HIP events around the kernel groups of the last assembly (on the caller's stream)
   hipEvent_t ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  double last_ms[4] = {0, 0, 0, 0};  // regular, adaptive, singular, free term + zeroing
+  double last_ms[4] = {0, 0, 0, 0};  // as mfb_mesh_timings gives them
+  bool time_groups = false;          // near pairs and free terms launched group by group
   int last_regular_launches = 0;
 };
 
@@ -2232,7 +2233,7 @@ static int mesh_ws(mfb_mesh_s* m, int slot, size_t bytes, P** out) {
 template <bool H>
 static void launch_near(const DevMesh& d, const QsiParams* qsp, const KernelParams* kpp,
                         NearArgs<typename Val<H>::T> a, int n_tree, hipStream_t s) {
-  const int most = n_tree < 0 ? a.na : n_tree;
+  const int most = n_tree < 0 ? a.na : std::min(n_tree, a.na);
   a.tree_wgs = std::min((most + kNearWaves - 1) / kNearWaves, 512);
   const long long wgs = (long long)a.tree_wgs + a.ns + (a.na + kNearWaves - 1) / kNearWaves +
                         (a.nfree + 255) / 256 + (a.nfree_mca + 255) / 256;
@@ -2895,12 +2896,20 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
   a.counters = m->counters;
   a.sing_points = m->sing_points;
   a.err = m->err;
-  launch_near<H>(d, m->d_qsp, kpp, a, learned ? -1 : m->n_tree, s);
-  if (events) {
-    MFB_HIP(hipEventRecord(m->ev[3], s));
-    MFB_HIP(hipEventRecord(m->ev[4], s));
+  const int n_tree = learned ? -1 : m->n_tree;
+  if (!events || !m->time_groups) {
+    launch_near<H>(d, m->d_qsp, kpp, a, n_tree, s);
+    if (events) MFB_HIP(hipEventRecord(m->ev[3], s));
+  } else {   // the same workgroups, group by group
+    for (int k = 0; k < 3; k++) {
+      NearArgs<T> g = a;
+      if (k != 0) g.na = 0;
+      if (k != 1) g.ns = 0, g.sing_points = 0;
+      if (k != 2) g.nfree = g.nfree_mca = 0;
+      launch_near<H>(d, m->d_qsp, kpp, g, n_tree, s);
+      MFB_HIP(hipEventRecord(m->ev[3 + k], s));
+    }
   }
-  if (events) MFB_HIP(hipEventRecord(m->ev[5], s));
   MFB_HIP(hipGetLastError());
   return MFB_OK;
 }
@@ -2992,16 +3001,15 @@ static int assemble(mfb_mesh_t m, const KernelParams& kp, double nu, double* Ara
     a.vec = vec;
     launch_near<H>(d, m->d_qsp, m->d_kp, a, m->n_tree, s);
     MFB_HIP(hipEventRecord(m->ev[3], s));
-    MFB_HIP(hipEventRecord(m->ev[4], s));
-    MFB_HIP(hipEventRecord(m->ev[5], s));
   }
   MFB_HIP(hipGetLastError());
   int herr = 0;
   MFB_HIP(hipMemcpyAsync(&herr, m->err, sizeof(int), hipMemcpyDeviceToHost, s));
   MFB_HIP(hipStreamSynchronize(s));
   {
-    float t[5];
-    for (int q = 0; q < 5; q++) MFB_HIP(hipEventElapsedTime(&t[q], m->ev[q], m->ev[q + 1]));
+    float t[5] = {};
+    const int groups = m->time_groups && !blocks && !vmode ? 5 : 3;
+    for (int q = 0; q < groups; q++) MFB_HIP(hipEventElapsedTime(&t[q], m->ev[q], m->ev[q + 1]));
     m->last_ms[0] = t[1];
     m->last_ms[1] = t[2];
     m->last_ms[2] = t[3];
@@ -3036,6 +3044,12 @@ extern "C" int mfb_mesh_timings(mfb_mesh_t m, double* ms, int* regular_launches)
   MFB_ARG(m && ms, "null argument");
   for (int q = 0; q < 4; q++) ms[q] = m->last_ms[q];
   if (regular_launches) *regular_launches = m->last_regular_launches;
+  return MFB_OK;
+}
+
+extern "C" int mfb_mesh_time_groups(mfb_mesh_t m, int on) {
+  MFB_ARG(m, "null argument");
+  m->time_groups = on != 0;
   return MFB_OK;
 }
 
