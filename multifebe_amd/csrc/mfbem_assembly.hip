@@ -2852,8 +2852,16 @@ static int enqueue_scatter(mfb_mesh_t m, const KernelParams* kpp, bool learned, 
   const TileOut<T> out{A, lda, b, (T*)extra};
   if (m->prezero) {
     const long long tot = (long long)n * n, nx = 3LL * d.nx * n;
-    const long long nblk = std::min<long long>((tot + 255) / 256, 1 << 14);   // 5.6 TB/s; 1 << 16: 5.1
-    hipLaunchKernelGGL(k_zero<T>, dim3((unsigned)nblk), dim3(256), 0, s, A, lda, n);
+    // the runtime's fill (6.1 TB/s at 30k) on a stream that is not being captured, a kernel under
+    // capture (memset nodes are kept out of graphs) and between padded columns
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    MFB_HIP(hipStreamIsCapturing(s, &cap));
+    if (cap == hipStreamCaptureStatusNone && lda == n) {
+      MFB_HIP(hipMemsetAsync(A, 0, sizeof(T) * (size_t)tot, s));
+    } else {
+      const long long nblk = std::min<long long>((tot + 255) / 256, 1 << 14);   // 5.6 TB/s; 1 << 16: 5.1
+      hipLaunchKernelGGL(k_zero<T>, dim3((unsigned)nblk), dim3(256), 0, s, A, lda, n);
+    }
     if (nx) hipLaunchKernelGGL(k_fill_zero<T>, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, s, out.X, nx);
   }
   {
