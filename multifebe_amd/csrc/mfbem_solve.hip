@@ -148,6 +148,18 @@ __device__ inline void wave_cand_max(double& v, int& i) {
   }
 }
 
+// Products with their roundings written out: which of the two products of an imaginary part is
+// rounded first would else be the compiler's choice in each kernel, and the factors of a block
+// would depend in the last bit on the kernel that takes it.
+__device__ inline double pmul(double a, double b) { return a * b; }
+__device__ inline float pmul(float a, float b) { return a * b; }
+__device__ inline cz pmul(cz a, cz b) {
+  return cz{__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im)};
+}
+__device__ inline cf pmul(cf a, cf b) {
+  return cf{__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.im, b.re, a.re * b.im)};
+}
+
 // One step of the narrow-block factorisation.  B: narrow block (m x w, ld), rows relative to its
 // top-left corner; one thread per row.  Step j >= 0: scale column j below the pivot and update
 // columns j+1..w-1 (pivot row staged in LDS, the thread's row held in registers).  Then
@@ -184,11 +196,11 @@ __global__ void __launch_bounds__(ROWS) k_col_step(T* B, long long ld, int m, in
       T l = tzero<T>();
 #pragma unroll
       for (int c = 0; c < IB; c++)
-        if (c == j) l = tmul(x[c], inv);
+        if (c == j) l = pmul(x[c], inv);
 #pragma unroll
       for (int c = 0; c < IB; c++) {
         if (c == j) x[c] = l;
-        else if (c > j && c < w) x[c] = tsub(x[c], tmul(l, prow[c]));
+        else if (c > j && c < w) x[c] = tsub(x[c], pmul(l, prow[c]));
       }
 #pragma unroll
       for (int c = 0; c < IB; c++)
@@ -411,18 +423,6 @@ struct PanelCtx {
   int* wi;    // LDS [ROWS / 64]
   T* stage;   // LDS [IB]: candidate row (posted one word per lane)
 };
-
-// Products with their roundings written out: which of the two products of an imaginary part is
-// rounded first would else be the compiler's choice in each kernel, and the factors of a block
-// would depend in the last bit on the kernel that takes it.
-__device__ inline double pmul(double a, double b) { return a * b; }
-__device__ inline float pmul(float a, float b) { return a * b; }
-__device__ inline cz pmul(cz a, cz b) {
-  return cz{__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im)};
-}
-__device__ inline cf pmul(cf a, cf b) {
-  return cf{__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.im, b.re, a.re * b.im)};
-}
 
 // Column J of the persistent panel (J a compile-time constant, so every register index of the
 // thread's row x is one too).  The pivot row is fetched when the pivot is known: reading the rows of
