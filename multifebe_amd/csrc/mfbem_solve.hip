@@ -294,6 +294,11 @@ __global__ void __launch_bounds__(ROWS) k_col_step(T* B, long long ld, int m, in
 constexpr int PANEL_GMAX = 256;   // workgroups of the persistent panel (rows <= 65,536)
 static_assert(PANEL_GMAX <= 256, "a record holds position << 8 | workgroup");
 
+// launches that have stamps of their own (31 bits of epoch x 32 + column); the buffers are cleared
+// before the next one
+constexpr unsigned PANEL_EPOCHS = 1u << 26;
+constexpr int CROW_MAX = 4 * (IB + 1);   // words of a posted row and its reciprocal, complex double
+
 // Every workgroup's record sits on its own 256-byte line: posts and polls of different
 // workgroups never touch the same line.
 constexpr int REC = 32;   // record stride in 8-byte words: |a|_1 (1 or 2 words), position and
@@ -1636,7 +1641,7 @@ struct Ctx {
   int ps_cap = 0;
   int device = -1;
   PanelSync pan{};          // persistent-panel posting buffers
-  unsigned pan_epoch = 0;   // launch counter of the persistent panel (tags of its posts)
+  unsigned pan_epoch = 0;   // launches of the persistent panel since its buffers were cleared
   SolveSync sol{};          // published-block tags of the persistent triangular solves
   unsigned sol_epoch = 0;
   int trsv_grid = 0;        // largest co-resident grid of k_trsv_blocked (all instantiations)
@@ -1742,8 +1747,7 @@ static int ensure_ctx(hipStream_t s, int n) {
     const size_t rb = sizeof(unsigned long long) * 2 * PANEL_GMAX * REC;
     MFB_HIP(hipMalloc(&c.pan.rec, rb));
     MFB_HIP(hipMalloc(&c.pan.err, sizeof(unsigned)));
-    // rows of complex128, four words per entry
-    const size_t rowb = sizeof(unsigned long long) * 4 * (IB + 1);
+    const size_t rowb = sizeof(unsigned long long) * CROW_MAX;
     MFB_HIP(hipMalloc(&c.pan.crow, rowb * 2 * PANEL_GMAX));
     MFB_HIP(hipMemset(c.pan.crow, 0, rowb * 2 * PANEL_GMAX));
     MFB_HIP(hipMemset(c.pan.rec, 0, rb));
@@ -2037,9 +2041,14 @@ static int getrf(LU<T>& f, T* A, long long lda, int n, hipStream_t s) {
           int mm_ = mm, w_ = w, g0_ = k1 + jj;
           int* info_ = c.ps.info;
           PanelSync pan = c.pan;
-          // epochs start at 1 (tags are zero-initialised); 2^32 launches before a repeat
-          unsigned ep = ++c.pan_epoch;
-          if (ep == 0) ep = ++c.pan_epoch;
+          if (c.pan_epoch == PANEL_EPOCHS) {   // the stamps begin again: no old word may match one
+            hipLaunchKernelGGL(k_zero_mat<double>, dim3(256), dim3(256), 0, s, (double*)pan.rec,
+                               (long long)REC, REC, 2 * PANEL_GMAX);
+            hipLaunchKernelGGL(k_zero_mat<double>, dim3(256), dim3(256), 0, s, (double*)pan.crow,
+                               (long long)CROW_MAX, CROW_MAX, 2 * PANEL_GMAX);
+            c.pan_epoch = 0;
+          }
+          const unsigned ep = ++c.pan_epoch;
           hipLaunchKernelGGL(k_panel<T>, dim3(grid), dim3(ROWS), 0, s, Bk, ld_, mm_, w_, piv, pan,
                              info_, g0_, ep);
         } else {
