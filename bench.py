@@ -40,9 +40,12 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP64 = 78.6e12          # MI355X FP64 vector (AMD public spec)
-# flops per quadrature point of the direct formulation (complex exponentials, nine components of t* and
-# of u*, 9 weights each); the kernel sums the symmetric u* as six and executes about 950
-FLOPS_PER_POINT_HARM = 1500
+# flops that k_regular_tile<harmonic> executes per quadrature point (FP64 vector flops x 64 lanes + matrix
+# MOPS x 512 by rocprofv3, three frequencies over the band): most of the soil surface needs t* alone
+FLOPS_PER_POINT = {"sphere": 1155, "soil": 984}
+# the direct formulation's (complex exponentials, nine components of t* and of u*, 9 weights each): an
+# equivalent rate, not work that is done
+FLOPS_PER_POINT_DIRECT = 1500
 QNET_DEFAULT = os.path.join(ROOT, "multifebe_amd", "data", "qnet_tau1e-10.npz")
 # HBM bytes per launch of k_regular_tile<harmonic> (mean over one assembly's launches), from
 # rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE scaled by a 1 GiB copy; None where not measured
@@ -208,7 +211,8 @@ def main():
         learned.time_groups(False)
         tm1, st1 = learned.timings(), learned.stats()
         del At1, b1
-        alone_ach = st1["regular_points"] * FLOPS_PER_POINT_HARM / (tm1["regular_ms"] * 1e-3)
+        alone_ach = (st1["regular_points"] * FLOPS_PER_POINT[args.workload]
+                     / (tm1["regular_ms"] * 1e-3))
         alone = {"launches": tm1["regular_launches"],
                  "avg_launch_ms": tm1["regular_ms"] / max(tm1["regular_launches"], 1),
                  "achieved": alone_ach / 1e12, "frac": alone_ach / PEAK_FP64, "kernel_ms": tm1,
@@ -241,19 +245,21 @@ def main():
 
     t_asm = sum(r[1] for r in recs)
     t_sol = sum(r[2] for r in recs)
-    # dominant assembly kernel: precalculated-rule pairs, FP64-VALU bound; algorithmic work =
-    # quadrature points of those pairs x flops per point of the harmonic kernel.  Its duration is
+    # dominant assembly kernel: precalculated-rule pairs, bound by its FP64 instructions; work =
+    # quadrature points of those pairs x flops the kernel executes per point.  Its duration is
     # the HIP-event time of its launches (recorded on the assembly's stream), summed over every
     # assembly of the timed sweep.
-    achieved = reg_points * FLOPS_PER_POINT_HARM / (reg_ms * 1e-3)
+    achieved = reg_points * FLOPS_PER_POINT[args.workload] / (reg_ms * 1e-3)
     roofline = {"kernel": "k_regular_tile<true> (harmonic, precalculated-rule pairs, scatter into A)",
                 "bound": "mfma",
-                "compute_pipe": "FP64 VALU (MI355X FP64 vector peak = FP64 matrix peak = 78.6 TFLOP/s)",
+                "compute_pipe": "FP64 vector and matrix units, one pipe (both peaks 78.6 TFLOP/s)",
                 "achieved": achieved / 1e12, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
                 "frac": achieved / PEAK_FP64, "traffic": TRAFFIC_PER_LAUNCH[args.workload],
                 "traffic_unit": "bytes per launch (mean)",
                 "launches": launches, "avg_launch_ms": reg_ms / max(launches, 1),
-                "regular_points": reg_points, "flops_per_point": FLOPS_PER_POINT_HARM,
+                "regular_points": reg_points, "flops_per_point": FLOPS_PER_POINT[args.workload],
+                "direct_formulation_equivalent": reg_points * FLOPS_PER_POINT_DIRECT
+                                                 / (reg_ms * 1e-3) / 1e12,
                 "timed": "every assembly of the timed sweep, each beside the LU of the previous "
                          "frequency",
                 "alone": alone}
