@@ -83,6 +83,9 @@ const char *mfb_last_error(void);
  * element shares) takes SBIE-MCA -- one collocation point in every element holding it, at
  * xi_node (1 - 0.05), all adding to the node's equations, free term (1/2) phi(xi) -- so truncated
  * open surfaces (a half-space free surface) are assembled as the reference assembles them.
+ * Such a node's points after its first have rows of their own while the matrix is assembled, in a device
+ * buffer of 9 nx nn entries for nx of them (288 MB for the 10,201 nodes and 196 points of a 50 x 50
+ * surface, complex), kept by the mesh, or one for all jobs of a batch.
  * Precomputed:
  * element characteristic lengths, gln_far and bounding balls (src/build_data_of_be_elements.f90:70-112),
  * precalculated Gauss-Legendre datasets (lib/fbem/src/bem_general.f90:163-759), node normals, and

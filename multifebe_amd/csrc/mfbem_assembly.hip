@@ -1587,15 +1587,18 @@ struct Leaf {
   int gln, pad;
 };
 constexpr int kLeaves = 32, kWalkWidth = 8;
-// The walk takes the kWalkWidth deepest sub-elements at a time, so at most 3 kWalkWidth wait per level
-// and 4 kWalkWidth on the last.
+// The walk takes the kWalkWidth topmost sub-elements of its stack at a time and puts the parts of those
+// that it splits, at most 4 kWalkWidth, in their place.  Of the parts that one step has put there, at most
+// 3 kWalkWidth are left below those of a later step, and the shallowest level that a step puts there is
+// deeper than what the step below put: there are fewer than kMaxNs steps' parts.  (Simulated with random
+// splits to level 20: 408 entries at most; with everything split to level 9: 160.)
 constexpr int kWalkStack = 3 * kWalkWidth * kMaxNs + 4 * kWalkWidth;
 struct WalkLds {
   unsigned long long stk[kWalkStack];   // level << 48 | ix << 24 | iy of the 2^(level-1) grid
   Leaf leaf[kLeaves];
 };
 
-// One step of the walk: the deepest sub-elements of the stack (a team of four lanes each) become
+// One step of the walk: the topmost sub-elements of the stack (a team of four lanes each) become
 // leaves or are replaced by their four parts.  sp, nl: entries on the stack, leaves.
 __device__ __attribute__((noinline)) void walk_step(const QsiParams& qsp, const double* X,
                                                     const double* x_i, int ns_max, int gln_far,
@@ -2177,9 +2180,9 @@ struct mfb_mesh_s {
   double h_tol = 1e-6;
   int* err = nullptr;
   long long* counters = nullptr;  // points, leaves of the adaptive and singular pairs
-  mfb::QsiParams* d_qsp = nullptr;     // estimator tables and kernel constants live in device memory:
-  mfb::QsiParams* d_qsp_li = nullptr;  // they are too large to travel as kernel arguments
-  mfb::KernelParams* d_kp = nullptr;
+  mfb::QsiParams* d_qsp = nullptr;     // estimator tables: too large to travel as kernel arguments
+  mfb::QsiParams* d_qsp_li = nullptr;
+  mfb::KernelParams* d_kp = nullptr;   // kernel constants, read as scalars through the constant cache
   long long decisions = 0;
   long long regular_points = 0;
   // HIP events around the kernel groups of the last assembly (on the caller's stream)
@@ -2425,7 +2428,9 @@ static void default_collocation(int nn, int ne, const double* x, const int* conn
 // takes more than the four of a structured surface (closed ones: six) once more by saturation
 // degree (Brelaz), which is kept if it needs fewer: every colour is a launch, and on a small mesh a
 // launch takes its latency (15 us on a cube of 24 elements, 44 on a sphere of 96 elements, each of two
-// launches fewer; the assemblies take 167 and 349 us).
+// launches fewer; the assemblies take 160 and 333 us).  Not beyond 4,096 elements, 49,000 unknowns: two
+// launches' latency is a thousandth of an assembly there (20 ms for 2,500 elements), the second search
+// takes 0.7 ms on the host at 4,056 elements, 2.1 at 9,600 and 3.1 at 21,600.
 constexpr int kMaxColors = 64;
 static int color_elements(int ne, const int* conn, const std::vector<int>& ip,
                           const std::vector<int>& ie, std::vector<int>& col) {
