@@ -885,9 +885,9 @@ __device__ inline void tile_body(const DevMesh& m, const KernelParams& kp,
 // registers of two waves per SIMD (61 spilled).
 // Bound by its FP64 instructions: the 4x4x4 matrix instruction and the vector FMA share one pipe, and
 // the sums over the element's nodes are contractions that the former does with a third of the issue
-// slots and no LDS traffic for the values.  An open harmonic surface of 26 x 26 elements: 410
+// slots and no LDS traffic for the values.  An open harmonic surface of 26 x 26 elements: 392
 // us a launch, 1340 with kernel values staged in LDS by workgroups of 256 and A cleared first; one of
-// 50 x 50: 5.1 ms a launch and 13.6 GB, 16.3 ms and 25.8 GB before; a static box of 454 elements 88
+// 50 x 50: 5.0 ms a launch and 13.6 GB, 16.3 ms and 25.8 GB before; a static box of 454 elements 85
 // and 157 us.
 // One launch over all colours with atomic additions needs no colours, but the chip does 27e9 of them a
 // second: 11.8 ms against 4 x 0.695 (26 x 26, this kernel before it stored).
@@ -1014,7 +1014,7 @@ __device__ inline void point_values(ConstKP k, const double* rv, const double* n
 // One wave per 16 points and `chunk` elements, the sums in registers over the elements.  Four lanes
 // share the quadrature points of a pair's own rule, the wave takes as many as the longest of its 16:
 // order, the points along a space-filling curve, keeps that close to what each needs, and lanes of one
-// rule load one address.  10,000 harmonic points, 216 elements: 0.83 ms; a lane per pair, 64 pairs a
+// rule load one address.  10,000 harmonic points, 216 elements: 0.76 ms; a lane per pair, 64 pairs a
 // wave, 1.2 ms; 64 pairs a wave by one rule after the other, its records as scalars, 2.9 ms.
 template <bool H>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(3)))
@@ -1965,8 +1965,8 @@ __device__ inline void free_term_mca(const DevMesh& m, int cp, T* A, long long l
 // each, in turn), singular pairs (a workgroup each), the other adaptive pairs (a wave each), free
 // terms (a thread each).  The parts are independent (atomic additions), each is a chain of a few
 // dependent loads and reductions and none fills the chip on a small mesh: one after the other they
-// took 150 of 480 us of a 1,158-DOF assembly (29 us against 61 on a cube of 24 elements,
-// 80 against 125 on a sphere of 96, 689 against 930 on an open surface of 26 x 26).  The longest come
+// took 150 of 480 us of a 1,158-DOF assembly (27 us against 61 on a cube of 24 elements,
+// 80 against 125 on a sphere of 96, 660 against 930 on an open surface of 26 x 26).  The longest come
 // first.
 // ------------------------------------------------------------------------------------------------
 template <typename T>
@@ -2428,7 +2428,7 @@ static void default_collocation(int nn, int ne, const double* x, const int* conn
 // takes more than the four of a structured surface (closed ones: six) once more by saturation
 // degree (Brelaz), which is kept if it needs fewer: every colour is a launch, and on a small mesh a
 // launch takes its latency (15 us on a cube of 24 elements, 44 on a sphere of 96 elements, each of two
-// launches fewer; the assemblies take 160 and 333 us).  Not beyond 4,096 elements, 49,000 unknowns: two
+// launches fewer; the assemblies take 155 and 320 us).  Not beyond 4,096 elements, 49,000 unknowns: two
 // launches' latency is a thousandth of an assembly there (20 ms for 2,500 elements), the second search
 // takes 0.7 ms on the host at 4,056 elements, 2.1 at 9,600 and 3.1 at 21,600.
 constexpr int kMaxColors = 64;

@@ -897,9 +897,9 @@ __host__ __device__ inline void exp_sums(zd z, zd g5, zd& e, zd& P, zd& R) {
 //   r^2 TT1 = lead2 + 3 A - 2 (V2 - q V1),  r^2 TT2 = lead3 + V2 + q Q1,  V = z^2 R,
 //   r^2 TT3 = lead4 + V1 + Q1 - 2 q V1 - q Q1 - Q2.
 // Largest error of TT1..TT3 (of the largest of them; nu 0.05..0.49, damping to 0.1) for |z| to 1, 2, 3
-// and 120: 5.3e-16, 1.2e-15, 2.9e-15, 4.3e-14.  The reference's E_n terms: 6.5e-16, 3.9e-15, 5.2e-15,
-// 1.4e-9; series of H = (1 - (1-z) e^z)/z^2 and e^z - 1 below |z| = 1, linear terms and all: 2.4e-15,
-// 9.4e-15, 2.8e-15, 4.3e-14, in about the same time (tiles of an open surface of 26 x 26 elements 1657
+// and 120: 4.4e-16, 1.3e-15, 3.5e-15, 3.1e-14.  The reference's E_n terms: 6.5e-16, 3.9e-15, 5.2e-15,
+// 1.1e-9; series of H = (1 - (1-z) e^z)/z^2 and e^z - 1 below |z| = 1, linear terms and all: 2.4e-15,
+// 9.4e-15, 2.8e-15, 3.1e-14, in about the same time (tiles of an open surface of 26 x 26 elements 1657
 // us, 1612 now; of a sphere of 96 185 and 155, of a cylinder of 384 545 and 548; 10,000 points 1.17 and
 // 1.16 ms).
 // Five complex constants, which stay in scalar registers: the same with kappa^2, q kappa, 6/kappa as
